@@ -26,62 +26,9 @@
 // allocations as the token rows, pool_base rows behind their start: pooled row b of a sequence is
 // row pool_base + table[b / pool_rows] * pool_rows + b % pool_rows.  In the order the kernels walk
 // a query's keys the pooled rows come first, then the window's tokens.
-#include "hybrid_merge.h"
+#include "hybrid_keys.h"
 
 using namespace hyb;
-
-struct KeyRule {
-    int window;             // 0: every earlier key is visible
-    int keep_first;
-    const float* slopes;    // [H] or null
-    int v_stride;           // elements from one (slot, KV head) value row to the next: E for a dense
-                            // V cache, more when the value rows are the leading part of wider rows
-                            // (values stored inside the key rows: v_cache then points into k_cache)
-    const float* temps;     // [H] or null: multiplies the scaled score of head h
-    float softcap;          // 0: none
-    int pool;               // 0: no pooled blocks (needs window > 0 and keep_first == 0)
-    int pool_rows;          // pooled rows per page
-    long pool_base;         // first pooled row, in rows from the start of the K (and of the V) cache
-    int chunk;              // 0: none (else keep_first == 0 and pool == 0)
-    // the first key a query at position i sees besides kept first tokens and pooled rows; it never
-    // falls as i grows
-    __device__ __forceinline__ int first_key(int i) const {
-        int lo = window > 0 ? max(0, i - window + 1) : 0;
-        if (chunk > 0) lo = max(lo, i / chunk * chunk);
-        return lo;
-    }
-    __device__ __forceinline__ float capped(float s) const {
-        return softcap > 0.f ? softcap * tanhf(s / softcap) : s;
-    }
-    __device__ __forceinline__ float head_scale(float scale, int h) const {
-        return temps ? scale * temps[h] : scale;
-    }
-    // pooled blocks a query that sees ctx keys without a window takes in
-    __device__ __forceinline__ int pooled_for(int ctx) const {
-        return (pool > 0 && ctx > window) ? (ctx - window) / pool : 0;
-    }
-    __device__ __forceinline__ long pooled_row(const int* table, int b) const {
-        return pool_base + (long)table[b / pool_rows] * pool_rows + b % pool_rows;
-    }
-};
-
-// The visible keys of a query that sees `ctx` keys without a window (its position is ctx - 1), as
-// one run of virtual indices: [0, kept) are keys 0 .. kept-1, the rest the window's keys from `lo`.
-struct VisibleKeys {
-    int kept, lo, count;
-    __device__ __forceinline__ VisibleKeys(int ctx, const KeyRule& r) {
-        lo = r.first_key(ctx - 1);
-        kept = r.pool > 0 ? r.pooled_for(ctx) : min(r.keep_first, lo);
-        count = kept + ctx - lo;
-    }
-    __device__ __forceinline__ int key(int v) const { return v < kept ? v : lo + (v - kept); }
-    // cache row of virtual key v (with pooled blocks the leading `kept` indices are pooled rows)
-    __device__ __forceinline__ long row(int v, const int* table, int block_size, const KeyRule& r) const {
-        if (r.pool > 0 && v < kept) return r.pooled_row(table, v);
-        const int j = key(v);
-        return (long)table[j / block_size] * block_size + j % block_size;
-    }
-};
 
 constexpr int TILE = 256;
 constexpr int RC = 4;       // query heads per workgroup
@@ -233,7 +180,8 @@ sink_attention_rows_kernel(const T* __restrict__ q, long q_row, long q_head,
 }
 
 // ---------------------------------------------------------------------------------------
-// Prompt portions: tiles on the matrix cores, everything in fp32.
+// Prompt portions: tiles on the matrix cores, everything in fp32 (bfloat16 caches with rows of whole
+// 16-byte runs have a kernel of their own, hybrid_prompts.hip).
 //
 // Workgroup = 4 waves = 128 consecutive queries of one (sequence, query head); a wave owns 32 of
 // them.  Keys are walked in tiles of 32 through LDS (K tile [32][DP+1], V tile [32][EP], both
@@ -248,13 +196,9 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
-// QK16 (bfloat16 caches only): the score products run as v_mfma_f32_32x32x16_bf16 on the raw
-// 16-bit K tile and q rows - the operands ARE bfloat16 values, so the products are exact and the
-// fp32 accumulation only differs in order from the fp32 instruction; the score scale is applied
-// to the fp32 result.  Weights and weighted sums stay on the fp32 instruction.
 // EXT: the instance that knows head temperatures, the soft cap and pooled rows; without it the
 // kernel is compiled free of them (their state costs registers the plain form has no room for).
-template <typename T, int DP, int EP, bool QK16, bool EXT>
+template <typename T, int DP, int EP, bool EXT>
 __global__ void __launch_bounds__(256)
 sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
                             const T* __restrict__ k_cache, const T* __restrict__ v_cache,
@@ -264,10 +208,8 @@ sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
                             long gate_row, T* __restrict__ out, float scale, int H, int G, int D,
                             int E, int seq0, int vec_k, int vec_v, KeyRule rule) {
     extern __shared__ float sm[];
-    constexpr int KS = QK16 ? (DP + 8) / 2 : DP + 1;      // floats per K row of the LDS image
-    constexpr int KSB = DP + 8;                             // (QK16) 16-bit elements per K row
+    constexpr int KS = DP + 1;                              // floats per K row of the LDS image
     float* Ks = sm;
-    uint16_t* Kb = reinterpret_cast<uint16_t*>(sm);
     float* Vs = sm + 32 * KS;
     const int b = blockIdx.x + seq0, tile = blockIdx.y, h = blockIdx.z;
     const int row0 = cu_q[b], qlen = cu_q[b + 1] - row0;
@@ -281,32 +223,17 @@ sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
     const int qpos = start + qi;
 
     const float hscale = EXT ? rule.head_scale(scale, h) : scale;
-    float qreg[QK16 ? 1 : DP / 2];
-    bf16x8 qv[QK16 ? DP / 16 : 1];
+    float qreg[DP / 2];
     {
         const T* qp = q + (long)(row0 + (qok ? qi : 0)) * q_row + (long)h * q_head;
-        if constexpr (QK16) {
 #pragma unroll
-            for (int s = 0; s < DP / 16; ++s) {
-                const int d = 16 * s + 8 * half;
-                uint4 raw = make_uint4(0, 0, 0, 0);
-                if (qok && d < D) raw = *reinterpret_cast<const uint4*>(qp + d);
-                qv[s] = __builtin_bit_cast(bf16x8, raw);
-            }
-            for (int i = tid; i < 32 * (KSB - D); i += 256) {   // padding columns of K stay zero
-                const int key = i / (KSB - D), c = D + i - key * (KSB - D);
-                Kb[key * KSB + c] = 0;
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < DP / 2; ++s) {
-                const int d = 2 * s + half;
-                qreg[s] = (qok && d < D) ? ld(qp + d) * hscale : 0.f;
-            }
-            for (int i = tid; i < 32 * (KS - D); i += 256) {      // padding columns of K stay zero
-                const int key = i / (KS - D), c = D + i - key * (KS - D);
-                Ks[key * KS + c] = 0.f;
-            }
+        for (int s = 0; s < DP / 2; ++s) {
+            const int d = 2 * s + half;
+            qreg[s] = (qok && d < D) ? ld(qp + d) * hscale : 0.f;
+        }
+        for (int i = tid; i < 32 * (KS - D); i += 256) {          // padding columns of K stay zero
+            const int key = i / (KS - D), c = D + i - key * (KS - D);
+            Ks[key * KS + c] = 0.f;
         }
     }
     float m = sink ? sink[h] : NO_SINK_MAX, lsum = sink ? 1.f : 0.f;
@@ -338,18 +265,7 @@ sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
                           : (long)table[j / block_size] * block_size + j % block_size;
         };
         // ---- K and V tile into LDS
-        if constexpr (QK16) {
-            const int D8 = D >> 3;
-            for (int i = tid; i < 32 * D8; i += 256) {
-                const int key = i / D8, c = (i - key * D8) << 3, j = k0 + key;
-                uint4 raw = make_uint4(0, 0, 0, 0);
-                if (j < k_lim) {
-                    const long slot = cache_row(j);
-                    raw = *reinterpret_cast<const uint4*>(k_cache + (slot * G + g) * (long)D + c);
-                }
-                *reinterpret_cast<uint4*>(Kb + key * KSB + c) = raw;
-            }
-        } else if (vec_k) {
+        if (vec_k) {
             const int D4 = D >> 2;
             for (int i = tid; i < 32 * D4; i += 256) {
                 const int key = i / D4, c = (i - key * D4) << 2, j = k0 + key;
@@ -401,21 +317,10 @@ sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
             f32x16 sacc;
 #pragma unroll
             for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
-            if constexpr (QK16) {
-                const uint16_t* ka = Kb + l32 * KSB + 8 * half;
+            const float* ka = Ks + l32 * KS + half;
 #pragma unroll
-                for (int s = 0; s < DP / 16; ++s) {
-                    const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(ka + 16 * s));
-                    sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qv[s], sacc, 0, 0, 0);
-                }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) sacc[r] *= hscale;
-            } else {
-                const float* ka = Ks + l32 * KS + half;
-#pragma unroll
-                for (int s = 0; s < DP / 2; ++s)
-                    sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[2 * s], qreg[s], sacc, 0, 0, 0);
-            }
+            for (int s = 0; s < DP / 2; ++s)
+                sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[2 * s], qreg[s], sacc, 0, 0, 0);
             float mt = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -471,31 +376,20 @@ static int launch_tiles(const void* q, long q_row, long q_head, const void* k_ca
                         const void* v_cache, const void* block_tables, int max_blocks,
                         int block_size, const void* cu_q, const void* positions, const void* sink,
                         const void* gate, long gate_row, void* out, float scale, int nseq,
-                        int seq0, int max_q, int H, int G, int D, int E, int esize,
+                        int seq0, int max_q, int H, int G, int D, int E,
                         KeyRule rule, hipStream_t s) {
     const int vec_k = (D % 4 == 0) && ((size_t)k_cache % 16 == 0);
     const int vec_v = (E % 4 == 0) && (rule.v_stride % 4 == 0) && ((size_t)v_cache % 16 == 0);
     const dim3 grid(nseq, (max_q + 127) / 128, H);
-#define TILES_LAUNCH_X(QK16, EXT, lds)                                                            \
-    hipLaunchKernelGGL((sink_attention_tiles_kernel<T, DP, EP, QK16, EXT>), grid, dim3(256), lds, s, \
+#define TILES_LAUNCH(EXT)                                                                         \
+    hipLaunchKernelGGL((sink_attention_tiles_kernel<T, DP, EP, EXT>), grid, dim3(256),            \
+                       (32 * (DP + 1) + 32 * EP) * sizeof(float), s,                              \
                        (const T*)q, q_row, q_head, (const T*)k_cache, (const T*)v_cache,          \
                        (const int*)block_tables, max_blocks, block_size, (const int*)cu_q,        \
                        (const int*)positions, (const float*)sink, (const T*)gate, gate_row,       \
                        (T*)out, scale, H, G, D, E, seq0, vec_k, vec_v, rule)
-#define TILES_LAUNCH(QK16, lds)                                                                   \
-    do { if (ext) TILES_LAUNCH_X(QK16, true, lds); else TILES_LAUNCH_X(QK16, false, lds); } while (0)
-    const bool ext = rule.temps || rule.softcap > 0.f || rule.pool > 0;
-    if constexpr (sizeof(T) == 2) {
-        // 16-bit caches: score products on the bf16 instruction when rows are 16-byte addressable
-        if (D % 16 == 0 && (size_t)k_cache % 16 == 0 && (size_t)q % 16 == 0 && q_row % 8 == 0 &&
-            q_head % 8 == 0) {
-            TILES_LAUNCH(true, (32 * ((DP + 8) / 2) + 32 * EP) * sizeof(float));
-            return HYB_LAUNCH_OK();
-        }
-    }
-    TILES_LAUNCH(false, (32 * (DP + 1) + 32 * EP) * sizeof(float));
+    if (rule.temps || rule.softcap > 0.f || rule.pool > 0) TILES_LAUNCH(true); else TILES_LAUNCH(false);
 #undef TILES_LAUNCH
-#undef TILES_LAUNCH_X
     return HYB_LAUNCH_OK();
 }
 
@@ -641,16 +535,6 @@ static int launch_split(const void* q, long q_row, long q_head, const void* k_ca
     return HYB_LAUNCH_OK();
 }
 
-static bool chunk_rule_ok(const KeyRule& r) {
-    return r.chunk == 0 || (r.chunk > 0 && r.keep_first == 0 && r.pool == 0);
-}
-
-// pooled blocks need a window, no kept first tokens, no distance penalty, and a place in the caches
-static bool pool_rule_ok(const KeyRule& r) {
-    return r.pool == 0 || (r.pool > 0 && r.window > 0 && r.keep_first == 0 && !r.slopes &&
-                           r.pool_rows > 0 && r.pool_base > 0);
-}
-
 extern "C" {
 
 // 1 when the split decode kernel has an instance for these head sizes
@@ -713,21 +597,25 @@ int hyb_sink_attention_tiles(const void* q, long q_row, long q_head, const void*
     if (G <= 0 || H % G || !hyb_sink_attention_tiles_ok(D, E)) return 1;
 #define TILES_ARGS q, q_row, q_head, k_cache, v_cache, block_tables, max_blocks, block_size, cu_q, \
                    positions, sink, gate, gate_row, out, scale, nseq, seq0, max_q, H, G, D, E
-#define TILES_E(T, DP, esz)                                                   \
-    do {                                                                      \
-        if (E <= 64) return launch_tiles<T, DP, 64>(TILES_ARGS, esz, rule, s);      \
-        if (E <= 128) return launch_tiles<T, DP, 128>(TILES_ARGS, esz, rule, s);    \
-        if (DP <= 128) return launch_tiles<T, (DP <= 128 ? DP : 64), 256>(TILES_ARGS, esz, rule, s); \
-        return 1;                                                             \
+    // bfloat16 operands that can be copied to LDS as they are: 8 times faster at 8 x 1k tokens of 128-wide
+    // heads, 4 times at 2 x 300 (hybrid_prompts.hip)
+    if (dt == 0 && prompt_attention_ok(q, q_row, q_head, k_cache, v_cache, out, nseq, max_q, D, E, rule.v_stride))
+        return prompt_attention(TILES_ARGS, rule, s);
+#define TILES_E(T, DP)                                                                       \
+    do {                                                                                     \
+        if (E <= 64) return launch_tiles<T, DP, 64>(TILES_ARGS, rule, s);                    \
+        if (E <= 128) return launch_tiles<T, DP, 128>(TILES_ARGS, rule, s);                  \
+        if (DP <= 128) return launch_tiles<T, (DP <= 128 ? DP : 64), 256>(TILES_ARGS, rule, s); \
+        return 1;                                                                            \
     } while (0)
-#define TILES_D(T, esz)                                   \
-    do {                                                  \
-        if (D <= 64) TILES_E(T, 64, esz);                 \
-        else if (D <= 128) TILES_E(T, 128, esz);          \
-        else TILES_E(T, 256, esz);                        \
+#define TILES_D(T)                                   \
+    do {                                             \
+        if (D <= 64) TILES_E(T, 64);                 \
+        else if (D <= 128) TILES_E(T, 128);          \
+        else TILES_E(T, 256);                        \
     } while (0)
-    if (dt == 0) TILES_D(hyb::bf16_t, 2);
-    else if (dt == 2) TILES_D(float, 4);
+    if (dt == 0) TILES_D(hyb::bf16_t);
+    else if (dt == 2) TILES_D(float);
     return 1;
 }
 

@@ -28,23 +28,12 @@
 // direct global -> LDS loads, requested a stage ahead.
 //
 // EP: value columns the accumulators hold (R <= EP, a multiple of 32); DP: key columns of the LDS
-// image (R + P <= DP, a multiple of 64).  The image is XOR-swizzled in 16-byte chunks so that both
-// the row reads (16 rows, one chunk) and the transposed reads (4 rows, 64 bytes) of a wave fall on
-// different banks, for row pitches of 256 bytes and of odd multiples of 128.
-#include "hybrid_merge.h"
-#include <type_traits>
+// image (R + P <= DP, a multiple of 64).
+#include "hybrid_tiles.h"
 
 using namespace hyb;
 
 namespace hyb_latent {
-
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) short s16x4;
-typedef __attribute__((ext_vector_type(8))) short s16x8;
-
-constexpr float LOG2E = 1.4426950408889634f;
-constexpr float RESCALE = 6.f;      // log2 units: weights stay <= 64 between rescales
 
 struct LatentArgs {
     const uint16_t* qa; long qa_row, qa_head;      // [rows, heads, R]
@@ -59,24 +48,6 @@ struct LatentArgs {
     float scale;
     int H, R, P, window, splits;
 };
-
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
-__device__ __forceinline__ uint16_t bf16_bits(float f) {
-    return __builtin_bit_cast(uint16_t, (__bf16)f);
-}
-
-// what the chunk number of a row is XORed with (see the header comment)
-template <int DP>
-__device__ __forceinline__ int swizzle(int row) {
-    return DP % 128 == 0 ? ((row & 3) << 2) | ((row >> 2) & 3) : (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
-}
 
 template <int EP, int DP, int RW>
 __global__ void __launch_bounds__(256, EP >= 256 ? 1 : 2)

@@ -1,0 +1,114 @@
+"""Prompt portions over bfloat16 caches (``csrc/hybrid/hybrid_prompts.hip``) against the plain form in
+fp32 on CPU copies: head sizes at the edges of the instances, pages smaller and larger than a key
+tile, portions around a wave's and a workgroup's queries, every option; and the operands that the
+general tile kernel takes instead."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from minivllm_amd.ops import hip_hybrid as hk
+from minivllm_amd.ops import torch_seqmix as ref
+
+LENS = [1, 31, 33, 64, 65, 127, 129, 300]          # contexts
+PORTIONS = [1, 31, 2, 64, 33, 127, 129, 200]       # their last tokens are this step's
+
+
+def close(got, want, top):
+    """Both round the same sum to bfloat16, whose numbers lie up to 2^-7 of their size apart, so one step;
+    and the fp32 sums of up to 300 products of weights <= 1 with values <= ``top`` differ themselves."""
+    got, want = got.float(), want.float()
+    d = (got - want).abs()
+    assert bool((d <= 2.0 ** -7 * torch.maximum(got.abs(), want.abs()) + 300 * 2.0 ** -22 * top).all()), float(d.max())
+
+
+def step(G, D, E, bs, seed=0, pooled=0):
+    g = torch.Generator().manual_seed(seed)
+    need = [-(-n // bs) for n in LENS]
+    ids = torch.randperm(sum(need), generator=g).int()
+    tables = torch.zeros(len(LENS), max(need) + 1, dtype=torch.int32)
+    at = 0
+    for b, n in enumerate(need):
+        tables[b, :n] = ids[at:at + n]
+        at += n
+    rows = sum(need) * bs
+    extra = sum(need) * -(-bs // pooled) if pooled else 0
+    k, v = (torch.randn((rows + extra) * G, n, generator=g).bfloat16() for n in (D, E))
+    cu_q = torch.tensor([0] + PORTIONS).cumsum(0).int()
+    cu_k = torch.tensor([0] + LENS).cumsum(0).int()
+    pos = torch.cat([torch.arange(L - n, L) for L, n in zip(LENS, PORTIONS)]).int()
+    return g, k, v, rows, tables, cu_q, cu_k, pos
+
+
+def caches(k, v, rows, G, D, E, bs, pooled):
+    n = rows // bs
+    kc, vc = k[:rows * G].view(n, bs, G, D), v[:rows * G].view(n, bs, G, E)
+    if not pooled:
+        return kc, vc, None, None
+    pr = -(-bs // pooled)
+    return kc, vc, k[rows * G:].view(n, pr, G, D), v[rows * G:].view(n, pr, G, E)
+
+
+@pytest.mark.parametrize("H,G,D,E", [(2, 1, 128, 128), (8, 4, 64, 64), (16, 2, 8, 16), (3, 3, 72, 136), (2, 2, 256, 120),
+                                     (1, 1, 40, 256), (4, 2, 136, 64), (2, 1, 128, 256)])
+@pytest.mark.parametrize("bs", [16, 64, 128])
+@pytest.mark.parametrize("opt", [dict(), dict(window=40, keep_first=5), dict(chunk=48), dict(slopes=True),
+                                 dict(window=33, pool=8, temps=True, softcap=5.0)])
+def test_every_instance_and_option(H, G, D, E, bs, opt):
+    opt = dict(opt)
+    pool = opt.get("pool", 0)
+    g, k, v, rows, tables, cu_q, cu_k, pos = step(G, D, E, bs, pooled=pool)
+    T = int(cu_q[-1])
+    proj = torch.randn(T, H * D + H, generator=g).bfloat16()
+    q, gate = proj[:, :H * D].view(T, H, D), proj[:, H * D:]
+    sink = torch.randn(H, generator=g) if opt.get("softcap") or not opt else None
+    if opt.pop("slopes", None):
+        opt["slopes"] = torch.rand(H, generator=g) * 0.2
+    if opt.pop("temps", None):
+        opt["temps"] = torch.randn(H, generator=g)
+    if H % 8:                                            # q rows of whole 16-byte runs only with H % 8 == 0
+        q = q.contiguous()
+
+    def call(f, to, **kw):
+        kc, vc, kp, vp = caches(to(k), to(v), rows, G, D, E, bs, pool)
+        o = {n: to(x) if torch.is_tensor(x) else x for n, x in opt.items()}
+        if pool:
+            o.update(k_pool=kp, v_pool=vp)
+        return f(to(q), kc, vc, to(cu_q), to(cu_k), to(tables), D ** -0.5, None if sink is None else to(sink),
+                 to(gate), to(torch.zeros(T, H, E, dtype=torch.bfloat16)), **kw, **o)
+
+    want = call(ref.sink_attention_prefill, lambda x: x)
+    got = call(hk.sink_attention_prefill, lambda x: x.cuda(), positions=pos.cuda(), max_q=max(PORTIONS)).cpu()
+    close(got, want, float(v.abs().max()))
+
+
+@pytest.mark.parametrize("D,E,shift", [(64, 64, 1), (36, 64, 0), (64, 20, 0), (128, 128, 4)])
+def test_operands_of_the_general_kernel(D, E, shift):
+    """Odd sizes and addresses stay with the kernel that takes any: same results."""
+    H, G, bs = 4, 2, 64
+    g, k, v, rows, tables, cu_q, cu_k, pos = step(G, D, E, bs)
+    T = int(cu_q[-1])
+    flat = torch.randn(T * H * D + shift, generator=g).bfloat16()
+    kc, vc, _, _ = caches(k, v, rows, G, D, E, bs, 0)
+    out = torch.zeros(T, H, E, dtype=torch.bfloat16)
+    want = ref.sink_attention_prefill(flat[shift:].view(T, H, D), kc, vc, cu_q, cu_k, tables, D ** -0.5, None, None, out)
+    got = hk.sink_attention_prefill(flat.cuda()[shift:].view(T, H, D), kc.cuda(), vc.cuda(), cu_q.cuda(), cu_k.cuda(),
+                                    tables.cuda(), D ** -0.5, None, None, torch.zeros_like(out).cuda(),
+                                    positions=pos.cuda(), max_q=max(PORTIONS)).cpu()
+    close(got, want, float(v.abs().max()))
+
+
+def test_values_inside_the_key_rows():
+    H, G, D, E, bs = 2, 1, 128, 64, 64
+    g, k, _, rows, tables, cu_q, cu_k, pos = step(G, D, E, bs)
+    T = int(cu_q[-1])
+    kc = k[:rows].view(-1, bs, G, D)
+    q = torch.randn(T, H, D, generator=g).bfloat16()
+    want = ref.sink_attention_prefill(q, kc, kc[..., :E], cu_q, cu_k, tables, D ** -0.5, None, None,
+                                      torch.zeros(T, H, E, dtype=torch.bfloat16))
+    kg = kc.cuda()
+    got = hk.sink_attention_prefill(q.cuda(), kg, kg[..., :E], cu_q.cuda(), cu_k.cuda(), tables.cuda(), D ** -0.5, None,
+                                    None, torch.zeros(T, H, E, dtype=torch.bfloat16).cuda(), positions=pos.cuda(),
+                                    max_q=max(PORTIONS)).cpu()
+    close(got, want, float(k.abs().max()))
