@@ -105,6 +105,21 @@ template <> __device__ __forceinline__ void store_run8<bf16_t>(bf16_t* p, const 
     *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Rows of a recurrence's output o [T, H, E] that no live sequence owns (ahead of the first sequence,
+// behind the last, those of a sequence without a state slot) read as zeros: workgroup (b, h, columns
+// [e0, e0 + cols)) of B sequences clears its share of them.
+__device__ __forceinline__ void clear_unowned(float* o, const int* cu_q, const int* slots, int b, int B, long T,
+                                              int H, int h, int E, int e0, int cols) {
+    const int n = min(cols, E - e0);
+    auto clear = [&](long from, long to) {
+        for (long i = threadIdx.x; i < (to - from) * n; i += blockDim.x)
+            o[((from + i / n) * H + h) * E + e0 + i % n] = 0.f;
+    };
+    if (b == 0 && cu_q) clear(0, cu_q[0]);
+    if (b + 1 == B) clear(cu_q ? cu_q[B] : B, T);
+    if (slots[b] < 0) clear(cu_q ? cu_q[b] : b, cu_q ? cu_q[b + 1] : b + 1);
+}
+
 #define HYB_DISPATCH(dt, ...)                                         \
     do {                                                              \
         if ((dt) == 0) { using T = hyb::bf16_t; __VA_ARGS__; }        \

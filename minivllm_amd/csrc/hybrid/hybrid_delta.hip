@@ -164,7 +164,7 @@ delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
                   const float* __restrict__ vv, const float* __restrict__ beta,
                   const float* __restrict__ decay, float* __restrict__ state,
                   const int* __restrict__ cu_q, const int* __restrict__ positions,
-                  const int* __restrict__ slots, float* __restrict__ o, int H, int G, int D, int E) {
+                  const int* __restrict__ slots, float* __restrict__ o, long T, int H, int G, int D, int E) {
     constexpr int CT = ScanChunk<NR>::tokens;
     constexpr int RS = NR + 4;                 // padded slice: the 4 lanes of a quad hit 4 bank groups
     constexpr int KQ = CT * 4 * RS;            // floats of one k (or q) chunk image
@@ -172,6 +172,7 @@ delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
     constexpr int NLD = (2 * CT * 4 * NR + CT * 64 + 2 * CT + 255) / 256;   // staged floats per thread
     extern __shared__ float sm[];
     const int b = blockIdx.x, h = blockIdx.y;
+    clear_unowned(o, cu_q, slots, b, gridDim.x, T, H, h, E, blockIdx.z * 64, 64);
     const int slot = slots[b];
     if (slot < 0) return;
     const long first = cu_q ? cu_q[b] : b;
@@ -284,13 +285,13 @@ delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
 template <int NR, bool DELTA>
 static void launch_scan(dim3 grid, hipStream_t s, const void* qn, const void* kn, const void* vv,
                         const void* beta, const void* decay, void* state, const void* cu_q,
-                        const void* positions, const void* slots, void* o, int H, int G, int D, int E) {
+                        const void* positions, const void* slots, void* o, long T_, int H, int G, int D, int E) {
     constexpr int CT = ScanChunk<NR>::tokens;
     constexpr int BUF = 2 * CT * 4 * (NR + 4) + CT * 64 + 2 * CT;
     hipLaunchKernelGGL((delta_scan_kernel<NR, DELTA>), grid, dim3(256), 2 * BUF * sizeof(float), s,
                        (const float*)qn, (const float*)kn, (const float*)vv, (const float*)beta,
                        (const float*)decay, (float*)state, (const int*)cu_q, (const int*)positions,
-                       (const int*)slots, (float*)o, H, G, D, E);
+                       (const int*)slots, (float*)o, T_, H, G, D, E);
 }
 
 extern "C" {
@@ -336,7 +337,7 @@ int hyb_delta_prepare(const void* proj, long row_stride, int b_off, const void* 
 
 int hyb_delta_scan(const void* qn, const void* kn, const void* vv, const void* beta,
                    const void* decay, void* state, const void* cu_q, const void* positions,
-                   const void* slots, void* o, int B, int H, int G, int D, int E, int correct,
+                   const void* slots, void* o, long T_, int B, int H, int G, int D, int E, int correct,
                    hipStream_t s) {
     if (B <= 0) return 0;
     if (H % G || D > 256) return 1;
@@ -344,9 +345,9 @@ int hyb_delta_scan(const void* qn, const void* kn, const void* vv, const void* b
 #define SCAN(NR)                                                                                       \
     do {                                                                                               \
         if (correct) launch_scan<NR, true>(grid, s, qn, kn, vv, beta, decay, state, cu_q, positions,   \
-                                           slots, o, H, G, D, E);                                      \
+                                           slots, o, T_, H, G, D, E);                                     \
         else launch_scan<NR, false>(grid, s, qn, kn, vv, beta, decay, state, cu_q, positions, slots,   \
-                                    o, H, G, D, E);                                                    \
+                                    o, T_, H, G, D, E);                                                   \
     } while (0)
     if (D <= 32) SCAN(8);
     else if (D <= 64) SCAN(16);

@@ -19,8 +19,8 @@
 // per-token scalars.  GLA, WKV and
 // MLSTM read the raw projections (bfloat16 or float rows of a wider projection output) and do
 // the gates' fp32 arithmetic while staging; CDELTA reads the fp32 outputs of delta_prepare.
-// MLSTM's running maximum is a sequential max-plus chain over tokens: wave 0 walks it once per
-// chunk (two dependent operations per token) and leaves the three factors of every token in LDS;
+// MLSTM's prompt portions over bfloat16 projections run on the matrix cores instead (hybrid_chunks.hip).
+// Its running maximum is a sequential max-plus chain over tokens: wave 0 walks it once per chunk (two dependent operations per token) and leaves the three factors of every token in LDS;
 // the normaliser n is kept by every lane group (its d-slice), since every column divides by n . q.
 // WKV's output is S^T q + (q . (u * k)) v: the factor of v is the same number for all columns and is
 // formed once per token, when a chunk has arrived in LDS, as ONE sum.  (A first token's output is
@@ -30,7 +30,7 @@
 // Sequence layout: `cu_q` [B+1] rows of each sequence (null: row b is sequence b), `positions`
 // (a sequence's first row holds the position its portion starts at; 0 = start from zeros),
 // `slots` [B] state slot per sequence (< 0: unused row of a padded batch).
-#include "hybrid_common.h"
+#include "hybrid_chunks.h"
 #include <stdlib.h>
 
 using namespace hyb;
@@ -53,6 +53,7 @@ struct ScanArgs {
     float *state, *nstate, *mstate; // [slots,H,D,E]; MLSTM: [slots,H,ZG,D], [slots,H,ZG], ZG = ceil(E/16)
     const int *cu_q, *positions, *slots;
     float* o;                       // [T, H, E]
+    long T;
     int H, G, D, E;
     float qscale;
 };
@@ -77,13 +78,15 @@ __global__ void __launch_bounds__(256) gated_scan_kernel(const ScanArgs a) {
     extern __shared__ float sm[];
     const int b = blockIdx.x, h = blockIdx.y;
     const int H = a.H, G = a.G, D = a.D, E = a.E;
+    const int e0 = blockIdx.z * COLS;
+    clear_unowned(a.o, a.cu_q, a.slots, b, gridDim.x, a.T, H, h, E, e0, COLS);
     const int slot = a.slots[b];
     if (slot < 0) return;
     const long first = a.cu_q ? a.cu_q[b] : b;
     const int n = a.cu_q ? a.cu_q[b + 1] - a.cu_q[b] : 1;
     if (n <= 0) return;
     const int tid = threadIdx.x, r = tid % LPC, c = tid / LPC;
-    const int e0 = blockIdx.z * COLS, e = e0 + c;
+    const int e = e0 + c;
     const bool col = e < E;
     const int g = h / (H / G);
     const int d0 = r * NR;
@@ -555,13 +558,13 @@ extern "C" {
 // q_row .. a_row; state [slots, H, D, E]; o [T, H, E] fp32.
 int hyb_gla_scan(const void* q, const void* k, const void* v, long q_row, long k_row, long v_row,
                  const void* a_raw, long a_row, const void* a_bias, float tau, void* state,
-                 const void* cu_q, const void* positions, const void* slots, void* o, int B, int H,
+                 const void* cu_q, const void* positions, const void* slots, void* o, long T_, int B, int H,
                  int D, int E, int dt, hipStream_t s) {
     ScanArgs a{};
     a.q = q; a.k = k; a.v = v; a.q_row = q_row; a.k_row = k_row; a.v_row = v_row;
     a.a = a_raw; a.a_row = a_row; a.a_bias = (const float*)a_bias; a.tau_inv = 1.f / tau;
     a.state = (float*)state; a.cu_q = (const int*)cu_q; a.positions = (const int*)positions;
-    a.slots = (const int*)slots; a.o = (float*)o; a.H = H; a.G = H; a.D = D; a.E = E;
+    a.slots = (const int*)slots; a.o = (float*)o; a.T = T_; a.H = H; a.G = H; a.D = D; a.E = E;
     a.qscale = 1.f / sqrtf((float)D);
     HYB_DISPATCH(dt, return (scan_by_size<T, GLA>(a, B, s)));
     return 1;
@@ -570,13 +573,13 @@ int hyb_gla_scan(const void* q, const void* k, const void* v, long q_row, long k
 // As hyb_gla_scan with the rule WKV: w_bias, bonus [H*D]; r and k are taken as they are (no D^-1/2).
 int hyb_wkv_scan(const void* r, const void* k, const void* v, long r_row, long k_row, long v_row,
                  const void* w_raw, long w_row, const void* w_bias, const void* bonus, void* state,
-                 const void* cu_q, const void* positions, const void* slots, void* o, int B, int H,
+                 const void* cu_q, const void* positions, const void* slots, void* o, long T_, int B, int H,
                  int D, int E, int dt, hipStream_t s) {
     ScanArgs a{};
     a.q = r; a.k = k; a.v = v; a.q_row = r_row; a.k_row = k_row; a.v_row = v_row;
     a.a = w_raw; a.a_row = w_row; a.a_bias = (const float*)w_bias; a.bonus = (const float*)bonus;
     a.state = (float*)state; a.cu_q = (const int*)cu_q; a.positions = (const int*)positions;
-    a.slots = (const int*)slots; a.o = (float*)o; a.H = H; a.G = H; a.D = D; a.E = E;
+    a.slots = (const int*)slots; a.o = (float*)o; a.T = T_; a.H = H; a.G = H; a.D = D; a.E = E;
     a.qscale = 1.f;
     HYB_DISPATCH(dt, return (scan_by_size<T, WKV>(a, B, s)));
     return 1;
@@ -587,14 +590,21 @@ int hyb_wkv_scan(const void* r, const void* k, const void* v, long r_row, long k
 int hyb_mlstm_scan(const void* q, const void* k, const void* v, long q_row, long k_row, long v_row,
                    const void* gi, const void* gf, long g_row, const void* bi, const void* bf,
                    float cap, void* state, void* nstate, void* mstate, const void* cu_q,
-                   const void* positions, const void* slots, void* o, int B, int H, int D, int E,
+                   const void* positions, const void* slots, void* o, long T_, int B, int H, int D, int E,
                    int dt, hipStream_t s) {
     ScanArgs a{};
     a.q = q; a.k = k; a.v = v; a.q_row = q_row; a.k_row = k_row; a.v_row = v_row;
     a.gi = gi; a.gf = gf; a.g_row = g_row; a.bi = (const float*)bi; a.bf = (const float*)bf;
     a.cap = cap; a.state = (float*)state; a.nstate = (float*)nstate; a.mstate = (float*)mstate;
+    if (dt == 0 && B > 0) {
+        const MlstmChunks c{(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, q_row, k_row, v_row,
+                            (const bf16_t*)gi, (const bf16_t*)gf, g_row, (const float*)bi, (const float*)bf, cap,
+                            (float*)state, (float*)nstate, (float*)mstate, (const int*)cu_q, (const int*)positions,
+                            (const int*)slots, (float*)o, T_, H, D, E, 1.f / sqrtf((float)D)};
+        if (mlstm_chunks_ok(c, B)) return mlstm_chunks(c, B, s);
+    }
     a.cu_q = (const int*)cu_q; a.positions = (const int*)positions; a.slots = (const int*)slots;
-    a.o = (float*)o; a.H = H; a.G = H; a.D = D; a.E = E; a.qscale = 1.f / sqrtf((float)D);
+    a.o = (float*)o; a.T = T_; a.H = H; a.G = H; a.D = D; a.E = E; a.qscale = 1.f / sqrtf((float)D);
     HYB_DISPATCH(dt, return (scan_by_size<T, MLSTM>(a, B, s)));
     return 1;
 }
@@ -602,13 +612,13 @@ int hyb_mlstm_scan(const void* q, const void* k, const void* v, long q_row, long
 // fp32 outputs of delta_prepare: qn, kn [T, G, D], vv [T, H, E], beta [T, H], decay [T, H, D].
 int hyb_channel_delta_scan(const void* qn, const void* kn, const void* vv, const void* beta,
                            const void* decay, void* state, const void* cu_q, const void* positions,
-                           const void* slots, void* o, int B, int H, int G, int D, int E,
+                           const void* slots, void* o, long T_, int B, int H, int G, int D, int E,
                            hipStream_t s) {
     ScanArgs a{};
     a.q = qn; a.k = kn; a.v = vv; a.q_row = (long)G * D; a.k_row = (long)G * D; a.v_row = (long)H * E;
     a.a = decay; a.a_row = (long)H * D; a.beta = (const float*)beta; a.state = (float*)state;
     a.cu_q = (const int*)cu_q; a.positions = (const int*)positions; a.slots = (const int*)slots;
-    a.o = (float*)o; a.H = H; a.G = G; a.D = D; a.E = E; a.qscale = 1.f;
+    a.o = (float*)o; a.T = T_; a.H = H; a.G = G; a.D = D; a.E = E; a.qscale = 1.f;
     return scan_by_size<float, CDELTA>(a, B, s);
 }
 

@@ -54,12 +54,12 @@ _split_ok.argtypes = [_I, _I]
 _split_ok.restype = _I
 _prep = _sig("hyb_delta_prepare", _P, _L, _I, _P, _L, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P,
              _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P)
-_scan = _sig("hyb_delta_scan", _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P)
-_cscan = _sig("hyb_channel_delta_scan", _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P)
-_gla = _sig("hyb_gla_scan", _P, _P, _P, _L, _L, _L, _P, _L, _P, _F, _P, _P, _P, _P, _P, _I, _I, _I, _I,
+_scan = _sig("hyb_delta_scan", _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P)
+_cscan = _sig("hyb_channel_delta_scan", _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _P)
+_gla = _sig("hyb_gla_scan", _P, _P, _P, _L, _L, _L, _P, _L, _P, _F, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I,
             _I, _P)
 _mlstm = _sig("hyb_mlstm_scan", _P, _P, _P, _L, _L, _L, _P, _P, _L, _P, _P, _F, _P, _P, _P, _P, _P, _P,
-              _P, _I, _I, _I, _I, _I, _P)
+              _P, _L, _I, _I, _I, _I, _I, _P)
 _esin = _sig("hyb_embed_sinusoid", _P, _P, _P, _P, _P, _L, _I, _I, _P)
 _rgn = _sig("hyb_residual_group_norm", _P, _P, _L, _P, _L, _P, _P, _L, _I, _I, _F, _I, _P)
 _anm = _sig("hyb_add_normed_mean", _P, _P, _L, _P, _P, _L, _P, _L, _I, _F, _I, _P)
@@ -91,7 +91,7 @@ _cns = _sig("hyb_conv_norm_store", _P, _L, _P, _P, _P, _P, _F, _P, _P, _P, _P, _
 _smx = _sig("hyb_shift_mix", _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _P)
 _rsq = _sig("hyb_relu_squared", _P, _L, _P, _L, _I, _I, _P)
 _tgt = _sig("hyb_token_gate", _P, _L, _P, _P, _L, _L, _P, _L, _I, _I, _P)
-_wkv = _sig("hyb_wkv_scan", _P, _P, _P, _L, _L, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P)
+_wkv = _sig("hyb_wkv_scan", _P, _P, _P, _L, _L, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _P)
 _lat = _sig("hyb_latent_attention", _P, _L, _L, _P, _L, _L, _P, _P, _I, _I, _P, _P, _P, _P, _P, _L, _L, _P,
             _F, _I, _I, _I, _I, _I, _I, _I, _P)
 _lat_ok = _lib.hyb_latent_attention_ok
@@ -360,6 +360,12 @@ def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale
                            chunk)
 
 
+def _rows_out(T, H, E, slots, device):
+    """The output rows of a recurrence: its kernel clears those that no sequence owns itself."""
+    new = torch.empty if slots.shape[0] else torch.zeros
+    return new((T, H, E), dtype=torch.float32, device=device)
+
+
 # ------------------------------------------------------------------ gated delta rule
 def delta_prepare(q, k, v, b, a, conv_w, a_log, dt_bias, conv_state, cu_q, positions, slots,
                   row_seq, conv_bias=None, ssd=False):
@@ -402,17 +408,17 @@ def delta_scan(qn, kn, vv, beta, decay, state, cu_q, positions, slots, correct=T
     T, G, D = qn.shape
     H, E = vv.shape[1], vv.shape[2]
     assert state.shape[1:] == (H, D, E)
-    o = torch.zeros((T, H, E), dtype=torch.float32, device=qn.device)
+    o = _rows_out(T, H, E, slots, qn.device)
     if decay.dim() == 3:                 # a decay per head and key channel
         assert decay.shape == (T, H, D) and decay.is_contiguous() and correct
         _check(_cscan(qn.data_ptr(), kn.data_ptr(), vv.data_ptr(), beta.data_ptr(), decay.data_ptr(),
                       _f32(state).data_ptr(), _ptr(_i32(cu_q)), _i32(positions).data_ptr(),
-                      _i32(slots).data_ptr(), o.data_ptr(), slots.shape[0], H, G, D, E, _stream()),
+                      _i32(slots).data_ptr(), o.data_ptr(), T, slots.shape[0], H, G, D, E, _stream()),
                "channel_delta_scan")
         return o
     _check(_scan(qn.data_ptr(), kn.data_ptr(), vv.data_ptr(), beta.data_ptr(), decay.data_ptr(),
                  _f32(state).data_ptr(), _ptr(_i32(cu_q)), _i32(positions).data_ptr(),
-                 _i32(slots).data_ptr(), o.data_ptr(), slots.shape[0], H, G, D, E, int(bool(correct)),
+                 _i32(slots).data_ptr(), o.data_ptr(), T, slots.shape[0], H, G, D, E, int(bool(correct)),
                  _stream()), "delta_scan")
     return o
 
@@ -549,12 +555,12 @@ def mlstm_scan(q, k, v, i_raw, f_raw, i_bias, f_bias, cap, state, norm_state, ma
     assert i_raw.shape == (T, H) and f_raw.shape == (T, H) and i_raw.stride(1) == 1 and f_raw.stride(1) == 1
     assert T == 1 or i_raw.stride(0) == f_raw.stride(0)
     assert k.dtype == q.dtype and v.dtype == q.dtype and i_raw.dtype == q.dtype and f_raw.dtype == q.dtype
-    o = torch.zeros((T, H, E), dtype=torch.float32, device=q.device)
+    o = _rows_out(T, H, E, slots, q.device)
     _check(_mlstm(q.data_ptr(), k.data_ptr(), v.data_ptr(), _heads_view(q, D), _heads_view(k, D),
                   _heads_view(v, E), i_raw.data_ptr(), f_raw.data_ptr(), _rows(i_raw),
                   _f32(i_bias).data_ptr(), _f32(f_bias).data_ptr(), cap, _f32(state).data_ptr(),
                   _f32(norm_state).data_ptr(), _f32(max_state).data_ptr(), _ptr(_i32(cu_q)),
-                  _i32(positions).data_ptr(), _i32(slots).data_ptr(), o.data_ptr(), slots.shape[0],
+                  _i32(positions).data_ptr(), _i32(slots).data_ptr(), o.data_ptr(), T, slots.shape[0],
                   H, D, E, _dt(q), _stream()), "mlstm_scan")
     return o
 
@@ -565,11 +571,11 @@ def gla_scan(q, k, v, a_raw, a_bias, tau, state, cu_q, positions, slots):
     assert state.shape[1:] == (H, D, E) and a_raw.shape == (T, H * D) and a_raw.stride(1) == 1
     assert k.dtype == q.dtype and v.dtype == q.dtype and a_raw.dtype == q.dtype
     assert a_bias.numel() == H * D
-    o = torch.zeros((T, H, E), dtype=torch.float32, device=q.device)
+    o = _rows_out(T, H, E, slots, q.device)
     _check(_gla(q.data_ptr(), k.data_ptr(), v.data_ptr(), _heads_view(q, D), _heads_view(k, D),
                 _heads_view(v, E), a_raw.data_ptr(), _rows(a_raw), _f32(a_bias).data_ptr(), tau,
                 _f32(state).data_ptr(), _ptr(_i32(cu_q)), _i32(positions).data_ptr(),
-                _i32(slots).data_ptr(), o.data_ptr(), slots.shape[0], H, D, E, _dt(q), _stream()),
+                _i32(slots).data_ptr(), o.data_ptr(), T, slots.shape[0], H, D, E, _dt(q), _stream()),
            "gla_scan")
     return o
 
@@ -944,11 +950,11 @@ def wkv_scan(r, k, v, w_raw, w_bias, bonus, state, cu_q, positions, slots):
     assert state.shape[1:] == (H, D, E) and w_raw.shape == (T, H * D) and w_raw.stride(1) == 1
     assert k.dtype == r.dtype and v.dtype == r.dtype and w_raw.dtype == r.dtype
     assert w_bias.numel() == H * D and bonus.numel() == H * D
-    o = torch.zeros((T, H, E), dtype=torch.float32, device=r.device)
+    o = _rows_out(T, H, E, slots, r.device)
     _check(_wkv(r.data_ptr(), k.data_ptr(), v.data_ptr(), _heads_view(r, D), _heads_view(k, D),
                 _heads_view(v, E), w_raw.data_ptr(), _rows(w_raw), _f32(w_bias).data_ptr(),
                 _f32(bonus).data_ptr(), _f32(state).data_ptr(), _ptr(_i32(cu_q)),
-                _i32(positions).data_ptr(), _i32(slots).data_ptr(), o.data_ptr(), slots.shape[0], H, D, E,
+                _i32(positions).data_ptr(), _i32(slots).data_ptr(), o.data_ptr(), T, slots.shape[0], H, D, E,
                 _dt(r), _stream()), "wkv_scan")
     return o
 

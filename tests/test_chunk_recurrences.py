@@ -1,0 +1,82 @@
+"""Recurrences over prompt portions in chunks on the matrix cores (``csrc/hybrid/hybrid_chunks.hip``)
+against the token-by-token form in fp64, and against the kernel that takes the recurrence literally
+(reached with the same numbers in rows that are no whole 16-byte runs): portions around a block of 16
+and a chunk of 64 tokens, head sizes at the edges of the instances, state carried in, sequences
+without rows or without a slot, rows of no sequence."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from minivllm_amd.ops import hip_hybrid as hk
+
+LENS = [1, 15, 0, 16, 17, 63, 64, 65, 129, 200, 5]
+PAST = [0, 9, 0, 0, 3, 0, 70, 0, 0, 1, 0]
+SLOTS = [3, 1, 2, 0, 12, 5, 7, 6, 8, 11, -1]
+TAIL = 3                                               # rows behind the last sequence
+
+
+def layout():
+    cu = [0]
+    for n in LENS:
+        cu.append(cu[-1] + n)
+    pos = [p + i for n, p in zip(LENS, PAST) for i in range(n)] + [0] * TAIL
+    return cu, [torch.tensor(x, dtype=torch.int32).cuda() for x in (cu, pos, SLOTS)]
+
+
+def off(got, want):
+    return float((got.double().cpu() - want).norm() / want.norm().clamp_min(1e-30))
+
+
+@pytest.mark.parametrize("H,D,E", [(2, 128, 128), (1, 8, 8), (3, 48, 40), (2, 64, 72), (1, 72, 32), (2, 120, 64)])
+@pytest.mark.parametrize("cap", [4.0, 15.0])
+def test_mlstm(H, D, E, cap):
+    g = torch.Generator().manual_seed(D + E)
+    cu, lay = layout()
+    T, Z, NS = cu[-1] + TAIL, (E + 15) // 16, 13
+    n_in = 2 * H * D + H * E + 2 * H
+    proj = torch.randn(T, n_in, generator=g)
+    proj[:, 2 * H * D + H * E:] *= 4                   # gates that reach the cap
+    proj = proj.bfloat16()
+    bi, bf = torch.randn(H, generator=g), 2 + torch.randn(H, generator=g)
+    init = [torch.randn(NS, H, D, E, generator=g), torch.randn(NS, H, 1, D, generator=g).expand(-1, -1, Z, -1).contiguous(),
+            torch.randn(NS, H, 1, generator=g).expand(-1, -1, Z).contiguous()]
+
+    def run(pad):
+        p = torch.zeros(T, n_in + pad, dtype=torch.bfloat16).cuda()
+        p[:, :n_in] = proj.cuda()
+        q, k, v, i, f = p[:, :n_in].split([H * D, H * D, H * E, H, H], -1)
+        st = [x.cuda() for x in init]
+        o = hk.mlstm_scan(q.view(T, H, D), k.view(T, H, D), v.view(T, H, E), i, f, bi.cuda(), bf.cuda(), cap, *st, *lay)
+        return [o.cpu()] + [x.cpu() for x in st]
+
+    q, k, v, i, f = proj.double().split([H * D, H * D, H * E, H, H], -1)
+    q, k, v = q.view(T, H, D) * D ** -0.5, k.view(T, H, D), v.view(T, H, E)
+    i = cap * torch.tanh((i + bi.double()) / cap)
+    f = torch.nn.functional.logsigmoid(cap * torch.tanh((f + bf.double()) / cap))
+    o = torch.zeros(T, H, E, dtype=torch.float64)
+    want = [x.double() for x in init]
+    for b, (n, s) in enumerate(zip(LENS, SLOTS)):
+        if s < 0 or n == 0:
+            continue
+        S, N, m = (x[s].clone() * (PAST[b] > 0) for x in want)
+        N, m = N[:, 0], m[:, 0]
+        for t in range(cu[b], cu[b + 1]):
+            m2 = torch.maximum(f[t] + m, i[t])
+            a, c = torch.exp(f[t] + m - m2), torch.exp(i[t] - m2)
+            S = a[:, None, None] * S + c[:, None, None] * k[t][:, :, None] * v[t][:, None]
+            N = a[:, None] * N + c[:, None] * k[t]
+            m = m2
+            den = torch.maximum((N * q[t]).sum(-1).abs(), torch.exp(-m)) + 1e-6
+            o[t] = torch.einsum("hde,hd->he", S, q[t]) / den[:, None]
+        want[0][s], want[1][s], want[2][s] = S, N[:, None], m[:, None]
+    got, literal = run((-n_in) % 8), run((-n_in) % 8 + 1)
+    for x, y, w in zip(got, literal, [o] + want):
+        # sums of up to 200 fp32 terms: 200 * 2^-24; no further off than the literal kernel is, but for that
+        assert off(x, w) <= 2 * off(y, w) + 200 * 2.0 ** -24, (off(x, w), off(y, w))
+    owned = torch.zeros(T, dtype=torch.bool)
+    for b, s in enumerate(SLOTS):
+        owned[cu[b]:cu[b + 1]] = s >= 0
+    for x in (got[0], literal[0]):
+        assert bool((x[~owned] == 0).all())
