@@ -1,8 +1,71 @@
-// Recurrences of hybrid_recurrent.hip over prompt portions in chunks (hybrid_chunks.hip).
+// Recurrences over prompt portions in chunks of tokens on the matrix cores: the matrix LSTM's
+// (hybrid_chunks.hip) and the delta rule's (hybrid_delta_chunks.hip); what their kernels share.
+//
+// An fp32 operand of a bf16 product is cut into three parts of eight bits, which hold all of its 24.
 #pragma once
-#include "hybrid_common.h"
+#include "hybrid_tiles.h"
 
 namespace hyb {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+// the upper halves of x and y side by side: eight bits of each
+__device__ __forceinline__ uint32_t upper(float x, float y) {
+    return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302);
+}
+__device__ __forceinline__ float rest(float x) { return x - __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+
+// eight numbers as three bfloat16 fragments whose sum they are
+__device__ __forceinline__ void split8(const float* x, bf16x8* p) {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float u = x[2 * j], v = x[2 * j + 1];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            w[k][j] = upper(u, v);
+            if (k < 2) { u = rest(u); v = rest(v); }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) p[k] = __builtin_bit_cast(bf16x8, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
+}
+
+#ifdef __HIP_DEVICE_COMPILE__
+__device__ __forceinline__ s16x4 read_tr(const char* lds) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(
+        (__attribute__((address_space(3))) char*)lds));
+}
+__device__ __forceinline__ bf16x8 join(s16x4 x, s16x4 y) {
+    const s16x8 v = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+    return __builtin_bit_cast(bf16x8, v);
+}
+__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+#endif
+
+// four numbers of a lane as three runs of bfloat16; at(k): where part k goes
+template <class F>
+__device__ __forceinline__ void put_parts(f32x4 x, F&& at) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        *reinterpret_cast<uint2*>(at(k)) = make_uint2(upper(x[0], x[1]), upper(x[2], x[3]));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = rest(x[r]);
+    }
+}
+
+// x of the lane N places before (behind) this one inside its row of 16, `none` where there is none
+template <int N> __device__ __forceinline__ float from_left(float x, float none) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(none), __float_as_uint(x), 0x110 | N, 0xf, 0xf, false));
+}
+template <int N> __device__ __forceinline__ float from_right(float x, float none) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(none), __float_as_uint(x), 0x100 | N, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float lane_of(float x, int lane) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), lane));
+}
 
 struct MlstmChunks {
     const uint16_t *q, *k, *v;      // rows of [*, H, D] / [*, H, E], element strides per token below
@@ -23,5 +86,21 @@ struct MlstmChunks {
 // addresses
 bool mlstm_chunks_ok(const MlstmChunks& a, int B);
 int mlstm_chunks(const MlstmChunks& a, int B, hipStream_t s);
+
+struct DeltaChunks {
+    const float *q, *k, *v;         // [T, G, D], [T, G, D], [T, H, E]
+    const float *beta, *decay;      // [T, H]
+    float* state;                   // [slots, H, D, E]
+    const int *cu_q, *positions, *slots;
+    float* o;                       // [T, H, E]
+    char* ws;                       // what the first kernel leaves for the second: delta_chunks_bytes
+    long T;
+    int B, H, G, D, E;
+};
+
+// bytes of workspace for portions of these sizes, 0 when the recurrence is to be walked token by token
+long delta_chunks_bytes(const DeltaChunks& a);
+// correct: with the delta rule's correction term
+int delta_chunks(const DeltaChunks& a, bool correct, hipStream_t s);
 
 }  // namespace hyb

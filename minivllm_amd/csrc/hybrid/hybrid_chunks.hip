@@ -30,54 +30,15 @@
 // and chunk at two waves per SIMD), 4.4 us a chunk.  8 portions of 512..1024 tokens, 8 heads of
 // 128: 70 us of 83 with the norm behind it, against 602 of 622 token by token.  With four waves of twice the
 // columns 112 us; two workgroups per CU (128 registers) spill: 177 us.
-#include "hybrid_tiles.h"
 #include "hybrid_chunks.h"
 
 using namespace hyb;
 
 namespace {
 
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
 constexpr int C = 64;                  // tokens per chunk
 constexpr int EB = 32;                 // state columns per workgroup
 constexpr float NEG_INF = -__builtin_inff();
-
-// the upper halves of x and y side by side: eight bits of each
-__device__ __forceinline__ uint32_t upper(float x, float y) {
-    return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302);
-}
-__device__ __forceinline__ float rest(float x) { return x - __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
-
-// eight numbers as three bfloat16 fragments whose sum they are
-__device__ __forceinline__ void split8(const float* x, bf16x8* p) {
-    uint32_t w[3][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        float u = x[2 * j], v = x[2 * j + 1];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            w[k][j] = upper(u, v);
-            if (k < 2) { u = rest(u); v = rest(v); }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) p[k] = __builtin_bit_cast(bf16x8, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
-}
-
-#ifdef __HIP_DEVICE_COMPILE__
-__device__ __forceinline__ s16x4 read_tr(const char* lds) {
-    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(
-        (__attribute__((address_space(3))) char*)lds));
-}
-__device__ __forceinline__ bf16x8 join(s16x4 x, s16x4 y) {
-    const s16x8 v = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-    return __builtin_bit_cast(bf16x8, v);
-}
-__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-#endif
 
 // per token of a chunk, in LDS
 struct Gates {
@@ -102,17 +63,6 @@ struct Lds {
 };
 
 __device__ __forceinline__ float logsigmoid_(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
-
-// x of the lane N places before (behind) this one inside its row of 16, `none` where there is none
-template <int N> __device__ __forceinline__ float from_left(float x, float none) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(none), __float_as_uint(x), 0x110 | N, 0xf, 0xf, false));
-}
-template <int N> __device__ __forceinline__ float from_right(float x, float none) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(none), __float_as_uint(x), 0x100 | N, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float lane_of(float x, int lane) {
-    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), lane));
-}
 
 template <int DP>
 __global__ void __launch_bounds__(512, 2)
@@ -252,15 +202,6 @@ mlstm_chunks_kernel(MlstmChunks a) {
             *reinterpret_cast<uint4*>(L.k + row * DP * 2 + ch * 16) = kr[i];
         }
         *reinterpret_cast<uint2*>(L.v + tid * 8) = vr;
-    };
-    // four numbers in a lane as three bfloat16 runs
-    auto put_parts = [&](f32x4 x, auto&& at) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            *reinterpret_cast<uint2*>(at(k)) = make_uint2(upper(x[0], x[1]), upper(x[2], x[3]));
-#pragma unroll
-            for (int r = 0; r < 4; ++r) x[r] = rest(x[r]);
-        }
     };
     // the state's parts: a row per column of the state
     auto publish = [&]() {

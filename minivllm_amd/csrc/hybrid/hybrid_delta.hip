@@ -9,7 +9,10 @@
 // (a sequence's first row holds the position its portion starts at; 0 = start from zeros),
 // `slots` [B] state slot per sequence (< 0: unused row of a padded batch), `row_seq` [T] the
 // sequence of each row in prefill form (< 0: no sequence).
-#include "hybrid_common.h"
+//
+// Prompt portions of the recurrence run in chunks on the matrix cores (hybrid_delta_chunks.hip) where the
+// operands and lengths allow; what is here takes single tokens and everything else.
+#include "hybrid_chunks.h"
 
 using namespace hyb;
 
@@ -335,12 +338,28 @@ int hyb_delta_prepare(const void* proj, long row_stride, int b_off, const void* 
     return HYB_LAUNCH_OK();
 }
 
+// Bytes of workspace hyb_delta_scan wants for these operands (0: none; the rows are walked token by token).
+long hyb_delta_scan_ws(const void* qn, const void* kn, const void* vv, const void* cu_q, const void* o,
+                       long T_, int B, int H, int G, int D, int E) {
+    DeltaChunks c{};
+    c.q = (const float*)qn; c.k = (const float*)kn; c.v = (const float*)vv; c.cu_q = (const int*)cu_q;
+    c.o = (float*)o; c.T = T_; c.B = B; c.H = H; c.G = G; c.D = D; c.E = E;
+    return delta_chunks_bytes(c);
+}
+
+// ws: hyb_delta_scan_ws bytes, or null
 int hyb_delta_scan(const void* qn, const void* kn, const void* vv, const void* beta,
                    const void* decay, void* state, const void* cu_q, const void* positions,
-                   const void* slots, void* o, long T_, int B, int H, int G, int D, int E, int correct,
-                   hipStream_t s) {
+                   const void* slots, void* o, void* ws, long T_, int B, int H, int G, int D, int E,
+                   int correct, hipStream_t s) {
     if (B <= 0) return 0;
     if (H % G || D > 256) return 1;
+    if (ws) {
+        const DeltaChunks c{(const float*)qn, (const float*)kn, (const float*)vv, (const float*)beta,
+                            (const float*)decay, (float*)state, (const int*)cu_q, (const int*)positions,
+                            (const int*)slots, (float*)o, (char*)ws, T_, B, H, G, D, E};
+        return delta_chunks(c, correct != 0, s);
+    }
     const dim3 grid(B, H, (E + 63) / 64);
 #define SCAN(NR)                                                                                       \
     do {                                                                                               \

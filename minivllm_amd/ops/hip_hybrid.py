@@ -54,7 +54,9 @@ _split_ok.argtypes = [_I, _I]
 _split_ok.restype = _I
 _prep = _sig("hyb_delta_prepare", _P, _L, _I, _P, _L, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P,
              _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P)
-_scan = _sig("hyb_delta_scan", _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P)
+_scan = _sig("hyb_delta_scan", _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P)
+_scan_ws = _sig("hyb_delta_scan_ws", _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I)
+_scan_ws.restype = _L
 _cscan = _sig("hyb_channel_delta_scan", _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _P)
 _gla = _sig("hyb_gla_scan", _P, _P, _P, _L, _L, _L, _P, _L, _P, _F, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I,
             _I, _P)
@@ -416,9 +418,15 @@ def delta_scan(qn, kn, vv, beta, decay, state, cu_q, positions, slots, correct=T
                       _i32(slots).data_ptr(), o.data_ptr(), T, slots.shape[0], H, G, D, E, _stream()),
                "channel_delta_scan")
         return o
+    # prompt portions in chunks on the matrix cores need a place for what a first kernel works out
+    ws = None
+    if cu_q is not None:
+        n = _scan_ws(qn.data_ptr(), kn.data_ptr(), vv.data_ptr(), cu_q.data_ptr(), o.data_ptr(), T,
+                     slots.shape[0], H, G, D, E)
+        ws = torch.empty((n,), dtype=torch.uint8, device=qn.device) if n else None
     _check(_scan(qn.data_ptr(), kn.data_ptr(), vv.data_ptr(), beta.data_ptr(), decay.data_ptr(),
                  _f32(state).data_ptr(), _ptr(_i32(cu_q)), _i32(positions).data_ptr(),
-                 _i32(slots).data_ptr(), o.data_ptr(), T, slots.shape[0], H, G, D, E, int(bool(correct)),
+                 _i32(slots).data_ptr(), o.data_ptr(), _ptr(ws), T, slots.shape[0], H, G, D, E, int(bool(correct)),
                  _stream()), "delta_scan")
     return o
 

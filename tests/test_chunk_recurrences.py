@@ -80,3 +80,52 @@ def test_mlstm(H, D, E, cap):
         owned[cu[b]:cu[b + 1]] = s >= 0
     for x in (got[0], literal[0]):
         assert bool((x[~owned] == 0).all())
+
+
+@pytest.mark.parametrize("H,G,D,E", [(2, 1, 128, 128), (3, 3, 8, 4), (4, 2, 48, 40), (2, 2, 64, 72), (6, 2, 72, 32), (33, 11, 120, 64)])
+@pytest.mark.parametrize("correct", [True, False])
+@pytest.mark.parametrize("fast", [True, False])
+def test_delta_rule(H, G, D, E, correct, fast):
+    """``fast``: decays down to 1e-9 per token (their products leave fp32's range inside a chunk), keys that
+    repeat each other."""
+    g = torch.Generator().manual_seed(D + E)
+    cu, lay = layout()
+    T, NS = cu[-1] + TAIL, 13
+    q, k = (torch.randn(T, G, D, generator=g) for _ in range(2))
+    if fast:
+        k = k[torch.arange(T) // 3]
+    q, k = q / q.norm(dim=-1, keepdim=True) * D ** -0.5, k / k.norm(dim=-1, keepdim=True)
+    v, beta = torch.randn(T, H, E, generator=g), torch.sigmoid(2 * torch.randn(T, H, generator=g))
+    decay = torch.exp(-torch.rand(T, H, generator=g) * (20.0 if fast else 0.2))
+    if fast:
+        decay[::7] = 1.0
+    state = torch.randn(NS, H, D, E, generator=g)
+
+    def run(shift):
+        def at(x):                                     # rows that do not start on 16 bytes go token by token
+            y = torch.empty(x.numel() + shift, dtype=x.dtype).cuda()
+            y[shift:] = x.reshape(-1).cuda()
+            return y[shift:].view(x.shape)
+        st = state.cuda()
+        return hk.delta_scan(at(q), at(k), at(v), beta.cuda(), decay.cuda(), st, *lay, correct).cpu(), st.cpu()
+
+    qd, kd = (x.double().repeat_interleave(H // G, 1) for x in (q, k))
+    o, want = torch.zeros(T, H, E, dtype=torch.float64), state.double()
+    for b, (n, s) in enumerate(zip(LENS, SLOTS)):
+        if s < 0:
+            continue
+        S = want[s] * (PAST[b] > 0)
+        for t in range(cu[b], cu[b + 1]):
+            S = S * decay[t].double()[:, None, None]
+            u = beta[t].double()[:, None] * (v[t].double() - (torch.einsum("hde,hd->he", S, kd[t]) if correct else 0))
+            S = S + kd[t][:, :, None] * u[:, None]
+            o[t] = torch.einsum("hde,hd->he", S, qd[t])
+        want[s] = S
+    got, literal = run(0), run(1)
+    for x, y, w in zip(got, literal, (o, want)):
+        assert off(x, w) <= 2 * off(y, w) + 200 * 2.0 ** -24, (off(x, w), off(y, w))
+    owned = torch.zeros(T, dtype=torch.bool)
+    for b, s in enumerate(SLOTS):
+        owned[cu[b]:cu[b + 1]] = s >= 0
+    for x in (got[0], literal[0]):
+        assert bool((x[~owned] == 0).all())
