@@ -24,10 +24,10 @@ constexpr int MAX_TAPS = 32;
 // head, DC = 1 (a decay per head) or D (one per head and key channel); dt_bias has H * DC
 // entries, decay out [T, H * DC].
 // conv_w [C, taps] (q, k, v rows stacked), conv_state [slots, taps-1, C].
-template <typename T, int TAPS>
+template <typename T>
 __global__ void delta_prepare_kernel(const T* __restrict__ proj, long row_stride, int b_off,
                                      const T* __restrict__ a, long a_row, int DC,
-                                     const float* __restrict__ conv_w, int taps_rt,
+                                     const float* __restrict__ conv_w, int taps,
                                      const float* __restrict__ conv_b, int ssd,
                                      const float* __restrict__ a_log,
                                      const float* __restrict__ dt_bias,
@@ -36,10 +36,8 @@ __global__ void delta_prepare_kernel(const T* __restrict__ proj, long row_stride
                                      const int* __restrict__ slots, const int* __restrict__ row_seq,
                                      float* __restrict__ qn, float* __restrict__ kn,
                                      float* __restrict__ vv, float* __restrict__ beta,
-                                     float* __restrict__ decay, int H, int G, int D, int E,
-                                     int vec8) {
+                                     float* __restrict__ decay, int H, int G, int D, int E) {
     extern __shared__ float y[];                     // [2GD] convolved + silu q, k
-    const int taps = TAPS ? TAPS : taps_rt;          // TAPS > 0: known at compile time (unrolled)
     const long t = blockIdx.x;
     const int b = row_seq ? row_seq[t] : (int)t;
     if (b < 0) return;
@@ -50,39 +48,6 @@ __global__ void delta_prepare_kernel(const T* __restrict__ proj, long row_stride
     const bool has_past = positions[first] > 0;
     const int C = 2 * G * D + H * E, GD = G * D;
     const float* tail = conv_state + (long)slot * (taps - 1) * C;
-    if (TAPS > 0 && vec8) {
-        // eight channels per thread and step, every load of the step issued before its first use:
-        // one 16-byte (bf16) load per tap and the channels' taps as whole rows of the tap table
-        constexpr int NT = TAPS ? TAPS : 1;
-        for (int c = threadIdx.x * 8; c < C; c += blockDim.x * 8) {
-            float x[NT][8], w[8][NT];
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const int back = NT - 1 - j;
-                if (i - back >= 0) load_run<T, 8>(proj + (t - back) * row_stride + c, x[j]);
-                else if (has_past) load_run<float, 8>(tail + (long)(NT - 1 + i - back) * C + c, x[j]);
-                else {
-#pragma unroll
-                    for (int z = 0; z < 8; ++z) x[j][z] = 0.f;
-                }
-            }
-#pragma unroll
-            for (int z = 0; z < 8; ++z)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) w[z][j] = conv_w[(long)(c + z) * NT + j];
-            float acc[8];
-#pragma unroll
-            for (int z = 0; z < 8; ++z) {
-                float a = conv_b ? conv_b[c + z] : 0.f;
-#pragma unroll
-                for (int j = 0; j < NT; ++j) a += x[j][z] * w[z][j];
-                acc[z] = siluf_(a);
-            }
-            float* dst = (c < 2 * GD) ? y + c : vv + t * (long)(H * E) + (c - 2 * GD);
-            *reinterpret_cast<float4*>(dst) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-            *reinterpret_cast<float4*>(dst + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
-        }
-    } else
     for (int c = threadIdx.x; c < C; c += blockDim.x) {
         float acc = conv_b ? conv_b[c] : 0.f;
         for (int j = 0; j < taps; ++j) {             // tap j reads the input `taps-1-j` tokens back
@@ -118,6 +83,136 @@ __global__ void delta_prepare_kernel(const T* __restrict__ proj, long row_stride
     }
 }
 
+// The same for the usual sizes (2 to 4 taps, channels in whole runs of eight): a workgroup takes `rows`
+// consecutive token rows and a block of channels that holds whole heads, a thread eight channels, whose
+// taps and last inputs stay in its registers from row to row.  A head's sum of squares runs over the
+// lanes that share it (LANES: a power of two of them, by exchanges; else through LDS).
+// The thread of a sequence's last row writes the slot's new tail where nobody else can still read the
+// old one: the sequence has no past, or all its rows are this workgroup's; delta_conv_tail takes the others.
+// Per row 2 C bytes in and 4 C out.  6100 rows of 4096 channels, 16 / 8 heads of 128: 57 us = 2.6 TB/s, of which
+// silu and the gates take a fifth and the stores a fifth, against 95 of one workgroup per row (the
+// taps, 16 C bytes, were read again for every row, four bytes a load); a decode batch of 64: 8 us as
+// before, and no second kernel (8 us) for the tails.
+template <typename T, int TAPS>
+__global__ void __launch_bounds__(256)
+delta_prepare_rows_kernel(const T* __restrict__ proj, long row_stride, int b_off,
+                          const T* __restrict__ a, long a_row, int DC,
+                          const float* __restrict__ conv_w, const float* __restrict__ conv_b, int ssd,
+                          const float* __restrict__ a_log, const float* __restrict__ dt_bias,
+                          float* __restrict__ conv_state, const int* __restrict__ cu_q,
+                          const int* __restrict__ positions, const int* __restrict__ slots,
+                          const int* __restrict__ row_seq, float* __restrict__ qn, float* __restrict__ kn,
+                          float* __restrict__ vv, float* __restrict__ beta, float* __restrict__ decay, long T_,
+                          int rows, int block, int H, int G, int D, int E) {
+    __shared__ float part[256];
+    const int tid = threadIdx.x, GD = G * D, C = 2 * GD + H * E;
+    const long t0 = (long)blockIdx.x * rows, t1 = min(t0 + rows, T_);
+    const int c = blockIdx.y * block + tid * 8;
+    const bool mine = tid * 8 < block && c < C;
+    const int lanes = D >> 3, lane0 = tid / lanes * lanes;       // the threads of this one's head
+    const bool exchange = (lanes & (lanes - 1)) == 0 && lanes <= kWave;
+    float w[8][TAPS], bias[8], past[TAPS - 1][8];
+    {   // the taps of eight channels are one run of 8 TAPS numbers
+        float run[8 * TAPS];
+        load_run<float, 8 * TAPS>(conv_w + (long)(mine ? c : 0) * TAPS, run);
+#pragma unroll
+        for (int z = 0; z < 8; ++z) {
+            bias[z] = mine && conv_b ? conv_b[c + z] : 0.f;
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) w[z][j] = run[z * TAPS + j];
+        }
+    }
+    int slot = -1;
+    long first = 0, last = t0 - 1;                   // the sequence whose rows are being walked
+    bool has_past = false, follows = false;          // follows: `past` holds the inputs of the rows above
+    float* tail = conv_state;
+    float x[8], next[8];
+    const T* in = proj + (mine ? c : 0);
+    load_run<T, 8>(in + t0 * row_stride, next);
+    for (long t = t0; t < t1; ++t) {
+#pragma unroll
+        for (int z = 0; z < 8; ++z) x[z] = mine ? next[z] : 0.f;
+        if (t + 1 < t1) load_run<T, 8>(in + (t + 1) * row_stride, next);     // on its way while this row is worked on
+        if (t > last) {                              // (uniform)
+            const int b = row_seq ? row_seq[t] : (int)t;
+            slot = b < 0 ? -1 : slots[b];
+            first = b >= 0 && cu_q ? cu_q[b] : t;
+            last = b >= 0 && cu_q ? cu_q[b + 1] - 1 : t;
+            has_past = slot >= 0 && positions[first] > 0;
+            tail = conv_state + (long)slot * (TAPS - 1) * C + c;
+            follows = false;
+        }
+        if (slot < 0) continue;
+        if (!follows) {
+#pragma unroll
+            for (int j = 0; j < TAPS - 1; ++j) {                   // past[j]: TAPS - 1 - j rows back
+                const long at = t - (TAPS - 1 - j);
+                if (mine && at >= first) load_run<T, 8>(in + at * row_stride, past[j]);
+                else if (mine && has_past) load_run<float, 8>(tail + (TAPS - 1 + at - first) * C, past[j]);
+                else {
+#pragma unroll
+                    for (int z = 0; z < 8; ++z) past[j][z] = 0.f;
+                }
+            }
+            follows = true;
+        }
+        float y[8], sq = 0.f;
+#pragma unroll
+        for (int z = 0; z < 8; ++z) {
+            float s = bias[z];
+#pragma unroll
+            for (int j = 0; j < TAPS - 1; ++j) s += past[j][z] * w[z][j];
+            s += x[z] * w[z][TAPS - 1];
+            y[z] = siluf_(s);
+            sq += y[z] * y[z];
+        }
+        if (!ssd) {
+            if (exchange) {
+                for (int o = 1; o < lanes; o <<= 1) sq += __shfl_xor(sq, o, kWave);
+            } else {
+                __syncthreads();                                   // (every thread is in the same row)
+                part[tid] = sq;
+                __syncthreads();
+                sq = 0.f;
+                for (int i = 0; i < lanes; ++i) sq += part[min(lane0 + i, 255)];
+            }
+        }
+        if (mine) {
+            float* dst = vv + t * (long)(H * E) + (c - 2 * GD);
+            if (c < 2 * GD) {
+                float r = ssd ? 1.f : rsqrtf(sq + 1e-6f);
+                if (!ssd && c < GD) r *= rsqrtf((float)D);
+#pragma unroll
+                for (int z = 0; z < 8; ++z) y[z] *= r;
+                dst = c < GD ? qn + t * GD + c : kn + t * GD + (c - GD);
+            }
+            store_run8(dst, y);
+            if (t == last && (!has_past || first >= t0)) {
+#pragma unroll
+                for (int j = 0; j + 1 < TAPS - 1; ++j) store_run8(tail + (long)j * C, past[j + 1]);
+                store_run8(tail + (long)(TAPS - 2) * C, x);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j + 1 < TAPS - 1; ++j)
+#pragma unroll
+            for (int z = 0; z < 8; ++z) past[j][z] = past[j + 1][z];
+#pragma unroll
+        for (int z = 0; z < 8; ++z) past[TAPS - 2][z] = x[z];
+    }
+    // the rows' gates, spread over the workgroups of all channel blocks
+    const int per = H * DC, n = (int)(t1 - t0) * per;
+    for (int i = blockIdx.y * 256 + tid; i < n; i += gridDim.y * 256) {
+        const long t = t0 + i / per;
+        const int h = i % per, b = row_seq ? row_seq[t] : (int)t;
+        if (b < 0 || slots[b] < 0) continue;
+        const float sp = softplusf_(ld(a + t * a_row + h) + dt_bias[h]);
+        if (ssd) beta[t * H + h] = sp;               // DC == 1: the step size of head h
+        else if (h % DC == 0) beta[t * H + h / DC] = sigmoidf_(ld(proj + t * row_stride + b_off + h / DC));
+        decay[t * (long)per + h] = expf(-expf(a_log[h / DC]) * sp);
+    }
+}
+
 // One workgroup per sequence: the convolution inputs of the portion's last taps-1 tokens become
 // the slot's tail (older entries shift when the portion is shorter).  Runs after delta_prepare.
 template <typename T>
@@ -125,7 +220,8 @@ __global__ void delta_conv_tail_kernel(const T* __restrict__ proj, long row_stri
                                        float* __restrict__ conv_state,
                                        const int* __restrict__ cu_q,
                                        const int* __restrict__ positions,
-                                       const int* __restrict__ slots, int C) {
+                                       const int* __restrict__ slots, int C, int rows) {
+    // rows > 0: delta_prepare_rows ran ahead with that many rows per workgroup and wrote the tails it could
     const int b = blockIdx.x;
     const int slot = slots[b];
     if (slot < 0 || taps <= 1) return;
@@ -133,6 +229,7 @@ __global__ void delta_conv_tail_kernel(const T* __restrict__ proj, long row_stri
     const int n = cu_q ? cu_q[b + 1] - cu_q[b] : 1;
     if (n <= 0) return;
     const bool has_past = positions[first] > 0;
+    if (rows > 0 && (!has_past || first / rows == (first + n - 1) / rows)) return;
     float* tail = conv_state + (long)slot * (taps - 1) * C;
     for (int c = blockIdx.y * blockDim.x + threadIdx.x; c < C; c += gridDim.y * blockDim.x) {
         float nv[MAX_TAPS];
@@ -310,30 +407,45 @@ int hyb_delta_prepare(const void* proj, long row_stride, int b_off, const void* 
     const int C = 2 * G * D + H * E;
     const size_t lds = 2 * (size_t)G * D * sizeof(float);
     if (lds > 64 * 1024) return 1;
-    const int vec8 = (G * D) % 8 == 0 && (H * E) % 8 == 0 && row_stride % 8 == 0 &&
-                     (size_t)proj % 16 == 0 && (size_t)conv_state % 16 == 0 && (size_t)vv % 16 == 0;
-#define PREP(TAPS)                                                                                 \
-    HYB_DISPATCH(dt, hipLaunchKernelGGL((delta_prepare_kernel<T, TAPS>), dim3(T_),                 \
-                                        dim3(C >= 2048 && T_ <= 1024 ? 1024 : 256), lds, s,        \
+    const int block = D <= 2048 ? 2048 / D * D : 0;       // channels per workgroup: whole heads, 8 a thread
+    const bool runs = taps >= 2 && taps <= 4 && D % 8 == 0 && block && (H * E) % 8 == 0 && row_stride % 8 == 0 &&
+                      ((size_t)proj | (size_t)conv_w | (size_t)conv_state | (size_t)qn | (size_t)kn | (size_t)vv) % 16 == 0;
+    // rows per workgroup: up to 16, as long as there are workgroups for every CU twice over (6100 rows of 4096
+    // channels: 8 rows 3 us more, 32 rows 12 us)
+    const int blocks = runs ? (C + block - 1) / block : 1;
+    int rows = 1;
+    while (cu_q && rows < 16 && T_ / (2 * rows) * blocks >= 512) rows *= 2;
+#define PREP_ROWS(TAPS)                                                                            \
+    HYB_DISPATCH(dt, hipLaunchKernelGGL((delta_prepare_rows_kernel<T, TAPS>),                      \
+                                        dim3((T_ + rows - 1) / rows, blocks), dim3(256), 0, s,     \
                                         (const T*)proj, row_stride, b_off, (const T*)a, a_row, DC, \
-                                        (const float*)conv_w, taps, (const float*)conv_b, ssd,     \
-                                        (const float*)a_log,                                       \
-                                        (const float*)dt_bias, (const float*)conv_state,           \
-                                        (const int*)cu_q, (const int*)positions, (const int*)slots,\
-                                        (const int*)row_seq, (float*)qn, (float*)kn, (float*)vv,   \
-                                        (float*)beta, (float*)decay, H, G, D, E, vec8))
-    if (taps == 4) PREP(4);
-    else if (taps == 3) PREP(3);
-    else if (taps == 2) PREP(2);
-    else PREP(0);
-#undef PREP
+                                        (const float*)conv_w, (const float*)conv_b, ssd,           \
+                                        (const float*)a_log, (const float*)dt_bias,                \
+                                        (float*)conv_state, (const int*)cu_q, (const int*)positions,\
+                                        (const int*)slots, (const int*)row_seq, (float*)qn,        \
+                                        (float*)kn, (float*)vv, (float*)beta, (float*)decay, T_,   \
+                                        rows, block, H, G, D, E))
+    if (runs && taps == 4) PREP_ROWS(4);
+    else if (runs && taps == 3) PREP_ROWS(3);
+    else if (runs) PREP_ROWS(2);
+    else
+        HYB_DISPATCH(dt, hipLaunchKernelGGL(delta_prepare_kernel<T>, dim3(T_),
+                                            dim3(C >= 2048 && T_ <= 1024 ? 1024 : 256), lds, s,
+                                            (const T*)proj, row_stride, b_off, (const T*)a, a_row, DC,
+                                            (const float*)conv_w, taps, (const float*)conv_b, ssd,
+                                            (const float*)a_log,
+                                            (const float*)dt_bias, (const float*)conv_state,
+                                            (const int*)cu_q, (const int*)positions, (const int*)slots,
+                                            (const int*)row_seq, (float*)qn, (float*)kn, (float*)vv,
+                                            (float*)beta, (float*)decay, H, G, D, E));
+#undef PREP_ROWS
     if (hipGetLastError() != hipSuccess) return 2;
-    if (taps > 1) {
+    if (taps > 1 && !(runs && !cu_q)) {
         HYB_DISPATCH(dt, hipLaunchKernelGGL(delta_conv_tail_kernel<T>, dim3(B, (C + 255) / 256),
                                             dim3(256), 0, s,
                                             (const T*)proj, row_stride, taps, (float*)conv_state,
                                             (const int*)cu_q, (const int*)positions,
-                                            (const int*)slots, C));
+                                            (const int*)slots, C, runs ? rows : 0));
     }
     return HYB_LAUNCH_OK();
 }

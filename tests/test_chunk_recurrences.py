@@ -129,3 +129,49 @@ def test_delta_rule(H, G, D, E, correct, fast):
         owned[cu[b]:cu[b + 1]] = s >= 0
     for x in (got[0], literal[0]):
         assert bool((x[~owned] == 0).all())
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,D,E,taps", [(2, 1, 8, 8, 4), (1, 1, 48, 40, 2), (3, 1, 16, 24, 3), (2, 2, 128, 64, 4)])
+@pytest.mark.parametrize("ssd,channel", [(False, False), (False, True), (True, False)])
+def test_delta_prepare_rows(dt, H, G, D, E, taps, ssd, channel):
+    """Several rows per workgroup: portions that start, end or lie inside its rows, shorter than the taps, with
+    and without a past, without a slot; then a step of single tokens on the tails it left."""
+    from minivllm_amd.ops import torch_seqmix as ref
+    g = torch.Generator().manual_seed(taps)
+    lens = [1, 2, 3, 700, 1, 0, 1500, 7, 9, 16, 2000, 5, 1, 2]
+    past = [5, 0, 9, 3, 0, 0, 0, 4, 0, 2, 8, 0, 3, 7]
+    slots = torch.tensor([3, 0, 12, 7, 13, 2, 1, 9, -1, 10, 11, 4, 5, 6], dtype=torch.int32)
+    cu = torch.tensor([0] + lens).cumsum(0).int()
+    T, C, N = int(cu[-1]), 2 * G * D + H * E, (H * D if channel else H)
+    pos = torch.cat([torch.arange(p, p + n) for n, p in zip(lens, past)]).int()
+    row_seq = torch.cat([torch.full((n,), b) for b, n in enumerate(lens)]).int()
+    conv_w, conv_b = torch.randn(C, taps, generator=g), torch.randn(C, generator=g) if ssd else None
+    a_log, dt_bias = torch.randn(H, generator=g), torch.randn(N, generator=g)
+    tail = torch.randn(14, taps - 1, C, generator=g)
+    width = -(-(C + H + N) // 8) * 8
+    steps = [(torch.randn(T, width, generator=g).to(dt), cu, pos, row_seq),
+             (torch.randn(14, width, generator=g).to(dt), None, torch.tensor([p + n for n, p in zip(lens, past)]).int(), None)]
+
+    def run(f, to):
+        st, outs = to(tail.clone()), []
+        for proj, c, p, rs in steps:
+            x = to(proj)
+            q, k, v, b, a = x[:, :C + H + N].split([G * D, G * D, H * E, H, N], -1)
+            n = x.shape[0]
+            args = [q.view(n, G, D), k.view(n, G, D), v.view(n, H, E), b, a, to(conv_w), to(a_log), to(dt_bias), st,
+                    None if c is None else to(c), to(p), to(slots)]
+            kw = dict(conv_bias=None if conv_b is None else to(conv_b), ssd=ssd)
+            if f is hk.delta_prepare:
+                kw["row_seq"] = None if rs is None else to(rs)
+            outs.append([y.cpu() for y in f(*args, **kw)])
+        return outs, st.cpu()
+
+    (w1, w2), wt = run(ref.delta_prepare, lambda x: x)
+    (g1, g2), gt = run(hk.delta_prepare, lambda x: x.cuda())
+    live = [(slots[row_seq.long()] >= 0), slots >= 0]
+    for got, want, ok in ((g1, w1, live[0]), (g2, w2, live[1])):
+        for x, y in zip(got, want):
+            # silu, softplus, exp and sums of up to 128 squares in fp32
+            torch.testing.assert_close(x[ok], y[ok], rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(gt, wt, rtol=0, atol=0)
