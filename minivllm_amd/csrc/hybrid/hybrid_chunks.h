@@ -103,4 +103,10 @@ long delta_chunks_bytes(const DeltaChunks& a);
 // correct: with the delta rule's correction term
 int delta_chunks(const DeltaChunks& a, bool correct, hipStream_t s);
 
+// hybrid_delta.hip: single next tokens of the delta rule with a decay per key channel; false when the sizes have
+// no instance
+bool channel_delta_step(const void* qn, const void* kn, const void* vv, const void* beta, const void* decay, void* state,
+                        const void* positions, const void* slots, void* o, long T_, int B, int H, int G, int D, int E,
+                        hipStream_t s, int* rc);
+
 }  // namespace hyb

@@ -614,6 +614,10 @@ int hyb_channel_delta_scan(const void* qn, const void* kn, const void* vv, const
                            const void* decay, void* state, const void* cu_q, const void* positions,
                            const void* slots, void* o, long T_, int B, int H, int G, int D, int E,
                            hipStream_t s) {
+    int rc = 0;
+    if (!cu_q && B > 0 && G > 0 && H % G == 0 && D > 0 && D <= 256 &&
+        channel_delta_step(qn, kn, vv, beta, decay, state, positions, slots, o, T_, B, H, G, D, E, s, &rc))
+        return rc;
     ScanArgs a{};
     a.q = qn; a.k = kn; a.v = vv; a.q_row = (long)G * D; a.k_row = (long)G * D; a.v_row = (long)H * E;
     a.a = decay; a.a_row = (long)H * D; a.beta = (const float*)beta; a.state = (float*)state;

@@ -175,3 +175,33 @@ def test_delta_prepare_rows(dt, H, G, D, E, taps, ssd, channel):
             # silu, softplus, exp and sums of up to 128 squares in fp32
             torch.testing.assert_close(x[ok], y[ok], rtol=1e-5, atol=1e-5)
     torch.testing.assert_close(gt, wt, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("H,G,D,E", [(4, 2, 128, 128), (2, 2, 8, 16), (3, 1, 100, 32), (2, 1, 256, 64), (1, 1, 33, 256), (2, 1, 64, 64)])
+@pytest.mark.parametrize("rule", ["delta", "channel", "plain"])
+def test_single_tokens(H, G, D, E, rule):
+    g = torch.Generator().manual_seed(D * E)
+    B = 7
+    slots = torch.tensor([2, 0, -1, 5, 4, 1, 3], dtype=torch.int32)
+    pos = torch.tensor([3, 0, 4, 9, 1, 0, 2], dtype=torch.int32)
+    q, k = (torch.randn(B, G, D, generator=g) for _ in range(2))
+    k = k / k.norm(dim=-1, keepdim=True)
+    v, beta = torch.randn(B, H, E, generator=g), torch.rand(B, H, generator=g)
+    decay = torch.rand(B, H, D, generator=g) if rule == "channel" else torch.rand(B, H, generator=g)
+    state = torch.randn(6, H, D, E, generator=g)
+    gs = state.cuda()
+    got = hk.delta_scan(q.cuda(), k.cuda(), v.cuda(), beta.cuda(), decay.cuda(), gs, None, pos.cuda(), slots.cuda(),
+                        rule != "plain").cpu()
+    qd, kd = (x.double().repeat_interleave(H // G, 1) for x in (q, k))
+    want, ws = torch.zeros(B, H, E, dtype=torch.float64), state.double()
+    for b, s in enumerate(slots.tolist()):
+        if s < 0:
+            continue
+        d = decay[b].double()
+        S = ws[s] * (int(pos[b]) > 0) * (d[:, :, None] if rule == "channel" else d[:, None, None])
+        u = beta[b].double()[:, None] * (v[b].double() - (torch.einsum("hde,hd->he", S, kd[b]) if rule != "plain" else 0))
+        ws[s] = S + kd[b][:, :, None] * u[:, None]
+        want[b] = torch.einsum("hde,hd->he", ws[s], qd[b])
+    # sums of up to 256 fp32 products
+    assert off(got, want) <= 256 * 2.0 ** -24 and off(gs, ws) <= 256 * 2.0 ** -24
+    assert bool((got[2] == 0).all())
