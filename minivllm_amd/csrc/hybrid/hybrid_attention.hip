@@ -180,8 +180,8 @@ sink_attention_rows_kernel(const T* __restrict__ q, long q_row, long q_head,
 }
 
 // ---------------------------------------------------------------------------------------
-// Prompt portions: tiles on the matrix cores, everything in fp32 (bfloat16 caches with rows of whole
-// 16-byte runs have a kernel of their own, hybrid_prompts.hip).
+// Prompt portions of any sizes and alignment: tiles on the matrix cores, everything in fp32 (rows of whole
+// 16-byte runs have kernels of their own, hybrid_prompts.hip).
 //
 // Workgroup = 4 waves = 128 consecutive queries of one (sequence, query head); a wave owns 32 of
 // them.  Keys are walked in tiles of 32 through LDS (K tile [32][DP+1], V tile [32][EP], both
@@ -597,10 +597,11 @@ int hyb_sink_attention_tiles(const void* q, long q_row, long q_head, const void*
     if (G <= 0 || H % G || !hyb_sink_attention_tiles_ok(D, E)) return 1;
 #define TILES_ARGS q, q_row, q_head, k_cache, v_cache, block_tables, max_blocks, block_size, cu_q, \
                    positions, sink, gate, gate_row, out, scale, nseq, seq0, max_q, H, G, D, E
-    // bfloat16 operands that can be copied to LDS as they are: 8 times faster at 8 x 1k tokens of 128-wide
-    // heads, 4 times at 2 x 300 (hybrid_prompts.hip)
-    if (dt == 0 && prompt_attention_ok(q, q_row, q_head, k_cache, v_cache, out, nseq, max_q, D, E, rule.v_stride))
-        return prompt_attention(TILES_ARGS, rule, s);
+    // operands in whole 16-byte runs: 8 times faster over bfloat16 at 8 x 1k tokens of 128-wide heads and 4
+    // times at 2 x 300; over float 2.3 times at 3 x 600 with a window (hybrid_prompts.hip)
+    if ((dt == 0 || dt == 2) &&
+        prompt_attention_ok(q, q_row, q_head, k_cache, v_cache, out, nseq, max_q, D, E, rule.v_stride, dt == 2))
+        return dt == 0 ? prompt_attention(TILES_ARGS, rule, s) : prompt_attention_f32(TILES_ARGS, rule, s);
 #define TILES_E(T, DP)                                                                       \
     do {                                                                                     \
         if (E <= 64) return launch_tiles<T, DP, 64>(TILES_ARGS, rule, s);                    \

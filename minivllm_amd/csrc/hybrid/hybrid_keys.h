@@ -68,14 +68,21 @@ inline bool pool_rule_ok(const KeyRule& r) {
                            r.pool_rows > 0 && r.pool_base > 0);
 }
 
-// hybrid_prompts.hip: prompt portions over bfloat16 caches (operands as hyb_sink_attention_tiles);
-// _ok: sizes in whole runs of eight numbers, 16-byte addresses, a grid that can be launched
+// hybrid_prompts.hip: prompt portions over bfloat16 and (_f32) float caches, operands as
+// hyb_sink_attention_tiles; _ok: sizes in whole runs of eight numbers, 16-byte addresses, a grid that can
+// be launched
 bool prompt_attention_ok(const void* q, long q_row, long q_head, const void* k_cache, const void* v_cache,
-                         const void* out, int nseq, int max_q, int D, int E, int v_stride);
+                         const void* out, int nseq, int max_q, int D, int E, int v_stride, bool f32);
 int prompt_attention(const void* q, long q_row, long q_head, const void* k_cache, const void* v_cache,
                      const void* block_tables, int max_blocks, int block_size, const void* cu_q,
                      const void* positions, const void* sink, const void* gate, long gate_row, void* out,
                      float scale, int nseq, int seq0, int max_q, int H, int G, int D, int E,
                      const KeyRule& rule, hipStream_t s);
+
+int prompt_attention_f32(const void* q, long q_row, long q_head, const void* k_cache, const void* v_cache,
+                         const void* block_tables, int max_blocks, int block_size, const void* cu_q,
+                         const void* positions, const void* sink, const void* gate, long gate_row, void* out,
+                         float scale, int nseq, int seq0, int max_q, int H, int G, int D, int E,
+                         const KeyRule& rule, hipStream_t s);
 
 }  // namespace hyb

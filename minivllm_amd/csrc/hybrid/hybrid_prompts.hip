@@ -23,7 +23,7 @@
 // would take 58 us and hold 16 bits of it; key tiles of 32 take 70 us, the two halves of a tile of 64
 // unrolled 73 us (registers spill).
 #include "hybrid_keys.h"
-#include "hybrid_tiles.h"
+#include "hybrid_chunks.h"
 
 using namespace hyb;
 
@@ -357,6 +357,250 @@ prompt_attention_kernel(PromptArgs a) {
 #endif
 }
 
+// The same over float caches: keys, values, queries and weights all fp32, each cut into three parts; a
+// product is the sum of the six products of parts that matter in 24 bits.  Key tiles of 32; K and V are
+// in registers a tile ahead and go to LDS as images of their parts, one buffer.  Exponentials are expf of
+// the difference, as in the general kernel.
+// Against the fp32 instruction (2.7 times the cycles) behind loads that nothing hid: 3 prompts of 300..611
+// tokens, window 256, 8 heads of 64: 90 -> 39 us with the fill of the output ahead of it, 2.0e-7 from 64 bits
+// instead of 2.7e-7.
+struct PromptArgs32 {
+    const float* q; long q_row, q_head;
+    const float *k_cache, *v_cache;
+    const int* tables; int max_blocks, block_size;
+    const int *cu_q, *positions;
+    const float* sink;
+    const float* gate; long gate_row;
+    float* out;
+    float scale;
+    int H, G, D, E, seq0;
+    KeyRule rule;
+};
+
+template <int DP, int EP, bool EXT>
+__global__ void __launch_bounds__(256, 1)
+prompt_attention_f32_kernel(PromptArgs32 a) {
+#ifdef __HIP_DEVICE_COMPILE__       // (the host pass only needs the launch stub)
+    constexpr int TK = 32, KS = DP / 16, NB = EP / 32;
+    constexpr int KT = TK * DP * 2, VT = TK * EP * 2;                         // bytes of a part's image
+    constexpr int KIT = TK * DP / 8 / 256, VIT = TK * EP / 8 / 256;           // runs of eight per thread
+    extern __shared__ __attribute__((aligned(256))) char smem[];
+    char *kim = smem, *vim = smem + 3 * KT;
+
+    const int H = a.H, hx = blockIdx.x;
+    const int h = H % 8 == 0 ? (hx & 7) * (H >> 3) + (hx >> 3) : hx;
+    const int b = blockIdx.y + a.seq0, tile_q0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * 128;
+    const int row0 = a.cu_q[b], qlen = a.cu_q[b + 1] - row0;
+    if (tile_q0 >= qlen) return;
+    const int start = a.positions[row0], G = a.G, g = h / (H / G);
+    const int* table = a.tables + (long)b * a.max_blocks;
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wq0 = tile_q0 + wave * 32, qi = wq0 + l32;
+    const bool qok = qi < qlen, wave_live = wq0 < qlen;
+    const int qpos = start + qi;
+    const float sc = EXT ? a.rule.head_scale(a.scale, h) : a.scale;
+    bf16x8 qf[KS][3];
+    {
+        const float* qp = a.q + (long)(row0 + min(qi, qlen - 1)) * a.q_row + (long)h * a.q_head;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const int d = 16 * s + 8 * half;
+            float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (d < a.D) load_run<float, 8>(qp + d, x);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] *= sc;
+            split8(x, qf[s]);
+        }
+    }
+    const KeyRule& rule = a.rule;
+    const int wg_ctx = start + min(qlen, tile_q0 + 128);
+    const int wave_first = start + wq0, wave_last = start + min(qlen - 1, wq0 + 31);
+    const int wg_lo = rule.first_key(start + tile_q0), wave_lo = rule.first_key(wave_first);
+    const int q_lo = rule.first_key(qpos), wave_top = rule.first_key(wave_last);
+    const int wg_nb = EXT ? rule.pooled_for(wg_ctx) : 0, wave_nb = EXT ? rule.pooled_for(wave_last + 1) : 0;
+    const int q_nb = EXT ? rule.pooled_for(qpos + 1) : 0;
+    const int ptiles = (wg_nb + TK - 1) / TK, first_tile = wg_lo / TK;
+    const int ktiles = min((rule.keep_first + TK - 1) / TK, first_tile);
+    const int n_tiles = ptiles + ktiles + (wg_ctx + TK - 1) / TK - first_tile;
+    auto tile_key = [&](int t) { return (t < ptiles ? t : t < ptiles + ktiles ? t - ptiles : t - ptiles - ktiles + first_tile) * TK; };
+    const bool whole = a.block_size % TK == 0;
+    typedef const __attribute__((address_space(4))) int* const_int_p;
+    auto page_of = [&](int t) { return *(const_int_p)(uintptr_t)(table + min(tile_key(t), wg_ctx - 1) / a.block_size); };
+    int page = page_of(0);
+    float kr[KIT][8], vr[VIT][8];
+    auto fetch = [&](int t) {
+        const int key0 = tile_key(t);
+        const bool pooled = EXT && t < ptiles;
+        const int lim = (pooled ? wg_nb : wg_ctx) - 1;               // (keys behind it repeat the last: masked)
+        const long base = (long)page * a.block_size + key0 % a.block_size - key0;
+        auto cache_row = [&](int j) -> long {
+            if (whole && !pooled) return base + j;
+            return pooled ? rule.pooled_row(table, j) : (long)table[j / a.block_size] * a.block_size + j % a.block_size;
+        };
+#pragma unroll
+        for (int i = 0; i < KIT; ++i) {
+            const int c = i * 256 + tid, d = c % (DP / 8) * 8;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) kr[i][j] = 0.f;
+            if (d < a.D) load_run<float, 8>(a.k_cache + (cache_row(min(key0 + c / (DP / 8), lim)) * G + g) * a.D + d, kr[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < VIT; ++i) {
+            const int c = i * 256 + tid, d = c % (EP / 8) * 8;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) vr[i][j] = 0.f;
+            if (d < a.E)
+                load_run<float, 8>(a.v_cache + (cache_row(min(key0 + c / (EP / 8), lim)) * G + g) * rule.v_stride + d, vr[i]);
+        }
+    };
+    auto stash = [&]() {
+#pragma unroll
+        for (int i = 0; i < KIT; ++i) {
+            const int c = i * 256 + tid, row = c / (DP / 8), ch = (c % (DP / 8)) ^ swizzle<DP>(row);
+            bf16x8 p[3];
+            split8(kr[i], p);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(kim + k * KT + row * DP * 2 + ch * 16) = p[k];
+        }
+#pragma unroll
+        for (int i = 0; i < VIT; ++i) {
+            const int c = i * 256 + tid, row = c / (EP / 8), ch = (c % (EP / 8)) ^ swizzle<EP>(row);
+            bf16x8 p[3];
+            split8(vr[i], p);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(vim + k * VT + row * EP * 2 + ch * 16) = p[k];
+        }
+    };
+    const int i16 = lane & 15, tr_row = 4 * half + (i16 >> 2);
+    const int tr_chunk = 2 * ((lane >> 4) & 1) + ((i16 & 3) >> 1);
+
+    f32x16 acc[NB];
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[n][e] = 0.f;
+    float m_run = NO_SINK_MAX, l_run = 0.f;
+    const float slope = rule.slopes ? rule.slopes[h] : 0.f;
+    fetch(0);
+    for (int t = 0; t < n_tiles; ++t) {
+        if (t > 0) __syncthreads();                                  // the images have been read
+        stash();
+        if (t + 1 < n_tiles) {
+            page = page_of(t + 1);
+            fetch(t + 1);
+        }
+        __syncthreads();
+        const int k0 = tile_key(t);
+        const bool pooled = EXT && t < ptiles;
+        const bool live = wave_live && (pooled ? k0 < wave_nb
+                                               : (k0 <= wave_last && (k0 < rule.keep_first || k0 + 32 > wave_lo)));
+        if (!live) continue;                                         // (uniform per wave)
+        f32x16 s_hi, s_lo;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) { s_hi[e] = 0.f; s_lo[e] = 0.f; }
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            bf16x8 kf[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                kf[k] = *reinterpret_cast<const bf16x8*>(kim + k * KT + l32 * DP * 2 + (((2 * s + half) ^ swizzle<DP>(l32)) << 4));
+            s_lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[2], qf[s][0], s_lo, 0, 0, 0);
+            s_lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[s][2], s_lo, 0, 0, 0);
+            s_lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[1], qf[s][1], s_lo, 0, 0, 0);
+            s_lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[1], qf[s][0], s_lo, 0, 0, 0);
+            s_lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[s][1], s_lo, 0, 0, 0);
+            s_hi = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[s][0], s_hi, 0, 0, 0);
+        }
+        float z[16], mt = -INFINITY;
+        const bool all_seen = pooled ? k0 + 32 <= rule.pooled_for(wave_first + 1) : k0 + 31 <= wave_first && k0 >= wave_top;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int key = k0 + (e & 3) + 8 * (e >> 2) + 4 * half;
+            float v = s_hi[e] + s_lo[e];
+            if (EXT) v = rule.capped(v);
+            if (!pooled) v -= slope * (float)(qpos - key);
+            if (!all_seen) {
+                const bool seen = pooled ? key < q_nb : (key <= qpos) & ((key >= q_lo) | (key < rule.keep_first));
+                v = seen ? v : -INFINITY;
+            }
+            z[e] = v;
+            mt = fmaxf(mt, v);
+        }
+        mt = fmaxf(mt, __shfl_xor(mt, 32, kWave));
+        if (!__all(mt - m_run <= 4.f)) {                             // the reference moves when a row outgrows it
+            const float m_new = fmaxf(m_run, mt), f = expf(m_run - m_new);
+            l_run *= f;
+#pragma unroll
+            for (int n = 0; n < NB; ++n) acc[n] *= f;
+            m_run = m_new;
+        }
+        bf16x8 p[2][3];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                x[j] = expf(z[8 * s + j] - m_run);
+                l_run += x[j];
+            }
+            split8(x, p[s]);
+        }
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                bf16x8 vf[3];
+                const int r0 = 16 * s + tr_row, ch = 4 * n + tr_chunk;
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    vf[k] = join(read_tr(vim + k * VT + r0 * EP * 2 + ((ch ^ swizzle<EP>(r0)) << 4) + (i16 & 1) * 8),
+                                 read_tr(vim + k * VT + (r0 + 8) * EP * 2 + ((ch ^ swizzle<EP>(r0 + 8)) << 4) + (i16 & 1) * 8));
+                acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[2], p[s][0], acc[n], 0, 0, 0);
+                acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0], p[s][2], acc[n], 0, 0, 0);
+                acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1], p[s][1], acc[n], 0, 0, 0);
+                acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1], p[s][0], acc[n], 0, 0, 0);
+                acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0], p[s][1], acc[n], 0, 0, 0);
+                acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0], p[s][0], acc[n], 0, 0, 0);
+            }
+    }
+    l_run += __shfl_xor(l_run, 32, kWave);
+    if (!qok) return;
+    float f;
+    if (a.sink) {
+        const float M = fmaxf(m_run, a.sink[h]);
+        f = expf(m_run - M);
+        f = f / (l_run * f + expf(a.sink[h] - M));
+    } else {
+        f = 1.f / l_run;
+    }
+    const long row = row0 + qi;
+    if (a.gate) f *= sigmoidf_(a.gate[row * a.gate_row + h]);
+    float* op = a.out + (row * H + h) * a.E;
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int e = 32 * n + 8 * r + 4 * half;
+            if (e < a.E)
+                *reinterpret_cast<float4*>(op + e) = make_float4(acc[n][4 * r] * f, acc[n][4 * r + 1] * f,
+                                                                 acc[n][4 * r + 2] * f, acc[n][4 * r + 3] * f);
+        }
+#endif
+}
+
+template <int DP, int EP>
+int launch_f32(const PromptArgs32& a, int nseq, int max_q, hipStream_t s) {
+    constexpr int lds = 3 * 32 * (DP + EP) * 2;
+    static_assert(lds <= 64 * 1024);
+    const dim3 grid(a.H, nseq, (max_q + 127) / 128);
+    if (a.rule.temps || a.rule.softcap > 0.f || a.rule.pool > 0)
+        hipLaunchKernelGGL((prompt_attention_f32_kernel<DP, EP, true>), grid, dim3(256), lds, s, a);
+    else
+        hipLaunchKernelGGL((prompt_attention_f32_kernel<DP, EP, false>), grid, dim3(256), lds, s, a);
+    return HYB_LAUNCH_OK();
+}
+
 template <int DP, int EP>
 int launch(const PromptArgs& a, int nseq, int max_q, hipStream_t s) {
     constexpr int TK = DP + EP <= 256 ? 64 : 32, lds = 2 * TK * (DP + EP) * 2;
@@ -374,7 +618,8 @@ int launch(const PromptArgs& a, int nseq, int max_q, hipStream_t s) {
 namespace hyb {
 
 bool prompt_attention_ok(const void* q, long q_row, long q_head, const void* k_cache, const void* v_cache,
-                         const void* out, int nseq, int max_q, int D, int E, int v_stride) {
+                         const void* out, int nseq, int max_q, int D, int E, int v_stride, bool f32) {
+    if (f32 && (D > 128 || E > 128)) return false;                    // (the queries' parts fill the registers)
     if (D < 8 || E < 8 || D % 8 || E % 8 || v_stride % 8 || D > 256 || E > 256 || (D > 128 && E > 128)) return false;
     if (((size_t)q | (size_t)k_cache | (size_t)v_cache | (size_t)out) % 16 || q_row % 8 || q_head % 8) return false;
     return nseq <= 65535 && (max_q + 127) / 128 <= 65535;             // (the grid)
@@ -399,6 +644,18 @@ int prompt_attention(const void* q, long q_row, long q_head, const void* k_cache
     PICK(256, 128);
 #undef PICK
     return 1;
+}
+
+int prompt_attention_f32(const void* q, long q_row, long q_head, const void* k_cache, const void* v_cache,
+                         const void* block_tables, int max_blocks, int block_size, const void* cu_q,
+                         const void* positions, const void* sink, const void* gate, long gate_row, void* out,
+                         float scale, int nseq, int seq0, int max_q, int H, int G, int D, int E,
+                         const KeyRule& rule, hipStream_t s) {
+    const PromptArgs32 a{(const float*)q, q_row, q_head, (const float*)k_cache, (const float*)v_cache,
+                         (const int*)block_tables, max_blocks, block_size, (const int*)cu_q, (const int*)positions,
+                         (const float*)sink, (const float*)gate, gate_row, (float*)out, scale, H, G, D, E, seq0, rule};
+    if (D <= 64) return E <= 64 ? launch_f32<64, 64>(a, nseq, max_q, s) : launch_f32<64, 128>(a, nseq, max_q, s);
+    return E <= 64 ? launch_f32<128, 64>(a, nseq, max_q, s) : launch_f32<128, 128>(a, nseq, max_q, s);
 }
 
 }  // namespace hyb

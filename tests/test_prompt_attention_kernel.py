@@ -1,4 +1,4 @@
-"""Prompt portions over bfloat16 caches (``csrc/hybrid/hybrid_prompts.hip``) against the plain form in
+"""Prompt portions over bfloat16 and float caches (``csrc/hybrid/hybrid_prompts.hip``) against the plain form in
 fp32 on CPU copies: head sizes at the edges of the instances, pages smaller and larger than a key
 tile, portions around a wave's and a workgroup's queries, every option; and the operands that the
 general tile kernel takes instead."""
@@ -16,14 +16,15 @@ PORTIONS = [1, 31, 2, 64, 33, 127, 129, 200]       # their last tokens are this 
 
 
 def close(got, want, top):
-    """Both round the same sum to bfloat16, whose numbers lie up to 2^-7 of their size apart, so one step;
+    """Both round the same sum (to bfloat16, whose numbers lie up to 2^-7 of their size apart: one step of it),
     and the fp32 sums of up to 300 products of weights <= 1 with values <= ``top`` differ themselves."""
+    step = 2.0 ** -7 if got.dtype == torch.bfloat16 else 0.0
     got, want = got.float(), want.float()
     d = (got - want).abs()
-    assert bool((d <= 2.0 ** -7 * torch.maximum(got.abs(), want.abs()) + 300 * 2.0 ** -22 * top).all()), float(d.max())
+    assert bool((d <= step * torch.maximum(got.abs(), want.abs()) + 300 * 2.0 ** -22 * top).all()), float(d.max())
 
 
-def step(G, D, E, bs, seed=0, pooled=0):
+def step(G, D, E, bs, seed=0, pooled=0, dt=torch.bfloat16):
     g = torch.Generator().manual_seed(seed)
     need = [-(-n // bs) for n in LENS]
     ids = torch.randperm(sum(need), generator=g).int()
@@ -34,7 +35,7 @@ def step(G, D, E, bs, seed=0, pooled=0):
         at += n
     rows = sum(need) * bs
     extra = sum(need) * -(-bs // pooled) if pooled else 0
-    k, v = (torch.randn((rows + extra) * G, n, generator=g).bfloat16() for n in (D, E))
+    k, v = (torch.randn((rows + extra) * G, n, generator=g).to(dt) for n in (D, E))
     cu_q = torch.tensor([0] + PORTIONS).cumsum(0).int()
     cu_k = torch.tensor([0] + LENS).cumsum(0).int()
     pos = torch.cat([torch.arange(L - n, L) for L, n in zip(LENS, PORTIONS)]).int()
@@ -55,12 +56,13 @@ def caches(k, v, rows, G, D, E, bs, pooled):
 @pytest.mark.parametrize("bs", [16, 64, 128])
 @pytest.mark.parametrize("opt", [dict(), dict(window=40, keep_first=5), dict(chunk=48), dict(slopes=True),
                                  dict(window=33, pool=8, temps=True, softcap=5.0)])
-def test_every_instance_and_option(H, G, D, E, bs, opt):
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_every_instance_and_option(H, G, D, E, bs, opt, dt):
     opt = dict(opt)
     pool = opt.get("pool", 0)
-    g, k, v, rows, tables, cu_q, cu_k, pos = step(G, D, E, bs, pooled=pool)
+    g, k, v, rows, tables, cu_q, cu_k, pos = step(G, D, E, bs, pooled=pool, dt=dt)
     T = int(cu_q[-1])
-    proj = torch.randn(T, H * D + H, generator=g).bfloat16()
+    proj = torch.randn(T, H * D + H, generator=g).to(dt)
     q, gate = proj[:, :H * D].view(T, H, D), proj[:, H * D:]
     sink = torch.randn(H, generator=g) if opt.get("softcap") or not opt else None
     if opt.pop("slopes", None):
@@ -76,22 +78,23 @@ def test_every_instance_and_option(H, G, D, E, bs, opt):
         if pool:
             o.update(k_pool=kp, v_pool=vp)
         return f(to(q), kc, vc, to(cu_q), to(cu_k), to(tables), D ** -0.5, None if sink is None else to(sink),
-                 to(gate), to(torch.zeros(T, H, E, dtype=torch.bfloat16)), **kw, **o)
+                 to(gate), to(torch.zeros(T, H, E, dtype=dt)), **kw, **o)
 
     want = call(ref.sink_attention_prefill, lambda x: x)
     got = call(hk.sink_attention_prefill, lambda x: x.cuda(), positions=pos.cuda(), max_q=max(PORTIONS)).cpu()
     close(got, want, float(v.abs().max()))
 
 
-@pytest.mark.parametrize("D,E,shift", [(64, 64, 1), (36, 64, 0), (64, 20, 0), (128, 128, 4)])
-def test_operands_of_the_general_kernel(D, E, shift):
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,E,shift", [(64, 64, 1), (36, 64, 0), (64, 20, 0), (128, 128, 2)])
+def test_operands_of_the_general_kernel(D, E, shift, dt):
     """Odd sizes and addresses stay with the kernel that takes any: same results."""
     H, G, bs = 4, 2, 64
-    g, k, v, rows, tables, cu_q, cu_k, pos = step(G, D, E, bs)
+    g, k, v, rows, tables, cu_q, cu_k, pos = step(G, D, E, bs, dt=dt)
     T = int(cu_q[-1])
-    flat = torch.randn(T * H * D + shift, generator=g).bfloat16()
+    flat = torch.randn(T * H * D + shift, generator=g).to(dt)
     kc, vc, _, _ = caches(k, v, rows, G, D, E, bs, 0)
-    out = torch.zeros(T, H, E, dtype=torch.bfloat16)
+    out = torch.zeros(T, H, E, dtype=dt)
     want = ref.sink_attention_prefill(flat[shift:].view(T, H, D), kc, vc, cu_q, cu_k, tables, D ** -0.5, None, None, out)
     got = hk.sink_attention_prefill(flat.cuda()[shift:].view(T, H, D), kc.cuda(), vc.cuda(), cu_q.cuda(), cu_k.cuda(),
                                     tables.cuda(), D ** -0.5, None, None, torch.zeros_like(out).cuda(),
