@@ -397,11 +397,46 @@ static int launch_tiles(const void* q, long q_row, long q_head, const void* k_ca
 // Decode rows at serving sizes: the context is split over workgroups and every K / V row is
 // read by 16 neighbouring lanes with 16-byte (bf16: EPL = 8 elements) loads, so a wave streams
 // four whole rows per step.  A 16-lane group walks its own keys (group kg of 16 per workgroup,
-// keys kg, kg + 16, ...) with a private running softmax for up to 4 query heads of the KV head;
-// the groups' partials meet in LDS, the workgroups' (one per context split) in a workspace that
-// `sink_attention_merge_kernel` folds together with the sink term and the gate.
+// keys kg, kg + 16, ...) with a private running softmax for NR query heads of the KV head, two keys per
+// trip, the next trip's rows on their way; the groups' partials meet in LDS, the workgroups' (one per
+// context split) in a workspace that `sink_attention_merge_kernel` folds together with the sink term
+// and the gate.
 // EPL / VPL: elements of a K / V row per lane (D = 16 EPL, E = 16 VPL).
-template <typename T, int EPL, int VPL, bool EXT>
+// Bound by the K / V stream and by what a workgroup does once.  64 rows of 512..1024 keys, 16 / 8 heads of 128,
+// bf16: 73 -> 51 us with the merge (210 MB), from registers for the heads there are, no division per key,
+// rows ahead that are not kept in the caches, one exponential per partial instead of one per output
+// column, and longer spans.  Four keys per trip: 54 us.
+template <typename T, int N> struct RawRun;          // N consecutive elements as loaded (used once: not cached)
+template <int N> struct RawRun<bf16_t, N> {
+    static constexpr int W = N >= 8 ? 4 : N / 2, M = N / 2 / W;       // words per load, loads
+    typedef __attribute__((ext_vector_type(W))) uint32_t vec;
+    vec v[M];
+    __device__ __forceinline__ void load(const bf16_t* p) {
+#pragma unroll
+        for (int i = 0; i < M; ++i) v[i] = __builtin_nontemporal_load(reinterpret_cast<const vec*>(p) + i);
+    }
+    __device__ __forceinline__ void widen(float* o) const {
+#pragma unroll
+        for (int i = 0; i < N / 2; ++i) {
+            o[2 * i] = __uint_as_float(v[i / W][i % W] << 16);
+            o[2 * i + 1] = __uint_as_float(v[i / W][i % W] & 0xffff0000u);
+        }
+    }
+};
+template <int N> struct RawRun<float, N> {
+    typedef __attribute__((ext_vector_type(4))) float vec;
+    vec v[N / 4];
+    __device__ __forceinline__ void load(const float* p) {
+#pragma unroll
+        for (int i = 0; i < N / 4; ++i) v[i] = __builtin_nontemporal_load(reinterpret_cast<const vec*>(p) + i);
+    }
+    __device__ __forceinline__ void widen(float* o) const {
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = v[i / 4][i % 4];
+    }
+};
+
+template <typename T, int EPL, int VPL, int NR, bool EXT>
 __global__ void __launch_bounds__(256)
 sink_attention_split_kernel(const T* __restrict__ q, long q_row, long q_head,
                             const T* __restrict__ k_cache, const T* __restrict__ v_cache,
@@ -410,58 +445,61 @@ sink_attention_split_kernel(const T* __restrict__ q, long q_row, long q_head,
                             float* __restrict__ ws, float scale, int H, int G, int splits,
                             KeyRule rule) {
     constexpr int D = 16 * EPL, E = 16 * VPL;
-    extern __shared__ float sm[];                 // [16 groups][RC][E + 2]
-    const int R = H / G, chunks = (R + RC - 1) / RC;
+    extern __shared__ float sm[];                 // [16 groups][NR][E + 2], [16 groups][NR]
+    const int R = H / G, chunks = (R + NR - 1) / NR;
     const int b = blockIdx.x, split = blockIdx.z;
-    const int g = blockIdx.y / chunks, h0 = g * R + (blockIdx.y % chunks) * RC;
-    const int nr = min(RC, g * R + R - h0);
+    const int g = blockIdx.y / chunks, h0 = g * R + (blockIdx.y % chunks) * NR;
+    const int nr = min(NR, g * R + R - h0);
     const int ctx = context_lens[b];
     const int tid = threadIdx.x, lane16 = tid & 15, kg = tid >> 4;
     const VisibleKeys vis(ctx, rule);
     const int span = ((vis.count + splits - 1) / splits + 15) & ~15;
     const int k_begin = split * span, k_end = min(vis.count, k_begin + span);
     const int* table = block_tables + (long)b * max_blocks;
+    const int shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctz(block_size) : -1;
 
-    float qf[RC][EPL], m[RC], l[RC], acc[RC][VPL], slope[RC];
+    float qf[NR][EPL], m[NR], l[NR], acc[NR][VPL], slope[NR];
 #pragma unroll
-    for (int r = 0; r < RC; ++r) {
-        if (r < nr) {
-            load_run<T, EPL>(q + b * q_row + (long)(h0 + r) * q_head + lane16 * EPL, qf[r]);
-            const float hs = EXT ? rule.head_scale(scale, h0 + r) : scale;
+    for (int r = 0; r < NR; ++r) {
+        const int h = h0 + min(r, nr - 1);        // (a head that is not there repeats the last: not written)
+        load_run<T, EPL>(q + b * q_row + (long)h * q_head + lane16 * EPL, qf[r]);
+        const float hs = EXT ? rule.head_scale(scale, h) : scale;
 #pragma unroll
-            for (int i = 0; i < EPL; ++i) qf[r][i] *= hs;
-            m[r] = sink ? sink[h0 + r] : NO_SINK_MAX;
-            slope[r] = rule.slopes ? rule.slopes[h0 + r] : 0.f;
-        } else {
-#pragma unroll
-            for (int i = 0; i < EPL; ++i) qf[r][i] = 0.f;
-            m[r] = 0.f;
-            slope[r] = 0.f;
-        }
+        for (int i = 0; i < EPL; ++i) qf[r][i] *= hs;
+        m[r] = sink ? sink[h] : NO_SINK_MAX;
+        slope[r] = rule.slopes ? rule.slopes[h] : 0.f;
         l[r] = 0.f;
 #pragma unroll
         for (int i = 0; i < VPL; ++i) acc[r][i] = 0.f;
     }
-    // two keys per trip: both rows' loads are in flight before the first one is used
-    for (int vj = k_begin + kg; vj < k_end; vj += 32) {
-        const bool two = vj + 16 < k_end;
-        const int j = vis.key(vj), j2 = two ? vis.key(vj + 16) : j;
-        const float dist[2] = {(float)(ctx - 1 - j), (float)(ctx - 1 - j2)};
-        const long slot = EXT ? vis.row(vj, table, block_size, rule)
-                              : (long)table[j / block_size] * block_size + j % block_size;
-        const long slot2 = !two ? slot : EXT ? vis.row(vj + 16, table, block_size, rule)
-                                             : (long)table[j2 / block_size] * block_size + j2 % block_size;
-        float kf[2][EPL], vf[2][VPL];
-        load_run<T, EPL>(k_cache + (slot * G + g) * (long)D + lane16 * EPL, kf[0]);
-        load_run<T, EPL>(k_cache + (slot2 * G + g) * (long)D + lane16 * EPL, kf[1]);
-        load_run<T, VPL>(v_cache + (slot * G + g) * (long)rule.v_stride + lane16 * VPL, vf[0]);
-        load_run<T, VPL>(v_cache + (slot2 * G + g) * (long)rule.v_stride + lane16 * VPL, vf[1]);
+    RawRun<T, EPL> kr[2];
+    RawRun<T, VPL> vr[2];
+    auto fetch = [&](int vj) {                    // keys vj, vj + 16 (behind the end: the last again)
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
-            if (x == 1 && !two) break;
+            const int v = min(vj + 16 * x, k_end - 1);
+            long slot;
+            if (EXT) slot = vis.row(v, table, block_size, rule);
+            else {
+                const int j = vis.key(v), p = shift >= 0 ? j >> shift : j / block_size;
+                slot = (long)table[p] * block_size + (j - p * block_size);
+            }
+            kr[x].load(k_cache + (slot * G + g) * (long)D + lane16 * EPL);
+            vr[x].load(v_cache + (slot * G + g) * (long)rule.v_stride + lane16 * VPL);
+        }
+    };
+    if (k_begin + kg < k_end) fetch(k_begin + kg);
+    for (int vj = k_begin + kg; vj < k_end; vj += 32) {
+        float kf[2][EPL], vf[2][VPL];
 #pragma unroll
-            for (int r = 0; r < RC; ++r) {
-                if (r >= nr) continue;
+        for (int x = 0; x < 2; ++x) { kr[x].widen(kf[x]); vr[x].widen(vf[x]); }
+        if (vj + 32 < k_end) fetch(vj + 32);
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            if (vj + 16 * x >= k_end) break;
+            const float dist = (float)(ctx - 1 - vis.key(vj + 16 * x));
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
                 float d = 0.f;
 #pragma unroll
                 for (int i = 0; i < EPL; ++i) d += kf[x][i] * qf[r][i];
@@ -469,7 +507,7 @@ sink_attention_split_kernel(const T* __restrict__ q, long q_row, long q_head,
                 d += __shfl_xor(d, 2, kWave);
                 d += __shfl_xor(d, 4, kWave);
                 d += __shfl_xor(d, 8, kWave);
-                d = (EXT ? rule.capped(d) : d) - slope[r] * dist[x];
+                d = (EXT ? rule.capped(d) : d) - slope[r] * dist;
                 if (d > m[r]) {                    // the running maximum moves: rescale (rare)
                     const float a = expf(m[r] - d);
                     l[r] *= a;
@@ -486,26 +524,31 @@ sink_attention_split_kernel(const T* __restrict__ q, long q_row, long q_head,
     }
     // the 16 groups' partials -> LDS -> one partial per (head, split)
     constexpr int PS = E + 2;
+    float* factor = sm + 16 * NR * PS;
 #pragma unroll
-    for (int r = 0; r < RC; ++r) {
-        float* dst = sm + (kg * RC + r) * PS;
+    for (int r = 0; r < NR; ++r) {
+        float* dst = sm + (kg * NR + r) * PS;
         if (lane16 == 0) { dst[0] = m[r]; dst[1] = l[r]; }
 #pragma unroll
         for (int i = 0; i < VPL; ++i) dst[2 + lane16 * VPL + i] = acc[r][i];
     }
     __syncthreads();
+    if (tid < 16 * NR) {                           // thread = (group, head): what its partial is multiplied by
+        const int r = tid % NR;
+        float M = sm[r * PS];
+        for (int k = 1; k < 16; ++k) M = fmaxf(M, sm[(k * NR + r) * PS]);
+        factor[tid] = expf(sm[tid * PS] - M);
+    }
+    __syncthreads();
     for (int c = tid; c < nr * PS; c += 256) {
         const int r = c / PS, x = c - r * PS;
-        float M = sm[r * PS];
-        for (int k = 1; k < 16; ++k) M = fmaxf(M, sm[(k * RC + r) * PS]);
         float v;
-        if (x == 0) v = M;
-        else {
+        if (x == 0) {
+            v = sm[r * PS];
+            for (int k = 1; k < 16; ++k) v = fmaxf(v, sm[(k * NR + r) * PS]);
+        } else {
             v = 0.f;
-            for (int k = 0; k < 16; ++k) {
-                const float* src = sm + (k * RC + r) * PS;
-                v += src[x] * expf(src[0] - M);
-            }
+            for (int k = 0; k < 16; ++k) v += sm[(k * NR + r) * PS + x] * factor[k * NR + r];
         }
         ws[(((long)b * H + h0 + r) * splits + split) * PS + x] = v;
     }
@@ -518,16 +561,23 @@ static int launch_split(const void* q, long q_row, long q_head, const void* k_ca
                         const void* gate, long gate_row, void* out, void* ws, float scale, int B,
                         int H, int G, int splits, KeyRule rule, hipStream_t s) {
     constexpr int E = 16 * VPL;
-    const int R = H / G, chunks = (R + RC - 1) / RC;
-    const size_t lds = 16 * RC * (E + 2) * sizeof(float);
-#define SPLIT_LAUNCH(EXT)                                                                         \
-    hipLaunchKernelGGL((sink_attention_split_kernel<T, EPL, VPL, EXT>), dim3(B, G * chunks, splits), \
-                       dim3(256), lds, s, (const T*)q, q_row, q_head, (const T*)k_cache,          \
+    const int R = H / G;
+#define SPLIT_LAUNCH_X(NR, EXT)                                                                   \
+    hipLaunchKernelGGL((sink_attention_split_kernel<T, EPL, VPL, NR, EXT>),                       \
+                       dim3(B, G * ((R + NR - 1) / NR), splits), dim3(256),                       \
+                       16 * NR * (E + 3) * sizeof(float), s, (const T*)q, q_row, q_head, (const T*)k_cache, \
                        (const T*)v_cache, (const int*)block_tables, max_blocks, block_size,       \
                        (const int*)context_lens, (const float*)sink, (float*)ws, scale, H, G, splits, \
                        rule)
+#define SPLIT_LAUNCH(EXT)                                                                         \
+    do {                                                                                          \
+        if (R == 1) SPLIT_LAUNCH_X(1, EXT);                                                       \
+        else if (R == 2) SPLIT_LAUNCH_X(2, EXT);                                                  \
+        else SPLIT_LAUNCH_X(4, EXT);                                                              \
+    } while (0)
     if (rule.temps || rule.softcap > 0.f || rule.pool > 0) SPLIT_LAUNCH(true); else SPLIT_LAUNCH(false);
 #undef SPLIT_LAUNCH
+#undef SPLIT_LAUNCH_X
     if (hipGetLastError() != hipSuccess) return 2;
     hipLaunchKernelGGL(sink_attention_merge_kernel<T>, dim3(B * H), dim3(E >= 128 ? 128 : 64), 0, s,
                        (const float*)ws, (const float*)sink, (const T*)gate, gate_row,

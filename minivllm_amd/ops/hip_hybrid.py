@@ -314,11 +314,13 @@ def _i32c(t):
     return t
 
 
-def decode_splits(batch: int, kv_heads: int, heads: int, max_context_len) -> int:
-    """Workgroups per (sequence, KV head group) of the split decode kernel: enough to fill the
-    256 CUs several times over, each with at least 128 keys of the longest context."""
+def decode_splits(batch: int, kv_heads: int, heads: int, max_context_len, wide: bool = False) -> int:
+    """Workgroups per (sequence, KV head group) of the split decode kernel: four per CU (``wide``, float
+    caches: eight; their rows keep a wave busy for longer), each with at least 128 keys of the longest
+    context.  64 sequences of 512..1024 keys, 8 KV heads: 51 us with four, 55 with eight, 75 with two; over
+    float 96 and 93."""
     groups = kv_heads * -(-(heads // kv_heads) // 4)
-    want = max(1, 2048 // max(batch * groups, 1))
+    want = max(1, (2048 if wide else 1024) // max(batch * groups, 1))
     room = max(1, (int(max_context_len) + 127) // 128) if max_context_len else 8
     return max(1, min(16, want, room))
 
@@ -342,7 +344,7 @@ def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale
             seen = min(int(seen), int(window) + int(keep_first) + (int(seen) // pool if pool else 0))
         if chunk and seen:
             seen = min(int(seen), int(chunk))
-        splits = decode_splits(B, G, H, seen)
+        splits = decode_splits(B, G, H, seen, es == 4)
         ws = torch.empty((B * H * splits * (E + 2),), dtype=torch.float32, device=q.device)
         if gate is not None:
             assert gate.stride(1) == 1 and gate.dtype == q.dtype
