@@ -20,7 +20,14 @@
 //
 // Workgroup = 4 waves.  RW = 4 (many rows): a wave per 32 rows, one key tile of 32 at a time for all.
 // RW = 2 (many rows, value rows too long for a wave's registers): two waves per 32 rows, each with
-// half of the value columns; both form the scores.
+// half of the value columns.  What bounds it is the chain tile -> scores -> weights -> values of a
+// workgroup.  With more workgroups than fit the card (PAIR) there are two of them on a CU: the waves
+// hold no more than 256 registers, 128 of accumulators and, as each takes half of the score product's
+// key columns, 72 (DP = 576) of queries; the halves of a score meet in LDS.  Otherwise both form the
+// whole score (18 products per tile for nothing, one workgroup on a CU, but a shorter chain).  8 prompts
+// of about 1024 tokens, 16 heads, R 512, P 64: 344 us with whole scores, 293 by halves, 236 with the
+// sequences' turn below, 182 with staging offsets in LDS and one key row read ahead instead of two (70
+// are the products alone at the instruction's rate).
 // RW = 1 (single next tokens of up to a few dozen heads): all waves share 32 rows; waves 0, 1 / 2, 3
 // take the left / right half of the value columns, waves 0, 2 / 1, 3 the even / odd key tiles; the
 // two halves of the keys meet in LDS at the end, the context may be split over workgroups too (fp32
@@ -49,22 +56,27 @@ struct LatentArgs {
     int H, R, P, window, splits;
 };
 
-template <int EP, int DP, int RW>
-__global__ void __launch_bounds__(256, EP >= 256 ? 1 : 2)
+template <int EP, int DP, int RW, bool PAIR>
+__global__ void __launch_bounds__(256, EP >= 256 && !PAIR ? 1 : 2)
 latent_attention_kernel(LatentArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__       // (the host pass only needs the launch stub)
-    static_assert(DP % 64 == 0 && EP % 64 == 0 && EP <= DP && (RW == 4 || RW == 2 || RW == 1));
+    static_assert((!PAIR || RW == 2) && DP % 64 == 0 && EP % 64 == 0 && EP <= DP && (RW == 4 || RW == 2 || RW == 1));
     constexpr int EW = RW == 4 ? 1 : 2;            // waves along the value columns
     constexpr int KW = 4 / RW / EW;                // key tiles per stage (= waves along the keys)
     constexpr int NB = EP / 32 / EW;               // 32-wide value blocks of a wave
-    constexpr int KS = DP / 16;                    // 16-wide steps of the score product
+    constexpr int KS = DP / 16 / (PAIR ? 2 : 1);   // 16-wide steps of a wave's score product
     constexpr int CPR = DP / 8;                    // 16-byte chunks of an LDS row
     constexpr int TILE = 32 * DP * 2;              // bytes
     constexpr int IT = CPR / 8;                    // 16-byte pieces per thread and tile
+    // PAIR: the staging offsets, 16 bits each, lie behind the buffers where two workgroups' LDS has the room
+    constexpr bool OFFS = PAIR && 2 * TILE + IT * 512 <= 80 * 1024;
     constexpr int SW = DP % 128 == 0 ? 16 : 8;     // chunks the swizzle permutes
     extern __shared__ __attribute__((aligned(256))) char smem[];
 
-    const int b = blockIdx.x, split = blockIdx.z;
+    // workgroups go to the 8 dies in turn: with the sequence as the fastest index alone, 8 sequences would
+    // stay on a die each, and the longest would be waited for (8 ragged prompts: 383 us for the layer, 327
+    // with a turn every 8 tiles; 326 with one every tile, 342 every 32, where a die's L2 sees fewer caches)
+    const int b = (blockIdx.x + blockIdx.y / 8) % gridDim.x, split = blockIdx.z;
     const int tile_row0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * (32 * RW);     // longest contexts first
     const int H = a.H, D = a.R + a.P;
     int row0, qlen, start;
@@ -96,7 +108,7 @@ latent_attention_kernel(LatentArgs a) {
         const uint16_t* pb = a.qb + (long)(row0 + tok) * a.qb_row + (long)head * a.qb_head;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
-            const int d = 16 * s + 8 * half;
+            const int d = 16 * (s + (PAIR ? ew * KS : 0)) + 8 * half;
             uint4 raw = make_uint4(0, 0, 0, 0);                     // columns from D on: zeros
             if (d < a.R) raw = *reinterpret_cast<const uint4*>(pa + d);
             else if (d < D) raw = *reinterpret_cast<const uint4*>(pb + d - a.R);
@@ -118,14 +130,24 @@ latent_attention_kernel(LatentArgs a) {
 
     // ---- staging: slot c of a tile's image (row c / CPR, chunk c % CPR) receives the cache chunk
     // that the swizzle puts there; chunks behind the row's end repeat chunk 0 (their queries are 0)
-    int s_row[IT], s_off[IT];
-#pragma unroll
-    for (int i = 0; i < IT; ++i) {
-        const int c = i * 256 + tid, row = c / CPR;
+    auto slot_of = [&](int i, int t, int& row, int& off) {
+        const int c = i * 256 + t;
+        row = c / CPR;
         int ch = (c - row * CPR) ^ swizzle<DP>(row);
         if (ch * 8 >= D) ch = 0;
-        s_row[i] = row;
-        s_off[i] = row * D * 2 + ch * 16;
+        off = row * D * 2 + ch * 16;
+    };
+    // (below 2^16: PAIR keeps them in LDS, or two to a register, as one to a register pushes others out)
+    uint16_t* const offs = reinterpret_cast<uint16_t*>(smem + 2 * TILE) + tid;
+    uint32_t s_off[OFFS ? 1 : PAIR ? (IT + 1) / 2 : IT];
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+        int row, off;
+        slot_of(i, tid, row, off);
+        if constexpr (OFFS) offs[i * 256] = (uint16_t)off;
+        else if constexpr (!PAIR) s_off[i] = off;
+        else if (i & 1) s_off[i / 2] |= (uint32_t)off << 16;
+        else s_off[i / 2] = off;
     }
     const bool uniform_rows = (a.block_size & 31) == 0;             // a tile's rows are consecutive
     // block ids of a stage's tiles, through the scalar unit (the table is read-only here) and a stage
@@ -138,6 +160,12 @@ latent_attention_kernel(LatentArgs a) {
             ids[k] = *(const_int_p)(uintptr_t)(table + min((t0 + k) * 32, n_keys - 1) / a.block_size);
     };
     auto stage = [&](int t0, int buf) {
+        int me = tid;
+        if constexpr (PAIR) {                       // (worked out or unpacked ahead of the loop they cost registers)
+            asm volatile("" : "+v"(me));
+#pragma unroll
+            for (int i = 0; i < (OFFS ? 0 : (IT + 1) / 2); ++i) asm volatile("" : "+v"(s_off[i]));
+        }
 #pragma unroll
         for (int k = 0; k < KW; ++k) {
             const int key0 = (t0 + k) * 32;
@@ -150,15 +178,20 @@ latent_attention_kernel(LatentArgs a) {
                 const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
                     const_cast<uint16_t*>(src), 0, bytes, 0x00020000);
 #pragma unroll
-                for (int i = 0; i < IT; ++i)
+                for (int i = 0; i < IT; ++i) {
+                    const int off = OFFS ? offs[i * 256] : !PAIR ? s_off[i]
+                                  : i & 1 ? s_off[i / 2] >> 16 : s_off[i / 2] & 0xffff;
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                        rsrc, (__attribute__((address_space(3))) void*)(dst + i * 4096), 16, s_off[i], 0, 0, 0);
+                        rsrc, (__attribute__((address_space(3))) void*)(dst + i * 4096), 16, off, 0, 0, 0);
+                }
             } else {
 #pragma unroll
                 for (int i = 0; i < IT; ++i) {
-                    const int key = min(key0 + s_row[i], n_keys - 1);
+                    int r0, off;
+                    slot_of(i, me, r0, off);
+                    const int key = min(key0 + r0, n_keys - 1);
                     const long row = (long)table[key / a.block_size] * a.block_size + key % a.block_size;
-                    const char* src = reinterpret_cast<const char*>(a.cache) + row * D * 2 + (s_off[i] - s_row[i] * D * 2);
+                    const char* src = reinterpret_cast<const char*>(a.cache) + row * D * 2 + (off - r0 * D * 2);
                     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                                      (__attribute__((address_space(3))) void*)(dst + i * 4096), 16, 0, 0);
                 }
@@ -168,21 +201,24 @@ latent_attention_kernel(LatentArgs a) {
 
     // ---- LDS addresses of this wave's fragments inside a buffer (one tile at kw)
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)smem + kw * TILE;
-    uint32_t k_addr[SW / 2];                        // row l32, chunk 2 s + half: distinct for s < SW / 2
-#pragma unroll
-    for (int s = 0; s < SW / 2; ++s) k_addr[s] = lds0 + l32 * (DP * 2) + (((2 * s + half) ^ swizzle<DP>(l32)) << 4);
+    // row l32, chunk 2 s + half: distinct for s < SW / 2.  (PAIR works them out anew from tile to tile:
+    // addresses that stay in registers would push others out to memory.)
+    auto k_address = [&](int s, int ln) {
+        const int r = ln & 31, hf = (ln >> 5) & 1;
+        return lds0 + r * (DP * 2) + (((2 * (s + (PAIR ? ew * KS : 0)) + hf) ^ swizzle<DP>(r)) << 4);
+    };
     // transposed reads: 16 lanes take 4 key rows x 16 columns and return 4 keys of one column each
     constexpr int NA = NB < SW / 4 ? NB : SW / 4;   // value blocks with addresses of their own
-    const int i16 = lane & 15, tr_row = 4 * half + (i16 >> 2);
-    const int tr_chunk = 2 * ((lane >> 4) & 1) + ((i16 & 3) >> 1);
-    uint32_t v_addr[NA][2];
+    auto v_address = [&](int n, int hi, int ln) {
+        const int i16 = ln & 15, row = 4 * ((ln >> 5) & 1) + (i16 >> 2) + 8 * hi;
+        const int ch = 4 * (ew * NB + n) + 2 * ((ln >> 4) & 1) + ((i16 & 3) >> 1);
+        return lds0 + row * (DP * 2) + ((ch ^ swizzle<DP>(row)) << 4) + (i16 & 1) * 8;
+    };
+    uint32_t k_addr[SW / 2], v_addr[NA][2];
 #pragma unroll
-    for (int n = 0; n < NA; ++n)
+    for (int s = 0; s < SW / 2; ++s) k_addr[s] = k_address(s, lane);
 #pragma unroll
-        for (int hi = 0; hi < 2; ++hi) {
-            const int row = tr_row + 8 * hi, ch = 4 * (ew * NB + n) + tr_chunk;
-            v_addr[n][hi] = lds0 + row * (DP * 2) + ((ch ^ swizzle<DP>(row)) << 4) + (i16 & 1) * 8;
-        }
+    for (int n = 0; n < NA; ++n) { v_addr[n][0] = v_address(n, 0, lane); v_addr[n][1] = v_address(n, 1, lane); }
 
     f32x16 acc[NB];
 #pragma unroll
@@ -203,19 +239,24 @@ latent_attention_kernel(LatentArgs a) {
         const bool live = wave_live && t + kw < t_end && key0 <= w_last &&
                           (a.window <= 0 || key0 + 31 > w_first - a.window);       // (uniform per wave)
         bf16x8 p_hi[2], p_lo[2];
-        if (t + KW < t_end) {                           // lands behind this tile's products
-            stage(t + KW, buf ^ 1);
-            if (t + 2 * KW < t_end) fetch_ids(t + 2 * KW);
-        }
+        auto stage_next = [&]() {                       // lands behind this tile's products
+            if (t + KW < t_end) {
+                stage(t + KW, buf ^ 1);
+                if (t + 2 * KW < t_end) fetch_ids(t + 2 * KW);
+            }
+        };
+        if constexpr (!PAIR) stage_next();
+        f32x16 s_acc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s_acc[e] = 0.f;
         if (live) {
-            f32x16 s_acc;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) s_acc[e] = 0.f;
             // (inline asm as for the value reads below: KA row reads in flight, no more registers)
-            constexpr int KA = 4;
+            constexpr int KA = PAIR ? 1 : 4;
             uint32_t ka[SW / 2];
+            int ln = lane;
+            if constexpr (PAIR) asm volatile("" : "+v"(ln));
 #pragma unroll
-            for (int s = 0; s < SW / 2; ++s) ka[s] = k_addr[s] + buf * (KW * TILE);
+            for (int s = 0; s < SW / 2; ++s) ka[s] = (PAIR ? k_address(s, ln) : k_addr[s]) + buf * (KW * TILE);
             s16x8 kf[KS];
             auto read_k = [&](auto ic) {
                 constexpr int i = decltype(ic)::value;
@@ -239,6 +280,30 @@ latent_attention_kernel(LatentArgs a) {
                 s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, x), qf[i], s_acc, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);    // (products sunk below later reads cost registers)
             });
+        }
+        if constexpr (PAIR) {
+            // the two halves of a score are added through the buffer that the next tile goes to afterwards
+            // (both waves of a pair are live or neither is)
+            float* x = reinterpret_cast<float*>(smem + (buf ^ 1) * (KW * TILE));
+            if (live) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    *reinterpret_cast<float4*>(x + ((wave * 4 + e) * 64 + lane) * 4) =
+                        make_float4(s_acc[4 * e], s_acc[4 * e + 1], s_acc[4 * e + 2], s_acc[4 * e + 3]);
+            }
+            __syncthreads();
+            if (live) {
+                const int other = rw + RW * (1 - ew);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float4 y = *reinterpret_cast<const float4*>(x + ((other * 4 + e) * 64 + lane) * 4);
+                    s_acc[4 * e] += y.x; s_acc[4 * e + 1] += y.y; s_acc[4 * e + 2] += y.z; s_acc[4 * e + 3] += y.w;
+                }
+            }
+            __syncthreads();
+            stage_next();
+        }
+        if (live) {
             // lane: query row l32, keys key0 + (e & 3) + 8 (e >> 2) + 4 half
             const bool all_seen = key0 + 31 <= w_first && (a.window <= 0 || w_last - key0 < a.window);
             const int oldest = a.window > 0 ? qpos - a.window : -1;
@@ -287,10 +352,12 @@ latent_attention_kernel(LatentArgs a) {
             constexpr int STEPS = 2 * NB, AHEAD = STEPS < 4 ? STEPS : 4;
             s16x4 lo4[STEPS], hi4[STEPS];
             uint32_t va[NA][2];
+            int ln = lane;
+            if constexpr (PAIR) asm volatile("" : "+v"(ln));
 #pragma unroll
             for (int n = 0; n < NA; ++n) {
-                va[n][0] = v_addr[n][0] + buf * (KW * TILE);
-                va[n][1] = v_addr[n][1] + buf * (KW * TILE);
+                va[n][0] = (PAIR ? v_address(n, 0, ln) : v_addr[n][0]) + buf * (KW * TILE);
+                va[n][1] = (PAIR ? v_address(n, 1, ln) : v_addr[n][1]) + buf * (KW * TILE);
             }
             auto read = [&](auto ic) {
                 constexpr int i = decltype(ic)::value, n = i >> 1, s = i & 1;
@@ -393,23 +460,33 @@ latent_attention_kernel(LatentArgs a) {
 #endif
 }
 
+// Workgroups above which halves of scores pay: two for each of the 256 CUs, fewer run at once anyway.  Layer
+// with 16 heads, R 512, P 64, whole scores / halves: 432 workgroups 97.6 / 103.0 us, 512 124.7 / 125.7 and
+// 190.4 / 193.2 (two sequences, one), 750 119.8 / 105.4, 768 173.9 / 144.1, 1024 181.1 / 152.3 (P 128: 195.4 /
+// 182.6; pages of 16 rows: 263.0 / 211.1).
+constexpr long PAIR_FROM = 512;
+
 template <int EP, int DP>
 int launch(const LatentArgs& a, int nseq, int max_rows, bool wide, hipStream_t s) {
     constexpr int tile = 32 * DP * 2;
-#define LATENT(RW)                                                                                 \
+#define LATENT(RW, PAIR)                                                                           \
     do {                                                                                           \
-        constexpr int lds = 2 * (RW == 1 ? 2 : 1) * tile;                                          \
+        constexpr int lds = 2 * (RW == 1 ? 2 : 1) * tile +                                         \
+            (PAIR && 2 * tile + DP / 64 * 512 <= 80 * 1024 ? DP / 64 * 512 : 0);                   \
         static_assert(lds <= 160 * 1024 && (RW > 1 || (EP / 2 + 4) * 256 <= lds));                  \
         if (lds > 64 * 1024) {                                                                     \
             static const hipError_t once = hipFuncSetAttribute(                                    \
-                (const void*)latent_attention_kernel<EP, DP, RW>,                                  \
+                (const void*)latent_attention_kernel<EP, DP, RW, PAIR>,                                  \
                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);                                  \
             if (once != hipSuccess) return 2;                                                      \
         }                                                                                          \
         const dim3 grid(nseq, (max_rows + 32 * RW - 1) / (32 * RW), a.splits);                     \
-        hipLaunchKernelGGL((latent_attention_kernel<EP, DP, RW>), grid, dim3(256), lds, s, a);      \
+        hipLaunchKernelGGL((latent_attention_kernel<EP, DP, RW, PAIR>), grid, dim3(256), lds, s, a);      \
     } while (0)
-    if (!wide) LATENT(1); else if constexpr (EP > 256) LATENT(2); else LATENT(4);
+    if (!wide) LATENT(1, false);
+    else if constexpr (EP <= 256) LATENT(4, false);
+    else if ((long)nseq * ((max_rows + 63) / 64) > PAIR_FROM) LATENT(2, true);
+    else LATENT(2, false);
 #undef LATENT
     return HYB_LAUNCH_OK();
 }
