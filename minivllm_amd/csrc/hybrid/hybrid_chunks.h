@@ -1,7 +1,9 @@
 // Recurrences over prompt portions in chunks of tokens on the matrix cores: the matrix LSTM's
 // (hybrid_chunks.hip) and the delta rule's (hybrid_delta_chunks.hip); what their kernels share.
 //
-// An fp32 operand of a bf16 product is cut into three parts of eight bits, which hold all of its 24.
+// An fp32 operand of a bf16 product is cut into three parts of eight bits, which hold all of its 24.  The parts are
+// rounded, not cut off: what they leave is half as large and of either sign, so that the three products of parts
+// that a product of two such operands leaves out (2^-27 of it in the mean, 2^-23 at most) do not add up over a sum.
 #pragma once
 #include "hybrid_tiles.h"
 
@@ -9,11 +11,17 @@ namespace hyb {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-// the upper halves of x and y side by side: eight bits of each
-__device__ __forceinline__ uint32_t upper(float x, float y) {
-    return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302);
+// x and y rounded to eight bits each, side by side
+__device__ __forceinline__ uint32_t rounded(float x, float y) {
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
 }
-__device__ __forceinline__ float rest(float x) { return x - __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+// what the two parts `w` leave of x and y (exact)
+__device__ __forceinline__ void rest(uint32_t w, float& x, float& y) {
+    x -= __uint_as_float(w << 16);
+    y -= __uint_as_float(w & 0xffff0000u);
+}
 
 // eight numbers as three bfloat16 fragments whose sum they are
 __device__ __forceinline__ void split8(const float* x, bf16x8* p) {
@@ -23,8 +31,8 @@ __device__ __forceinline__ void split8(const float* x, bf16x8* p) {
         float u = x[2 * j], v = x[2 * j + 1];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            w[k][j] = upper(u, v);
-            if (k < 2) { u = rest(u); v = rest(v); }
+            w[k][j] = rounded(u, v);
+            if (k < 2) rest(w[k][j], u, v);
         }
     }
 #pragma unroll
@@ -48,11 +56,13 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
 // four numbers of a lane as three runs of bfloat16; at(k): where part k goes
 template <class F>
 __device__ __forceinline__ void put_parts(f32x4 x, F&& at) {
+    float a = x[0], b = x[1], c = x[2], d = x[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        *reinterpret_cast<uint2*>(at(k)) = make_uint2(upper(x[0], x[1]), upper(x[2], x[3]));
-#pragma unroll
-        for (int r = 0; r < 4; ++r) x[r] = rest(x[r]);
+        const uint2 w = make_uint2(rounded(a, b), rounded(c, d));
+        *reinterpret_cast<uint2*>(at(k)) = w;
+        rest(w.x, a, b);
+        rest(w.y, c, d);
     }
 }
 

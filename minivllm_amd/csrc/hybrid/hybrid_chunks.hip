@@ -11,8 +11,7 @@
 //   A = (Q K^T) o W;  O = diag(c) Q S_0 + A V;  n . q = c_t n_0 . q_t + sum_i A_ti
 //   S_end = c_end S_0 + K^T diag(W_end) V,  n_end = c_end n_0 + K^T W_end
 //
-// Every factor is a product of the same a and b the recurrence multiplies by, all <= 1 except for the
-// first token's b: no quotients, no logarithms of products.  W comes from the products inside blocks of 16
+// Every factor is a product of the same a and b the recurrence multiplies by, all <= 1: no quotients, no logarithms of products.  W comes from the products inside blocks of 16
 // tokens: in a pair of different blocks it is (a .. to t inside its block) (whole blocks between) (a .. from
 // i to its block's end) b_i, on the diagonal the running product.
 //
@@ -158,7 +157,10 @@ mlstm_chunks_kernel(MlstmChunks a) {
         }
         m_run = before;
         const float m = fmaxf(M, m0 + F), mp = from_left<1>(m, m0);
-        const float fa = ok ? expf(f + mp - m) : 1.f, fb = ok ? expf(i - m) : 0.f;
+        // (of the difference that decides the maximum, as in the recurrence, and not of m, whose own rounding would
+        // come on top; not by fminf, which would lose a NaN)
+        const float x = f + mp - i;
+        const float fa = ok ? expf(x >= 0.f ? 0.f : x) : 1.f, fb = ok ? expf(x <= 0.f ? 0.f : -x) : 0.f;
         float pre = fa, suf = fa;
         static_for<0, 4>([&](auto dc) {
             constexpr int d = 1 << decltype(dc)::value;
@@ -186,11 +188,12 @@ mlstm_chunks_kernel(MlstmChunks a) {
         g.wl[lane] = G.wl;
         g.em[lane] = G.em;
         if (l16 == 15) g.blk[q4] = G.pre;
-        float x = G.wl;
+        float x = G.wl, y = 0.f;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            g.wp[k][lane] = (uint16_t)(__float_as_uint(x) >> 16);
-            x = rest(x);
+            const uint32_t w = rounded(x, y);
+            g.wp[k][lane] = (uint16_t)w;
+            rest(w, x, y);
         }
     };
     // what was fetched last into LDS

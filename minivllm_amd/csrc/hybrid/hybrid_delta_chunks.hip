@@ -22,8 +22,11 @@
 // rows are on their way all the while.
 //
 // Everything is fp32 here, so every operand is cut into three parts of eight bits and a product is the sum
-// of the six products of parts that matter in 24 bits, on v_mfma_f32_16x16x32_bf16 with fp32 sums (2.7
-// times the rate of the fp32 instruction).
+// of the six largest products of parts, on v_mfma_f32_16x16x32_bf16 with fp32 sums (2.7 times the rate of the
+// fp32 instruction).  An instruction rounds its sum once, so the small products are summed apart from, or
+// ahead of, the large one.  From 64 bits, 4 portions of 1024 tokens, decays of a trained range: outputs 1.0e-7,
+// state 6.9e-8, against 1.1e-7 and 7.2e-8 token by token (2.3e-7 and 1.4e-7 with parts cut off and one sum for
+// all products).
 //
 // 8 portions of 512..1024 tokens, 16 / 8 heads of 128: 54 + 140 us, against 645 us token by token.  The walk
 // takes 9 us a chunk of 64 columns; its six phases between barriers use the matrix units, the
@@ -55,7 +58,7 @@ __device__ __forceinline__ void load8(__amdgpu_buffer_rsrc_t b, int off, float* 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_of(const float* p, int row, int nt, int width) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, ((nt - 1) * row + width) * 4, 0x00020000);
 }
-// sum of the six products of parts, the small ones first
+// sum of the six products of parts that reach 24 bits, the small ones first
 __device__ __forceinline__ f32x4 mfma6(const bf16x8* a, const bf16x8* b, f32x4 c) {
     c = mfma(a[2], b[0], c);
     c = mfma(a[0], b[2], c);
@@ -64,6 +67,20 @@ __device__ __forceinline__ f32x4 mfma6(const bf16x8* a, const bf16x8* b, f32x4 c
     c = mfma(a[0], b[1], c);
     return mfma(a[0], b[0], c);
 }
+// A product of fp32 operands: the six products of parts that reach 24 bits.  The small five have a sum of
+// their own, so that a step rounds the result once and not six times.
+struct Product {
+    f32x4 hi = {0.f, 0.f, 0.f, 0.f}, lo = {0.f, 0.f, 0.f, 0.f};
+    __device__ __forceinline__ void add(const bf16x8* a, const bf16x8* b) {
+        lo = mfma(a[2], b[0], lo);
+        hi = mfma(a[0], b[0], hi);
+        lo = mfma(a[0], b[2], lo);
+        lo = mfma(a[1], b[1], lo);
+        lo = mfma(a[1], b[0], lo);
+        lo = mfma(a[0], b[1], lo);
+    }
+    __device__ __forceinline__ f32x4 sum() const { return hi + lo; }
+};
 #endif
 
 template <int DP, bool DELTA>
@@ -118,15 +135,18 @@ delta_weights_kernel(DeltaChunks a) {
             qk[kb2] = kk[kb2];
             if (kb2 > tb) continue;
             const int row = 16 * kb2 + l16;
+            Product pk, pq;
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
                 bf16x8 x[3];
 #pragma unroll
                 for (int p = 0; p < 3; ++p)
                     x[p] = *reinterpret_cast<const bf16x8*>(kparts + p * C * DP * 2 + row * DP * 2 + (((4 * s + q4) ^ swizzle<DP>(row)) << 4));
-                if (DELTA) kk[kb2] = mfma6(x, kf[s], kk[kb2]);
-                qk[kb2] = mfma6(x, qf[s], qk[kb2]);
+                if (DELTA) pk.add(x, kf[s]);
+                pq.add(x, qf[s]);
             }
+            kk[kb2] = pk.sum();
+            qk[kb2] = pq.sum();
         }
     }
     for (int r = 0; r < R; ++r) {
@@ -334,6 +354,12 @@ delta_chunks_kernel(DeltaChunks a) {
     const int t = 16 * tb + l16;
     float raw[KS][8];
     bf16x8 xp[KS][3];                                // the chunk's k (or q) rows as operand, in parts
+    // (addresses worked out ahead of the loop, for every phase, cost the registers that the products need: each phase
+    // works its own out)
+    auto again = [](int x) {
+        asm volatile("" : "+v"(x));
+        return x;
+    };
     auto fetch = [&](int ch) {
         const int nt = min(C, n - ch * C);
         const __amdgpu_buffer_rsrc_t rows = rows_of((update ? a.k : a.q) + ((long)first + ch * C) * G * D + (long)g * D, G * D, nt, D);
@@ -373,13 +399,35 @@ delta_chunks_kernel(DeltaChunks a) {
     };
     // the parts of columns 16 x .. of an image as operand: rows row0 + 4 (quarter of the wave's lanes) + j, then
     // those `step` behind them
-    auto get_cols = [&](char (*im)[C * ROW], int x, int row0, int step, bf16x8* p) {
-        const int r0 = row0 + (l16 >> 2), r1 = r0 + step, ch = 2 * x + ((l16 & 3) >> 1);
+    auto get_cols = [&](char (*im)[C * ROW], int ln, int x, int row0, int step, bf16x8* p) {
+        const int l16 = ln & 15, r0 = row0 + 4 * (ln >> 4) + (l16 >> 2), r1 = r0 + step, ch = 2 * x + ((l16 & 3) >> 1);
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             p[k] = join(read_tr(im[k] + place(r0, ch) + (l16 & 1) * 8), read_tr(im[k] + place(r1, ch) + (l16 & 1) * 8));
     };
     constexpr int NE = 2 * ET;                       // 16-wide blocks of columns
+    // the fragments m (of M or A) times columns 16 x .. of an image: the small products of parts first, so that
+    // two steps round the whole sum
+    auto chunk_product = [&](char (*im)[C * ROW], int ln, int x, const bf16x8 (*m)[3]) {
+        bf16x8 p[2][3];
+        f32x4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            if (2 * s <= tb) {
+                get_cols(im, ln, x, 32 * s, 16, p[s]);
+                y = mfma(p[s][2], m[s][0], y);
+                y = mfma(p[s][0], m[s][2], y);
+                y = mfma(p[s][1], m[s][1], y);
+                y = mfma(p[s][1], m[s][0], y);
+                y = mfma(p[s][0], m[s][1], y);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+            if (2 * s <= tb) y = mfma(p[s][0], m[s][0], y);
+        __builtin_amdgcn_sched_barrier(0);
+        return y;
+    };
 
     const int nchunks = (n + C - 1) / C;
     fetch(0);
@@ -411,21 +459,24 @@ delta_chunks_kernel(DeltaChunks a) {
         const float bt = !DELTA && update && t < left ? a.beta[(t0 + t) * H + h] : 0.f;
         __syncthreads();                                     // the images of k and of the state are there
         f32x4 X[NE];                                         // K S (Q S)
+        if (DELTA || !update) {
+            const int ln = again(lane), l16 = ln & 15, q4 = ln >> 4;
 #pragma unroll
-        for (int x = 0; x < NE; ++x) X[x] = {0.f, 0.f, 0.f, 0.f};
-        if (DELTA || !update)
+            for (int x = 0; x < NE; ++x) {
+                Product p;
 #pragma unroll
-            for (int s = 0; s < KS; ++s)
-#pragma unroll
-                for (int x = 0; x < NE; ++x) {
+                for (int s = 0; s < KS; ++s) {
                     const int row = 16 * x + l16;
                     bf16x8 sf[3];
 #pragma unroll
                     for (int k = 0; k < 3; ++k)
                         sf[k] = *reinterpret_cast<const bf16x8*>(L.s[k] + row * DP * 2 + (((4 * s + q4) ^ swizzle<DP>(row)) << 4));
-                    X[x] = mfma6(sf, xp[s], X[x]);
+                    p.add(sf, xp[s]);
                     __builtin_amdgcn_sched_barrier(0);       // (reads hoisted over the products cost registers)
                 }
+                X[x] = p.sum();
+            }
+        }
         __builtin_amdgcn_sched_barrier(0);
         if (ch + 1 < nchunks) fetch(ch + 1);                 // (into the registers of the operand)
         __syncthreads();                                     // the state's image has been read
@@ -436,18 +487,9 @@ delta_chunks_kernel(DeltaChunks a) {
                 for (int x = 0; x < NE; ++x) put_cols(L.x, x, v[x] - ct * X[x]);
             __syncthreads();
             if (update) {
+                const int ln = again(lane);
 #pragma unroll
-                for (int x = 0; x < NE; ++x) U[x] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-                    if (2 * s <= tb)
-#pragma unroll
-                        for (int x = 0; x < NE; ++x) {
-                            bf16x8 p[3];
-                            get_cols(L.x, x, 32 * s + 4 * q4, 16, p);
-                            U[x] = mfma6(p, mf[s], U[x]);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
+                for (int x = 0; x < NE; ++x) U[x] = chunk_product(L.x, ln, x, mf);
             }
         } else if (update) {
 #pragma unroll
@@ -461,18 +503,9 @@ delta_chunks_kernel(DeltaChunks a) {
 #pragma unroll
             for (int x = 0; x < NE; ++x) put_cols(L.x, x, wt * U[x]);
         } else {
+            const int ln = again(lane);
 #pragma unroll
-            for (int x = 0; x < NE; ++x) X[x] *= ct;
-#pragma unroll
-            for (int s = 0; s < 2; ++s)
-                if (2 * s <= tb)
-#pragma unroll
-                    for (int x = 0; x < NE; ++x) {
-                        bf16x8 p[3];
-                        get_cols(L.u, x, 32 * s + 4 * q4, 16, p);
-                        X[x] = mfma6(p, mf[s], X[x]);
-                            __builtin_amdgcn_sched_barrier(0);
-                    }
+            for (int x = 0; x < NE; ++x) X[x] = ct * X[x] + chunk_product(L.u, ln, x, mf);
             if (t < left)
 #pragma unroll
                 for (int x = 0; x < NE; ++x) {
@@ -487,9 +520,10 @@ delta_chunks_kernel(DeltaChunks a) {
             for (int x = 0; x < ET; ++x) S[j][x] *= ce;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
+            const int ln = again(lane), l16 = ln & 15, q4 = ln >> 4;
             bf16x8 up[ET][3];
 #pragma unroll
-            for (int x = 0; x < ET; ++x) get_cols(L.x, eh * ET + x, 32 * s + 4 * q4, 16, up[x]);
+            for (int x = 0; x < ET; ++x) get_cols(L.x, ln, eh * ET + x, 32 * s, 16, up[x]);
             const int row = 32 * s + 4 * q4 + (l16 >> 2);
 #pragma unroll
             for (int j = 0; j < DT; ++j) {

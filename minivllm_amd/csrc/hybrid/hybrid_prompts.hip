@@ -358,11 +358,11 @@ prompt_attention_kernel(PromptArgs a) {
 }
 
 // The same over float caches: keys, values, queries and weights all fp32, each cut into three parts; a
-// product is the sum of the six products of parts that matter in 24 bits.  Key tiles of 32; K and V are
+// product is the sum of the six largest products of parts.  Key tiles of 32; K and V are
 // in registers a tile ahead and go to LDS as images of their parts, one buffer.  Exponentials are expf of
 // the difference, as in the general kernel.
 // Against the fp32 instruction (2.7 times the cycles) behind loads that nothing hid: 3 prompts of 300..611
-// tokens, window 256, 8 heads of 64: 90 -> 39 us with the fill of the output ahead of it, 2.0e-7 from 64 bits
+// tokens, window 256, 8 heads of 64: 90 -> 39 us with the fill of the output ahead of it, 1.9e-7 from 64 bits
 // instead of 2.7e-7.
 struct PromptArgs32 {
     const float* q; long q_row, q_head;

@@ -101,13 +101,9 @@ def test_delta_rule(H, G, D, E, correct, fast):
         decay[::7] = 1.0
     state = torch.randn(NS, H, D, E, generator=g)
 
-    def run(shift):
-        def at(x):                                     # rows that do not start on 16 bytes go token by token
-            y = torch.empty(x.numel() + shift, dtype=x.dtype).cuda()
-            y[shift:] = x.reshape(-1).cuda()
-            return y[shift:].view(x.shape)
+    def run(shift):                                    # rows that do not start on 16 bytes go token by token
         st = state.cuda()
-        return hk.delta_scan(at(q), at(k), at(v), beta.cuda(), decay.cuda(), st, *lay, correct).cpu(), st.cpu()
+        return hk.delta_scan(at(q, shift), at(k, shift), at(v, shift), beta.cuda(), decay.cuda(), st, *lay, correct).cpu(), st.cpu()
 
     qd, kd = (x.double().repeat_interleave(H // G, 1) for x in (q, k))
     o, want = torch.zeros(T, H, E, dtype=torch.float64), state.double()
@@ -129,6 +125,89 @@ def test_delta_rule(H, G, D, E, correct, fast):
         owned[cu[b]:cu[b + 1]] = s >= 0
     for x in (got[0], literal[0]):
         assert bool((x[~owned] == 0).all())
+
+
+def at(x, shift):
+    """x on the GPU, ``shift`` numbers behind a 16-byte address."""
+    y = torch.empty(x.numel() + shift, dtype=x.dtype, device="cuda")
+    y[shift:] = x.reshape(-1).cuda()
+    return y[shift:].view(x.shape)
+
+
+def portions(B, n):
+    return [torch.tensor(x, dtype=torch.int32).cuda() for x in (list(range(0, B * n + 1, n)), list(range(n)) * B, list(range(B)))]
+
+
+@pytest.mark.parametrize("n", [200, 512])
+@pytest.mark.parametrize("correct", [True, False])
+def test_bits_of_the_delta_rule(n, correct):
+    """Operands in parts lose nothing against the fp32 arithmetic of the literal kernel: over decays of a trained
+    range neither the outputs nor the state are further from 64 bits (a tenth for the sample's own spread)."""
+    g = torch.Generator().manual_seed(n)
+    B, H, G, D, E = 2, 4, 2, 128, 128
+    T = B * n
+    q, k = (torch.nn.functional.normalize(torch.randn(T, G, D, generator=g), dim=-1) for _ in range(2))
+    q, v, beta = q * D ** -0.5, torch.randn(T, H, E, generator=g), torch.sigmoid(torch.randn(T, H, generator=g))
+    rate = 1 + 15 * torch.rand(H, generator=g)
+    decay = torch.exp(-rate * torch.nn.functional.softplus(torch.randn(T, H, generator=g) - 4.6))
+    lay = portions(B, n)
+    args = [x.cuda() for x in (beta, decay)]
+    got = []
+    for shift in (0, 1):
+        st = torch.zeros(B, H, D, E, device="cuda")
+        got.append((hk.delta_scan(at(q, shift), at(k, shift), at(v, shift), *args, st, *lay, correct), st))
+    qd, kd = (x.cuda().double().repeat_interleave(H // G, 1).view(B, n, H, D) for x in (q, k))
+    vd, bd, gd = v.cuda().double().view(B, n, H, E), args[0].double().view(B, n, H), args[1].double().view(B, n, H)
+    S, o = torch.zeros(B, H, D, E, dtype=torch.float64, device="cuda"), torch.empty(B, n, H, E, dtype=torch.float64, device="cuda")
+    for t in range(n):
+        S = S * gd[:, t, :, None, None]
+        u = vd[:, t] - (torch.matmul(kd[:, t, :, None], S)[:, :, 0] if correct else 0)
+        S = S + kd[:, t, :, :, None] * (bd[:, t, :, None] * u)[:, :, None]
+        o[:, t] = torch.matmul(qd[:, t, :, None], S)[:, :, 0]
+    for x, y, w in zip(*got, (o.view(T, H, E), S)):
+        chunks, literal = off(x, w.cpu()), off(y, w.cpu())
+        assert chunks <= 1.1 * literal, (chunks, literal)
+
+
+@pytest.mark.parametrize("forget", [4.0, 0.0])
+def test_bits_of_the_matrix_lstm(forget):
+    """As above; a row's error is counted against the row, as small denominators make some rows a thousand times the
+    others, and the running maximum's against its last bit.  (W_end v is rounded once more than in the literal kernel:
+    2^-26 in the mean, which shows where little else is rounded, as with half of the state forgotten per token.)"""
+    g = torch.Generator().manual_seed(int(forget))
+    B, n, H, D, E, cap = 2, 500, 4, 128, 128, 15.0
+    T, n_in = B * n, 2 * H * D + H * E + 2 * H
+    proj = torch.randn(T, n_in, generator=g)
+    proj[:, -2 * H:] *= 2
+    proj = proj.bfloat16().cuda()
+    bi, bf = torch.randn(H, generator=g).cuda(), (forget + torch.randn(H, generator=g)).cuda()
+    lay, got = portions(B, n), []
+    for pad in ((-n_in) % 8, (-n_in) % 8 + 1):
+        p = torch.zeros(T, n_in + pad, dtype=torch.bfloat16, device="cuda")
+        p[:, :n_in] = proj
+        q, k, v, i, f = p[:, :n_in].split([H * D, H * D, H * E, H, H], -1)
+        st = [torch.zeros(B, H, D, E, device="cuda"), torch.zeros(B, H, E // 16, D, device="cuda"),
+              torch.zeros(B, H, E // 16, device="cuda")]
+        got.append([hk.mlstm_scan(q.view(T, H, D), k.view(T, H, D), v.view(T, H, E), i, f, bi, bf, cap, *st, *lay)] + st)
+    q, k, v, i, f = proj.double().split([H * D, H * D, H * E, H, H], -1)
+    q, k, v = q.view(B, n, H, D) * D ** -0.5, k.view(B, n, H, D), v.view(B, n, H, E)
+    i = (cap * torch.tanh((i + bi.double()) / cap)).view(B, n, H)
+    f = torch.nn.functional.logsigmoid(cap * torch.tanh((f + bf.double()) / cap)).view(B, n, H)
+    S, o = torch.zeros(B, H, D, E, dtype=torch.float64, device="cuda"), torch.empty(B, n, H, E, dtype=torch.float64, device="cuda")
+    N, m = S[..., 0].clone(), S[..., 0, 0].clone()
+    for t in range(n):
+        m2 = torch.maximum(f[:, t] + m, i[:, t])
+        a, c = torch.exp(f[:, t] + m - m2), torch.exp(i[:, t] - m2)
+        S = a[..., None, None] * S + c[..., None, None] * k[:, t, :, :, None] * v[:, t, :, None]
+        N, m = a[..., None] * N + c[..., None] * k[:, t], m2
+        den = torch.maximum((N * q[:, t]).sum(-1).abs(), torch.exp(-m)) + 1e-6
+        o[:, t] = torch.matmul(q[:, t, :, None], S)[:, :, 0] / den[..., None]
+    rows = [float(((x[0].double() - o.view(T, H, E)).norm(dim=-1) / o.view(T, H, E).norm(dim=-1)).median()) for x in got]
+    assert rows[0] <= 1.1 * rows[1], rows
+    for x, y, w in zip(got[0][1:3], got[1][1:3], (S, N[:, :, None].expand(-1, -1, E // 16, -1))):
+        chunks, literal = off(x, w.cpu()), off(y, w.cpu())
+        assert chunks <= 1.1 * literal + 2.0 ** -26, (chunks, literal)
+    assert off(got[0][3], m[..., None].expand(-1, -1, E // 16).cpu()) <= 2.0 ** -23
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
