@@ -44,6 +44,64 @@ struct PromptArgs {
     KeyRule rule;
 };
 
+// rows of the wave (lane: a row and half of its columns, acc times f) with an infinity or a NaN
+template <int NB>
+__device__ __forceinline__ uint32_t rows_not_finite(const f32x16* acc, float f, bool ok) {
+    f32x16 sum = acc[0];
+#pragma unroll
+    for (int n = 1; n < NB; ++n) sum += acc[n];
+#pragma unroll
+    for (int w = 8; w > 0; w >>= 1)
+#pragma unroll
+        for (int e = 0; e < w; ++e) sum[e] += sum[e + w];
+    const uint64_t odd = __ballot(ok && sum[0] * f * 0.f != 0.f);
+    return (uint32_t)odd | (uint32_t)(odd >> 32);
+}
+
+// Infinities and NaN.  A key may be infinite without the row being lost (its score is -infinity and its weight
+// zero), and so may a value (the row's entry in that column is infinite, and no other row's); but part times
+// part, padding column times anything, and zero weight times what no query sees would make NaN of them.  NaN and
+// infinities stay in a row's sums once they are there, so a row that comes out finite met none, and the others are
+// worked out again by all lanes of their wave: one query, key after key, nothing in parts.
+template <typename T, bool EXT>
+__device__ void row_by_keys(const T* q, const T* k_cache, const T* v_cache, const int* table, int block_size, int ctx,
+                            float scale, float slope, const float* sink, const T* gate, T* out, int G, int g, int h,
+                            int D, int E, const KeyRule& rule) {
+    constexpr int N = 256 / kWave;                 // of up to 256 columns, lane + 64 i are this lane's
+    const int lane = threadIdx.x & 63;
+    const VisibleKeys vis(ctx, rule);
+    float qf[N], acc[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        qf[i] = lane + 64 * i < D ? ld(q + lane + 64 * i) * scale : 0.f;
+        acc[i] = 0.f;
+    }
+    float m = sink ? sink[h] : NO_SINK_MAX, l = sink ? 1.f : 0.f;
+    for (int v = 0; v < vis.count; ++v) {
+        const long row = vis.row(v, table, block_size, rule) * G + g;
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if (lane + 64 * i < D) s += ld(k_cache + row * D + lane + 64 * i) * qf[i];
+        s = wave_sum(s);
+        if (EXT) s = rule.capped(s);
+        s -= slope * (float)(ctx - 1 - vis.key(v));
+        const float top = fmaxf(m, s), f = expf(m - top), w = expf(s - top);
+        l = l * f + w;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int e = lane + 64 * i;
+            acc[i] = acc[i] * f + w * (e < E ? ld(v_cache + row * (long)rule.v_stride + e) : 0.f);
+        }
+        m = top;
+    }
+    float f = 1.f / l;
+    if (gate) f *= sigmoidf_(ld(gate));
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        if (lane + 64 * i < E) st(out + lane + 64 * i, acc[i] * f);
+}
+
 template <int DP, int EP, int TK, bool EXT>
 __global__ void __launch_bounds__(256, DP + EP > 256 ? 1 : 2)
 prompt_attention_kernel(PromptArgs a) {
@@ -336,6 +394,7 @@ prompt_attention_kernel(PromptArgs a) {
     }
     const long row = row0 + min(qi, qlen - 1);
     if (a.gate) f *= sigmoidf_(ld(a.gate + row * a.gate_row + h));
+    uint32_t lost = rows_not_finite<NB>(acc, f, qok);
     // both halves of the wave hold every second run of four columns of a row: swapped so that a
     // lane stores eight neighbouring ones
     uint16_t* op = a.out + (row * H + h) * a.E;
@@ -352,8 +411,17 @@ prompt_attention_kernel(PromptArgs a) {
             const uint32_t g0 = __shfl_xor(s0, 32, kWave), g1 = __shfl_xor(s1, 32, kWave);
             const uint4 v = half ? make_uint4(g0, g1, w[2], w[3]) : make_uint4(w[0], w[1], g0, g1);
             const int e = 32 * n + 8 * r + 8 * half;
-            if (qok && e < a.E) *reinterpret_cast<uint4*>(op + e) = v;
+            if (qok && e < a.E && !(lost >> l32 & 1)) *reinterpret_cast<uint4*>(op + e) = v;
         }
+    for (; lost; lost &= lost - 1) {
+        const int i = __builtin_ctz(lost);
+        const long r = row0 + wq0 + i;
+        row_by_keys<bf16_t, EXT>((const bf16_t*)a.q + r * a.q_row + (long)h * a.q_head, (const bf16_t*)a.k_cache,
+                                 (const bf16_t*)a.v_cache, table, a.block_size, start + wq0 + i + 1,
+                                 EXT ? rule.head_scale(a.scale, h) : a.scale, rule.slopes ? rule.slopes[h] : 0.f, a.sink,
+                                 a.gate ? a.gate + r * a.gate_row + h : nullptr, (bf16_t*)a.out + (r * H + h) * a.E, G, g,
+                                 h, a.D, a.E, rule);
+    }
 #endif
 }
 
@@ -564,8 +632,8 @@ prompt_attention_f32_kernel(PromptArgs32 a) {
                 acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0], p[s][0], acc[n], 0, 0, 0);
             }
     }
+    if (!wave_live) return;
     l_run += __shfl_xor(l_run, 32, kWave);
-    if (!qok) return;
     float f;
     if (a.sink) {
         const float M = fmaxf(m_run, a.sink[h]);
@@ -574,18 +642,26 @@ prompt_attention_f32_kernel(PromptArgs32 a) {
     } else {
         f = 1.f / l_run;
     }
-    const long row = row0 + qi;
+    const long row = row0 + min(qi, qlen - 1);
     if (a.gate) f *= sigmoidf_(a.gate[row * a.gate_row + h]);
+    uint32_t lost = rows_not_finite<NB>(acc, f, qok);
     float* op = a.out + (row * H + h) * a.E;
 #pragma unroll
     for (int n = 0; n < NB; ++n)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int e = 32 * n + 8 * r + 4 * half;
-            if (e < a.E)
+            if (qok && e < a.E && !(lost >> l32 & 1))
                 *reinterpret_cast<float4*>(op + e) = make_float4(acc[n][4 * r] * f, acc[n][4 * r + 1] * f,
                                                                  acc[n][4 * r + 2] * f, acc[n][4 * r + 3] * f);
         }
+    for (; lost; lost &= lost - 1) {
+        const int i = __builtin_ctz(lost);
+        const long r = row0 + wq0 + i;
+        row_by_keys<float, EXT>(a.q + r * a.q_row + (long)h * a.q_head, a.k_cache, a.v_cache, table, a.block_size,
+                                start + wq0 + i + 1, sc, slope, a.sink, a.gate ? a.gate + r * a.gate_row + h : nullptr,
+                                a.out + (r * H + h) * a.E, G, g, h, a.D, a.E, rule);
+    }
 #endif
 }
 

@@ -115,3 +115,49 @@ def test_values_inside_the_key_rows():
                                     None, torch.zeros(T, H, E, dtype=torch.bfloat16).cuda(), positions=pos.cuda(),
                                     max_q=max(PORTIONS)).cpu()
     close(got, want, float(k.abs().max()))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,E,bs", [(128, 128, 64), (40, 72, 64), (64, 64, 16)])
+@pytest.mark.parametrize("opt", [dict(), dict(window=40, keep_first=5)])
+def test_infinities_stay_where_they_are(D, E, bs, dt, opt):
+    """A key of infinity has no weight where its score is -infinity; a value of infinity makes its column of the rows
+    that see it infinite; what is not a number makes the rows (key) or entries (value) that see it so; no other
+    entry changes (float64, over the keys that a row sees)."""
+    H, G, inf = 4, 2, float("inf")
+    g, k, v, rows, tables, cu_q, cu_k, pos = step(G, D, E, bs, dt=dt)
+    kc, vc, _, _ = caches(k, v, rows, G, D, E, bs, 0)
+
+    def put(cache, b, j, head, column, x):
+        cache[tables[b, j // bs], j % bs, head, column] = x
+
+    put(kc, 2, 32, 0, 1, inf)                            # (sequence, key): the last key, one of a tile's middle, the first
+    put(kc, 5, 70, 1, D - 1, -inf)
+    put(kc, 7, 0, 0, 9, inf)
+    put(kc, 7, 250, 1, 0, float("nan"))
+    put(vc, 4, 40, 0, 3, -inf)
+    put(vc, 6, 3, 1, E - 1, inf)
+    put(vc, 6, 100, 0, 0, float("nan"))
+    T = int(cu_q[-1])
+    q = torch.randn(T, H, D, generator=g).to(dt)
+    sink = torch.randn(H, generator=g)
+    got = hk.sink_attention_prefill(q.cuda(), kc.cuda(), vc.cuda(), cu_q.cuda(), cu_k.cuda(), tables.cuda(), D ** -0.5,
+                                    sink.cuda(), None, torch.zeros(T, H, E, dtype=dt).cuda(), positions=pos.cuda(),
+                                    max_q=max(PORTIONS), **opt).cpu()
+    want = torch.empty(T, H, E, dtype=torch.float64)
+    for t in range(T):
+        b, p = int(torch.searchsorted(cu_q[1:].contiguous(), t, right=True)), int(pos[t])
+        lo = max(0, p - opt.get("window", p + 1) + 1)
+        keys = list(range(min(opt.get("keep_first", 0), lo))) + list(range(lo, p + 1))
+        at = [(int(tables[b, j // bs]), j % bs) for j in keys]
+        kk, vv = (torch.stack([c[i, j] for i, j in at], 1).double() for c in (kc, vc))               # [G, keys, :]
+        s = torch.einsum("hd,hnd->hn", q[t].double(), kk.repeat_interleave(H // G, 0)) * D ** -0.5
+        s = torch.cat([s, sink.double()[:, None]], 1)
+        w = torch.exp(s - s.max(1, keepdim=True)[0])
+        w = (w / w.sum(1, keepdim=True))[:, :-1]
+        x = w[:, :, None] * vv.repeat_interleave(H // G, 0)
+        want[t] = torch.where((w > 0)[:, :, None] | w.isnan()[:, :, None], x, torch.zeros_like(x)).sum(1)
+    assert int(want.isnan().any(2).sum()) > 20 and int(want.isinf().any(2).sum()) > 20
+    assert bool(want.isfinite().all(2).sum() > T * H // 3)
+    tol = dict(rtol=2 ** -7, atol=1e-5) if dt == torch.bfloat16 else dict(rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(got.double(), want, equal_nan=True, **tol)
