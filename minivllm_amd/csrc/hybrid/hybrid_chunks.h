@@ -53,6 +53,16 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
 }
 #endif
 
+#ifdef __HIP_DEVICE_COMPILE__
+// A kernel's only argument, loaded again: what a rare path needs of it is not kept in registers all along.
+template <class A>
+__device__ __forceinline__ A arguments_anew() {
+    uintptr_t p = (uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const __attribute__((address_space(4))) A*)p;
+}
+#endif
+
 // four numbers of a lane as three runs of bfloat16; at(k): where part k goes
 template <class F>
 __device__ __forceinline__ void put_parts(f32x4 x, F&& at) {

@@ -25,6 +25,10 @@
 // as operands for all waves.  The next chunk's q, k, v and gates are in registers while this one
 // is worked on; three barriers per chunk.
 //
+// An infinity or a NaN in a row of a chunk meets the zero weights of the tokens ahead of it, and its parts are NaN.
+// It stays in the sums once it is there, so a portion whose outputs and state come out finite met none; any other is
+// walked again from its first token by the recurrence itself (same workgroup, its own columns).
+//
 // Bound by the vector instructions around the products (splitting, weights, addresses: 1300 per wave
 // and chunk at two waves per SIMD), 4.4 us a chunk.  8 portions of 512..1024 tokens, 8 heads of
 // 128: 70 us of 83 with the norm behind it, against 602 of 622 token by token.  With four waves of twice the
@@ -59,12 +63,73 @@ struct Lds {
     char s[3][EB * DP * 2];                // the state's parts, a row per state column
     char n[3][DP * 2];                     // the normaliser's parts
     Gates g;
+    int lost;                              // an output or a state is not finite
 };
 
 __device__ __forceinline__ float logsigmoid_(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
+// The portion's tokens one after the other: thread = a column and a sixteenth of the channels, sums through LDS
+// (`red`: 8 KB).
 template <int DP>
-__global__ void __launch_bounds__(512, 2)
+__device__ __forceinline__ void walk_tokens(const MlstmChunks a, float* red) {
+    constexpr int CH = DP / 16;
+    const int b = blockIdx.x, h = blockIdx.y, e0 = blockIdx.z * EB, slot = a.slots[b];
+    const long first = a.cu_q[b];
+    const int n = a.cu_q[b + 1] - (int)first;
+    const bool has_past = a.positions[first] > 0;
+    const int c = threadIdx.x & 31, r = threadIdx.x >> 5, e = e0 + c, d0 = r * CH;
+    const int H = a.H, D = a.D, E = a.E, ZG = (E + 15) / 16, z = e0 / 16;
+    float* sp = a.state + ((long)slot * H + h) * D * E;
+    float* np = a.nstate + (((long)slot * H + h) * ZG + z) * D;
+    float* mp = a.mstate + ((long)slot * H + h) * ZG + z;
+    float S[CH], N[CH], m = has_past ? *mp : 0.f;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        S[i] = has_past && d0 + i < D && e < E ? sp[(long)(d0 + i) * E + e] : 0.f;
+        N[i] = has_past && d0 + i < D ? np[d0 + i] : 0.f;
+    }
+    for (int x = 0; x < n; ++x) {
+        const long t = first + x;
+        const float gi = a.cap * tanhf((ld(a.gi + t * a.g_row + h) + a.bi[h]) / a.cap);
+        const float gf = logsigmoid_(a.cap * tanhf((ld(a.gf + t * a.g_row + h) + a.bf[h]) / a.cap));
+        const float m2 = fmaxf(gf + m, gi), fs = expf(gf + m - m2), is = expf(gi - m2);
+        m = m2;
+        const float kv = e < E ? is * ld((const bf16_t*)a.v + t * a.v_row + (long)h * E + e) : 0.f;
+        float po = 0.f, pn = 0.f;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            if (d0 + i >= D) continue;
+            const float k = ld((const bf16_t*)a.k + t * a.k_row + (long)h * D + d0 + i);
+            const float q = ld((const bf16_t*)a.q + t * a.q_row + (long)h * D + d0 + i) * a.qscale;
+            S[i] = fs * S[i] + k * kv;
+            po += S[i] * q;
+            N[i] = fs * N[i] + is * k;
+            pn += N[i] * q;
+        }
+        float* at = red + (x & 1) * 1024;              // two of them: one barrier per token
+        at[r * 32 + c] = po;
+        at[512 + r * 32 + c] = pn;
+        __syncthreads();
+        if (r == 0 && e < E) {
+            po = pn = 0.f;
+            for (int i = 0; i < 16; ++i) {
+                po += at[i * 32 + c];
+                pn += at[512 + i * 32 + c];
+            }
+            a.o[(t * H + h) * (long)E + e] = po / (fmaxf(fabsf(pn), expf(-m)) + 1e-6f);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        if (d0 + i >= D) continue;
+        if (e < E) sp[(long)(d0 + i) * E + e] = S[i];
+        if (c < 2 && z + c < ZG) np[c * D + d0 + i] = N[i];
+    }
+    if (r == 0 && c < 2 && z + c < ZG) mp[c] = m;
+}
+
+template <int DP>
+__global__ void __launch_bounds__(512, DP > 64 ? 2 : 4)      // (two workgroups on a CU where the LDS has room for them)
 mlstm_chunks_kernel(MlstmChunks a) {
 #ifdef __HIP_DEVICE_COMPILE__       // (the host pass only needs the launch stub)
     constexpr int KS = DP / 32, DT = DP / 64;      // steps over the key channels; a wave's 16-wide blocks of them
@@ -217,6 +282,8 @@ mlstm_chunks_kernel(MlstmChunks a) {
     };
 
     const int nchunks = (n + C - 1) / C;
+    float seen = 0.f;                              // the sum of all outputs and states: finite if they are
+    if (tid == 0) L.lost = 0;
     fetch(0);
     if (wave == GATES) {
         gates(0);
@@ -314,9 +381,10 @@ mlstm_chunks_kernel(MlstmChunks a) {
         sum += __shfl_xor(sum, 16, kWave);
         sum += __shfl_xor(sum, 32, kWave);
         den = 1.f / (fmaxf(fabsf(den + sum), g.em[t]) + 1e-6f);
+        O *= den;
         if (t < left && e0 + 16 * et + 4 * q4 < E)
-            *reinterpret_cast<float4*>(a.o + ((first + ch * C + t) * H + h) * (long)E + e0 + 16 * et + 4 * q4) =
-                make_float4(O[0] * den, O[1] * den, O[2] * den, O[3] * den);
+            *reinterpret_cast<f32x4*>(a.o + ((first + ch * C + t) * H + h) * (long)E + e0 + 16 * et + 4 * q4) = O;
+        seen += (O[0] + O[1]) + (O[2] + O[3]);              // (zeros behind the portion, as q is)
         }
         if (wave == GATES && ch + 1 < nchunks) gates(ch + 1);
         __syncthreads();                                    // W_end v is there
@@ -362,6 +430,16 @@ mlstm_chunks_kernel(MlstmChunks a) {
             publish();
             __syncthreads();
         }
+    }
+#pragma unroll
+    for (int j = 0; j < DT; ++j) seen += (S[j][0] + S[j][1]) + (S[j][2] + S[j][3]);
+    if (seen * 0.f != 0.f) L.lost = 1;
+    __syncthreads();
+    if (L.lost) {
+        __threadfence();                                    // (the outputs are written again, by other waves)
+        __syncthreads();
+        walk_tokens<DP>(arguments_anew<MlstmChunks>(), reinterpret_cast<float*>(smem));
+        return;
     }
     // ---- the state after the portion
 #pragma unroll

@@ -284,3 +284,52 @@ def test_single_tokens(H, G, D, E, rule):
     # sums of up to 256 fp32 products
     assert off(got, want) <= 256 * 2.0 ** -24 and off(gs, ws) <= 256 * 2.0 ** -24
     assert bool((got[2] == 0).all())
+
+
+INF, NAN = float("inf"), float("nan")
+
+
+def same_but_for_rounding(got, want):
+    """Infinities and NaN in the same places, and elsewhere the same numbers (how closely is tested above: two
+    roundings of a small denominator, 2^-23 of its terms, may differ by a thousand times that)."""
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()], want[want.isinf()])
+    ok = want.isfinite()
+    assert off(got[ok], want[ok].double()) <= 2.0 ** -13
+
+
+@pytest.mark.parametrize("D,E", [(128, 128), (64, 72), (8, 8)])
+@pytest.mark.parametrize("what", ["k inf", "k nan", "v inf", "v nan", "q inf", "f nan", "i nan", "state inf"])
+def test_mlstm_infinities(D, E, what):
+    """What is not finite reaches the outputs and states that it reaches token by token, and no earlier token, no
+    other column, no other sequence."""
+    g = torch.Generator().manual_seed(D)
+    H, cap = 2, 15.0
+    cu, lay = layout()
+    T, Z, NS = cu[-1] + TAIL, (E + 15) // 16, 13
+    n_in = 2 * H * D + H * E + 2 * H
+    proj = torch.randn(T, n_in, generator=g)
+    bi, bf = torch.randn(H, generator=g), 4 + torch.randn(H, generator=g)
+    init = [torch.randn(NS, H, D, E, generator=g), torch.randn(NS, H, 1, D, generator=g).expand(-1, -1, Z, -1).contiguous(),
+            torch.randn(NS, H, 1, generator=g).expand(-1, -1, Z).contiguous()]
+    t, h = cu[8] + 70, 1                               # token 70 of 129: its chunk has tokens ahead of it
+    x = INF if "inf" in what else NAN
+    at = {"k": H * D + h * D + 3, "v": 2 * H * D + h * E + E // 2, "q": h * D + 5, "i": n_in - 2 * H + h, "f": n_in - H + h}
+    if what[0] in at:
+        proj[t, at[what[0]]] = x
+    else:
+        init[0][SLOTS[6], h, 2, 1] = x                 # (a sequence with a past)
+    proj = proj.bfloat16()
+
+    def run(pad):
+        p = torch.zeros(T, n_in + pad, dtype=torch.bfloat16).cuda()
+        p[:, :n_in] = proj.cuda()
+        q, k, v, i, f = p[:, :n_in].split([H * D, H * D, H * E, H, H], -1)
+        st = [y.cuda() for y in init]
+        o = hk.mlstm_scan(q.view(T, H, D), k.view(T, H, D), v.view(T, H, E), i, f, bi.cuda(), bf.cuda(), cap, *st, *lay)
+        return [o.cpu()] + [y.cpu() for y in st]
+
+    got, literal = run((-n_in) % 8), run((-n_in) % 8 + 1)
+    assert not bool(got[0].isfinite().all()) and bool(got[0][cu[8]:t].isfinite().all())
+    for y, w in zip(got, literal):
+        same_but_for_rounding(y, w)
