@@ -28,6 +28,10 @@
 // state 6.9e-8, against 1.1e-7 and 7.2e-8 token by token (2.3e-7 and 1.4e-7 with parts cut off and one sum for
 // all products).
 //
+// An infinity or a NaN in a row of a chunk meets the zero weights of the tokens ahead of it, and its parts are NaN.
+// It stays in the sums once it is there, so a portion whose outputs and state come out finite met none; any other is
+// walked again from its first token by the recurrence itself (same workgroup, its own columns).
+//
 // 8 portions of 512..1024 tokens, 16 / 8 heads of 128: 54 + 140 us, against 645 us token by token.  The walk
 // takes 9 us a chunk of 64 columns; its six phases between barriers use the matrix units, the
 // vector units (cutting) and the LDS for about 2.5 us each and hardly overlap: one workgroup per CU is all that
@@ -314,7 +318,56 @@ struct Lds {
         char s[3][EB * DP * 2];        // the state's parts, a row per state column
         struct { char x[3][C * ROW], u[3][C * ROW]; };   // rows of tokens: V - diag(c) K S, later diag(W_end) U; U
     };
+    int lost;                          // an output or a state is not finite
 };
+
+// The portion's tokens one after the other: a thread has a column and some of the channels, sums through LDS
+// (`red`: 4 KB).
+template <int DP, int EB, bool DELTA>
+__device__ __forceinline__ void walk_tokens(const DeltaChunks a, float* red) {
+    constexpr int NS = 512 / EB, CH = DP / NS;
+    const int b = blockIdx.x, h = blockIdx.y, slot = a.slots[b], first = a.cu_q[b], n = a.cu_q[b + 1] - first;
+    const bool has_past = a.positions[first] > 0;
+    const int c = threadIdx.x % EB, r = threadIdx.x / EB, e = blockIdx.z * EB + c, d0 = r * CH;
+    const int H = a.H, G = a.G, D = a.D, E = a.E, g = h / (H / G);
+    float* sp = a.state + ((long)slot * H + h) * D * E;
+    float S[CH];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) S[i] = has_past && d0 + i < D && e < E ? sp[(long)(d0 + i) * E + e] : 0.f;
+    auto column_sum = [&](float* at, float x) {
+        at[r * EB + c] = x;
+        __syncthreads();
+        x = 0.f;
+        for (int i = 0; i < NS; ++i) x += at[i * EB + c];
+        return x;
+    };
+    for (long t = first; t < first + n; ++t) {
+        const float* kp = a.k + (t * G + g) * D + d0;
+        const float* qp = a.q + (t * G + g) * D + d0;
+        const float dec = a.decay[t * H + h];
+        float u = e < E ? a.v[(t * H + h) * E + e] : 0.f, dot = 0.f, po = 0.f;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            S[i] *= dec;
+            if (DELTA && d0 + i < D) dot += S[i] * kp[i];
+        }
+        if (DELTA) u -= column_sum(red, dot);
+        u *= a.beta[t * H + h];
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            if (d0 + i >= D) continue;
+            S[i] += kp[i] * u;
+            po += S[i] * qp[i];
+        }
+        // (the barriers of this sum and of the one above stand between a sum's reads and the next token's writes; with
+        // this one alone two places take turns)
+        po = column_sum(red + (DELTA ? 512 : (t & 1) * 512), po);
+        if (r == 0 && e < E) a.o[(t * H + h) * E + e] = po;
+    }
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+        if (d0 + i < D && e < E) sp[(long)(d0 + i) * E + e] = S[i];
+}
 
 template <int DP, int ET, bool DELTA>
 __global__ void __launch_bounds__(512, 2)
@@ -380,6 +433,7 @@ delta_chunks_kernel(DeltaChunks a) {
             }
     };
     auto stash = [&]() {
+        const int ln = again(lane), t = 16 * tb + (ln & 15), q4 = ln >> 4;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             split8(raw[s], xp[s]);
@@ -430,6 +484,8 @@ delta_chunks_kernel(DeltaChunks a) {
     };
 
     const int nchunks = (n + C - 1) / C;
+    float seen = 0.f;                                // the sum of all outputs and states: finite if they are
+    if (tid == 0) L.lost = 0;
     fetch(0);
     stash();
     publish();
@@ -506,6 +562,8 @@ delta_chunks_kernel(DeltaChunks a) {
             const int ln = again(lane);
 #pragma unroll
             for (int x = 0; x < NE; ++x) X[x] = ct * X[x] + chunk_product(L.u, ln, x, mf);
+#pragma unroll
+            for (int x = 0; x < NE; ++x) seen += (X[x][0] + X[x][1]) + (X[x][2] + X[x][3]);      // (zeros behind the portion)
             if (t < left)
 #pragma unroll
                 for (int x = 0; x < NE; ++x) {
@@ -544,6 +602,18 @@ delta_chunks_kernel(DeltaChunks a) {
             __builtin_amdgcn_sched_barrier(0);
             stash();
         }
+    }
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+        for (int x = 0; x < ET; ++x) seen += (S[j][x][0] + S[j][x][1]) + (S[j][x][2] + S[j][x][3]);
+    if (seen * 0.f != 0.f) L.lost = 1;
+    __syncthreads();
+    if (L.lost) {
+        __threadfence();                                     // (the outputs are written again, by other waves)
+        __syncthreads();
+        walk_tokens<DP, EB, DELTA>(arguments_anew<DeltaChunks>(), reinterpret_cast<float*>(smem));
+        return;
     }
 #pragma unroll
     for (int j = 0; j < DT; ++j)

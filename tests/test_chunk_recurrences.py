@@ -333,3 +333,40 @@ def test_mlstm_infinities(D, E, what):
     assert not bool(got[0].isfinite().all()) and bool(got[0][cu[8]:t].isfinite().all())
     for y, w in zip(got, literal):
         same_but_for_rounding(y, w)
+
+
+@pytest.mark.parametrize("H,G,D,E", [(2, 1, 128, 128), (40, 40, 64, 72), (2, 1, 8, 4)])
+@pytest.mark.parametrize("correct", [True, False])
+@pytest.mark.parametrize("what", ["k inf", "k nan", "v inf", "v nan", "q inf", "beta nan", "decay nan", "state inf", "large"])
+def test_delta_infinities(H, G, D, E, correct, what):
+    """As above; ``large``: a finite value whose rounded part is none.  (40 heads of 72 columns: 64 per workgroup.)"""
+    g = torch.Generator().manual_seed(D)
+    cu, lay = layout()
+    T, NS, h = cu[-1] + TAIL, 13, H - 1
+    q, k = (torch.nn.functional.normalize(torch.randn(T, G, D, generator=g), dim=-1) for _ in range(2))
+    ops = {"q": q * D ** -0.5, "k": k, "v": torch.randn(T, H, E, generator=g), "beta": torch.rand(T, H, generator=g),
+           "decay": torch.exp(-torch.rand(T, H, generator=g) * 0.2)}
+    state = torch.randn(NS, H, D, E, generator=g)
+    t, x, name = cu[8] + 70, INF if "inf" in what else NAN, what.split()[0]
+    if name in ("q", "k"):
+        ops[name][t, G - 1, 3] = x
+    elif name in ("beta", "decay"):
+        ops[name][t, h] = x
+    elif name == "v":
+        ops[name][t, h, E // 2] = x
+    elif name == "large":
+        ops["v"][t, h, E // 2], ops["beta"][t, h] = torch.finfo(torch.float32).max, 1.0
+    else:
+        state[SLOTS[6], h, 2, 1] = x
+
+    def run(shift):
+        st = state.cuda()
+        o = hk.delta_scan(at(ops["q"], shift), at(ops["k"], shift), at(ops["v"], shift), ops["beta"].cuda(),
+                          ops["decay"].cuda(), st, *lay, correct)
+        return o.cpu(), st.cpu()
+
+    got, literal = run(0), run(1)
+    assert name == "large" or not bool(got[0].isfinite().all())
+    assert bool(got[0][cu[8]:t].isfinite().all())
+    for y, w in zip(got, literal):
+        same_but_for_rounding(y / 2.0 ** 70, w / 2.0 ** 70) if name == "large" else same_but_for_rounding(y, w)
