@@ -196,9 +196,14 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
+// QK16 (bfloat16 caches, D % 16 == 0): the score products run as v_mfma_f32_32x32x16_bf16 on the raw
+// 16-bit K tile and q rows - the operands ARE bfloat16 values, so the products are exact and the
+// fp32 accumulation only differs in order from the fp32 instruction; the score scale is applied
+// to the fp32 result.  Weights and weighted sums stay on the fp32 instruction.  8 x 1024 tokens, 16 heads,
+// scores on the fp32 / on the bf16 instruction: D 128, E 100 849 / 552 us, E 36 648 / 290, D 64, E 20 372 / 249.
 // EXT: the instance that knows head temperatures, the soft cap and pooled rows; without it the
 // kernel is compiled free of them (their state costs registers the plain form has no room for).
-template <typename T, int DP, int EP, bool EXT>
+template <typename T, int DP, int EP, bool QK16, bool EXT>
 __global__ void __launch_bounds__(256)
 sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
                             const T* __restrict__ k_cache, const T* __restrict__ v_cache,
@@ -208,8 +213,10 @@ sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
                             long gate_row, T* __restrict__ out, float scale, int H, int G, int D,
                             int E, int seq0, int vec_k, int vec_v, KeyRule rule) {
     extern __shared__ float sm[];
-    constexpr int KS = DP + 1;                              // floats per K row of the LDS image
+    constexpr int KS = QK16 ? (DP + 8) / 2 : DP + 1;      // floats per K row of the LDS image
+    constexpr int KSB = DP + 8;                             // (QK16) 16-bit elements per K row
     float* Ks = sm;
+    uint16_t* Kb = reinterpret_cast<uint16_t*>(sm);
     float* Vs = sm + 32 * KS;
     const int b = blockIdx.x + seq0, tile = blockIdx.y, h = blockIdx.z;
     const int row0 = cu_q[b], qlen = cu_q[b + 1] - row0;
@@ -223,17 +230,32 @@ sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
     const int qpos = start + qi;
 
     const float hscale = EXT ? rule.head_scale(scale, h) : scale;
-    float qreg[DP / 2];
+    float qreg[QK16 ? 1 : DP / 2];
+    bf16x8 qv[QK16 ? DP / 16 : 1];
     {
         const T* qp = q + (long)(row0 + (qok ? qi : 0)) * q_row + (long)h * q_head;
+        if constexpr (QK16) {
 #pragma unroll
-        for (int s = 0; s < DP / 2; ++s) {
-            const int d = 2 * s + half;
-            qreg[s] = (qok && d < D) ? ld(qp + d) * hscale : 0.f;
-        }
-        for (int i = tid; i < 32 * (KS - D); i += 256) {          // padding columns of K stay zero
-            const int key = i / (KS - D), c = D + i - key * (KS - D);
-            Ks[key * KS + c] = 0.f;
+            for (int s = 0; s < DP / 16; ++s) {
+                const int d = 16 * s + 8 * half;
+                uint4 raw = make_uint4(0, 0, 0, 0);
+                if (qok && d < D) raw = *reinterpret_cast<const uint4*>(qp + d);
+                qv[s] = __builtin_bit_cast(bf16x8, raw);
+            }
+            for (int i = tid; i < 32 * (KSB - D); i += 256) {   // padding columns of K stay zero
+                const int key = i / (KSB - D), c = D + i - key * (KSB - D);
+                Kb[key * KSB + c] = 0;
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < DP / 2; ++s) {
+                const int d = 2 * s + half;
+                qreg[s] = (qok && d < D) ? ld(qp + d) * hscale : 0.f;
+            }
+            for (int i = tid; i < 32 * (KS - D); i += 256) {      // padding columns of K stay zero
+                const int key = i / (KS - D), c = D + i - key * (KS - D);
+                Ks[key * KS + c] = 0.f;
+            }
         }
     }
     float m = sink ? sink[h] : NO_SINK_MAX, lsum = sink ? 1.f : 0.f;
@@ -265,7 +287,18 @@ sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
                           : (long)table[j / block_size] * block_size + j % block_size;
         };
         // ---- K and V tile into LDS
-        if (vec_k) {
+        if constexpr (QK16) {
+            const int D8 = D >> 3;
+            for (int i = tid; i < 32 * D8; i += 256) {
+                const int key = i / D8, c = (i - key * D8) << 3, j = k0 + key;
+                uint4 raw = make_uint4(0, 0, 0, 0);
+                if (j < k_lim) {
+                    const long slot = cache_row(j);
+                    raw = *reinterpret_cast<const uint4*>(k_cache + (slot * G + g) * (long)D + c);
+                }
+                *reinterpret_cast<uint4*>(Kb + key * KSB + c) = raw;
+            }
+        } else if (vec_k) {
             const int D4 = D >> 2;
             for (int i = tid; i < 32 * D4; i += 256) {
                 const int key = i / D4, c = (i - key * D4) << 2, j = k0 + key;
@@ -317,10 +350,21 @@ sink_attention_tiles_kernel(const T* __restrict__ q, long q_row, long q_head,
             f32x16 sacc;
 #pragma unroll
             for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
-            const float* ka = Ks + l32 * KS + half;
+            if constexpr (QK16) {
+                const uint16_t* ka = Kb + l32 * KSB + 8 * half;
 #pragma unroll
-            for (int s = 0; s < DP / 2; ++s)
-                sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[2 * s], qreg[s], sacc, 0, 0, 0);
+                for (int s = 0; s < DP / 16; ++s) {
+                    const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(ka + 16 * s));
+                    sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qv[s], sacc, 0, 0, 0);
+                }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sacc[r] *= hscale;
+            } else {
+                const float* ka = Ks + l32 * KS + half;
+#pragma unroll
+                for (int s = 0; s < DP / 2; ++s)
+                    sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[2 * s], qreg[s], sacc, 0, 0, 0);
+            }
             float mt = -INFINITY;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -376,19 +420,26 @@ static int launch_tiles(const void* q, long q_row, long q_head, const void* k_ca
                         const void* v_cache, const void* block_tables, int max_blocks,
                         int block_size, const void* cu_q, const void* positions, const void* sink,
                         const void* gate, long gate_row, void* out, float scale, int nseq,
-                        int seq0, int max_q, int H, int G, int D, int E,
+                        int seq0, int max_q, int H, int G, int D, int E, bool scores16,
                         KeyRule rule, hipStream_t s) {
     const int vec_k = (D % 4 == 0) && ((size_t)k_cache % 16 == 0);
     const int vec_v = (E % 4 == 0) && (rule.v_stride % 4 == 0) && ((size_t)v_cache % 16 == 0);
     const dim3 grid(nseq, (max_q + 127) / 128, H);
-#define TILES_LAUNCH(EXT)                                                                         \
-    hipLaunchKernelGGL((sink_attention_tiles_kernel<T, DP, EP, EXT>), grid, dim3(256),            \
-                       (32 * (DP + 1) + 32 * EP) * sizeof(float), s,                              \
+#define TILES_LAUNCH(QK16, EXT)                                                                   \
+    hipLaunchKernelGGL((sink_attention_tiles_kernel<T, DP, EP, QK16, EXT>), grid, dim3(256),      \
+                       (32 * (QK16 ? (DP + 8) / 2 : DP + 1) + 32 * EP) * sizeof(float), s,        \
                        (const T*)q, q_row, q_head, (const T*)k_cache, (const T*)v_cache,          \
                        (const int*)block_tables, max_blocks, block_size, (const int*)cu_q,        \
                        (const int*)positions, (const float*)sink, (const T*)gate, gate_row,       \
                        (T*)out, scale, H, G, D, E, seq0, vec_k, vec_v, rule)
-    if (rule.temps || rule.softcap > 0.f || rule.pool > 0) TILES_LAUNCH(true); else TILES_LAUNCH(false);
+    const bool ext = rule.temps || rule.softcap > 0.f || rule.pool > 0;
+    if constexpr (sizeof(T) == 2) {
+        if (scores16) {
+            if (ext) TILES_LAUNCH(true, true); else TILES_LAUNCH(true, false);
+            return HYB_LAUNCH_OK();
+        }
+    }
+    if (ext) TILES_LAUNCH(false, true); else TILES_LAUNCH(false, false);
 #undef TILES_LAUNCH
     return HYB_LAUNCH_OK();
 }
@@ -629,6 +680,18 @@ int hyb_sink_attention_split(const void* q, long q_row, long q_head, const void*
 // 1 when the tile kernel has an instance for these head sizes (else the row kernel serves)
 int hyb_sink_attention_tiles_ok(int D, int E) { return D <= 256 && E <= 256 && !(D > 128 && E > 128); }
 
+// Which kernel takes the prompts.  2: operands in whole 16-byte runs, 8 times faster than the general kernel over
+// bfloat16 at 8 x 1k tokens of 128-wide heads and 4 times at 2 x 300, over float 2.3 times at 3 x 600 with a window
+// (hybrid_prompts.hip).  The general kernel takes the others: 1: score products of 16-bit rows that are whole runs,
+// whatever the value rows are (QK16 above); 0: everything else.
+int hyb_sink_attention_tiles_form(const void* q, long q_row, long q_head, const void* k_cache, const void* v_cache,
+                                  const void* out, int nseq, int max_q, int D, int E, int v_stride, int dt) {
+    if ((dt == 0 || dt == 2) &&
+        prompt_attention_ok(q, q_row, q_head, k_cache, v_cache, out, nseq, max_q, D, E, v_stride, dt == 2))
+        return 2;
+    return dt == 0 && D % 16 == 0 && ((size_t)k_cache | (size_t)q) % 16 == 0 && q_row % 8 == 0 && q_head % 8 == 0;
+}
+
 // Sequences seq0 .. seq0 + nseq - 1 of a prefill-form step (cu_q / block_tables indexed by the
 // absolute sequence number); max_q: longest portion among them.
 int hyb_sink_attention_tiles(const void* q, long q_row, long q_head, const void* k_cache,
@@ -647,16 +710,14 @@ int hyb_sink_attention_tiles(const void* q, long q_row, long q_head, const void*
     if (G <= 0 || H % G || !hyb_sink_attention_tiles_ok(D, E)) return 1;
 #define TILES_ARGS q, q_row, q_head, k_cache, v_cache, block_tables, max_blocks, block_size, cu_q, \
                    positions, sink, gate, gate_row, out, scale, nseq, seq0, max_q, H, G, D, E
-    // operands in whole 16-byte runs: 8 times faster over bfloat16 at 8 x 1k tokens of 128-wide heads and 4
-    // times at 2 x 300; over float 2.3 times at 3 x 600 with a window (hybrid_prompts.hip)
-    if ((dt == 0 || dt == 2) &&
-        prompt_attention_ok(q, q_row, q_head, k_cache, v_cache, out, nseq, max_q, D, E, rule.v_stride, dt == 2))
-        return dt == 0 ? prompt_attention(TILES_ARGS, rule, s) : prompt_attention_f32(TILES_ARGS, rule, s);
+    const int form = hyb_sink_attention_tiles_form(q, q_row, q_head, k_cache, v_cache, out, nseq, max_q, D, E,
+                                                   rule.v_stride, dt);
+    if (form == 2) return dt == 0 ? prompt_attention(TILES_ARGS, rule, s) : prompt_attention_f32(TILES_ARGS, rule, s);
 #define TILES_E(T, DP)                                                                       \
     do {                                                                                     \
-        if (E <= 64) return launch_tiles<T, DP, 64>(TILES_ARGS, rule, s);                    \
-        if (E <= 128) return launch_tiles<T, DP, 128>(TILES_ARGS, rule, s);                  \
-        if (DP <= 128) return launch_tiles<T, (DP <= 128 ? DP : 64), 256>(TILES_ARGS, rule, s); \
+        if (E <= 64) return launch_tiles<T, DP, 64>(TILES_ARGS, form == 1, rule, s);         \
+        if (E <= 128) return launch_tiles<T, DP, 128>(TILES_ARGS, form == 1, rule, s);       \
+        if (DP <= 128) return launch_tiles<T, (DP <= 128 ? DP : 64), 256>(TILES_ARGS, form == 1, rule, s); \
         return 1;                                                                            \
     } while (0)
 #define TILES_D(T)                                   \

@@ -47,6 +47,7 @@ _tiles = _sig("hyb_sink_attention_tiles", _P, _L, _L, _P, _P, _P, _I, _I, _P, _P
 _tiles_ok = _lib.hyb_sink_attention_tiles_ok
 _tiles_ok.argtypes = [_I, _I]
 _tiles_ok.restype = _I
+_tiles_form = _sig("hyb_sink_attention_tiles_form", _P, _L, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I)
 _split = _sig("hyb_sink_attention_split", _P, _L, _L, _P, _P, _P, _I, _I, _P, _P, _P, _L, _P, _P, _F,
               _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, *_POOL, _I, _P)
 _split_ok = _lib.hyb_sink_attention_split_ok

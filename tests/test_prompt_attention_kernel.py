@@ -51,13 +51,12 @@ def caches(k, v, rows, G, D, E, bs, pooled):
     return kc, vc, k[rows * G:].view(n, pr, G, D), v[rows * G:].view(n, pr, G, E)
 
 
-@pytest.mark.parametrize("H,G,D,E", [(2, 1, 128, 128), (8, 4, 64, 64), (16, 2, 8, 16), (3, 3, 72, 136), (2, 2, 256, 120),
-                                     (1, 1, 40, 256), (4, 2, 136, 64), (2, 1, 128, 256)])
-@pytest.mark.parametrize("bs", [16, 64, 128])
-@pytest.mark.parametrize("opt", [dict(), dict(window=40, keep_first=5), dict(chunk=48), dict(slopes=True),
-                                 dict(window=33, pool=8, temps=True, softcap=5.0)])
-@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
-def test_every_instance_and_option(H, G, D, E, bs, opt, dt):
+OPTIONS = [dict(), dict(window=40, keep_first=5), dict(chunk=48), dict(slopes=True),
+           dict(window=33, pool=8, temps=True, softcap=5.0)]
+
+
+def compare(H, G, D, E, bs, opt, dt, shift=0):
+    """The kernel that takes these operands (q ``shift`` numbers off 16 bytes) against the plain form."""
     opt = dict(opt)
     pool = opt.get("pool", 0)
     g, k, v, rows, tables, cu_q, cu_k, pos = step(G, D, E, bs, pooled=pool, dt=dt)
@@ -69,20 +68,40 @@ def test_every_instance_and_option(H, G, D, E, bs, opt, dt):
         opt["slopes"] = torch.rand(H, generator=g) * 0.2
     if opt.pop("temps", None):
         opt["temps"] = torch.randn(H, generator=g)
-    if H % 8:                                            # q rows of whole 16-byte runs only with H % 8 == 0
+    if H % 8 or shift:                                   # q rows of whole 16-byte runs only with H % 8 == 0
         q = q.contiguous()
 
-    def call(f, to, **kw):
+    def call(f, to, q, **kw):
         kc, vc, kp, vp = caches(to(k), to(v), rows, G, D, E, bs, pool)
         o = {n: to(x) if torch.is_tensor(x) else x for n, x in opt.items()}
         if pool:
             o.update(k_pool=kp, v_pool=vp)
-        return f(to(q), kc, vc, to(cu_q), to(cu_k), to(tables), D ** -0.5, None if sink is None else to(sink),
+        return f(q, kc, vc, to(cu_q), to(cu_k), to(tables), D ** -0.5, None if sink is None else to(sink),
                  to(gate), to(torch.zeros(T, H, E, dtype=dt)), **kw, **o)
 
-    want = call(ref.sink_attention_prefill, lambda x: x)
-    got = call(hk.sink_attention_prefill, lambda x: x.cuda(), positions=pos.cuda(), max_q=max(PORTIONS)).cpu()
+    want = call(ref.sink_attention_prefill, lambda x: x, q)
+    gq = q.cuda()
+    if shift:
+        gq = torch.empty(q.numel() + shift, dtype=dt, device="cuda")[shift:].view(q.shape).copy_(q)
+    got = call(hk.sink_attention_prefill, lambda x: x.cuda(), gq, positions=pos.cuda(), max_q=max(PORTIONS)).cpu()
     close(got, want, float(v.abs().max()))
+
+
+@pytest.mark.parametrize("H,G,D,E", [(2, 1, 128, 128), (8, 4, 64, 64), (16, 2, 8, 16), (3, 3, 72, 136), (2, 2, 256, 120),
+                                     (1, 1, 40, 256), (4, 2, 136, 64), (2, 1, 128, 256)])
+@pytest.mark.parametrize("bs", [16, 64, 128])
+@pytest.mark.parametrize("opt", OPTIONS)
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_every_instance_and_option(H, G, D, E, bs, opt, dt):
+    compare(H, G, D, E, bs, opt, dt)
+
+
+@pytest.mark.parametrize("H,G,D,E,shift", [(4, 2, 128, 100, 0), (8, 4, 64, 20, 0), (3, 1, 144, 36, 0),    # whole key rows
+                                           (4, 2, 36, 64, 0), (2, 1, 64, 64, 1), (2, 2, 128, 128, 3)])    # neither
+@pytest.mark.parametrize("opt", OPTIONS)
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_every_option_of_the_general_kernel(H, G, D, E, shift, opt, dt):
+    compare(H, G, D, E, 64, opt, dt, shift)
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
