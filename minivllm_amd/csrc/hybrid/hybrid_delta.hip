@@ -24,10 +24,14 @@ constexpr int MAX_TAPS = 32;
 // head, DC = 1 (a decay per head) or D (one per head and key channel); dt_bias has H * DC
 // entries, decay out [T, H * DC].
 // conv_w [C, taps] (q, k, v rows stacked), conv_state [slots, taps-1, C].
-template <typename T>
+// TAPS: how many taps, if known at compile time (2 to 4: unrolled), else 0.  6000 rows, head sizes that
+// delta_prepare_rows_kernel does not take: D 100, 16 / 8 heads, 3200 channels in runs of eight, bfloat16 140 us with taps
+// of run time and a channel per thread, 77 like this; D 36, 1600 channels 76 / 46; rows off 16 bytes (no runs),
+// float, 6 / 3 heads of 128 55 / 50.
+template <typename T, int TAPS>
 __global__ void delta_prepare_kernel(const T* __restrict__ proj, long row_stride, int b_off,
                                      const T* __restrict__ a, long a_row, int DC,
-                                     const float* __restrict__ conv_w, int taps,
+                                     const float* __restrict__ conv_w, int taps_rt,
                                      const float* __restrict__ conv_b, int ssd,
                                      const float* __restrict__ a_log,
                                      const float* __restrict__ dt_bias,
@@ -36,8 +40,10 @@ __global__ void delta_prepare_kernel(const T* __restrict__ proj, long row_stride
                                      const int* __restrict__ slots, const int* __restrict__ row_seq,
                                      float* __restrict__ qn, float* __restrict__ kn,
                                      float* __restrict__ vv, float* __restrict__ beta,
-                                     float* __restrict__ decay, int H, int G, int D, int E) {
+                                     float* __restrict__ decay, int H, int G, int D, int E,
+                                     int vec8) {
     extern __shared__ float y[];                     // [2GD] convolved + silu q, k
+    const int taps = TAPS ? TAPS : taps_rt;
     const long t = blockIdx.x;
     const int b = row_seq ? row_seq[t] : (int)t;
     if (b < 0) return;
@@ -48,6 +54,39 @@ __global__ void delta_prepare_kernel(const T* __restrict__ proj, long row_stride
     const bool has_past = positions[first] > 0;
     const int C = 2 * G * D + H * E, GD = G * D;
     const float* tail = conv_state + (long)slot * (taps - 1) * C;
+    if (TAPS > 0 && vec8) {
+        // eight channels per thread and step, every load of the step issued before its first use:
+        // one 16-byte (bf16) load per tap and the channels' taps as whole rows of the tap table
+        constexpr int NT = TAPS ? TAPS : 1;
+        for (int c = threadIdx.x * 8; c < C; c += blockDim.x * 8) {
+            float x[NT][8], w[8][NT];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const int back = NT - 1 - j;
+                if (i - back >= 0) load_run<T, 8>(proj + (t - back) * row_stride + c, x[j]);
+                else if (has_past) load_run<float, 8>(tail + (long)(NT - 1 + i - back) * C + c, x[j]);
+                else {
+#pragma unroll
+                    for (int z = 0; z < 8; ++z) x[j][z] = 0.f;
+                }
+            }
+#pragma unroll
+            for (int z = 0; z < 8; ++z)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) w[z][j] = conv_w[(long)(c + z) * NT + j];
+            float acc[8];
+#pragma unroll
+            for (int z = 0; z < 8; ++z) {
+                float a = conv_b ? conv_b[c + z] : 0.f;
+#pragma unroll
+                for (int j = 0; j < NT; ++j) a += x[j][z] * w[z][j];
+                acc[z] = siluf_(a);
+            }
+            float* dst = (c < 2 * GD) ? y + c : vv + t * (long)(H * E) + (c - 2 * GD);
+            *reinterpret_cast<float4*>(dst) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+            *reinterpret_cast<float4*>(dst + 4) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+        }
+    } else
     for (int c = threadIdx.x; c < C; c += blockDim.x) {
         float acc = conv_b ? conv_b[c] : 0.f;
         for (int j = 0; j < taps; ++j) {             // tap j reads the input `taps-1-j` tokens back
@@ -506,6 +545,15 @@ bool channel_delta_step(const void* qn, const void* kn, const void* vv, const vo
 
 extern "C" {
 
+// Which kernel prepares the rows.  2: delta_prepare_rows_kernel (heads of whole runs of eight channels, 2 to 4 taps);
+// 1: a workgroup per row, channels in runs of eight, whatever the heads' size is; 0: a channel per thread and step.
+int hyb_delta_prepare_form(const void* proj, long row_stride, const void* conv_w, const void* conv_state, const void* qn,
+                           const void* kn, const void* vv, int taps, int H, int G, int D, int E) {
+    if (taps < 2 || taps > 4 || (H * E) % 8 || row_stride % 8 || ((size_t)proj | (size_t)conv_state | (size_t)vv) % 16) return 0;
+    if (D % 8 == 0 && D <= 2048 && ((size_t)conv_w | (size_t)qn | (size_t)kn) % 16 == 0) return 2;
+    return (G * D) % 8 == 0;
+}
+
 int hyb_delta_prepare(const void* proj, long row_stride, int b_off, const void* a, long a_row,
                       int DC, const void* conv_w, int taps, const void* conv_b, int ssd,
                       const void* a_log, const void* dt_bias, void* conv_state,
@@ -517,9 +565,9 @@ int hyb_delta_prepare(const void* proj, long row_stride, int b_off, const void* 
     const int C = 2 * G * D + H * E;
     const size_t lds = 2 * (size_t)G * D * sizeof(float);
     if (lds > 64 * 1024) return 1;
-    const int block = D <= 2048 ? 2048 / D * D : 0;       // channels per workgroup: whole heads, 8 a thread
-    const bool runs = taps >= 2 && taps <= 4 && D % 8 == 0 && block && (H * E) % 8 == 0 && row_stride % 8 == 0 &&
-                      ((size_t)proj | (size_t)conv_w | (size_t)conv_state | (size_t)qn | (size_t)kn | (size_t)vv) % 16 == 0;
+    const int form = hyb_delta_prepare_form(proj, row_stride, conv_w, conv_state, qn, kn, vv, taps, H, G, D, E);
+    const bool runs = form == 2;
+    const int block = runs ? 2048 / D * D : 0;            // channels per workgroup: whole heads, 8 a thread
     // rows per workgroup: up to 16, as long as there are workgroups for every CU twice over (6100 rows of 4096
     // channels: 8 rows 3 us more, 32 rows 12 us)
     const int blocks = runs ? (C + block - 1) / block : 1;
@@ -538,16 +586,23 @@ int hyb_delta_prepare(const void* proj, long row_stride, int b_off, const void* 
     if (runs && taps == 4) PREP_ROWS(4);
     else if (runs && taps == 3) PREP_ROWS(3);
     else if (runs) PREP_ROWS(2);
-    else
-        HYB_DISPATCH(dt, hipLaunchKernelGGL(delta_prepare_kernel<T>, dim3(T_),
-                                            dim3(C >= 2048 && T_ <= 1024 ? 1024 : 256), lds, s,
-                                            (const T*)proj, row_stride, b_off, (const T*)a, a_row, DC,
-                                            (const float*)conv_w, taps, (const float*)conv_b, ssd,
-                                            (const float*)a_log,
-                                            (const float*)dt_bias, (const float*)conv_state,
-                                            (const int*)cu_q, (const int*)positions, (const int*)slots,
-                                            (const int*)row_seq, (float*)qn, (float*)kn, (float*)vv,
-                                            (float*)beta, (float*)decay, H, G, D, E));
+    else {
+#define PREP(TAPS)                                                                                 \
+    HYB_DISPATCH(dt, hipLaunchKernelGGL((delta_prepare_kernel<T, TAPS>), dim3(T_),                 \
+                                        dim3(C >= 2048 && T_ <= 1024 ? 1024 : 256), lds, s,        \
+                                        (const T*)proj, row_stride, b_off, (const T*)a, a_row, DC, \
+                                        (const float*)conv_w, taps, (const float*)conv_b, ssd,     \
+                                        (const float*)a_log,                                       \
+                                        (const float*)dt_bias, (const float*)conv_state,           \
+                                        (const int*)cu_q, (const int*)positions, (const int*)slots,\
+                                        (const int*)row_seq, (float*)qn, (float*)kn, (float*)vv,   \
+                                        (float*)beta, (float*)decay, H, G, D, E, form == 1))
+        if (taps == 4) PREP(4);
+        else if (taps == 3) PREP(3);
+        else if (taps == 2) PREP(2);
+        else PREP(0);
+#undef PREP
+    }
 #undef PREP_ROWS
     if (hipGetLastError() != hipSuccess) return 2;
     if (taps > 1 && !(runs && !cu_q)) {

@@ -55,6 +55,7 @@ _split_ok.argtypes = [_I, _I]
 _split_ok.restype = _I
 _prep = _sig("hyb_delta_prepare", _P, _L, _I, _P, _L, _I, _P, _I, _P, _I, _P, _P, _P, _P, _P, _P, _P,
              _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P)
+_prep_form = _sig("hyb_delta_prepare_form", _P, _L, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I)
 _scan = _sig("hyb_delta_scan", _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _P)
 _scan_ws = _sig("hyb_delta_scan_ws", _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I)
 _scan_ws.restype = _L

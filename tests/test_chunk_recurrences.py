@@ -211,7 +211,9 @@ def test_bits_of_the_matrix_lstm(forget):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("H,G,D,E,taps", [(2, 1, 8, 8, 4), (1, 1, 48, 40, 2), (3, 1, 16, 24, 3), (2, 2, 128, 64, 4)])
+@pytest.mark.parametrize("H,G,D,E,taps", [(2, 1, 8, 8, 4), (1, 1, 48, 40, 2), (3, 1, 16, 24, 3), (2, 2, 128, 64, 4),
+                                          # heads that are no whole runs in rows that are, rows that are none
+                                          (4, 2, 12, 16, 4), (2, 2, 20, 4, 2), (8, 4, 6, 3, 3), (3, 1, 10, 7, 4), (2, 1, 8, 8, 6)])
 @pytest.mark.parametrize("ssd,channel", [(False, False), (False, True), (True, False)])
 def test_delta_prepare_rows(dt, H, G, D, E, taps, ssd, channel):
     """Several rows per workgroup: portions that start, end or lie inside its rows, shorter than the taps, with

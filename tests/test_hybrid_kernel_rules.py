@@ -18,3 +18,21 @@ def test_prompt_attention(D, E, v_stride, shift, q_row, form):
     # a value cache or an output off 16 bytes takes nothing from the score products
     if form == 2:
         assert hk._tiles_form(*a[:4], AT + 2, *a[5:], 0) == 1 and hk._tiles_form(*a[:5], AT + 2, *a[6:], 0) == 1
+
+
+@pytest.mark.parametrize("H,G,D,E,taps,row,form", [
+    (16, 8, 128, 128, 4, 6208, 2), (2, 1, 8, 8, 2, 32, 2), (2, 1, 2048, 8, 3, 4128, 2), (16, 8, 128, 128, 5, 6208, 0),
+    # heads that are no whole runs in rows that are; no runs at all
+    (16, 8, 100, 128, 4, 3680, 1), (16, 8, 36, 64, 2, 1632, 1), (8, 4, 2050, 8, 3, 16480, 1),
+    (15, 15, 12, 12, 3, 572, 0), (3, 3, 12, 12, 3, 120, 0), (6, 3, 128, 128, 4, 1548, 0)])
+def test_delta_preparation(H, G, D, E, taps, row, form):
+    a = [AT, row, AT, AT, AT, AT, AT, taps, H, G, D, E]
+    assert hk._prep_form(*a) == form
+    for off in (2, 4, 5):                              # the taps' table and the unit vectors' address: the rows kernel only
+        b = list(a)
+        b[off] += 4
+        assert hk._prep_form(*b) == (min(form, 1) if G * D % 8 == 0 else form)
+    for off in (0, 3, 6):
+        b = list(a)
+        b[off] += 4
+        assert hk._prep_form(*b) == 0
