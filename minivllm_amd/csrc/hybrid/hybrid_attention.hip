@@ -449,22 +449,25 @@ static int launch_tiles(const void* q, long q_row, long q_head, const void* k_ca
 // read by 16 neighbouring lanes with 16-byte (bf16: EPL = 8 elements) loads, so a wave streams
 // four whole rows per step.  A 16-lane group walks its own keys (group kg of 16 per workgroup,
 // keys kg, kg + 16, ...) with a private running softmax for NR query heads of the KV head, two keys per
-// trip, the next trip's rows on their way; the groups' partials meet in LDS, the workgroups' (one per
-// context split) in a workspace that `sink_attention_merge_kernel` folds together with the sink term
-// and the gate.
-// EPL / VPL: elements of a K / V row per lane (D = 16 EPL, E = 16 VPL).
-// Bound by the K / V stream and by what a workgroup does once.  64 rows of 512..1024 keys, 16 / 8 heads of 128,
-// bf16: 73 -> 51 us with the merge (210 MB), from registers for the heads there are, no division per key,
-// rows ahead that are not kept in the caches, one exponential per partial instead of one per output
-// column, and longer spans.  Four keys per trip: 54 us.
-template <typename T, int N> struct RawRun;          // N consecutive elements as loaded (used once: not cached)
+// trip; the groups' partials meet in LDS, the workgroups' (one per context split) in a workspace that
+// `sink_attention_merge_kernel` folds together with the sink term and the gate.
+// EPL / VPL: elements of a K / V row per lane (D = 16 EPL, E = 16 VPL).  ONCE: rows that one workgroup alone reads
+// are not kept in the caches (bfloat16; float rows come faster through them, 85 against 92 us).
+// Bound by the K / V stream and by waves enough to keep it busy, so by registers: nothing is loaded ahead of the
+// trip it is used in (that took 36 registers and a wave per SIMD or two).  64 rows of 512..1024 keys, 8 KV heads
+// of 128, with the merge, at 1 / 2 / 3 / 4 / 6 / 8 query heads per KV head: bfloat16 47 / 50 / 55 / 63 / 92 / 108 us,
+// float 81 / 84 / 86 / 90 / 110 / 122 (4 of 4 with rows ahead: 100 and 112).
+template <typename T, int N> struct RawRun;          // N consecutive elements as loaded
 template <int N> struct RawRun<bf16_t, N> {
     static constexpr int W = N >= 8 ? 4 : N / 2, M = N / 2 / W;       // words per load, loads
     typedef __attribute__((ext_vector_type(W))) uint32_t vec;
     vec v[M];
-    __device__ __forceinline__ void load(const bf16_t* p) {
+    template <bool ONCE> __device__ __forceinline__ void load(const bf16_t* p) {
 #pragma unroll
-        for (int i = 0; i < M; ++i) v[i] = __builtin_nontemporal_load(reinterpret_cast<const vec*>(p) + i);
+        for (int i = 0; i < M; ++i) {
+            const vec* at = reinterpret_cast<const vec*>(p) + i;
+            v[i] = ONCE ? __builtin_nontemporal_load(at) : *at;
+        }
     }
     __device__ __forceinline__ void widen(float* o) const {
 #pragma unroll
@@ -477,9 +480,12 @@ template <int N> struct RawRun<bf16_t, N> {
 template <int N> struct RawRun<float, N> {
     typedef __attribute__((ext_vector_type(4))) float vec;
     vec v[N / 4];
-    __device__ __forceinline__ void load(const float* p) {
+    template <bool ONCE> __device__ __forceinline__ void load(const float* p) {
 #pragma unroll
-        for (int i = 0; i < N / 4; ++i) v[i] = __builtin_nontemporal_load(reinterpret_cast<const vec*>(p) + i);
+        for (int i = 0; i < N / 4; ++i) {
+            const vec* at = reinterpret_cast<const vec*>(p) + i;
+            v[i] = ONCE ? __builtin_nontemporal_load(at) : *at;
+        }
     }
     __device__ __forceinline__ void widen(float* o) const {
 #pragma unroll
@@ -487,7 +493,7 @@ template <int N> struct RawRun<float, N> {
     }
 };
 
-template <typename T, int EPL, int VPL, int NR, bool EXT>
+template <typename T, int EPL, int VPL, int NR, bool ONCE, bool EXT>
 __global__ void __launch_bounds__(256)
 sink_attention_split_kernel(const T* __restrict__ q, long q_row, long q_head,
                             const T* __restrict__ k_cache, const T* __restrict__ v_cache,
@@ -523,28 +529,24 @@ sink_attention_split_kernel(const T* __restrict__ q, long q_row, long q_head,
 #pragma unroll
         for (int i = 0; i < VPL; ++i) acc[r][i] = 0.f;
     }
-    RawRun<T, EPL> kr[2];
-    RawRun<T, VPL> vr[2];
-    auto fetch = [&](int vj) {                    // keys vj, vj + 16 (behind the end: the last again)
+    for (int vj = k_begin + kg; vj < k_end; vj += 32) {
+        RawRun<T, EPL> kr[2];
+        RawRun<T, VPL> vr[2];
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
-            const int v = min(vj + 16 * x, k_end - 1);
+            const int v = min(vj + 16 * x, k_end - 1);         // (behind the end: the last again)
             long slot;
             if (EXT) slot = vis.row(v, table, block_size, rule);
             else {
                 const int j = vis.key(v), p = shift >= 0 ? j >> shift : j / block_size;
                 slot = (long)table[p] * block_size + (j - p * block_size);
             }
-            kr[x].load(k_cache + (slot * G + g) * (long)D + lane16 * EPL);
-            vr[x].load(v_cache + (slot * G + g) * (long)rule.v_stride + lane16 * VPL);
+            kr[x].template load<ONCE>(k_cache + (slot * G + g) * (long)D + lane16 * EPL);
+            vr[x].template load<ONCE>(v_cache + (slot * G + g) * (long)rule.v_stride + lane16 * VPL);
         }
-    };
-    if (k_begin + kg < k_end) fetch(k_begin + kg);
-    for (int vj = k_begin + kg; vj < k_end; vj += 32) {
         float kf[2][EPL], vf[2][VPL];
 #pragma unroll
         for (int x = 0; x < 2; ++x) { kr[x].widen(kf[x]); vr[x].widen(vf[x]); }
-        if (vj + 32 < k_end) fetch(vj + 32);
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
             if (vj + 16 * x >= k_end) break;
@@ -605,6 +607,14 @@ sink_attention_split_kernel(const T* __restrict__ q, long q_row, long q_head,
     }
 }
 
+// Query heads of a KV head (of R) that a workgroup takes: as few workgroups as four each allow, as they all read the
+// same rows, and as many heads in each as that needs (5: 3 + 2 and not 4 + 1, where the second would work out 3 that
+// are not there).
+extern "C" int hyb_sink_attention_split_heads(int R) {
+    const int chunks = (R + 3) / 4;
+    return (R + chunks - 1) / chunks;
+}
+
 template <typename T, int EPL, int VPL>
 static int launch_split(const void* q, long q_row, long q_head, const void* k_cache,
                         const void* v_cache, const void* block_tables, int max_blocks,
@@ -612,9 +622,10 @@ static int launch_split(const void* q, long q_row, long q_head, const void* k_ca
                         const void* gate, long gate_row, void* out, void* ws, float scale, int B,
                         int H, int G, int splits, KeyRule rule, hipStream_t s) {
     constexpr int E = 16 * VPL;
+    constexpr bool ONCE = sizeof(T) == 2;
     const int R = H / G;
-#define SPLIT_LAUNCH_X(NR, EXT)                                                                   \
-    hipLaunchKernelGGL((sink_attention_split_kernel<T, EPL, VPL, NR, EXT>),                       \
+#define SPLIT_LAUNCH_X(NR, ONCE, EXT)                                                             \
+    hipLaunchKernelGGL((sink_attention_split_kernel<T, EPL, VPL, NR, ONCE, EXT>),                 \
                        dim3(B, G * ((R + NR - 1) / NR), splits), dim3(256),                       \
                        16 * NR * (E + 3) * sizeof(float), s, (const T*)q, q_row, q_head, (const T*)k_cache, \
                        (const T*)v_cache, (const int*)block_tables, max_blocks, block_size,       \
@@ -622,9 +633,12 @@ static int launch_split(const void* q, long q_row, long q_head, const void* k_ca
                        rule)
 #define SPLIT_LAUNCH(EXT)                                                                         \
     do {                                                                                          \
-        if (R == 1) SPLIT_LAUNCH_X(1, EXT);                                                       \
-        else if (R == 2) SPLIT_LAUNCH_X(2, EXT);                                                  \
-        else SPLIT_LAUNCH_X(4, EXT);                                                              \
+        if (R == 1) SPLIT_LAUNCH_X(1, ONCE, EXT);                                                 \
+        else if (R == 2) SPLIT_LAUNCH_X(2, ONCE, EXT);                                            \
+        else if (R == 3) SPLIT_LAUNCH_X(3, ONCE, EXT);                                            \
+        else if (R == 4) SPLIT_LAUNCH_X(4, ONCE, EXT);                                            \
+        else if (hyb_sink_attention_split_heads(R) == 3) SPLIT_LAUNCH_X(3, false, EXT);           \
+        else SPLIT_LAUNCH_X(4, false, EXT);                                                       \
     } while (0)
     if (rule.temps || rule.softcap > 0.f || rule.pool > 0) SPLIT_LAUNCH(true); else SPLIT_LAUNCH(false);
 #undef SPLIT_LAUNCH

@@ -50,6 +50,7 @@ _tiles_ok.restype = _I
 _tiles_form = _sig("hyb_sink_attention_tiles_form", _P, _L, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I)
 _split = _sig("hyb_sink_attention_split", _P, _L, _L, _P, _P, _P, _I, _I, _P, _P, _P, _L, _P, _P, _F,
               _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, *_POOL, _I, _P)
+_split_heads = _sig("hyb_sink_attention_split_heads", _I)
 _split_ok = _lib.hyb_sink_attention_split_ok
 _split_ok.argtypes = [_I, _I]
 _split_ok.restype = _I
@@ -316,15 +317,15 @@ def _i32c(t):
     return t
 
 
-def decode_splits(batch: int, kv_heads: int, heads: int, max_context_len, wide: bool = False) -> int:
-    """Workgroups per (sequence, KV head group) of the split decode kernel: four per CU (``wide``, float
-    caches: eight; their rows keep a wave busy for longer), each with at least 128 keys of the longest
-    context.  64 sequences of 512..1024 keys, 8 KV heads: 51 us with four, 55 with eight, 75 with two; over
-    float 96 and 93."""
-    groups = kv_heads * -(-(heads // kv_heads) // 4)
-    want = max(1, (2048 if wide else 1024) // max(batch * groups, 1))
-    room = max(1, (int(max_context_len) + 127) // 128) if max_context_len else 8
-    return max(1, min(16, want, room))
+def decode_splits(batch: int, kv_heads: int, heads: int, max_context_len) -> int:
+    """Workgroups per (sequence, KV head group) of the split decode kernel: four per CU, each with at least 128
+    keys of the longest context; up to eight per CU where one of them would walk more than 2048 keys, for the batch
+    that waits for its longest sequence.  64 sequences of 512..1024 keys, 8 KV heads, 2 heads each: 50 us with four,
+    54 with eight (float 84 and 88); 64 of 200 keys and one of 8192: 287 and 174 (float 358 and 220)."""
+    groups = max(1, batch * kv_heads * -(-(heads // kv_heads) // 4))
+    longest = int(max_context_len) if max_context_len else 1024
+    want = max(1, 1024 // groups, min(2048 // groups, -(-longest // 2048)))
+    return min(16, want, max(1, (longest + 127) // 128))
 
 
 def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale, sink, gate, out,
@@ -346,7 +347,7 @@ def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale
             seen = min(int(seen), int(window) + int(keep_first) + (int(seen) // pool if pool else 0))
         if chunk and seen:
             seen = min(int(seen), int(chunk))
-        splits = decode_splits(B, G, H, seen, es == 4)
+        splits = decode_splits(B, G, H, seen)
         ws = torch.empty((B * H * splits * (E + 2),), dtype=torch.float32, device=q.device)
         if gate is not None:
             assert gate.stride(1) == 1 and gate.dtype == q.dtype

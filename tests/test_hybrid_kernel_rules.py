@@ -36,3 +36,18 @@ def test_delta_preparation(H, G, D, E, taps, row, form):
         b = list(a)
         b[off] += 4
         assert hk._prep_form(*b) == 0
+
+
+def test_heads_of_a_decode_workgroup():
+    """No workgroup more than groups of four need, no head worked out twice that could be left out."""
+    assert [hk._split_heads(r) for r in range(1, 13)] == [1, 2, 3, 4, 3, 3, 4, 4, 3, 4, 4, 4]
+
+
+@pytest.mark.parametrize("batch,kv_heads,heads,longest,splits", [
+    (64, 8, 16, 1024, 2), (64, 8, 16, 2048, 2), (32, 8, 16, 4096, 4), (1, 8, 16, 100, 1), (1, 8, 16, 8192, 16),
+    # a long context in a batch that fills the card: spans of up to 2048 keys, eight workgroups per CU at most
+    (64, 8, 16, 8192, 4), (128, 8, 16, 4096, 2), (128, 8, 16, 2048, 1), (256, 8, 16, 1 << 17, 1), (16, 8, 64, 1 << 17, 8),
+    # an unknown context
+    (64, 8, 16, 0, 2), (1, 8, 16, None, 8)])
+def test_splits_of_a_decode_batch(batch, kv_heads, heads, longest, splits):
+    assert hk.decode_splits(batch, kv_heads, heads, longest) == splits

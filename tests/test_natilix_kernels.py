@@ -159,7 +159,10 @@ def test_sink_attention_prefill_long_portions(dt, H, G, D, E):
 
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("H,G,D,E,maxctx", [(4, 2, 128, 128, 2000), (8, 1, 64, 64, None), (2, 2, 256, 128, 300),
-                                            (6, 2, 128, 64, 100000)])
+                                            (6, 2, 128, 64, 100000),
+                                            # further numbers of heads per KV head: 5 as 3 + 2, 7 as 4 + 3, 9 as three of 3
+                                            (3, 3, 64, 64, 2000), (10, 2, 128, 128, 2000), (7, 1, 64, 128, 300),
+                                            (9, 1, 256, 64, None), (12, 2, 64, 64, 1500)])
 def test_sink_attention_decode_split_contexts(dt, H, G, D, E, maxctx):
     """The head sizes of the split-context decode kernel: several splits, contexts shorter
     than a split, rows without a sequence, q rows strided as inside a projection output."""
