@@ -625,8 +625,9 @@ class ModelRunner:
             budget = int(total * cfg.gpu_memory_utilization) - used - max(peak - current, 0)
             if self.hybrid:
                 # no warm-up ran: keep room for a step's activations (fp32 stream + the widest
-                # projection outputs) and for the recurrent state slots
+                # projection outputs), for what a mixer needs beside them and for the recurrent state slots
                 budget -= self._state_bytes() + cfg.max_num_batched_tokens * self._widest_row_bytes()
+                budget -= self._step_workspace()
             num_blocks = budget // block_bytes
             if self.world_size > 1:        # every rank must agree on the block count
                 t = torch.tensor([num_blocks], dtype=torch.int64, device=self.device)
@@ -659,6 +660,12 @@ class ModelRunner:
     def _state_bytes(self) -> int:
         return sum(self.num_state_slots * 4 * int(np.prod(shape, dtype=np.int64))
                    for d in self.model.state_layers() for _, shape in d.state_spec())
+
+    def _step_workspace(self) -> int:
+        """The layers run one after the other, so the largest of their workspaces."""
+        cfg = self.cfg
+        return max([m.step_workspace(cfg.max_num_batched_tokens, cfg.max_num_sequences)
+                    for m in self.model.modules() if hasattr(m, "step_workspace")] + [0])
 
     def _widest_row_bytes(self) -> int:
         widest = max([p.shape[0] for p in self.model.parameters() if p.dim() == 2] + [1])

@@ -55,6 +55,12 @@ class GatedDeltaRule(nn.Module):
         H, D, E = self.num_heads, self.head_dim, self.v_head_dim
         return [("state", (H, D, E)), ("conv_state", (max(self.taps - 1, 0), self.conv_channels))]
 
+    def step_workspace(self, tokens: int, seqs: int) -> int:
+        """Bytes a step of up to that many tokens and sequences needs on the GPU beside its activations."""
+        if self.channel_decay:
+            return 0
+        return ops.delta_scan_workspace(tokens, seqs, self.num_heads, self.num_kv_heads, self.head_dim, self.v_head_dim)
+
     def split_sizes(self):
         """Column blocks of the fused input projection: q, k, v, gate, beta, decay (with
         ``channel_decay``: q, k, v, beta; decay and gate come as arguments of ``forward``)."""

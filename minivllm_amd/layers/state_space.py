@@ -59,6 +59,10 @@ class StateSpaceDuality(nn.Module):
         spec = [("state", (H, N, E)), ("conv_state", (max(self.taps - 1, 0), C))]
         self.slots: List[StateSlots] = [StateSlots(spec) for _ in range(passes)]
 
+    def step_workspace(self, tokens: int, seqs: int) -> int:
+        """Bytes a step of up to that many tokens and sequences needs on the GPU beside its activations."""
+        return ops.delta_scan_workspace(tokens, seqs, self.num_heads, self.groups, self.state_size, self.v_head_dim)
+
     def split_sizes(self):
         """Column blocks of the fused input projection in the order this module reads them:
         C, B, x (the convolved channels), the gate z, the step size's pre-activation."""

@@ -336,6 +336,12 @@ def delta_scan(qn, kn, vv, beta, decay, state, cu_q, positions, slots, correct=T
     return _seqmix(qn).delta_scan(qn, kn, vv, beta, decay, state, cu_q, positions, slots, correct)
 
 
+def delta_scan_workspace(tokens, seqs, H, G, D, E):
+    """Bytes that ``delta_scan`` takes on the GPU, beyond its results, in a step of up to that many tokens and
+    sequences."""
+    return _hybrid().delta_scan_workspace(tokens, seqs, H, G, D, E)
+
+
 def gated_head_norm(o, w, gate, eps, out_dtype, act="silu"):
     return _seqmix(o).gated_head_norm(o, w, gate, eps, out_dtype, act)
 

@@ -436,6 +436,14 @@ def delta_scan(qn, kn, vv, beta, decay, state, cu_q, positions, slots, correct=T
     return o
 
 
+def delta_scan_workspace(tokens: int, seqs: int, H: int, G: int, D: int, E: int) -> int:
+    """The most bytes ``delta_scan`` takes for itself in a step of up to that many tokens and sequences: it grows with
+    both, and steps of too few tokens for their sequences take none."""
+    seqs = min(seqs, tokens, max(tokens // 20, tokens - 1024))
+    aligned = 256
+    return _scan_ws(aligned, aligned, aligned, aligned, aligned, tokens, seqs, H, G, D, E) if seqs > 0 else 0
+
+
 def gated_head_norm(o, w, gate, eps, out_dtype, act="silu"):
     T, H, E = o.shape
     assert gate.stride(-1) == 1 and gate.dtype == out_dtype and w.numel() in (E, H * E)
