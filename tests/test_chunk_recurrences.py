@@ -73,8 +73,9 @@ def test_mlstm(H, D, E, cap):
         want[0][s], want[1][s], want[2][s] = S, N[:, None], m[:, None]
     got, literal = run((-n_in) % 8), run((-n_in) % 8 + 1)
     for x, y, w in zip(got, literal, [o] + want):
-        # sums of up to 200 fp32 terms: 200 * 2^-24; no further off than the literal kernel is, but for that
-        assert off(x, w) <= 2 * off(y, w) + 200 * 2.0 ** -24, (off(x, w), off(y, w))
+        # the same sums in fp32, rounded in other places: twice the literal kernel's error and one rounding in the
+        # mean (a part of eight bits less in any operand is 2^-17)
+        assert off(x, w) <= 2 * off(y, w) + 2.0 ** -26, (off(x, w), off(y, w))
     owned = torch.zeros(T, dtype=torch.bool)
     for b, s in enumerate(SLOTS):
         owned[cu[b]:cu[b + 1]] = s >= 0
@@ -119,7 +120,7 @@ def test_delta_rule(H, G, D, E, correct, fast):
         want[s] = S
     got, literal = run(0), run(1)
     for x, y, w in zip(got, literal, (o, want)):
-        assert off(x, w) <= 2 * off(y, w) + 200 * 2.0 ** -24, (off(x, w), off(y, w))
+        assert off(x, w) <= 2 * off(y, w) + 2.0 ** -26, (off(x, w), off(y, w))      # as above
     owned = torch.zeros(T, dtype=torch.bool)
     for b, s in enumerate(SLOTS):
         owned[cu[b]:cu[b + 1]] = s >= 0
