@@ -289,6 +289,32 @@ def test_single_tokens(H, G, D, E, rule):
     assert bool((got[2] == 0).all())
 
 
+@pytest.mark.parametrize("H,G,D,E", [(16, 8, 128, 128), (8, 4, 64, 64), (4, 4, 256, 64), (2, 2, 64, 256), (8, 8, 128, 16)])
+@pytest.mark.parametrize("rule", ["delta", "channel", "plain"])
+def test_bits_of_single_tokens(H, G, D, E, rule):
+    """Neither the outputs nor the state are further from 64 bits than those of the token-by-token kernels, which
+    take the same rows as portions of one token (a twentieth for the sample's spread)."""
+    g = torch.Generator().manual_seed(D + E)
+    B = 64
+    q, k = (torch.nn.functional.normalize(torch.randn(B, G, D, generator=g), dim=-1).cuda() for _ in range(2))
+    q = q * D ** -0.5
+    v, beta = torch.randn(B, H, E, generator=g).cuda(), torch.rand(B, H, generator=g).cuda()
+    decay = (0.7 + 0.3 * (torch.rand(B, H, D, generator=g) if rule == "channel" else torch.rand(B, H, generator=g))).cuda()
+    state = torch.randn(B, H, D, E, generator=g).cuda()
+    pos, slots = torch.ones(B, dtype=torch.int32).cuda(), torch.arange(B, dtype=torch.int32).cuda()
+    got = []
+    for cu in (None, torch.arange(B + 1, dtype=torch.int32).cuda()):
+        st = state.clone()
+        got.append((hk.delta_scan(q, k, v, beta, decay, st, cu, pos, slots, rule != "plain"), st))
+    qd, kd = (x.double().repeat_interleave(H // G, 1) for x in (q, k))
+    S = state.double() * (decay.double()[..., None] if rule == "channel" else decay.double()[..., None, None])
+    u = v.double() - ((S * kd[..., None]).sum(2) if rule != "plain" else 0)
+    S = S + kd[..., None] * (beta.double()[..., None] * u)[:, :, None]
+    for x, y, w in zip(*got, ((S * qd[..., None]).sum(2), S)):
+        single, literal = off(x, w.cpu()), off(y, w.cpu())
+        assert single <= 1.05 * literal, (single, literal)
+
+
 INF, NAN = float("inf"), float("nan")
 
 
