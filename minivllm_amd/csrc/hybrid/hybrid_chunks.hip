@@ -11,9 +11,10 @@
 //   A = (Q K^T) o W;  O = diag(c) Q S_0 + A V;  n . q = c_t n_0 . q_t + sum_i A_ti
 //   S_end = c_end S_0 + K^T diag(W_end) V,  n_end = c_end n_0 + K^T W_end
 //
-// Every factor is a product of the same a and b the recurrence multiplies by, all <= 1: no quotients, no logarithms of products.  W comes from the products inside blocks of 16
-// tokens: in a pair of different blocks it is (a .. to t inside its block) (whole blocks between) (a .. from
-// i to its block's end) b_i, on the diagonal the running product.
+// Every factor is a product of the same a and b the recurrence multiplies by, all <= 1: no quotients, no
+// logarithms of products.  W comes from the products inside blocks of 16 tokens: in a pair of different blocks it
+// is (a .. to t inside its block) (whole blocks between) (a .. from i to its block's end) b_i, on the diagonal the
+// running product.
 //
 // q, k, v ARE bfloat16; what is fp32 (the weighted scores, the state, the weighted values) is cut into
 // three parts of eight bits, all of its 24, and multiplied part by part on

@@ -32,8 +32,8 @@
 // It stays in the sums once it is there, so a portion whose outputs and state come out finite met none; any other is
 // walked again from its first token by the recurrence itself (same workgroup, its own columns).
 //
-// 8 portions of 512..1024 tokens, 16 / 8 heads of 128: 54 + 140 us, against 645 us token by token.  The walk
-// takes 9 us a chunk of 64 columns; its six phases between barriers use the matrix units, the
+// 8 portions of 512..1024 tokens, 16 / 8 heads of 128: 55 + 155 us, against 645 us token by token.  The walk
+// takes 9.7 us a chunk of 64 columns; its six phases between barriers use the matrix units, the
 // vector units (cutting) and the LDS for about 2.5 us each and hardly overlap: one workgroup per CU is all that
 // LDS and registers hold.  32 columns per workgroup 160 us; all waves in both roles, two workgroups per CU
 // 213 us (registers spill); k's rows fetched a whole chunk ahead 193 us (spill).

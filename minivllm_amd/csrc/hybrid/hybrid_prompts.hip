@@ -17,7 +17,7 @@
 // and pooled rows look every row up.  Heads of one KV head go to one XCD, long contexts start first.
 //
 // Bound by the wave's own chain of score product, softmax and value product with two waves per SIMD
-// (about 220 registers).  8 prompts of 512..1024 tokens, 16 / 8 heads of 128, sink and gate: 68 us
+// (about 220 registers).  8 prompts of 512..1024 tokens, 16 / 8 heads of 128, sink and gate: 69 us
 // = 350 TFLOP/s of the products a bf16 softmax would need, against 566 us of the fp32 instruction over
 // tiles widened to fp32 in LDS and loaded between two barriers.  Two parts per weight instead of three
 // would take 58 us and hold 16 bits of it; key tiles of 32 take 70 us, the two halves of a tile of 64

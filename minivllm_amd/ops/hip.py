@@ -497,7 +497,7 @@ def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
 # ------------------------------------------------------- weight-streaming GEMM
 SKINNY_MAX_ROWS = 16
 SKINNY_PAYS_ROWS = 16                 # up to here the kernel beats the library (see skinny_gemm_pays)
-SKINNY_MIN_WEIGHT_BYTES = 8 << 20     # below this a projection is launch-latency bound anyway
+SKINNY_MIN_WEIGHT_BYTES = 8 << 20     # below this an unmeasured projection goes to the library (see skinny_gemm_pays)
 
 
 def skinny_gemm_ok(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False) -> bool:
@@ -528,7 +528,10 @@ def skinny_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False
     Qwen3-32B gate_up+SwiGLU 124 vs 91 us against it, and its down projection 81 vs 134 us for
     it again), so the engine measures both on its own weights at start-up (tune_skinny_gemm)
     and this function looks the answer up.  Unmeasured shapes: the kernel for fused SwiGLU and
-    for N, K <= 4096 when the matrix is large enough to cover the chip, the library otherwise."""
+    for N, K <= 4096 when the matrix is large enough to cover the chip, the library otherwise.
+    Below 8 MB that is not the faster choice for few rows (kernel / library, 1, 4 and 16 rows:
+    1024 x 3072 6.3 / 9.2, 6.9 / 9.2 and 8.8 / 9.3 us, 2048 x 1024 3.9 / 5.9, 4.3 / 6.0 and
+    6.1 / 6.0); the measurement at start-up, which engines run unless it is switched off, finds that."""
     if x.dim() != 2 or x.shape[0] > SKINNY_PAYS_ROWS or not skinny_gemm_ok(x, weight, swiglu):
         return False
     n, k = weight.shape
@@ -537,7 +540,7 @@ def skinny_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False
         return choice
     n_out = n // 2 if swiglu else n
     if n_out // 16 < 192 or n * k * 2 < SKINNY_MIN_WEIGHT_BYTES:
-        return False                       # too few tiles to cover the chip / launch-bound anyway
+        return False                       # too few tiles to cover the chip
     return swiglu or (n <= 4096 and k <= 4096)
 
 
