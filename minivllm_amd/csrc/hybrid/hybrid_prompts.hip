@@ -10,18 +10,26 @@
 // is cut into parts of eight bits (PARTS of them; three hold all 24) that are multiplied one after the
 // other.  The score accumulators are the B operand as they stand, V^T fragments are transposed LDS reads.
 //
-// Workgroup = 4 waves x 32 consecutive queries of one (sequence, query head); keys in tiles of TK, K and
-// V each an LDS image filled by direct global -> LDS loads, two buffers, the next tile requested
-// before the current one's products.  A page that holds whole tiles is read through one buffer
-// descriptor per tile (rows behind the context are out of its range and read as zeros); smaller pages
-// and pooled rows look every row up.  Heads of one KV head go to one XCD, long contexts start first.
+// Workgroup = 4 waves x 32 consecutive queries of one (sequence, query head); keys in tiles of 32, K and V each an
+// LDS image filled by direct global -> LDS loads two tiles ahead (three buffers of keys, four of values: a tile's
+// values are read a tile later than its keys).  Where a page holds whole tiles (WHOLE) a tile is read through one
+// buffer descriptor, where it holds runs of eight tokens a wave's rows are (rows behind the context are out of its
+// range and read as zeros); other pages and pooled rows look every row up.  Heads of one KV head go to one XCD, long
+// contexts start first.
 //
-// Bound by the wave's own chain of score product, softmax and value product with two waves per SIMD
-// (about 220 registers).  8 prompts of 512..1024 tokens, 16 / 8 heads of 128, sink and gate: 69 us
-// = 350 TFLOP/s of the products a bf16 softmax would need, against 566 us of the fp32 instruction over
-// tiles widened to fp32 in LDS and loaded between two barriers.  Two parts per weight instead of three
-// would take 58 us and hold 16 bits of it; key tiles of 32 take 70 us, the two halves of a tile of 64
-// unrolled 73 us (registers spill).
+// A wave issues in order, and a matrix instruction leaves the unit busy for 32 cycles after the 8 of its issue: what
+// the softmax does in vector instructions has to stand between them.  So a tile's exponentials and the first half
+// of its parts are formed between the value products of the tile BEFORE, the second half between the score products of
+// the tile AFTER, a few instructions behind each product.  No maximum is formed ahead of the exponentials: they are
+// taken against the last reference, and formed again where that turns out too low.  The scalar work of a tile
+// (where the next lies) was a fifth of its time as expressions of the tile's number: it is kept up instead.
+//
+// 8 prompts of 512..1024 tokens, 16 / 8 heads of 128, sink and gate: 68 -> 63.8 us for the layer, 5 to 7 of which the clearing
+// of the output takes; one of 1024 tokens alone 46 -> 36 (a tile in 2260 cycles of a lone wave: 1024 of products,
+// some 1000 of vector issue beside them; two waves on a SIMD take 1600 each).  Before that the waves formed score
+// product, softmax and value product one after the other (a tile of 32 in 3350 cycles).  What is left: the clock (1.9
+// GHz under this load), 6 us at the two ends of a workgroup, and the last workgroups, of which not all CUs have one.
+// Two parts per weight instead of three would hold 16 bits of it.
 #include "hybrid_keys.h"
 #include "hybrid_chunks.h"
 
@@ -29,11 +37,9 @@ using namespace hyb;
 
 namespace {
 
-constexpr int PARTS = 3;
-
 struct PromptArgs {
     const uint16_t* q; long q_row, q_head;
-    const uint16_t *k_cache, *v_cache;
+    const uint16_t *k_cache, *v_cache;             // latent attention: the formed keys and values [H, formed_rows, D | E]
     const int* tables; int max_blocks, block_size;
     const int *cu_q, *positions;
     const float* sink;
@@ -42,6 +48,20 @@ struct PromptArgs {
     float scale;
     int H, G, D, E, seq0;
     KeyRule rule;
+    // latent attention: the turned key part of a token (its cache row's last P numbers) and of the queries
+    const uint16_t* q_turned; long turned_row;     // [T, H, P]
+    const uint16_t* latents; int latent_row, P;    // cache rows of latent_row numbers
+    long formed_rows;
+    uint32_t page_magic;                           // key / block_size == key * page_magic >> 32 for every key there can be (0: none)
+};
+
+// what a wave needs of the key rows' second part in row_by_keys
+struct NoTail {};
+struct LatentTail {
+    const bf16_t *q, *rows;
+    int row, P;
+    const int* table;
+    int block_size;
 };
 
 // rows of the wave (lane: a row and half of its columns, acc times f) with an infinity or a NaN
@@ -63,10 +83,10 @@ __device__ __forceinline__ uint32_t rows_not_finite(const f32x16* acc, float f, 
 // part, padding column times anything, and zero weight times what no query sees would make NaN of them.  NaN and
 // infinities stay in a row's sums once they are there, so a row that comes out finite met none, and the others are
 // worked out again by all lanes of their wave: one query, key after key, nothing in parts.
-template <typename T, bool EXT>
+template <typename T, bool EXT, class Tail = NoTail>
 __device__ void row_by_keys(const T* q, const T* k_cache, const T* v_cache, const int* table, int block_size, int ctx,
                             float scale, float slope, const float* sink, const T* gate, T* out, int G, int g, int h,
-                            int D, int E, const KeyRule& rule) {
+                            int D, int E, const KeyRule& rule, Tail tail = {}) {
     constexpr int N = 256 / kWave;                 // of up to 256 columns, lane + 64 i are this lane's
     const int lane = threadIdx.x & 63;
     const VisibleKeys vis(ctx, rule);
@@ -77,9 +97,15 @@ __device__ void row_by_keys(const T* q, const T* k_cache, const T* v_cache, cons
         acc[i] = 0.f;
     }
     float m = sink ? sink[h] : NO_SINK_MAX, l = sink ? 1.f : 0.f;
+    constexpr bool TAIL = !std::is_same<Tail, NoTail>::value;
     for (int v = 0; v < vis.count; ++v) {
-        const long row = vis.row(v, table, block_size, rule) * G + g;
+        const long row = TAIL ? vis.key(v) : vis.row(v, table, block_size, rule) * G + g;
         float s = 0.f;
+        if constexpr (TAIL) {
+            const T* r = tail.rows + ((long)tail.table[row / tail.block_size] * tail.block_size + row % tail.block_size + 1) *
+                                         tail.row - tail.P;
+            for (int i = lane; i < tail.P; i += 64) s += ld(r + i) * (ld(tail.q + i) * scale);
+        }
 #pragma unroll
         for (int i = 0; i < N; ++i)
             if (lane + 64 * i < D) s += ld(k_cache + row * D + lane + 64 * i) * qf[i];
@@ -102,23 +128,39 @@ __device__ void row_by_keys(const T* q, const T* k_cache, const T* v_cache, cons
         if (lane + 64 * i < E) st(out + lane + 64 * i, acc[i] * f);
 }
 
-template <int DP, int EP, int TK, bool EXT>
-__global__ void __launch_bounds__(256, DP + EP > 256 ? 1 : 2)
+// tiles of 32 keys that the sequences ahead of b have (by all lanes of a wave)
+__device__ __forceinline__ int formed_tiles_before(const int* cu_q, const int* positions, int b, int lane) {
+    int n = 0;
+    for (int i = lane; i < b; i += 64) {
+        const int r = cu_q[i], len = cu_q[i + 1] - r;
+        if (len > 0) n += (positions[r] + len + 31) / 32;
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) n += __shfl_xor(n, o, kWave);
+    return __builtin_amdgcn_readfirstlane(n);
+}
+
+// DP, EP: columns of the K and V images; RP: columns of a second key image (0: none), the shared key part of
+// latent attention; PARTS: parts a weight is cut into.
+template <int DP, int RP, int EP, int PARTS, bool EXT, bool WHOLE>
+__global__ void __launch_bounds__(256, DP + RP + EP > 256 + (RP ? 128 : 0) ? 1 : 2)
 prompt_attention_kernel(PromptArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__       // (the host pass only needs the launch stub)
-    static_assert(DP % 64 == 0 && EP % 64 == 0 && TK % 32 == 0);
-    constexpr int KS = DP / 16, NB = EP / 32;      // steps of the score product; 32-wide value blocks
-    constexpr int KT = TK * DP * 2, VT = TK * EP * 2, BUF = KT + VT;          // bytes
-    constexpr int KIT = KT / 4096, VIT = VT / 4096;                           // 16-byte pieces per thread
-    constexpr int KSW = DP % 128 == 0 ? 16 : 8, VSW = EP % 128 == 0 ? 16 : 8; // chunks a swizzle permutes
+    static_assert(DP % 64 == 0 && EP % 64 == 0 && RP % 64 == 0 && (PARTS == 2 || PARTS == 3) && !(RP && !WHOLE) && !(EXT && WHOLE));
+    constexpr bool LAT = RP > 0;
+    constexpr int TK = 32, KS = DP / 16, RS = RP / 16, NB = EP / 32;  // steps of the score product; 32-wide value blocks
+    constexpr int KT = TK * DP * 2, RT = TK * RP * 2, VT = TK * EP * 2;                     // bytes of an image
+    constexpr int KIT = KT / 4096, RIT = RT / 4096, VIT = VT / 4096, LOADS = KIT + RIT + VIT; // 16-byte pieces per thread
+    constexpr int KSW = DP % 128 == 0 ? 16 : 8, RSW = RP % 128 == 0 ? 16 : 8, VSW = EP % 128 == 0 ? 16 : 8; // chunks a swizzle permutes
+    constexpr int R_AT = 3 * KT, V_AT = 3 * (KT + RT);                // three buffers of keys, four of values
     extern __shared__ __attribute__((aligned(256))) char smem[];
 
     const int H = a.H, hx = blockIdx.x;
     const int h = H % 8 == 0 ? (hx & 7) * (H >> 3) + (hx >> 3) : hx;
     const int b = blockIdx.y + a.seq0, tile_q0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * 128;
-    const int row0 = a.cu_q[b], qlen = a.cu_q[b + 1] - row0;
+    const int row0 = __builtin_amdgcn_readfirstlane(a.cu_q[b]), qlen = __builtin_amdgcn_readfirstlane(a.cu_q[b + 1]) - row0;
     if (tile_q0 >= qlen) return;
-    const int start = a.positions[row0], G = a.G, g = h / (H / G);
+    const int start = __builtin_amdgcn_readfirstlane(a.positions[row0]), G = a.G, g = h / (H / G);
     const int* table = a.tables + (long)b * a.max_blocks;
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -126,7 +168,7 @@ prompt_attention_kernel(PromptArgs a) {
     const int wq0 = tile_q0 + wave * 32, qi = wq0 + l32;
     const bool qok = qi < qlen, wave_live = wq0 < qlen;
     const int qpos = start + qi;
-    bf16x8 qf[KS];
+    bf16x8 qf[KS + RS];
     {
         const uint16_t* qp = a.q + (long)(row0 + min(qi, qlen - 1)) * a.q_row + (long)h * a.q_head;
 #pragma unroll
@@ -136,7 +178,21 @@ prompt_attention_kernel(PromptArgs a) {
             if (d < a.D) raw = *reinterpret_cast<const uint4*>(qp + d);
             qf[s] = __builtin_bit_cast(bf16x8, raw);
         }
+        if constexpr (LAT) {
+            const uint16_t* rp = a.q_turned + (long)(row0 + min(qi, qlen - 1)) * a.turned_row + (long)h * a.P;
+#pragma unroll
+            for (int s = 0; s < RS; ++s) {
+                const int d = 16 * s + 8 * half;
+                uint4 raw = make_uint4(0, 0, 0, 0);
+                if (d < a.P) raw = *reinterpret_cast<const uint4*>(rp + d);
+                qf[KS + s] = __builtin_bit_cast(bf16x8, raw);
+            }
+        }
     }
+
+    // (asked for here: at the end they would be waited for)
+    const float gate = a.gate ? ld(a.gate + (long)(row0 + min(qi, qlen - 1)) * a.gate_row + h) : 0.f;
+    const float sink = a.sink ? a.sink[h] * LOG2E : 0.f;
 
     // ---- the tiles this workgroup walks: pooled rows, kept first tokens, the tokens its window reaches
     const KeyRule& rule = a.rule;
@@ -153,77 +209,182 @@ prompt_attention_kernel(PromptArgs a) {
     auto tile_key = [&](int t) { return (t < ptiles ? t : t < ptiles + ktiles ? t - ptiles : t - ptiles - ktiles + first_tile) * TK; };
 
     // ---- staging: slot c of an image (row c / chunks per row) receives the chunk that the swizzle puts
-    // there; chunks behind a row's end repeat chunk 0 (their queries are zeros, their columns not stored)
+    // there; chunks behind a row's end repeat chunk 0 (their queries are zeros, their columns not stored).
+    // A wave's piece of an image is a whole number of rows: they lie in one page where a page holds whole runs of
+    // eight tokens, and a descriptor reads them (rows behind the context are out of its range and read as zeros);
+    // where it holds whole tiles (WHOLE), one descriptor does for all pieces.
+    const int cols_k = a.D, cols_v = a.E;
     const int krow = G * a.D * 2, vrow = G * rule.v_stride * 2;     // bytes from one token's row to the next
-    int k_off[KIT], v_off[VIT];
-#pragma unroll
-    for (int i = 0; i < KIT; ++i) {
-        const int c = i * 256 + tid, row = c / (DP / 8);
-        int ch = (c % (DP / 8)) ^ swizzle<DP>(row);
-        if (ch * 8 >= a.D) ch = 0;
-        k_off[i] = row * krow + ch * 16;
-    }
-#pragma unroll
-    for (int i = 0; i < VIT; ++i) {
-        const int c = i * 256 + tid, row = c / (EP / 8);
-        int ch = (c % (EP / 8)) ^ swizzle<EP>(row);
-        if (ch * 8 >= a.E) ch = 0;
-        v_off[i] = row * vrow + ch * 16;
-    }
-    const bool whole = a.block_size % TK == 0;           // a tile of tokens lies in one page
-    typedef const __attribute__((address_space(4))) int* const_int_p;
-    auto page_of = [&](int t) {                          // through the scalar unit (the table is read-only here)
-        return *(const_int_p)(uintptr_t)(table + min(tile_key(t), wg_ctx - 1) / a.block_size);
+    const int rrow = LAT ? a.latent_row * 2 : 0;
+    int k_off[KIT], v_off[VIT], r_off[RIT > 0 ? RIT : 1];
+    auto slot_of = [&](auto cols, int i, int n, int row_bytes) {    // lane's source offset from the tile's first row
+        constexpr int C = decltype(cols)::value;
+        const int c = i * 256 + tid, row = c / (C / 8);
+        int ch = (c % (C / 8)) ^ swizzle<C>(row);
+        if (ch * 8 >= n) ch = 0;
+        return row * row_bytes + ch * 16;
     };
-    int page = 0;                                        // of the tile to be staged next
-    auto stage = [&](int t, int buf) {
-        const int key0 = tile_key(t);
-        const bool pooled = EXT && t < ptiles;
-        char* dst = smem + buf * BUF + wave * 1024;
-        if (whole && !pooled) {
-            const long slot = (long)page * a.block_size + key0 % a.block_size;
-            const int rows = min(TK, wg_ctx - key0) - 1;
-            const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<uint16_t*>(a.k_cache + (slot * G + g) * a.D), 0, rows * krow + a.D * 2, 0x00020000);
-            const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<uint16_t*>(a.v_cache + (slot * G + g) * rule.v_stride), 0, rows * vrow + a.E * 2, 0x00020000);
 #pragma unroll
-            for (int i = 0; i < KIT; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    kr, (__attribute__((address_space(3))) void*)(dst + i * 4096), 16, k_off[i], 0, 0, 0);
+    for (int i = 0; i < KIT; ++i) k_off[i] = slot_of(std::integral_constant<int, DP>{}, i, cols_k, LAT ? a.D * 2 : krow);
 #pragma unroll
-            for (int i = 0; i < VIT; ++i)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    vr, (__attribute__((address_space(3))) void*)(dst + KT + i * 4096), 16, v_off[i], 0, 0, 0);
+    for (int i = 0; i < VIT; ++i) v_off[i] = slot_of(std::integral_constant<int, EP>{}, i, cols_v, LAT ? a.E * 2 : vrow);
+    if constexpr (LAT) {
+#pragma unroll
+        for (int i = 0; i < RIT; ++i) r_off[i] = slot_of(std::integral_constant<int, RP>{}, i, a.P, rrow);
+    }
+    const bool runs = WHOLE || (a.page_magic && a.block_size % 8 == 0);
+    // (a division is some 40 instructions of a tile's 400)
+    auto page_index = [&](int key) { return (int)__umulhi((uint32_t)key, a.page_magic); };
+    auto in_page = [&](int key) { return key - page_index(key) * a.block_size; };
+    // bytes of a row inside a page (page_magic: a page's bytes fit 31 bits)
+    auto place = [&](int page, int in, int row_bytes) {
+        return (uint64_t)(uint32_t)page * (uint32_t)(a.block_size * row_bytes) + (uint32_t)(in * row_bytes);
+    };
+    const char* k_head = reinterpret_cast<const char*>(a.k_cache) + g * a.D * 2;
+    const char* v_head = reinterpret_cast<const char*>(a.v_cache) + (long)g * rule.v_stride * 2;
+    typedef const __attribute__((address_space(4))) int* const_int_p;
+    auto page_of = [&](int key) {                        // through the scalar unit (the table is read-only here)
+        return *(const_int_p)(uintptr_t)(table + page_index(min(key, wg_ctx - 1)));
+    };
+    const int last_page = page_index(wg_ctx - 1);
+    // LAT: rows of the formed keys and values ahead of this sequence's
+    long formed0 = 0;
+    if constexpr (LAT) formed0 = (long)formed_tiles_before(a.cu_q, a.positions, b, lane) * 32;
+    constexpr int RPK = 512 / (LAT ? RP : DP), RPV = 512 / EP;   // rows of a piece that is looked up by page
+    constexpr int PIT = LAT ? RIT : KIT;
+    // the tile to be staged next, kept up from tile to tile (as expressions of its number they were a fifth of the
+    // loop's time): its number, its first key, its LDS buffers; WHOLE: where it lies, tiles until the page or the run ends
+    int ahead = 0, s_key = 0, s_kbuf = 0, s_vbuf = 0, s_run = 0;
+    const char *s_k = nullptr, *s_v = nullptr, *s_r = nullptr;
+    int kpage[PIT], vpage[VIT];                          // requested ahead
+    auto locate = [&]() {                                // WHOLE: tile `ahead` begins a page, a run of tiles or the work
+        const int page = *(const_int_p)(uintptr_t)(table + min(page_index(s_key), last_page)), in = in_page(s_key);
+        s_run = (a.block_size - in) / TK;
+        if (ahead < ktiles) s_run = min(s_run, ktiles - ahead);
+        if constexpr (LAT) {
+            s_r = reinterpret_cast<const char*>(a.latents) + place(page, in, rrow) + rrow - a.P * 2;
+        } else {
+            s_k = k_head + place(page, in, krow);
+            s_v = v_head + place(page, in, vrow);
+        }
+    };
+    auto fetch_pages = [&]() {
+        if constexpr (!WHOLE) {
+            if (!runs || (EXT && ahead < ptiles)) return;
+#pragma unroll
+            for (int i = 0; i < PIT; ++i) kpage[i] = page_of(s_key + (4 * i + wave) * RPK);
+#pragma unroll
+            for (int i = 0; i < VIT; ++i) vpage[i] = page_of(s_key + (4 * i + wave) * RPV);
+        }
+    };
+    auto next_tile = [&]() {
+        ++ahead;
+        s_kbuf = s_kbuf == 2 * KT ? 0 : s_kbuf + KT;
+        s_vbuf = s_vbuf == 3 * VT ? 0 : s_vbuf + VT;
+        if constexpr (WHOLE) {
+            s_key += TK;
+            if constexpr (LAT) {
+                s_r += TK * rrow;
+                s_k += TK * a.D * 2;
+                s_v += TK * a.E * 2;
+            } else {
+                s_k += TK * krow;
+                s_v += TK * vrow;
+            }
+            if (--s_run == 0) {
+                const int jump = tile_key(ahead) - s_key;
+                s_key += jump;
+                if constexpr (LAT) {
+                    s_k += (long)jump * a.D * 2;
+                    s_v += (long)jump * a.E * 2;
+                }
+                locate();
+            }
+        } else {
+            s_key = tile_key(ahead);
+            fetch_pages();
+        }
+    };
+    // rows of a tile: `first` lies `rb` rows into it, `left` rows from the tile's start are there
+    auto source = [](const char* first, int rb, int left, int row_bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(first - (long)rb * row_bytes), 0, left * row_bytes, 0x00020000);
+    };
+    auto to_lds = [](__amdgpu_buffer_rsrc_t r, char* dst, int off) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, off, 0, 0, 0);
+    };
+    auto stage = [&]() {
+        const int key0 = s_key;
+        int left = min(TK, wg_ctx - key0);                           // (behind the last tile: zeros are staged)
+        asm volatile("" : "+s"(left));                               // (min and max in one are a vector instruction)
+        left = max(left, 0);
+        const bool pooled = EXT && ahead < ptiles;
+        char* kd = smem + s_kbuf + wave * 1024;
+        char* vd = smem + V_AT + s_vbuf + wave * 1024;
+        if constexpr (WHOLE) {
+            const int rows = !LAT ? left : left > 0 ? TK : 0;        // (formed rows fill their last tile)
+            const auto kr = source(s_k, 0, rows, LAT ? a.D * 2 : krow), vr = source(s_v, 0, rows, LAT ? a.E * 2 : vrow);
+#pragma unroll
+            for (int i = 0; i < KIT; ++i) to_lds(kr, kd + i * 4096, k_off[i]);
+#pragma unroll
+            for (int i = 0; i < VIT; ++i) to_lds(vr, vd + i * 4096, v_off[i]);
+            if constexpr (LAT) {
+                const auto rr = source(s_r, 0, left, rrow);
+                char* rd = smem + R_AT + s_kbuf / KT * RT + wave * 1024;
+#pragma unroll
+                for (int i = 0; i < RIT; ++i) to_lds(rr, rd + i * 4096, r_off[i]);
+            }
+        } else if (runs && !pooled) {
+#pragma unroll
+            for (int i = 0; i < KIT; ++i) {
+                const int rb = (4 * i + wave) * RPK;
+                to_lds(source(k_head + place(kpage[i], in_page(key0 + rb), krow), rb, left, krow), kd + i * 4096, k_off[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < VIT; ++i) {
+                const int rb = (4 * i + wave) * RPV;
+                to_lds(source(v_head + place(vpage[i], in_page(key0 + rb), vrow), rb, left, vrow), vd + i * 4096, v_off[i]);
+            }
         } else {
             const int lim = (pooled ? wg_nb : wg_ctx) - 1;
             auto cache_row = [&](int j) -> long {
                 return pooled ? rule.pooled_row(table, j) : (long)table[j / a.block_size] * a.block_size + j % a.block_size;
             };
+            int me = tid;
+            asm volatile("" : "+v"(me));                             // (worked out ahead of the loop it costs registers)
 #pragma unroll
             for (int i = 0; i < KIT; ++i) {
-                const int row = (i * 256 + tid) / (DP / 8);
+                const int row = (i * 256 + me) / (DP / 8);
                 const char* src = reinterpret_cast<const char*>(a.k_cache) +
                                   (cache_row(min(key0 + row, lim)) * G + g) * a.D * 2 + (k_off[i] - row * krow);
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                                 (__attribute__((address_space(3))) void*)(dst + i * 4096), 16, 0, 0);
+                                                 (__attribute__((address_space(3))) void*)(kd + i * 4096), 16, 0, 0);
             }
 #pragma unroll
             for (int i = 0; i < VIT; ++i) {
-                const int row = (i * 256 + tid) / (EP / 8);
+                const int row = (i * 256 + me) / (EP / 8);
                 const char* src = reinterpret_cast<const char*>(a.v_cache) +
                                   (cache_row(min(key0 + row, lim)) * G + g) * (long)rule.v_stride * 2 + (v_off[i] - row * vrow);
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                                 (__attribute__((address_space(3))) void*)(dst + KT + i * 4096), 16, 0, 0);
+                                                 (__attribute__((address_space(3))) void*)(vd + i * 4096), 16, 0, 0);
             }
         }
+    };
+    // all but the last tile's requests have landed, for all waves
+    auto tile_done = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" :: "n"(LOADS) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
     };
 
     // ---- LDS addresses of this lane's fragments inside a buffer
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)smem;
-    uint32_t k_addr[KSW / 2];                       // row l32, chunk 2 s + half: distinct for s < KSW / 2
+    uint32_t k_addr[KSW / 2], r_addr[LAT ? RSW / 2 : 1]; // row l32, chunk 2 s + half: distinct for s < KSW / 2
 #pragma unroll
     for (int s = 0; s < KSW / 2; ++s) k_addr[s] = lds0 + l32 * (DP * 2) + (((2 * s + half) ^ swizzle<DP>(l32)) << 4);
+    if constexpr (LAT) {
+#pragma unroll
+        for (int s = 0; s < RSW / 2; ++s) r_addr[s] = lds0 + R_AT + l32 * (RP * 2) + (((2 * s + half) ^ swizzle<RP>(l32)) << 4);
+    }
     // transposed reads: 16 lanes take 4 key rows x 16 columns and return 4 keys of one column each
     constexpr int NA = NB < VSW / 4 ? NB : VSW / 4; // value blocks with addresses of their own
     const int i16 = lane & 15, tr_row = 4 * half + (i16 >> 2);
@@ -234,7 +395,7 @@ prompt_attention_kernel(PromptArgs a) {
 #pragma unroll
         for (int hi = 0; hi < 2; ++hi) {
             const int row = tr_row + 8 * hi;
-            v_addr[n][hi] = lds0 + KT + row * (EP * 2) + (((4 * n + tr_chunk) ^ swizzle<EP>(row)) << 4) + (i16 & 1) * 8;
+            v_addr[n][hi] = lds0 + V_AT + row * (EP * 2) + (((4 * n + tr_chunk) ^ swizzle<EP>(row)) << 4) + (i16 & 1) * 8;
         }
 
     f32x16 acc[NB];
@@ -243,64 +404,183 @@ prompt_attention_kernel(PromptArgs a) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[n][e] = 0.f;
     float m_run = NO_SINK_MAX, l_run = 0.f;         // in log2 units of the scores
-    const float sc = (EXT ? rule.head_scale(a.scale, h) : a.scale) * (EXT ? 1.f : LOG2E);
     const float slope = rule.slopes ? rule.slopes[h] * LOG2E : 0.f;
+    // scores are scaled inside the exponential's argument where nothing but a positive factor is between
+    const float sc_all = (EXT ? rule.head_scale(a.scale, h) : a.scale) * (EXT ? 1.f : LOG2E);
+    const bool scaled_first = EXT || rule.slopes || !(sc_all > 0.f);
+    const float sc = scaled_first ? 1.f : sc_all;
 
-    page = page_of(0);
-    stage(0, 0);
-    if (n_tiles > 1) page = page_of(1);
-    __syncthreads();
-    for (int t = 0, buf = 0; t < n_tiles; ++t, buf ^= 1) {
-        if (t + 1 < n_tiles) {
-            stage(t + 1, buf ^ 1);
-            if (t + 2 < n_tiles) page = page_of(t + 2);
+    // ---- a tile's weights: the exponentials of both halves of its keys (e < 8, e >= 8 of a lane's 16) and the parts
+    // of the first are formed between the value products of the tile before, the parts of the second between the
+    // score products of the tile after
+    uint32_t pw[PARTS][2][4];                       // [part][half][pair]: the operand of the value products
+    float late[8];                                  // weights of the second half, not yet in parts
+    auto stay = [](auto& x, auto& y) { asm volatile("" : "+v"(x), "+v"(y)); };     // (the compiler would sink it all to its use)
+    constexpr int SPLITS = 4 * (PARTS - 1);         // steps in which a half's weights are cut
+    auto cut = [&](auto ic, float* w, int s) {      // step i: pair i / (PARTS - 1)
+        constexpr int i = decltype(ic)::value, j = i / (PARTS - 1), k = i % (PARTS - 1);
+        float x = w[2 * j], y = w[2 * j + 1];
+        if constexpr (PARTS == 3) {                 // the upper halves of what the parts before left over
+            if constexpr (k == 0) pw[0][s][j] = __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302);
+            x -= __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+            y -= __uint_as_float(__float_as_uint(y) & 0xffff0000u);
+            pw[k + 1][s][j] = __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302);
+            w[2 * j] = x;
+            w[2 * j + 1] = y;
+            stay(pw[0][s][j], pw[k + 1][s][j]);
+        } else {                                    // rounded parts
+            pw[0][s][j] = rounded(x, y);
+            rest(pw[0][s][j], x, y);
+            pw[1][s][j] = rounded(x, y);
+            stay(pw[0][s][j], pw[1][s][j]);
         }
-        const int key0 = tile_key(t);
-        const bool pooled = EXT && t < ptiles;
-#pragma unroll 1
-        for (int j = 0; j < TK / 32; ++j) {
-            const int k0 = key0 + 32 * j;
-            const bool live = wave_live && (pooled ? k0 < wave_nb
-                                                   : (k0 <= wave_last && (k0 < rule.keep_first || k0 + 32 > wave_lo)));
-            if (!live) continue;                                     // (uniform per wave)
-            f32x16 s_acc;
+    };
+    auto part = [&](int k, int s) { return __builtin_bit_cast(bf16x8, make_uint4(pw[k][s][0], pw[k][s][1], pw[k][s][2], pw[k][s][3])); };
+    // step i of n takes its share of the `of` pieces of work
+    auto share = [](auto ic, auto nc, auto ofc, auto&& f) {
+        constexpr int i = decltype(ic)::value, n = decltype(nc)::value, of = decltype(ofc)::value;
+        static_for<i * of / n, (i + 1) * of / n>(f);
+    };
+    // value products of the tile whose values lie at va, half s of its keys after the other; between them work(step)
+    // (inline asm: through the builtin the compiler would wait for the stage's loads in flight ahead of the first
+    // read; a pair of blocks is requested ahead)
+    constexpr int PAIRS = NB / 2, HALF = NB * PARTS, STEPS = 2 * HALF;
+    s16x4 vlo[2][2], vhi[2][2];
+    uint32_t va[NA][2];
+    auto read_v = [&](auto gc) {                    // group g: half g / PAIRS, blocks 2 (g % PAIRS) ..
+        constexpr int gi = decltype(gc)::value, s = gi / PAIRS;
+        static_for<0, 2>([&](auto dc) {
+            constexpr int d = decltype(dc)::value, n = 2 * (gi % PAIRS) + d;
+            constexpr int off = (n / NA) * NA * 64 + s * 16 * EP * 2;
+            const uint32_t a0 = va[n % NA][0], a1 = va[n % NA][1];
+            s16x4 x, y;
+            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(x) : "v"(a0), "n"(off));
+            asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(y) : "v"(a1), "n"(off));
+            vlo[gi & 1][d] = x;
+            vhi[gi & 1][d] = y;
+        });
+    };
+    auto open_values = [&](int buf) {               // (ahead of value_products, as soon as the addresses are free)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) s_acc[e] = 0.f;
-            uint32_t ka[KSW / 2];
+        for (int n = 0; n < NA; ++n) {
+            va[n][0] = v_addr[n][0] + buf;
+            va[n][1] = v_addr[n][1] + buf;
+        }
+        read_v(std::integral_constant<int, 0>{});
+    };
+    auto value_products = [&](auto&& work) {
+        static_for<0, 2 * PAIRS>([&](auto gc) {
+            constexpr int gi = decltype(gc)::value, s = gi / PAIRS, n0 = 2 * (gi % PAIRS);
+            if constexpr (gi + 1 < 2 * PAIRS) read_v(std::integral_constant<int, gi + 1>{});
+            s16x4 x0 = vlo[gi & 1][0], y0 = vhi[gi & 1][0], x1 = vlo[gi & 1][1], y1 = vhi[gi & 1][1];
+            asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(x0), "+v"(y0), "+v"(x1), "+v"(y1) : "n"(gi + 1 < 2 * PAIRS ? 4 : 0));
+            const bf16x8 v0 = join(x0, y0), v1 = join(x1, y1);
+            static_for<0, 2 * PARTS>([&](auto ic) {
+                constexpr int i = decltype(ic)::value, k = i / 2, d = i % 2;
+                acc[n0 + d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(d ? v1 : v0, part(k, s), acc[n0 + d], 0, 0, 0);
+                work(std::integral_constant<int, gi * 2 * PARTS + i>{});
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
+    };
+
+    // (behind the last tile more are requested, of keys that are not there: the pages stay those of the table)
+    if constexpr (LAT) {
+        const long at = h * a.formed_rows + formed0 + tile_key(0);
+        s_k = reinterpret_cast<const char*>(a.k_cache) + at * a.D * 2;
+        s_v = reinterpret_cast<const char*>(a.v_cache) + at * a.E * 2;
+    }
+    s_key = tile_key(0);
+    if constexpr (WHOLE) locate(); else fetch_pages();
+    stage();
+    next_tile();
+    stage();
+    next_tile();
+    tile_done();
+    // the tiles this wave has a share in (uniform): of the pooled ones the first, then those with kept first tokens,
+    // then from the first its window reaches to that of its last query
+    const int p_end = EXT ? (wave_nb + TK - 1) / TK : 0, keep_end = ptiles + (rule.keep_first + TK - 1) / TK;
+    const int win_begin = ptiles + ktiles + wave_lo / TK - first_tile, win_end = ptiles + ktiles + wave_last / TK - first_tile;
+    auto live_tile = [&](int t) -> int {
+        return wave_live && (EXT && t < ptiles ? t < p_end : (t < keep_end || t >= win_begin) && t <= win_end);
+    };
+    // buffers of the current tile; that of the tile whose value products are still to come (< 0: none)
+    int kbuf = 0, vbuf = 0, open = -1, t = 0;
+    auto turn = [&]() {
+        tile_done();
+        kbuf = kbuf == 2 * KT ? 0 : kbuf + KT;
+        vbuf = vbuf == 3 * VT ? 0 : vbuf + VT;
+        ++t;
+    };
+    while (true) {
+        for (; t < n_tiles && !live_tile(t); turn()) {
+            stage();
+            next_tile();
+        }
+        if (t >= n_tiles) break;
 #pragma unroll
-            for (int s = 0; s < KSW / 2; ++s) ka[s] = k_addr[s] + buf * BUF + j * (32 * DP * 2);
-            // (inline asm: through the builtin the compiler would wait for the stage's loads in flight
-            // ahead of the first read; AHEAD reads are in flight)
-            constexpr int KA = 4;
-            s16x8 kf[KS];
+        for (int k = 0; k < PARTS; ++k)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pw[k][i / 4][i % 4] = 0u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) late[i] = 0.f;
+        open = -1;
+        do {
+            const int k0 = tile_key(t);
+            const bool pooled = EXT && t < ptiles;
+            if constexpr (!WHOLE) stage();
+            // (K reads: inline asm, as through the builtin the compiler would wait for the stage's loads in flight ahead
+            // of the first; KA of them are in flight)
+            constexpr int N = KS + RS, KA = N < 8 ? N : 8;
+            s16x8 kf[N];
+            uint32_t ka[KSW / 2], ra[LAT ? RSW / 2 : 1];
             auto read_k = [&](auto ic) {
-                constexpr int i = decltype(ic)::value;
-                constexpr int off = (i / (KSW / 2)) * (KSW * 16);
-                const uint32_t a0 = ka[i % (KSW / 2)];
+                constexpr int i = decltype(ic)::value, j = i < KS ? i : i - KS;
+                constexpr int off = i < KS ? (j / (KSW / 2)) * (KSW * 16) : (j / (RSW / 2)) * (RSW * 16);
+                const uint32_t a0 = i < KS ? ka[j % (KSW / 2)] : ra[LAT ? j % (RSW / 2) : 0];
                 s16x8 x;
                 asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(x) : "v"(a0), "n"(off));
                 kf[i] = x;
             };
-            static_for<0, (KA < KS ? KA : KS)>(read_k);
-            static_for<0, KS>([&](auto ic) {
+            {
+#pragma unroll
+                for (int s = 0; s < KSW / 2; ++s) ka[s] = k_addr[s] + kbuf;
+                if constexpr (LAT) {
+#pragma unroll
+                    for (int s = 0; s < RSW / 2; ++s) ra[s] = r_addr[s] + kbuf / KT * RT;
+                }
+                static_for<0, KA>(read_k);
+            }
+            if constexpr (WHOLE) stage();                // (while the first reads are on their way)
+            f32x16 s_acc;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s_acc[e] = 0.f;
+            static_for<0, N>([&](auto ic) {
                 constexpr int i = decltype(ic)::value;
-                if constexpr (i + KA < KS) read_k(std::integral_constant<int, i + KA>{});
-                constexpr int left = KS - 1 - i < KA ? KS - 1 - i : KA;      // reads still in flight
+                if constexpr (i + KA < N) read_k(std::integral_constant<int, i + KA>{});
+                constexpr int left = N - 1 - i < KA ? N - 1 - i : KA;        // reads still in flight
                 s16x8 x = kf[i];
                 asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(x) : "n"(left));
                 s_acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, x), qf[i], s_acc, 0, 0, 0);
+                share(ic, std::integral_constant<int, N>{}, std::integral_constant<int, SPLITS>{},
+                      [&](auto jc) { cut(jc, late, 1); });
                 __builtin_amdgcn_sched_barrier(0);
             });
+            // (nothing open: the weights are zeros, of any values that are there)
+            open_values(open < 0 ? vbuf : open);
+            __builtin_amdgcn_sched_barrier(0);
             // lane: query qi, keys k0 + (e & 3) + 8 (e >> 2) + 4 half
+            if (scaled_first) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) s_acc[e] = EXT ? rule.capped(s_acc[e] * sc) * LOG2E : s_acc[e] * sc;
-            if (rule.slopes && !pooled) {
+                for (int e = 0; e < 16; ++e) s_acc[e] = EXT ? rule.capped(s_acc[e] * sc_all) * LOG2E : s_acc[e] * sc_all;
+                if (rule.slopes && !pooled) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) s_acc[e] -= slope * (float)(qpos - (k0 + (e & 3) + 8 * (e >> 2) + 4 * half));
+                    for (int e = 0; e < 16; ++e) s_acc[e] -= slope * (float)(qpos - (k0 + (e & 3) + 8 * (e >> 2) + 4 * half));
+                }
             }
-            const bool all_seen = pooled ? k0 + 32 <= rule.pooled_for(wave_first + 1)
-                                         : k0 + 31 <= wave_first && k0 >= wave_top;
-            if (!all_seen) {                                         // (one uniform branch, not one per score)
+            const bool all_seen = pooled ? k0 + TK <= rule.pooled_for(wave_first + 1)
+                                         : k0 + TK - 1 <= wave_first && k0 >= wave_top;
+            if (!all_seen) {                                             // (one uniform branch, not one per score)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     const int key = k0 + (e & 3) + 8 * (e >> 2) + 4 * half;
@@ -308,96 +588,84 @@ prompt_attention_kernel(PromptArgs a) {
                     s_acc[e] = seen ? s_acc[e] : -INFINITY;
                 }
             }
-            float mt = s_acc[0];
+            float w[16], l_new = 0.f, top = 0.f, f = 1.f;
+            bool grows = false;
+            const float neg = -m_run;
+            value_products([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                if constexpr (i < HALF) {
+                    share(ic, std::integral_constant<int, HALF>{}, std::integral_constant<int, 8>{}, [&](auto jc) {
+                        constexpr int j = decltype(jc)::value;
+                        w[2 * j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[2 * j], sc, neg));
+                        w[2 * j + 1] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[2 * j + 1], sc, neg));
+                        stay(w[2 * j], w[2 * j + 1]);
+                        l_new += w[2 * j];
+                        l_new += w[2 * j + 1];
+                        top = fmaxf(top, fmaxf(w[2 * j], w[2 * j + 1]));
+                        stay(l_new, top);
+                    });
+                    // The reference of the exponentials only moves when some row outgrows it by RESCALE (a tile's weights
+                    // are NaN or infinite or too large, so is the first one's): they are formed again.  The sums follow
+                    // once the products of the tile before are in them.
+                    if constexpr (i == HALF - 1) {
+                        grows = !__all(top <= 64.f && l_new == l_new);       // (2^RESCALE)
+                        if (grows) {
+                            float mt = s_acc[0];
 #pragma unroll
-            for (int e = 1; e < 16; ++e) mt = fmaxf(mt, s_acc[e]);
-            mt = fmaxf(mt, __shfl_xor(mt, 32, kWave));
-            // the reference of the exponentials only moves when some row outgrows it by RESCALE
-            if (!__all(mt - m_run <= RESCALE)) {
-                const float m_new = fmaxf(m_run, mt);
-                const float f = __builtin_amdgcn_exp2f(m_run - m_new);
-                l_run *= f;
+                            for (int e = 1; e < 16; ++e) mt = fmaxf(mt, s_acc[e]);
+                            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+                            const float m_new = fmaxf(m_run, fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) * sc);
+                            f = __builtin_amdgcn_exp2f(m_run - m_new);
+                            l_run *= f;
+                            m_run = m_new;
+                            l_new = 0.f;
 #pragma unroll
-                for (int n = 0; n < NB; ++n) acc[n] *= f;
-                m_run = m_new;
-            }
-            // part k of a pair of weights: the upper halves of what the parts before it left over
-            bf16x8 p[PARTS][2];
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                uint32_t w[PARTS][4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float x = __builtin_amdgcn_exp2f(s_acc[8 * s + 2 * j] - m_run);
-                    float y = __builtin_amdgcn_exp2f(s_acc[8 * s + 2 * j + 1] - m_run);
-                    l_run += x;
-                    l_run += y;
-#pragma unroll
-                    for (int k = 0; k < PARTS; ++k) {
-                        const uint32_t ux = __float_as_uint(x), uy = __float_as_uint(y);
-                        w[k][j] = __builtin_amdgcn_perm(uy, ux, 0x07060302);
-                        if (k + 1 < PARTS) {
-                            x -= __uint_as_float(ux & 0xffff0000u);
-                            y -= __uint_as_float(uy & 0xffff0000u);
+                            for (int e = 0; e < 16; ++e) {
+                                w[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[e], sc, -m_new));
+                                l_new += w[e];
+                            }
                         }
+                        l_run += l_new;
                     }
                 }
-#pragma unroll
-                for (int k = 0; k < PARTS; ++k)
-                    p[k][s] = __builtin_bit_cast(bf16x8, make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]));
-            }
-            // step i: value block i / 2, keys 16 (i & 1) .. of the 32; requested AHEAD steps early
-            constexpr int STEPS = 2 * NB, AHEAD = STEPS < 4 ? STEPS : 4;
-            s16x4 lo4[STEPS], hi4[STEPS];
-            uint32_t va[NA][2];
-#pragma unroll
-            for (int n = 0; n < NA; ++n) {
-                va[n][0] = v_addr[n][0] + buf * BUF + j * (32 * EP * 2);
-                va[n][1] = v_addr[n][1] + buf * BUF + j * (32 * EP * 2);
-            }
-            auto read_v = [&](auto ic) {
-                constexpr int i = decltype(ic)::value, n = i >> 1, s = i & 1;
-                constexpr int off = (n / NA) * NA * 64 + s * 16 * EP * 2;
-                const uint32_t a0 = va[n % NA][0], a1 = va[n % NA][1];
-                s16x4 x, y;
-                asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(x) : "v"(a0), "n"(off));
-                asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(y) : "v"(a1), "n"(off));
-                lo4[i] = x;
-                hi4[i] = y;
-            };
-            static_for<0, AHEAD>(read_v);
-            static_for<0, STEPS>([&](auto ic) {
-                constexpr int i = decltype(ic)::value, n = i >> 1, s = i & 1;
-                if constexpr (i + AHEAD < STEPS) read_v(std::integral_constant<int, i + AHEAD>{});
-                constexpr int left = 2 * (STEPS - 1 - i < AHEAD ? STEPS - 1 - i : AHEAD);   // reads still in flight
-                s16x4 x = lo4[i], y = hi4[i];
-                asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(x), "+v"(y) : "n"(left));
-                const s16x8 v = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-                const bf16x8 vf = __builtin_bit_cast(bf16x8, v);
-#pragma unroll
-                for (int k = 0; k < PARTS; ++k)
-                    acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, p[k][s], acc[n], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (i >= HALF)
+                    share(std::integral_constant<int, i - HALF>{}, std::integral_constant<int, HALF>{},
+                          std::integral_constant<int, SPLITS>{}, [&](auto jc) { cut(jc, w, 0); });
             });
-        }
-        __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) late[i] = w[8 + i];
+            if constexpr (WHOLE) next_tile();
+            if (grows) {
+#pragma unroll
+                for (int n = 0; n < NB; ++n) acc[n] *= f;
+            }
+            open = vbuf;
+            if constexpr (!WHOLE) next_tile();
+            turn();
+        } while (t < n_tiles && live_tile(t));
+        // tiles that are not this wave's may follow, and its values' buffer be used again: the products now
+        static_for<0, SPLITS>([&](auto jc) { cut(jc, late, 1); });
+        open_values(open);
+        value_products([](auto) {});
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // (the requests behind the last tile)
     if (!wave_live) return;
+    const PromptArgs z = arguments_anew<PromptArgs>();
     l_run += __shfl_xor(l_run, 32, kWave);
     float f;
-    if (a.sink) {
-        const float sk = a.sink[h] * LOG2E, M = fmaxf(m_run, sk);
+    if (z.sink) {
+        const float M = fmaxf(m_run, sink);
         f = __builtin_amdgcn_exp2f(m_run - M);
-        f = f / (l_run * f + __builtin_amdgcn_exp2f(sk - M));
+        f = f / (l_run * f + __builtin_amdgcn_exp2f(sink - M));
     } else {
         f = 1.f / l_run;
     }
     const long row = row0 + min(qi, qlen - 1);
-    if (a.gate) f *= sigmoidf_(ld(a.gate + row * a.gate_row + h));
+    if (z.gate) f *= sigmoidf_(gate);
     uint32_t lost = rows_not_finite<NB>(acc, f, qok);
     // both halves of the wave hold every second run of four columns of a row: swapped so that a
     // lane stores eight neighbouring ones
-    uint16_t* op = a.out + (row * H + h) * a.E;
+    uint16_t* op = z.out + (row * z.H + h) * z.E;
 #pragma unroll
     for (int n = 0; n < NB; ++n)
 #pragma unroll
@@ -407,20 +675,29 @@ prompt_attention_kernel(PromptArgs a) {
             for (int k = 0; k < 4; ++k)
                 w[k] = (uint32_t)bf16_bits(acc[n][4 * r + 2 * k] * f) |
                        ((uint32_t)bf16_bits(acc[n][4 * r + 2 * k + 1] * f) << 16);
-            const uint32_t s0 = half ? w[0] : w[2], s1 = half ? w[1] : w[3];
-            const uint32_t g0 = __shfl_xor(s0, 32, kWave), g1 = __shfl_xor(s1, 32, kWave);
-            const uint4 v = half ? make_uint4(g0, g1, w[2], w[3]) : make_uint4(w[0], w[1], g0, g1);
+            const auto r0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+            const auto r1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
             const int e = 32 * n + 8 * r + 8 * half;
-            if (qok && e < a.E && !(lost >> l32 & 1)) *reinterpret_cast<uint4*>(op + e) = v;
+            if (qok && e < z.E && !(lost >> l32 & 1)) *reinterpret_cast<uint4*>(op + e) = make_uint4(r0[0], r1[0], r0[1], r1[1]);
         }
     for (; lost; lost &= lost - 1) {
         const int i = __builtin_ctz(lost);
         const long r = row0 + wq0 + i;
-        row_by_keys<bf16_t, EXT>((const bf16_t*)a.q + r * a.q_row + (long)h * a.q_head, (const bf16_t*)a.k_cache,
-                                 (const bf16_t*)a.v_cache, table, a.block_size, start + wq0 + i + 1,
-                                 EXT ? rule.head_scale(a.scale, h) : a.scale, rule.slopes ? rule.slopes[h] : 0.f, a.sink,
-                                 a.gate ? a.gate + r * a.gate_row + h : nullptr, (bf16_t*)a.out + (r * H + h) * a.E, G, g,
-                                 h, a.D, a.E, rule);
+        const float scale = EXT ? z.rule.head_scale(z.scale, h) : z.scale;
+        if constexpr (LAT) {
+            const long at = h * z.formed_rows + formed0;
+            row_by_keys<bf16_t, false>((const bf16_t*)z.q + r * z.q_row + (long)h * z.q_head, (const bf16_t*)z.k_cache + at * z.D,
+                                       (const bf16_t*)z.v_cache + at * z.E, nullptr, 0, start + wq0 + i + 1, scale, 0.f,
+                                       z.sink, nullptr, (bf16_t*)z.out + (r * z.H + h) * z.E, 1, 0, h, z.D, z.E, z.rule,
+                                       LatentTail{(const bf16_t*)z.q_turned + r * z.turned_row + (long)h * z.P,
+                                                  (const bf16_t*)z.latents, z.latent_row, z.P, table, z.block_size});
+        } else {
+            row_by_keys<bf16_t, EXT>((const bf16_t*)z.q + r * z.q_row + (long)h * z.q_head, (const bf16_t*)z.k_cache,
+                                     (const bf16_t*)z.v_cache, table, z.block_size, start + wq0 + i + 1, scale,
+                                     z.rule.slopes ? z.rule.slopes[h] : 0.f, z.sink,
+                                     z.gate ? z.gate + r * z.gate_row + h : nullptr, (bf16_t*)z.out + (r * z.H + h) * z.E, z.G, g,
+                                     h, z.D, z.E, z.rule);
+        }
     }
 #endif
 }
@@ -665,6 +942,11 @@ prompt_attention_f32_kernel(PromptArgs32 a) {
 #endif
 }
 
+// floor(2^32 / n) + 1 is off by less than n / 2^32 of itself: exact below 2^32 / n
+uint32_t page_magic(int n, int max_blocks, long row_bytes) {
+    return n > 1 && (long)max_blocks * n * n < (1L << 32) && n * row_bytes < (1L << 31) ? (uint32_t)((1ull << 32) / n + 1) : 0;
+}
+
 template <int DP, int EP>
 int launch_f32(const PromptArgs32& a, int nseq, int max_q, hipStream_t s) {
     constexpr int lds = 3 * 32 * (DP + EP) * 2;
@@ -677,16 +959,25 @@ int launch_f32(const PromptArgs32& a, int nseq, int max_q, hipStream_t s) {
     return HYB_LAUNCH_OK();
 }
 
+template <int DP, int RP, int EP, int PARTS, bool EXT, bool WHOLE>
+int launch_form(const PromptArgs& a, int nseq, int max_q, hipStream_t s) {
+    constexpr int lds = 32 * 2 * (3 * (DP + RP) + 4 * EP);
+    static_assert(lds <= 160 * 1024);
+    if (lds > 64 * 1024) {
+        static const hipError_t once = hipFuncSetAttribute((const void*)prompt_attention_kernel<DP, RP, EP, PARTS, EXT, WHOLE>,
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (once != hipSuccess) return 2;
+    }
+    hipLaunchKernelGGL((prompt_attention_kernel<DP, RP, EP, PARTS, EXT, WHOLE>), dim3(a.H, nseq, (max_q + 127) / 128), dim3(256),
+                       lds, s, a);
+    return HYB_LAUNCH_OK();
+}
+
 template <int DP, int EP>
 int launch(const PromptArgs& a, int nseq, int max_q, hipStream_t s) {
-    constexpr int TK = DP + EP <= 256 ? 64 : 32, lds = 2 * TK * (DP + EP) * 2;
-    static_assert(lds <= 64 * 1024);
-    const dim3 grid(a.H, nseq, (max_q + 127) / 128);
-    if (a.rule.temps || a.rule.softcap > 0.f || a.rule.pool > 0)
-        hipLaunchKernelGGL((prompt_attention_kernel<DP, EP, TK, true>), grid, dim3(256), lds, s, a);
-    else
-        hipLaunchKernelGGL((prompt_attention_kernel<DP, EP, TK, false>), grid, dim3(256), lds, s, a);
-    return HYB_LAUNCH_OK();
+    if (a.rule.temps || a.rule.softcap > 0.f || a.rule.pool > 0) return launch_form<DP, 0, EP, 3, true, false>(a, nseq, max_q, s);
+    return a.page_magic && a.block_size % 32 == 0 ? launch_form<DP, 0, EP, 3, false, true>(a, nseq, max_q, s)
+                                                  : launch_form<DP, 0, EP, 3, false, false>(a, nseq, max_q, s);
 }
 
 }  // namespace
@@ -708,7 +999,8 @@ int prompt_attention(const void* q, long q_row, long q_head, const void* k_cache
                      const KeyRule& rule, hipStream_t s) {
     const PromptArgs a{(const uint16_t*)q, q_row, q_head, (const uint16_t*)k_cache, (const uint16_t*)v_cache,
                        (const int*)block_tables, max_blocks, block_size, (const int*)cu_q, (const int*)positions,
-                       (const float*)sink, (const bf16_t*)gate, gate_row, (uint16_t*)out, scale, H, G, D, E, seq0, rule};
+                       (const float*)sink, (const bf16_t*)gate, gate_row, (uint16_t*)out, scale, H, G, D, E, seq0, rule, nullptr, 0, nullptr, 0, 0, 0, 
+                       page_magic(block_size, max_blocks, 2L * G * (D > rule.v_stride ? D : rule.v_stride))};
 #define PICK(DP, EP) if (D <= DP && E <= EP) return launch<DP, EP>(a, nseq, max_q, s)
     PICK(64, 64);
     PICK(64, 128);
