@@ -7,10 +7,10 @@
 // (reference: src/myvllm/layers/attention.py:283-473).  This kernel is organised around the
 // KV stream instead, which is what bounds decode on HBM3E:
 //
-//  * one workgroup (4 waves) serves ALL query heads that share a KV head (up to 16 per
+//  * one workgroup (4 or 8 waves) serves ALL query heads that share a KV head (up to 16 per
 //    group), so every K/V byte is fetched once per sequence, not once per query head;
 //  * grid = (context splits, KV heads, sequences); each wave walks its own 32-token tiles
-//    and keeps a private online-softmax state, the 4 waves and then the splits are merged
+//    and keeps a private online-softmax state, the waves and then the splits are merged
 //    flash-decoding style (the splits by whichever of their workgroups finishes last, inside
 //    this kernel), so small batches still fill 256 CUs;
 //  * a tile is fetched with 16-byte-per-lane coalesced loads (a (block, kv-head) slab is
@@ -42,7 +42,20 @@ typedef __attribute__((ext_vector_type(8))) short s16x8_t;
 namespace {
 
 constexpr int kTile = 32;          // tokens per wave iteration
-constexpr int kWaves = 4;
+
+// Context splits that do any work for a context of `tiles` tiles, of the `nsplit` the grid holds
+// (workgroups of WAVES waves).  The grid of a captured step is sized for the longest context the
+// engine admits, and a split costs the merge (write-through partials, a ticket, reading them
+// back: 2 us, more with every split).  A context of up to 1.25 tiles per wave therefore stays in one
+// workgroup, without partials; a longer one is bound by what one CU reads (a workgroup's
+// 256 tokens take 0.9 us) and takes a split for every half workgroup of tiles (one for every whole one is slower
+// below 2000 tokens: 8.2 us at 512, one for every two tiles 7.4).  4 sequences, 16 / 8 heads of 128, grid for 2048 tokens, us a launch
+// before (16 splits of 4 waves, all of them merged) and now: 128 tokens 8.1 -> 4.5, 264 7.9 -> 6.4,
+// 512 9.2 -> 7.0, 1024 10.0 -> 7.8, 2048 10.4 -> 8.8.
+template <int WAVES>
+__device__ __forceinline__ int splits_in_use(int tiles, int nsplit) {
+    return tiles <= WAVES + WAVES / 4 ? 1 : min(nsplit, (2 * tiles + WAVES - 1) / WAVES);
+}
 
 // Device-scope ("agent") relaxed accesses to global memory: stores are written through to
 // where every XCD sees them, loads are served from there.
@@ -80,14 +93,14 @@ struct DecodeFuse {
     float eps;
 };
 
-template <int CODE, int D, bool KV8, bool FUSE = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void paged_decode_kernel(
+template <int CODE, int D, bool KV8, int kWaves, bool FUSE = false>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))) void paged_decode_kernel(
         const uint16_t* __restrict__ q, long q_stride_b, long q_stride_h,
         char* __restrict__ k_cache, char* __restrict__ v_cache,
         long cs_b, long cs_t, long cs_h, const int* __restrict__ block_tables, int bt_stride,
         const int* __restrict__ context_lens, uint16_t* __restrict__ out, long o_stride_b,
         long o_stride_h, float* part_acc, float* part_ml, int* tickets,
-        float scale_log2, int Hq, int Hkv, int bs_log2, int nsplit, DecodeFuse fu) {
+        float scale_log2, int Hq, int Hkv, int bs_log2, int nsplit_grid, DecodeFuse fu) {
     static_assert(!(FUSE && KV8), "the fused form writes a 16-bit cache");
     using DT = DType<CODE>;
     using vec8 = typename DT::vec8;
@@ -121,6 +134,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     const int bs_mask = (1 << bs_log2) - 1;
 
     const int total_tiles = (L + kTile - 1) / kTile;
+    const int nsplit = splits_in_use<kWaves>(total_tiles, nsplit_grid);   // the same for all splits of b
+    if (split >= nsplit) return;
     const int tps = (total_tiles + nsplit - 1) / nsplit;
     const int t0 = split * tps;
     const int t1 = min(t0 + tps, total_tiles);
@@ -402,7 +417,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         }
     }
 
-    // ---- merge the 4 waves through LDS (each wave reuses its own staging region)
+    // ---- merge the waves through LDS (each wave reuses its own staging region)
     l_run += __shfl_xor(l_run, 16, 64);
     l_run += __shfl_xor(l_run, 32, 64);
     float* wbuf = reinterpret_cast<float*>(smem + w * WAVE_LDS);
@@ -412,7 +427,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         *reinterpret_cast<f32x4_t*>(wbuf + 32 + c16 * ACC_LD + 16 * n + 4 * q4) = acc_o[n];
     __syncthreads();
 
-    for (int e = threadIdx.x; e < 16 * D; e += 256) {
+    for (int e = threadIdx.x; e < 16 * D; e += 64 * kWaves) {
         const int c = e / D, d = e - c * D;
         if (c >= nheads) continue;
         float M = -INFINITY;
@@ -434,7 +449,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         } else {
             // partial results cross to another workgroup, possibly on another XCD (private
             // L2): device-scope (write-through) stores, read back below by device-scope loads
-            const long pi = ((long)b * Hq + head) * nsplit + split;
+            const long pi = ((long)b * Hq + head) * nsplit_grid + split;   // (splits in use differ between sequences)
             st_agent(part_acc + pi * D + d, o);
             if (d == 0) { st_agent(part_ml + pi * 2, M); st_agent(part_ml + pi * 2 + 1, l); }
         }
@@ -464,7 +479,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
     float* s_f = reinterpret_cast<float*>(smem);       // [16 heads][64 splits] weights of the splits
     float* s_l = s_f + 16 * 64;                        // [16 heads] merged normalisers
     for (int c = w; c < nheads; c += kWaves) {         // lane = split (nsplit <= 64)
-        const long base = ((long)b * Hq + head0 + c) * nsplit;
+        const long base = ((long)b * Hq + head0 + c) * nsplit_grid;
         const float ms = lane < nsplit ? ld_agent(part_ml + (base + lane) * 2) : -INFINITY;
         const float ls = lane < nsplit ? ld_agent(part_ml + (base + lane) * 2 + 1) : 0.f;
         const float M = wave_max(ms);
@@ -474,23 +489,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         if (lane == 0) s_l[c] = l;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < nheads * D; e += 256) {
+    for (int e = threadIdx.x; e < nheads * D; e += 64 * kWaves) {
         const int c = e / D, d = e - c * D;
-        const long base = ((long)b * Hq + head0 + c) * nsplit;
+        const long base = ((long)b * Hq + head0 + c) * nsplit_grid;
         const float* sf = s_f + c * 64;
         float o = 0.f;
-        int s = 0;
-        for (; s + 8 <= nsplit; s += 8) {              // 8 loads in flight: a chain of round trips otherwise
+        for (int s = 0; s < nsplit; s += 8) {          // 8 loads in flight: a chain of round trips otherwise
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = ld_agent(part_acc + (base + s + j) * D + d);
+            for (int j = 0; j < 8; ++j) v[j] = s + j < nsplit ? ld_agent(part_acc + (base + s + j) * D + d) : 0.f;
 #pragma unroll
             for (int j = 0; j < 8; ++j) o += v[j] * sf[s + j];
         }
-        for (; s < nsplit; ++s) o += ld_agent(part_acc + (base + s) * D + d) * sf[s];
         const float l = s_l[c];
         out[b * o_stride_b + (head0 + c) * o_stride_h + d] = DT::from_float(l > 0.f ? o / l : 0.f);
     }
+}
+
+template <int CODE, int D, bool KV8, int WAVES, bool FUSE>
+int launch_decode_as(const void* q, long qsb, long qsh, void* kc, void* vc, long csb,
+                     long cst, long csh, const int* bt, int bt_stride, const int* ctx, void* out,
+                     long osb, long osh, float* part_acc, float* part_ml, int* tickets, float scale,
+                     int B, int Hq, int Hkv, int bs_log2, int nsplit, DecodeFuse fu, hipStream_t st) {
+    const int ngrp = (Hq / Hkv + 15) / 16;
+    const size_t lds = (size_t)WAVES * 2 * kTile * D * 2;
+    auto kern = paged_decode_kernel<CODE, D, KV8, WAVES, FUSE>;
+    if constexpr (WAVES * 2 * kTile * D * 2 > 64 * 1024) {
+        static const hipError_t once = hipFuncSetAttribute(
+            (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, WAVES * 2 * kTile * D * 2);
+        if (once != hipSuccess) return -1;
+    }
+    kern<<<dim3(nsplit, Hkv * ngrp, B), 64 * WAVES, lds, st>>>(
+        (const uint16_t*)q, qsb, qsh, (char*)kc, (char*)vc, csb, cst, csh, bt,
+        bt_stride, ctx, (uint16_t*)out, osb, osh, part_acc, part_ml, tickets, scale * kLog2e,
+        Hq, Hkv, bs_log2, nsplit, fu);
+    return MVL_CHECK_LAUNCH();
 }
 
 template <int CODE, int D, bool KV8>
@@ -505,25 +538,17 @@ int launch_decode(const void* q, long qsb, long qsh, void* kc, void* vc, long cs
     if (csb <= 0 || cst <= 0 || csh < 0 || csb * EB >= (1L << 32) || cst * EB >= (1L << 24) ||
         ((long)block_size * cst + (long)Hkv * csh) * EB + D * EB >= (1L << 31))
         return -1;
-    const int G = Hq / Hkv;
-    const int ngrp = (G + 15) / 16;
-    dim3 grid(nsplit, Hkv * ngrp, B);
-    const size_t lds = (size_t)kWaves * 2 * kTile * D * 2;
+    // 8 waves (one workgroup fills a CU) where every workgroup finds a CU of its own, 4 waves (two
+    // on a CU) otherwise: twice the tokens under one workgroup are half the partials to merge
+    const bool wide = (long)nsplit * Hkv * ((Hq / Hkv + 15) / 16) * B <= 256;
+#define MVL_DEC_AS(W, F) launch_decode_as<CODE, D, KV8, W, F>(q, qsb, qsh, kc, vc, csb, cst, csh, bt,  \
+        bt_stride, ctx, out, osb, osh, part_acc, part_ml, tickets, scale, B, Hq, Hkv, bs_log2, nsplit, fu, st)
     if constexpr (!KV8) {
-        if (fu.k_new != nullptr) {
-            paged_decode_kernel<CODE, D, KV8, true><<<grid, 256, lds, st>>>(
-                (const uint16_t*)q, qsb, qsh, (char*)kc, (char*)vc, csb, cst, csh, bt,
-                bt_stride, ctx, (uint16_t*)out, osb, osh, part_acc, part_ml, tickets, scale * kLog2e,
-                Hq, Hkv, bs_log2, nsplit, fu);
-            return MVL_CHECK_LAUNCH();
-        }
+        if (fu.k_new != nullptr) return wide ? MVL_DEC_AS(8, true) : MVL_DEC_AS(4, true);
     }
     if (fu.k_new != nullptr) return -1;
-    paged_decode_kernel<CODE, D, KV8><<<grid, 256, lds, st>>>(
-        (const uint16_t*)q, qsb, qsh, (char*)kc, (char*)vc, csb, cst, csh, bt,
-        bt_stride, ctx, (uint16_t*)out, osb, osh, part_acc, part_ml, tickets, scale * kLog2e, Hq,
-        Hkv, bs_log2, nsplit, fu);
-    return MVL_CHECK_LAUNCH();
+    return wide ? MVL_DEC_AS(8, false) : MVL_DEC_AS(4, false);
+#undef MVL_DEC_AS
 }
 
 }  // namespace

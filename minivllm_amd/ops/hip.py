@@ -396,14 +396,21 @@ def prefill_item_slots(num_tokens: int, num_seqs: int) -> int:
 
 
 def decode_num_splits(batch: int, num_kv_heads: int, max_context_len: Optional[int]) -> int:
-    """Context splits so that ~2 workgroups per CU exist even at batch 1; never more splits
-    than 128-token chunks of the longest context."""
+    """Context splits so that 8 waves per CU exist even at batch 1: workgroups of 8 waves, one
+    per CU, where their number comes as close to that as workgroups of 4, two per CU, do (the
+    launcher takes 8 waves for grids of at most 256 workgroups), otherwise of 4; never more
+    splits than the longest context uses (``splits_in_use`` of the kernel: shorter ones leave the
+    rest of theirs unused)."""
     wgs = max(batch * num_kv_heads, 1)
     # one workgroup per CU or more: no split (batch 256 x 1 KV head at 1024 tokens: 24.5 us
     # unsplit, 27 us in two splits; what the second split adds is its merge, not bandwidth)
-    n = 1 if wgs >= 256 else max(1, min(32, 512 // wgs))
+    if wgs >= 256:
+        return 1
+    wide, narrow = min(32, 256 // wgs), min(32, 512 // wgs)
+    n, waves = (wide, 8) if 2 * wide >= narrow else (narrow, 4)
     if max_context_len is not None:
-        n = max(1, min(n, (max_context_len + 127) // 128))
+        tiles = (max_context_len + 31) // 32
+        n = 1 if tiles <= waves + waves // 4 else min(n, (2 * tiles + waves - 1) // waves)
     return n
 
 

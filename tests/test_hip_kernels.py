@@ -304,6 +304,41 @@ def test_paged_decode(hip, dtype, hq, hkv, d, bs):
     close(got, want, dtype)
 
 
+@pytest.mark.parametrize("d,fp8", [(128, False), (64, False), (128, True)])
+@pytest.mark.parametrize("bs", [16, 256])
+@pytest.mark.parametrize("ns", [1, 2, 5, 16, 40])
+def test_paged_decode_splits_in_use(hip, d, fp8, bs, ns):
+    """A sequence uses as many of the grid's splits as its own context needs: contexts on both
+    sides of where a second split, a third and all of them set in (8 waves: above 10 tiles of 32 tokens, then one
+    for every 4; 4 waves, which the larger grids take: above 5, then one for every 2), mixed in a batch, launched
+    twice over the same tickets.  Against attention in 64 bits over the cache as it is stored."""
+    torch.manual_seed(9)
+    hq, hkv, dtype, scale = 8, 2, torch.bfloat16, d ** -0.5
+    lens = [1, 160, 161, 0, 320, 321, 384, 385, 193, 1025, 32, 2049]
+    need = [-(-n // bs) for n in lens]
+    perm = torch.randperm(sum(need)).to(torch.int32)
+    tables, at = torch.zeros(len(lens), max(need), dtype=torch.int32), 0
+    for i, n in enumerate(need):
+        tables[i, :n] = perm[at:at + n]
+        at += n
+    kc, vc = (torch.randn(sum(need), hkv, bs, d, device=DEV).to(torch.float8_e4m3fn if fp8 else dtype)
+              .permute(0, 2, 1, 3) for _ in "kv")
+    q = torch.randn(len(lens), hq, d, device=DEV, dtype=dtype)
+    ctx = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    for _ in range(2):
+        got = hip.paged_attention_decode(q, kc, vc, tables.to(DEV), ctx, scale, num_splits=ns)
+    for i, n in enumerate(lens):
+        if n == 0:
+            assert not got[i].any()
+            continue
+        k, v = (c[tables[i, :need[i]].long().to(DEV)].reshape(-1, hkv, d)[:n].double()
+                .repeat_interleave(hq // hkv, 1) for c in (kc, vc))
+        p = torch.softmax((q[i].double()[:, None] * k.transpose(0, 1)).sum(-1) * scale, -1)
+        want = (p[..., None] * v.transpose(0, 1)).sum(1)
+        # weights and result are rounded to bfloat16 (8 bits): 2^-9 each, relative to the output's size
+        assert float((got[i].double() - want).norm() / want.norm()) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (16, 8, 128), (8, 1, 128), (16, 8, 64), (4, 4, 128),
                                       (40, 8, 128), (64, 4, 128), (40, 2, 128)])
