@@ -76,8 +76,8 @@ _skinny = _sig("mvl_skinny_gemm", _c_void, _c_long, _c_void, _c_void, _c_void, _
 
 _skinny_splitk = _sig("mvl_skinny_gemm_splitk", _c_void, _c_long, _c_void, _c_void, _c_int, _c_int,
                       _c_int, _c_int, _c_int, _c_void)
-_skinny_norm = _sig("mvl_skinny_norm_gemm", _c_void, _c_long, _c_void, _c_long, _c_void, _c_long,
-                    _c_float, _c_void, _c_void, _c_void, _c_long, _c_int, _c_int, _c_int,
+_skinny_norm = _sig("mvl_skinny_norm_gemm", _c_void, _c_long, _c_void, _c_int, _c_void, _c_void, _c_long,
+                    _c_void, _c_long, _c_float, _c_void, _c_void, _c_void, _c_long, _c_int, _c_int, _c_int,
                     _c_int, _c_int, _c_void)
 
 _mid = _sig("mvl_mid_gemm", _c_void, _c_long, _c_void, _c_void, _c_void, _c_long, _c_void, _c_int,
@@ -551,14 +551,27 @@ def skinny_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False
     return swiglu or (n <= 4096 and k <= 4096)
 
 
-def skinny_gemm_splits(x: torch.Tensor, weight: torch.Tensor) -> int:
+def skinny_gemm_splits(x: torch.Tensor, weight: torch.Tensor) -> Optional[int]:
     """For a projection whose output goes straight into residual add + RMSNorm: the K split
-    (over workgroups) that was measured fastest together with that norm, 0 = library GEMM,
-    None = never measured (the caller falls back to ``skinny_gemm_pays``)."""
+    (over workgroups) that was measured fastest together with that norm, 0 = library GEMM.
+    Never measured: ``skinny_narrow_splits`` where the output is narrow, otherwise None (the caller
+    falls back to ``skinny_gemm_pays``)."""
     if x.dim() != 2 or x.shape[0] > SKINNY_PAYS_ROWS or not skinny_gemm_ok(x, weight):
         return None
     n, k = weight.shape
-    return _SKINNY_CHOICE.get((_row_bucket(x.shape[0]), n, k, "norm"))
+    return _SKINNY_CHOICE.get((_row_bucket(x.shape[0]), n, k, "norm"), skinny_narrow_splits(n, k))
+
+
+def skinny_narrow_splits(n: int, k: int) -> Optional[int]:
+    """K split of a projection to norm that was never measured, None: no opinion.  Up to 2048
+    output columns are at most 128 tiles of 16, so K goes over up to four workgroups, no more than fill the
+    chip once, with 1024 of K or more for each.  us at 4 / 16 rows, library, unsplit, split so: 1024 x 2048
+    8.0 / 8.0, 5.2 / 7.1, 4.2 / 5.9; 1024 x 3072 9.0 / 9.0, 6.8 / 8.4, 4.4 / 6.0; 2048 x 4096 14.5 / 14.3,
+    7.8 / 9.6, 6.2 / 7.8; 2048 x 6144 10.9 / 11.1, 11.3 / 15.7, 7.6 / 9.2; 1536 x 8960 28.9 / 28.9, 16.0 / 21.8,
+    11.5 / 12.9.  Wider ones lose by it: 2560 x 9728 15.0 / 15.5, 17.4 / 22.9, 17.2 / 24.0."""
+    if n > 2048 or n * k * 2 < (1 << 20):
+        return None
+    return next((s for s in (4, 3, 2) if skinny_splits_ok(k, s) and k // s >= 1024 and n // 16 * s <= _NUM_CUS), 1)
 
 
 def tune_skinny_to_norm(weights, margin: float = 0.97) -> dict:
@@ -677,37 +690,72 @@ def skinny_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Te
     return out
 
 
-SKINNY_NORM_MAX_ROWS = 2          # beyond this the two-kernel path is faster (measured)
+SKINNY_NORM_MAX_ROWS = 2          # beyond this the two-kernel path is faster for rows of more than 1024 values
+_STAGED_ROWS_BYTES = 112 << 10    # rows the kernel can hold in LDS (csrc/skinny_norm_gemm.hip)
 
 
 def skinny_norm_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False) -> bool:
     """Shapes for which (residual add + RMSNorm + projection) runs as ONE weight-streaming
     kernel: 1-2 rows and a projection the plain weight-streaming kernel takes (also QKV-sized
-    outputs, where dropping the norm launch outweighs the library's small GEMM advantage)."""
-    if x.dim() != 2 or x.shape[0] > SKINNY_NORM_MAX_ROWS or not skinny_gemm_ok(x, weight, swiglu):
+    outputs, where dropping the norm launch outweighs the library's small GEMM advantage), or up to 16 rows
+    of up to 1024 values, where every workgroup can afford to form the rows itself (us, two kernels / one, 4, 8
+    and 16 rows: 4096 x 1024 7.6 / 4.8, 8.7 / 5.3, 10.6 / 6.4, SwiGLU of 2 x 3072 x 1024 7.6 / 6.0, 8.0 / 6.6,
+    8.4 / 7.7; but 6144 x 4096 16.3 / 17.3, 18.1 / 21.2, 22.3 / 29.4)."""
+    if x.dim() != 2 or not skinny_gemm_ok(x, weight, swiglu):
         return False
-    return swiglu or weight.shape[0] <= 8192
+    n, k = weight.shape
+    if x.shape[0] > SKINNY_NORM_MAX_ROWS and (k > 1024 or k % 256 or n > 8192 or x.stride(0) % 8
+                                              or x.data_ptr() % 16):
+        return False
+    return swiglu or n <= 8192
 
 
-def skinny_norm_linear(x: torch.Tensor, residual: Optional[torch.Tensor], eps: float,
+def skinny_norm_partials_pays(part: SplitKPartials, residual: Optional[torch.Tensor], weight: torch.Tensor,
+                              swiglu: bool = False) -> bool:
+    """The same for the K slices of the projection before, which every workgroup then reads and
+    sums (norm kernel that sums + projection / one kernel, us, two slices, 4, 8 and 16 rows: 4096 x 1024 7.4 / 5.2,
+    8.4 / 6.2, 10.4 / 8.2; 4096 x 2048 9.5 / 8.2, 10.3 / 10.1, 12.4 / 14.2; SwiGLU of 2 x 3072 x 1024 7.6 / 6.8,
+    7.8 / 8.1, 8.2 / 10.6; of 2 x 6144 x 2048 16.8 / 21.7 at 4 rows)."""
+    slices, m, k = part.ws.shape
+    n = weight.shape[0]
+    if (slices > 4 or m > SKINNY_MAX_ROWS or n > 8192 or k % 256 or n % (32 if swiglu else 16)
+            or weight.dtype != part.dtype or weight.shape[1] != k or not weight.is_contiguous()
+            or part.dtype not in _DT or m * (k + 8) * 2 > _STAGED_ROWS_BYTES):
+        return False
+    if residual is not None and (residual.shape != (m, k) or residual.dtype != part.dtype or residual.stride(1) != 1
+                                 or residual.stride(0) % 8 or residual.data_ptr() % 16):
+        return False
+    return (m <= 4 or not swiglu) if k <= 1024 else (k <= 2048 and m <= 4 and not swiglu)
+
+
+def skinny_norm_linear(x, residual: Optional[torch.Tensor], eps: float,
                        weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                        swiglu: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
     """``r = x + residual`` (``x`` when residual is None); returns
     ``(linear_or_swiglu(r * rsqrt(mean(r^2) + eps)), r)`` for a ``weight`` that already carries
     the norm's scale vector.  ``r`` is a new tensor: the inputs are left untouched (other
-    workgroups of the kernel are still reading them)."""
+    workgroups of the kernel are still reading them).  ``x`` may be the ``SplitKPartials`` of the
+    projection before (at most 4 slices): the kernel sums them as it reads them."""
     M, K = x.shape
     N = weight.shape[0]
-    out = torch.empty((M, N // 2 if swiglu else N), dtype=x.dtype, device=x.device)
+    dt = weight.dtype
+    out = torch.empty((M, N // 2 if swiglu else N), dtype=dt, device=weight.device)
+    r, rin, rin_s, rout, rout_s = x, None, 0, None, 0
     if residual is not None:
-        assert residual.shape == x.shape and residual.stride(1) == 1
-        r = torch.empty((M, K), dtype=x.dtype, device=x.device)
-        rin, rin_s, rout, rout_s = residual.data_ptr(), residual.stride(0), r.data_ptr(), K
+        assert residual.shape == x.shape and residual.dtype == dt and residual.stride(1) == 1
+        rin, rin_s = residual.data_ptr(), residual.stride(0)
+    src = (None, 0, None, 0, None)
+    if isinstance(x, SplitKPartials):
+        assert x.ws.is_contiguous() and x.dtype == dt
+        src = (None, 0, x.ws.data_ptr(), x.ws.shape[0], x.bias.data_ptr() if x.bias is not None else None)
     else:
-        r, rin, rin_s, rout, rout_s = x, None, 0, None, 0
-    _check(_skinny_norm(x.data_ptr(), x.stride(0), rin, rin_s, rout, rout_s, eps,
+        src = (x.data_ptr(), x.stride(0), None, 0, None)
+    if residual is not None or src[2] is not None:
+        r = torch.empty((M, K), dtype=dt, device=weight.device)
+        rout, rout_s = r.data_ptr(), K
+    _check(_skinny_norm(*src, rin, rin_s, rout, rout_s, eps,
                         weight.data_ptr(), bias.data_ptr() if bias is not None else None,
-                        out.data_ptr(), out.stride(0), M, N, K, 1 if swiglu else 0, _dt(x),
+                        out.data_ptr(), out.stride(0), M, N, K, 1 if swiglu else 0, _DT[dt],
                         _stream()), "skinny_norm_gemm")
     return out, r
 

@@ -779,6 +779,48 @@ def test_skinny_norm_gemm(hip, dtype, M, K, N, swiglu, with_res):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N,swiglu,slices,with_res,with_bias", [
+    (1, 256, 16, False, 2, True, False), (4, 1024, 4096, False, 3, True, True), (4, 1024, 6144, True, 4, True, False),
+    (16, 1024, 4112, False, 2, True, True), (3, 768, 96, True, 1, False, True), (4, 2048, 4096, False, 2, False, False),
+    (5, 1024, 4096, False, 0, True, False), (16, 1024, 6144, True, 0, True, True), (9, 512, 32, False, 0, False, False),
+    (2, 1280, 48, False, 3, True, False)])
+def test_skinny_norm_gemm_staged_rows(hip, dtype, M, K, N, swiglu, slices, with_res, with_bias):
+    """The form whose workgroups form the rows in LDS, from fp32 slices or from a tensor: the stream bit
+    for bit the rounded sum that the norm kernel over slices gives, the product against 64 bits over that stream."""
+    from minivllm_amd import ops
+    torch.manual_seed(31)
+    res = torch.randn(M, K + 8, device=DEV, dtype=dtype)[:, :K] if with_res else None
+    w = (torch.randn(N, K, device=DEV) * 0.03).to(dtype)
+    bias = torch.randn(N, device=DEV, dtype=dtype) if with_bias else None
+    if slices:
+        x = hip.SplitKPartials(torch.randn(slices, M, K, device=DEV),
+                               torch.randn(K, device=DEV, dtype=dtype) if with_bias else None, dtype)
+        r_want = x.add_rms_norm(res.clone() if with_res else None, torch.ones(K, device=DEV, dtype=dtype), 1e-6)[1]
+        assert hip.skinny_norm_partials_pays(x, res, w, swiglu)
+    else:
+        x = torch.randn(M, K + 16, device=DEV, dtype=dtype)[:, :K]
+        r_want = (x.float() + res.float()).to(dtype) if with_res else x
+        assert hip.skinny_norm_gemm_pays(x, w, swiglu)
+    res0 = res.clone() if with_res else None
+    out, r = ops.norm_linear(x, res, torch.ones(K, device=DEV, dtype=dtype), 1e-6, w, bias, swiglu, gamma_folded=True)
+    assert torch.equal(r, r_want) and (not with_res or torch.equal(res, res0))
+    rd = r.double()
+    y = (rd @ w.double().T) * torch.rsqrt(rd.pow(2).mean(-1, keepdim=True) + 1e-6)
+    if with_bias:
+        y = y + bias.double()
+    want = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:] if swiglu else y
+    # one rounding of the result: 2^-9 (bfloat16) or 2^-12 (float16) of it, plus fp32 sums of K terms
+    assert float((out.double() - want).norm() / want.norm()) < (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
+
+
+@pytest.mark.parametrize("n,k,want", [(1024, 2048, 2), (1024, 3072, 3), (1024, 4096, 4), (2048, 4096, 2),
+                                      (1536, 8960, 2), (1024, 1024, 1), (4096, 4096, None), (64, 256, None),
+                                      (1024, 1152, 1), (1024, 4224, 3)])
+def test_narrow_projections_split_without_measurement(hip, n, k, want):
+    assert hip.skinny_narrow_splits(n, k) == want
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 7, 16])
 def test_skinny_gemm_swiglu(hip, dtype, M):
     torch.manual_seed(17)
