@@ -21,7 +21,8 @@
 //    of tiles that lie entirely above its own 32 rows, and the mask is applied on diagonal
 //    tiles only;
 //  * the 1-D grid is remapped so that workgroups sharing an XCD (and its L2) walk the query
-//    heads of one KV head and adjacent Q tiles of one sequence, heaviest Q tiles first.
+//    heads of one KV head and adjacent Q tiles of one sequence, heaviest Q tiles first, and that
+//    every XCD gets its share of every sequence.
 #include "common.h"
 #include <type_traits>
 #include <cstdlib>
@@ -146,12 +147,15 @@ __global__ __launch_bounds__(kThreads, 2) void flash_prefill_kernel(PrefillArgs 
         int id = blockIdx.x;
         const int n = a.total_wg;
         const int q8 = n >> 3, r8 = n & 7, x = id & 7;
-        // blocks with equal (id % 8) share an XCD: give each XCD a contiguous range
+        // Blocks with equal (id % 8) share an XCD: give each XCD a contiguous range, KV heads
+        // outermost.  With the sequences outermost an XCD had two of 16 prompts, and the one
+        // with the two longest finished last: 16 prompts of 512..1024 tokens, 32 / 8 heads of 128, 146 us
+        // against 124 (no two alike: 8 of 1024..2048, 40 / 8 heads, 349 against 271; all alike: no change).
         id = (x < r8 ? x * (q8 + 1) : r8 * (q8 + 1) + (x - r8) * q8) + (id >> 3);
         g = id % G;                id /= G;
         qti = id % a.n_items;      id /= a.n_items;
-        kvh = id % a.Hkv;
-        b = id / a.Hkv;
+        b = id % a.B;
+        kvh = id / a.B;
     }
     const int head = kvh * G + g;
 
@@ -163,9 +167,8 @@ __global__ __launch_bounds__(kThreads, 2) void flash_prefill_kernel(PrefillArgs 
     // under the causal mask tile i attends to i + 1 key blocks, so the pair (n - 1 - p, p) always
     // costs n + 1 of them; every workgroup of a sequence then runs equally long and the fixed
     // cost of a workgroup (launch, ramp-up, drain) is paid once per 2 g tiles.
-    // with a work list the pairs are formed per sequence (from its own tile count), without one
-    // from the longest sequence's (shorter ones skip the tiles they do not have)
-    const int n_qtiles = a.items != nullptr ? (q_len + kBM - 1) / kBM : a.n_qtiles;
+    // The pairs are formed per sequence, from its own tile count.
+    const int n_qtiles = (q_len + kBM - 1) / kBM;
     const int n_pairs = (n_qtiles + 1) >> 1;
     const int n_pass = a.pair ? 2 * a.pair : 1;
 #pragma unroll 1
@@ -178,9 +181,9 @@ __global__ __launch_bounds__(kThreads, 2) void flash_prefill_kernel(PrefillArgs 
         qt = (pass & 1) ? p : n_qtiles - 1 - p;
     } else {
         qt = n_qtiles - 1 - qti;                         // heaviest tiles first
+        if (qt < 0) break;                               // (uniform: a sequence shorter than the longest)
     }
     const int q0 = qt * kBM;
-    if (q0 >= q_len) continue;                           // uniform for the workgroup
     if (pass) __syncthreads();                           // every wave is done with the LDS tiles
     // every per-lane constant is derived inside the pass from a value the compiler cannot see
     // through: hoisted out of the loop they would stay live across it and spill
@@ -685,12 +688,13 @@ extern "C" int mvl_flash_attention_prefill(
     a.B = B; a.Hq = Hq; a.Hkv = Hkv;
     a.n_qtiles = (max_q_len + kBM - 1) / kBM;
     static const char* pair_env = getenv("MVL_PREFILL_PAIR");
-    // one heavy / light pair per workgroup (MVL_PREFILL_PAIR: 0 = one Q tile per workgroup, g = g
-    // pairs).  Several pairs per workgroup once paid for the workgroup's fixed cost; since the
-    // prologue got short, more and smaller workgroups balance better (32 x 512, 16 q heads:
-    // 0.073 ms with two pairs, 0.068 ms with one)
+    // One Q tile per workgroup, or one heavy / light pair (MVL_PREFILL_PAIR: 0 = tiles, g = g pairs).
+    // Tiles find better places on 512 slots than pairs do and a lone prompt's chain is half as long; a pair saves
+    // one of two prologues, which shows where prompts are short and the chip is filled twice over.
+    // us, pairs / tiles, heads of 128: 4 x 256 (16 / 8) 15.0 / 10.0, 1 x 2048 (16 / 8) 48.8 / 43.4, 3 x 1000 (32 / 8)
+    // 42.7 / 33.5, 8 x 2048 (40 / 8) 271 / 262, 16 x 1024 (32 / 8) 124.8 / 124.1; but 32 x 512 (16 / 8) 60.7 / 67.4.
     const int n_pairs = (a.n_qtiles + 1) / 2;
-    a.pair = pair_env ? atoi(pair_env) : 1;
+    a.pair = pair_env ? atoi(pair_env) : a.n_qtiles <= 4 && (long)B * Hq * n_pairs >= 1024 ? 1 : 0;
     a.n_items = a.pair ? (n_pairs + a.pair - 1) / a.pair : a.n_qtiles;
     a.total_wg = B * Hq * a.n_items;
     a.items = items;

@@ -635,6 +635,21 @@ def test_prefill_many_uneven_sequences(hip, hq, hkv, d):
     close(got, want, dtype)
 
 
+@pytest.mark.parametrize("hq,hkv", [(16, 2), (18, 3), (3, 3)])
+@pytest.mark.parametrize("longest", [512, 513])
+def test_prefill_tiles_and_pairs_of_uneven_sequences(hip, hq, hkv, longest):
+    """A workgroup takes a pair of Q tiles (up to 4 tiles a prompt, 1024 workgroups and more) or one tile:
+    prompts of no, one and all rows and at the tiles' edges in one step, KV heads that do not divide over the XCDs."""
+    torch.manual_seed(3)
+    d, dtype = 64, torch.bfloat16
+    lens = [0, 1, 127, 128, 129, 255, 256, 257, 384, 385, longest, 0] + [37 * i % 400 + 1 for i in range(50)]
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), device=DEV, dtype=torch.int32)
+    q = torch.randn(sum(lens), hq, d, device=DEV, dtype=dtype)
+    k, v = (torch.randn(sum(lens), hkv, d, device=DEV, dtype=dtype) for _ in "kv")
+    got = hip.flash_attention_prefill(q, k, v, cu, d ** -0.5, longest)
+    close(got, ref.flash_attention_prefill(q, k, v, cu, d ** -0.5), dtype)
+
+
 def test_flash_prefill_long_and_softmax_rescale(hip):
     """4k tokens (many KV tiles) with a spiked key late in the sequence, which forces the
     running-max rescale branch of the online softmax on rows that already accumulated."""
