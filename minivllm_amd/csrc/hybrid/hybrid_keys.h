@@ -85,4 +85,12 @@ int prompt_attention_f32(const void* q, long q_row, long q_head, const void* k_c
                          float scale, int nseq, int seq0, int max_q, int H, int G, int D, int E,
                          const KeyRule& rule, hipStream_t s);
 
+// the same over formed keys and values of latent attention (hybrid_latent_form.hip, with the operands of
+// hyb_latent_formed_prompts); _pages_ok: what the pages have to be
+bool latent_prompts_pages_ok(int block_size, int max_blocks, int latent_row);
+int latent_prompts(const void* q, long q_row, long q_head, const void* qr, long qr_row, const void* cache,
+                   const void* block_tables, int max_blocks, int block_size, const void* cu_q, const void* positions,
+                   const void* sink, const void* k, const void* v, long formed_rows, void* out, float scale, int nseq,
+                   int max_q, int H, int D, int E, int R, int P, int window, hipStream_t s);
+
 }  // namespace hyb

@@ -249,7 +249,10 @@ prompt_attention_kernel(PromptArgs a) {
     const int last_page = page_index(wg_ctx - 1);
     // LAT: rows of the formed keys and values ahead of this sequence's
     long formed0 = 0;
-    if constexpr (LAT) formed0 = (long)formed_tiles_before(a.cu_q, a.positions, b, lane) * 32;
+    if constexpr (LAT) {
+        formed0 = (long)formed_tiles_before(a.cu_q, a.positions, b, lane) * 32;
+        if (formed0 + (wg_ctx + 31) / 32 * 32 > a.formed_rows) return;      // (a longest context given too short: nothing there)
+    }
     constexpr int RPK = 512 / (LAT ? RP : DP), RPV = 512 / EP;   // rows of a piece that is looked up by page
     constexpr int PIT = LAT ? RIT : KIT;
     // the tile to be staged next, kept up from tile to tile (as expressions of its number they were a fifth of the
@@ -1024,6 +1027,27 @@ int prompt_attention_f32(const void* q, long q_row, long q_head, const void* k_c
                          (const float*)sink, (const float*)gate, gate_row, (float*)out, scale, H, G, D, E, seq0, rule};
     if (D <= 64) return E <= 64 ? launch_f32<64, 64>(a, nseq, max_q, s) : launch_f32<64, 128>(a, nseq, max_q, s);
     return E <= 64 ? launch_f32<128, 64>(a, nseq, max_q, s) : launch_f32<128, 128>(a, nseq, max_q, s);
+}
+
+bool latent_prompts_pages_ok(int block_size, int max_blocks, int latent_row) {
+    return block_size > 0 && block_size % 32 == 0 && page_magic(block_size, max_blocks, 2L * latent_row) != 0;
+}
+
+int latent_prompts(const void* q, long q_row, long q_head, const void* qr, long qr_row, const void* cache,
+                   const void* block_tables, int max_blocks, int block_size, const void* cu_q, const void* positions,
+                   const void* sink, const void* k, const void* v, long formed_rows, void* out, float scale, int nseq,
+                   int max_q, int H, int D, int E, int R, int P, int window, hipStream_t s) {
+    if (!latent_prompts_pages_ok(block_size, max_blocks, R + P)) return 1;
+    KeyRule rule{};
+    rule.window = window;
+    rule.v_stride = E;
+    const PromptArgs a{(const uint16_t*)q, q_row, q_head, (const uint16_t*)k, (const uint16_t*)v,
+                       (const int*)block_tables, max_blocks, block_size, (const int*)cu_q, (const int*)positions,
+                       (const float*)sink, nullptr, 0, (uint16_t*)out, scale, H, 1, D, E, 0, rule,
+                       (const uint16_t*)qr, qr_row, (const uint16_t*)cache, R + P, P, formed_rows,
+                       page_magic(block_size, max_blocks, 2L * (R + P))};
+    return P <= 64 ? launch_form<128, 64, 128, 2, false, true>(a, nseq, max_q, s)
+                   : launch_form<128, 128, 128, 2, false, true>(a, nseq, max_q, s);
 }
 
 }  // namespace hyb

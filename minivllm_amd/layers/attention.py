@@ -327,12 +327,14 @@ class LatentAttention(nn.Module):
     """Attention whose keys and values are expansions of one cached latent per token: key of
     head h = [W_uk_h c | r], value = W_uv_h c, with c the RMS-normed latent (R numbers) and r one
     rotated key part (P numbers) shared by all heads.  Only c and r are cached, and the
-    expansions are never formed: with a_h = W_uk_h^T q_h the score is (a_h . c + q_rot_h . r) *
+    expansions are as a rule not formed: with a_h = W_uk_h^T q_h the score is (a_h . c + q_rot_h . r) *
     scale, and the weighted sum of values is W_uv_h applied to the weighted sum of latents.  So
     this is attention with ONE key/value head whose key row is [c | r] (R + P) and whose value row
     is c (R), run by ``SinkAttention`` (with its window and sink, when asked for), between two
     batched products per head; in bfloat16 on the GPU by a matrix-core kernel of its own that takes
-    the two parts of a query where they are (``SinkAttention.forward_latent``).  ``up_k`` [H, D, R] and ``up_v`` [H, R, E] are the per-head
+    the two parts of a query where they are (``SinkAttention.forward_latent``).  Prompts that are most of
+    their contexts are the exception: there keys and values ARE formed, in one pass ahead of the attention
+    (``ops.latent_formed_prompts``), which takes a quarter of the operations.  ``up_k`` [H, D, R] and ``up_v`` [H, R, E] are the per-head
     expansion matrices, each laid out as the right operand of its product; ``rotation``: a
     ``HalfRotation`` / ``NeighbourRotation`` over the first entries of the P-part.  Only c and r
     are cached, once: the values are read from the key rows (``value_in_key``)."""
@@ -374,8 +376,17 @@ class LatentAttention(nn.Module):
         core = core or self.core
         T = q.shape[0]
         H, D, R, E = self.num_heads, self.head_dim, self.kv_rank, self.v_head_dim
-        q_abs = torch.bmm(q[:, :, :D].transpose(0, 1), self.up_k)                    # [H, T, R]
         rot = self.rotation
+        if ctx.is_prefill and not ctx.num_decode_seqs and core.value_in_key and ops.latent_formed_ok(
+                q, dkv, self.up_k, self.up_v, core.k_cache, ctx.block_tables, ctx.cu_seqlens_q.shape[0] - 1, ctx.max_seqlen_q,
+                ctx.max_seqlen_k):
+            qr = ops.latent_rope_store(None, q, dkv, self.latent_norm, self.eps, ctx.positions, rot.inv_freq,
+                                       rot.rotary_dim, core.k_cache, None, ctx.slot_mapping, rot.neighbours, rot.mult,
+                                       assemble=False)
+            return ops.latent_formed_prompts(q, qr, core.k_cache, self.up_k, self.up_v, ctx.cu_seqlens_q,
+                                             ctx.block_tables, ctx.positions, core.scale, core.sink,
+                                             ctx.max_seqlen_q, ctx.max_seqlen_k, core.window)
+        q_abs = torch.bmm(q[:, :, :D].transpose(0, 1), self.up_k)                    # [H, T, R]
         parts = core.value_in_key and ops.latent_attention_ok(q_abs, core.k_cache, self.rot_dim)
         qr = ops.latent_rope_store(q_abs, q, dkv, self.latent_norm, self.eps, ctx.positions,
                                    rot.inv_freq, rot.rotary_dim, core.k_cache,

@@ -417,6 +417,19 @@ def latent_attention_ok(q_abs, k_cache, rot_dim):
     return _on_gpu(q_abs) and _hybrid().latent_attention_ok(q_abs, k_cache, rot_dim)
 
 
+def latent_formed_ok(q, dkv, up_k, up_v, k_cache, block_tables, seqs, max_q, max_k):
+    """True when prompt portions of latent attention run with keys and values formed per head
+    (``latent_formed_prompts``) instead of in the latents' coordinates."""
+    return _on_gpu(q) and _hybrid().latent_formed_ok(q, dkv, up_k, up_v, k_cache, block_tables, seqs, max_q, max_k)
+
+
+def latent_formed_prompts(q, q_rot, k_cache, up_k, up_v, cu_q, block_tables, positions, scale, sink, max_q, max_k,
+                          window=0):
+    """GPU only (``hip_hybrid``)."""
+    return _hybrid().latent_formed_prompts(q, q_rot, k_cache, up_k, up_v, cu_q, block_tables, positions, scale,
+                                           sink, max_q, max_k, window)
+
+
 def latent_attention_prefill(q_abs, q_rot, k_cache, cu_q, block_tables, positions, scale, sink, out,
                              max_q=None, window=0):
     """GPU only (``hip_hybrid``); elsewhere the queries are assembled and ``sink_attention_*`` runs."""

@@ -99,6 +99,11 @@ _tgt = _sig("hyb_token_gate", _P, _L, _P, _P, _L, _L, _P, _L, _I, _I, _P)
 _wkv = _sig("hyb_wkv_scan", _P, _P, _P, _L, _L, _L, _P, _L, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _P)
 _lat = _sig("hyb_latent_attention", _P, _L, _L, _P, _L, _L, _P, _P, _I, _I, _P, _P, _P, _P, _P, _L, _L, _P,
             _F, _I, _I, _I, _I, _I, _I, _I, _P)
+_latf = _sig("hyb_latent_formed_prompts", _P, _L, _L, _P, _L, _P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _P, _L, _P,
+             _F, _I, _I, _I, _I, _I, _I, _I, _I, _P)
+_latf_ok = _lib.hyb_latent_formed_ok
+_latf_ok.argtypes = [_I] * 6
+_latf_ok.restype = _I
 _lat_ok = _lib.hyb_latent_attention_ok
 _lat_ok.argtypes = [_I, _I]
 _lat_ok.restype = _I
@@ -650,10 +655,11 @@ def row_norm_store(q, k, v, qw, kw, eps, k_cache, v_cache, slot_mapping):
 
 def latent_rope_store(q_abs, q, dkv, w, eps, positions, inv_freq, rot_dims, k_cache, v_cache,
                       slot_mapping, neighbours=False, mult=1.0, assemble=True):
-    H, T, R = q_abs.shape
+    T, H, R = q.shape[0], q.shape[1], w.numel()
     P = dkv.shape[1] - R
     D = q.shape[2] - P
-    assert q_abs.is_contiguous() and q_abs.dtype == q.dtype and dkv.dtype == q.dtype
+    assert dkv.dtype == q.dtype and (q_abs is not None or not assemble)
+    assert q_abs is None or (q_abs.is_contiguous() and q_abs.dtype == q.dtype and q_abs.shape == (H, T, R))
     assert q.shape[:2] == (T, H) and q.stride(2) == 1 and q.stride(1) == D + P and dkv.stride(1) == 1
     assert w.numel() == R and inv_freq.numel() * 2 == rot_dims
     if k_cache is not None:
@@ -724,6 +730,57 @@ def latent_attention_decode(q_abs, q_rot, k_cache, block_tables, context_lens, s
     B, H, R = out.shape
     return _latent(q_abs, q_rot, k_cache, block_tables, None, None, _i32c(context_lens), scale, sink, out,
                    B, 1, window, latent_splits(B, H, R, max_context_len, window))
+
+
+def latent_formed_rows(seqs: int, max_k: int) -> int:
+    """Rows of formed keys and values that hold any ``seqs`` contexts of up to ``max_k`` tokens, each
+    rounded up to whole tiles of 32."""
+    return seqs * (-(-int(max_k) // 32) * 32)
+
+
+def latent_formed_ok(q, dkv, up_k, up_v, k_cache, block_tables, seqs, max_q, max_k) -> bool:
+    """Whether prompt portions run with their keys and values formed: bfloat16, sizes the kernels
+    have, pages of whole tiles of 32, and formed rows that take no more memory than the absorbed
+    queries and the sums of latents of the other form do.  With that a context is at most 2 R / (D + E)
+    times (R 512, D = E = 128: four times) the step's new tokens, sequence by sequence as long as the longest.
+    On that line the forming pays too: us, absorbed / formed, 16 heads, R 512, 512 tokens behind 1536 146 / 100, 64 behind 192
+    42.8 / 39.9, 8 times 32 behind 96 44.4 / 41.0; 16 tokens alone 29.5 / 29.5.  Beyond it a token forms more than it saves, and
+    for R 128, where the two come out alike (8 prompts of about 1024: 109.6 / 108.7), the line lies at contexts without a prefix."""
+    T, H, width = q.shape
+    D, R, E = up_k.shape[1], up_k.shape[2], up_v.shape[2]
+    P = width - D
+    if not (max_q and max_k and seqs > 0 and T > 0) or max_q > max_k:
+        return False
+    if any(t is None or t.dtype != torch.bfloat16 for t in (q, dkv, up_k, up_v, k_cache)):
+        return False
+    if latent_formed_rows(seqs, max_k) * (D + E) > 2 * T * R or P <= 0 or dkv.shape[1] != R + P:
+        return False
+    return bool(k_cache.is_contiguous() and up_k.is_contiguous() and up_v.is_contiguous() and q.stride(2) == 1
+                and q.stride(1) == width and width % 8 == 0 and (T == 1 or q.stride(0) % 8 == 0)
+                and block_tables is not None and block_tables.dtype == torch.int32 and block_tables.stride(1) == 1
+                and all(t.data_ptr() % 16 == 0 for t in (q, up_k, up_v, k_cache))
+                and _latf_ok(D, E, R, P, k_cache.shape[1], block_tables.stride(0)))
+
+
+def latent_formed_prompts(q, q_rot, k_cache, up_k, up_v, cu_q, block_tables, positions, scale, sink, max_q, max_k,
+                          window=0):
+    """``q`` [T, H, D + P] (the D-parts are read), ``q_rot`` [T, H, P] turned, cache rows [c | r] of the
+    step's tokens already stored; sequence b owns rows cu_q[b] .. cu_q[b+1] and block table row b.
+    Returns [T, H, E] (rows of no sequence hold anything)."""
+    T, H, width = q.shape
+    D, R, E = up_k.shape[1], up_k.shape[2], up_v.shape[2]
+    nseq = cu_q.shape[0] - 1
+    rows = latent_formed_rows(nseq, max_k)
+    k = torch.empty((H, rows, D), dtype=q.dtype, device=q.device)
+    v = torch.empty((H, rows, E), dtype=q.dtype, device=q.device)
+    out = torch.empty((T, H, E), dtype=q.dtype, device=q.device)
+    assert q_rot.shape == (T, H, width - D) and q_rot.is_contiguous() and block_tables.shape[0] >= nseq
+    _check(_latf(q.data_ptr(), q.stride(0), width, q_rot.data_ptr(), q_rot.stride(0), k_cache.data_ptr(),
+                 block_tables.data_ptr(), block_tables.stride(0), k_cache.shape[1], _i32c(cu_q).data_ptr(),
+                 _i32(positions).data_ptr(), up_k.data_ptr(), up_v.data_ptr(), _ptr(_f32(sink)) if sink is not None else None,
+                 k.data_ptr(), v.data_ptr(), rows, out.data_ptr(), float(scale), nseq, int(max_q), H, D, E, R,
+                 width - D, int(window), _stream()), "latent_formed_prompts")
+    return out
 
 
 def xielu(u, ap, aq, out_dtype):
