@@ -7,7 +7,8 @@
 //
 //  * one workgroup (8 waves) owns a BM x BN output tile and a slice of K; BM covers every row
 //    of the batch (64 / 128 / 256), so each weight byte is fetched from HBM exactly once, and
-//    BN x split-K is chosen on the host so that the grid fills the chip;
+//    BN x split-K is chosen on the host so that the grid fills the chip (257 to 1024 rows of narrow
+//    projections run in several row tiles: there the grid that fills the chip once counts for more);
 //  * x and W tiles go global -> LDS by LDS-DMA in pieces of 8 rows x 128 bytes (whole cache
 //    lines), into a ring of D stages of 64 k-elements; the loads of the next D - 1 k-steps
 //    stay in flight across the one barrier per k-step (counted vmcnt, raw s_barrier);
@@ -94,7 +95,7 @@ void mid_gemm_kernel(MidArgs a) {
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wv / WN, wn = wv % WN;
     const bool extra = wv < PREM;                      // this wave moves PFULL + 1 pieces
-    const int n_tile = blockIdx.x, split = blockIdx.y;
+    const int n_tile = blockIdx.x, split = blockIdx.y, row0 = blockIdx.z * BM;
     const int ks0 = split * a.ksteps_per_split;
     const int nsteps = min(a.ksteps_per_split, a.ksteps - ks0);
 
@@ -109,7 +110,7 @@ void mid_gemm_kernel(MidArgs a) {
     for (int i = 0; i < PMAX; ++i) {
         const int p = i * 8 + wv;
         if (i * 8 < XPIECES) {
-            const int row = min(p * 8 + prow, a.M - 1);               // rows >= M: duplicates
+            const int row = min(row0 + p * 8 + prow, a.M - 1);        // rows >= M: duplicates
             src[i] = a.x + (long)row * a.x_stride + (long)ks0 * kBK + pchunk * 8;
         } else {
             const int j = min(p - XPIECES, BN / 8 - 1) * 8 + prow;    // row of the W tile image
@@ -259,7 +260,7 @@ void mid_gemm_kernel(MidArgs a) {
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        const int row = wm * TM + m * 16 + frow;
+        const int row = row0 + wm * TM + m * 16 + frow;
         if (row >= a.M) continue;
         if (EPI == 2) {
             float* wp = a.ws + ((long)split * a.M + row) * a.N;
@@ -407,7 +408,7 @@ template <int CODE, int BM, int BN, int WM, int D, bool SWI, bool NT>
 int launch_tile(MidArgs a, int splits, hipStream_t st) {
     const int tiles = a.N / BN;
     const size_t lds = (size_t)D * (BM + BN) * 128;
-    dim3 grid(tiles, splits);
+    dim3 grid(tiles, splits, (a.M + BM - 1) / BM);
     if (splits > 1) {
         auto k = mid_gemm_kernel<CODE, BM, BN, WM, D, 2, SWI, NT>;
         static const hipError_t once = hipFuncSetAttribute(
@@ -443,13 +444,13 @@ int launch_shape(MidArgs a, int bm, int bn, int splits, hipStream_t st) {
 }  // namespace
 
 // out[M, N_out] = x . W^T (+ bias) [SwiGLU: W = [gate; up], N_out = N / 2].
-// bm in {64, 128, 256} >= M; bn in {64, 96 (bm 256 only), 128} with N % bn == 0; splits >= 1 K slices (workspace
+// bm in {64, 128, 256} (M > bm: several row tiles); bn in {64, 96 (bm 256 only), 128} with N % bn == 0; splits >= 1 K slices (workspace
 // `ws` of splits * M * N floats when splits > 1); nt: non-temporal weight loads.
 extern "C" int mvl_mid_gemm(const void* x, long x_stride, const void* w, const void* bias,
                             void* out, long o_stride, void* ws, int M, int N, int K, int swiglu,
                             int bm, int bn, int splits, int nt, int dtype, void* stream) {
     if (M == 0) return 0;
-    if (M > bm || K % kBK != 0 || N % bn != 0 || splits < 1 || (dtype != 0 && dtype != 1)) return -1;
+    if (bm <= 0 || (M + bm - 1) / bm > 65535 || K % kBK != 0 || N % bn != 0 || splits < 1 || (dtype != 0 && dtype != 1)) return -1;
     if (swiglu && (N % 2 != 0 || (N / 2) % (bn / 2) != 0)) return -1;
     if (splits > 1 && ws == nullptr) return -1;
     MidArgs a;

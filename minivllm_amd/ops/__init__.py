@@ -136,7 +136,8 @@ def paged_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scal
 def linear(x, weight, bias=None, to_norm=False, residual=None):
     """``x @ weight.T (+ bias)``: the library GEMM, except for the GPU inputs (<= 16 rows: skinny
     kernel; 17..256 rows: mid-batch kernel; more: the 256 x 256-tile prefill kernel) of the
-    shapes where the hand-written kernels were measured to be faster on this machine.  ``to_norm``: the
+    shapes where the hand-written kernels were measured to be faster on this machine, and for 257..1024 rows of narrow
+    projections that were not measured (``hip.tiled_gemm_sizes``).  ``to_norm``: the
     caller passes the result straight to ``norm_linear`` / ``add_rms_norm`` (and to nothing
     else), which lets a K-split mid-batch GEMM hand over its unsummed slices
     (``SplitKPartials``) for the norm kernel to sum.  ``residual`` (with ``to_norm``): the
@@ -162,6 +163,9 @@ def linear(x, weight, bias=None, to_norm=False, residual=None):
             return h.big_linear_resid(x, weight, bias, residual)
         if h.big_gemm_pays(x, weight):
             return h.big_linear(x, weight, bias)
+        c = h.tiled_gemm_choice(x, weight, to_norm=to_norm)
+        if c is not None:
+            return h.mid_linear(x, weight, bias, False, c[1], c[2], False, c[0], defer=to_norm)
     return F.linear(x, weight, bias)
 
 
@@ -179,8 +183,13 @@ def swiglu_linear(x, weight, bias=None):
             c = h.mid_gemm_choice(x, weight, swiglu=True)
             if c is not None:
                 return h.mid_linear(x, weight, bias, True, c[0], c[1], c[2])
-    elif _on_gpu(x) and x.dim() == 2 and _hip().big_gemm_pays(x, weight, swiglu=True):
-        return _hip().big_linear(x, weight, bias, swiglu=True)     # prefill: GEMM + SwiGLU in one kernel
+    elif _on_gpu(x) and x.dim() == 2:
+        h = _hip()
+        if h.big_gemm_pays(x, weight, swiglu=True):
+            return h.big_linear(x, weight, bias, swiglu=True)      # prefill: GEMM + SwiGLU in one kernel
+        c = h.tiled_gemm_choice(x, weight, swiglu=True)
+        if c is not None:
+            return h.mid_linear(x, weight, bias, True, c[1], c[2], False, c[0])
     return silu_and_mul(F.linear(x, weight, bias))
 
 

@@ -9,6 +9,7 @@ tensors).
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional, Tuple
 
@@ -768,7 +769,11 @@ _NUM_CUS = 256
 def mid_gemm_ok(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False) -> bool:
     """Operands the mid-batch kernel takes: <= 256 rows with 16-byte aligned rows, K a multiple
     of 64, N a multiple of 64 (SwiGLU: N/2 a multiple of 32), contiguous same-dtype weights."""
-    if x.dim() != 2 or x.shape[0] == 0 or x.shape[0] > MID_MAX_ROWS or x.dtype not in _DT:
+    return x.dim() == 2 and x.shape[0] <= MID_MAX_ROWS and _mid_operands_ok(x, weight, swiglu)
+
+
+def _mid_operands_ok(x: torch.Tensor, weight: torch.Tensor, swiglu: bool) -> bool:
+    if x.dim() != 2 or x.shape[0] == 0 or x.dtype not in _DT:
         return False
     n, k = weight.shape
     return (weight.dtype == x.dtype and weight.is_contiguous() and x.stride(1) == 1
@@ -832,12 +837,12 @@ def mid_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
                swiglu: bool = False, bn: int = 128, splits: int = 1, nt: bool = True,
                bm: Optional[int] = None, defer: bool = False):
     """``x @ weight.T (+ bias)`` (``swiglu``: ``silu(gate) * up`` of the fused weight) for up to
-    256 rows with the weight-streaming MFMA kernel; ``splits`` > 1 slices K over workgroups
+    256 rows (more with a row tile ``bm`` given, see ``tiled_gemm_choice``) with the weight-streaming MFMA kernel; ``splits`` > 1 slices K over workgroups
     (fp32 partial sums in a scratch buffer, summed by a second kernel).  ``defer`` (with a K
     split, no SwiGLU) returns the slices unsummed as ``SplitKPartials`` for a norm to consume."""
     M, K = x.shape
     N = weight.shape[0]
-    if not mid_gemm_ok(x, weight, swiglu):
+    if not _mid_operands_ok(x, weight, swiglu) or (bm is None and M > MID_MAX_ROWS):
         raise ValueError(f"mid_linear cannot take x {tuple(x.shape)} / weight {tuple(weight.shape)}")
     bm = bm or mid_row_tile(M)
     if defer and not swiglu and splits > 1 and (eff := _mid_eff_splits(K, splits)) > 1:
@@ -853,6 +858,45 @@ def mid_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
                 ws.data_ptr() if ws is not None else None, M, N, K, int(swiglu), bm, bn, splits,
                 int(nt), _dt(x), _stream()), "mid_gemm")
     return out
+
+
+# us a k-step of 64 takes in one workgroup per CU (fitted to 64 measured times), by row and column tile
+_TILE_US = {(64, 64): 0.2, (64, 128): 0.31, (128, 64): 0.31, (128, 128): 0.5, (256, 64): 0.5, (256, 96): 0.8,
+            (256, 128): 0.88}
+
+
+@functools.lru_cache(maxsize=4096)
+def tiled_gemm_sizes(m: int, n: int, k: int, swiglu: bool, to_norm: bool) -> Optional[Tuple[int, int, int]]:
+    """(row tile, column tile, K split) with which the mid-batch kernel's grid takes 257 to 1024 rows of a
+    projection that was not measured at start-up, None: the library.  Up to 4 M outputs (6 M for gate and up, whose SiLU the
+    kernel does in passing) and 16 MB of weights the chip is hardly filled once, and a tile that fills it beats the library's
+    choice; beyond, larger tiles and streams win.  The choice: rounds of the grid over 256 CUs, times k-steps, times what one
+    takes; K is split only towards a norm, which sums the slices, at what they cost to write and read.  us, library /
+    kernel: 960 rows, 1024 x 2048 10.7 / 10.3, 1024 x 3072 14.5 / 14.2, SwiGLU of 2 x 3072 x 1024 23.8 / 16.6, 4096 x 1024
+    12.7 / 12.7, 2048 x 2048 14.8 / 14.1; 512 rows, 4096 x 1024 10.1 / 8.9, 1024 x 3072 11.8 / 8.6 (slices for the norm);
+    past the lines 960 rows 6144 x 4096 51.5 / 57.8, 2048 x 6144 39.2 / 44.3, 1500 rows 2048 x 2048 18.0 / 19.8.  And a call of the
+    library costs the host 24 us where tables of its variants are loaded, one of the kernel 8."""
+    if (not BIG_MIN_ROWS <= m <= 1024 or m * n > (6 << 20 if swiglu else 4 << 20) or n * k > 8 << 20
+            or n < 512 or k < 512):
+        return None
+    best = None
+    for (bm, bn), us in _TILE_US.items():
+        if n % bn or (swiglu and (n // 2) % (bn // 2)):
+            continue
+        for s in (1, 2, 3, 4) if to_norm and not swiglu else (1,):
+            rounds = -(-(-(-m // bm) * (n // bn) * s) // _NUM_CUS)
+            t = rounds * (3.5 + -(-(k // 64) // s) * us) + (s > 1) * s * m * n * 8 / 5e6
+            if best is None or t < best[0]:
+                best = (t, (bm, bn, s))
+    return best and best[1]
+
+
+def tiled_gemm_choice(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False, to_norm: bool = False):
+    """``tiled_gemm_sizes`` for this call, None where the start-up has measured its shape or the operands do not fit."""
+    m, (n, k) = x.shape[0], weight.shape
+    if m > 1024 or (big_row_bucket(m), n, k, swiglu) in _BIG_CHOICE or not _mid_operands_ok(x, weight, swiglu):
+        return None
+    return tiled_gemm_sizes(m, n, k, swiglu, to_norm)
 
 
 def splitk_materialize(part: SplitKPartials) -> torch.Tensor:

@@ -828,6 +828,39 @@ def test_skinny_norm_gemm_staged_rows(hip, dtype, M, K, N, swiglu, slices, with_
     assert float((out.double() - want).norm() / want.norm()) < (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,swiglu,to_norm,tile", [
+    (257, 1024, 2048, False, True, (64, 64, 3)), (960, 1024, 3072, False, True, (64, 64, 1)),
+    (960, 6144, 1024, True, False, (256, 96, 1)), (512, 4096, 1024, False, False, (64, 128, 1)), (500, 1024, 3072, False, True, (64, 64, 2)),
+    (1024, 4096, 512, False, False, (128, 128, 1)), (300, 576, 576, False, False, (64, 64, 1)),
+    (769, 704, 1536, True, False, None), (321, 4160, 1024, True, False, None)])
+def test_tiled_gemm_of_rows_in_several_tiles(hip, dtype, M, N, K, swiglu, to_norm, tile):
+    """257 to 1024 rows on the mid-batch kernel: last row tiles that are not full, strided rows, every kind of result."""
+    from minivllm_amd import ops
+    torch.manual_seed(5)
+    x = torch.randn(M, K + 64, device=DEV, dtype=dtype)[:, :K]
+    w, bias = (torch.randn(N, K, device=DEV) * K ** -0.5).to(dtype), torch.randn(N, device=DEV, dtype=dtype)
+    c = hip.tiled_gemm_choice(x, w, swiglu, to_norm)
+    assert c is not None and (tile is None or c == tile), c
+    out = ops.swiglu_linear(x, w, bias) if swiglu else ops.linear(x, w, bias, to_norm=to_norm)
+    assert isinstance(out, hip.SplitKPartials) == (c[2] > 1)
+    if c[2] > 1:
+        out = out.materialize()
+    y = x.double() @ w.double().T + bias.double()
+    want = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:] if swiglu else y
+    # one rounding of the result: 2^-9 (bfloat16) or 2^-12 (float16) of it, plus fp32 sums of K terms
+    assert float((out.double() - want).norm() / want.norm()) < (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
+
+
+@pytest.mark.parametrize("m,n,k,swiglu", [(256, 1024, 1024, False), (1025, 1024, 1024, False), (960, 6144, 1024, False),
+                                          (1024, 8192, 1024, True), (300, 2048, 6144, False), (300, 448, 1024, False), (300, 1024, 448, False)])
+def test_tiled_gemm_leaves_other_sizes_to_the_library(hip, m, n, k, swiglu):
+    assert hip.tiled_gemm_sizes(m, n, k, swiglu, True) is None
+    x, w = torch.zeros(960, 1024, device=DEV, dtype=torch.bfloat16), torch.zeros(1024, 1024, device=DEV, dtype=torch.bfloat16)
+    assert hip.tiled_gemm_choice(x, w) and not hip.tiled_gemm_choice(x.float(), w.float())
+    assert not hip.tiled_gemm_choice(x, w[:, ::2]) and not hip.tiled_gemm_choice(x[:, 1:], w[:, 1:])
+
+
 @pytest.mark.parametrize("n,k,want", [(1024, 2048, 2), (1024, 3072, 3), (1024, 4096, 4), (2048, 4096, 2),
                                       (1536, 8960, 2), (1024, 1024, 1), (4096, 4096, None), (64, 256, None),
                                       (1024, 1152, 1), (1024, 4224, 3)])
