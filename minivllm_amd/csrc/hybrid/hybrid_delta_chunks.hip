@@ -32,7 +32,7 @@
 // It stays in the sums once it is there, so a portion whose outputs and state come out finite met none; any other is
 // walked again from its first token by the recurrence itself (same workgroup, its own columns).
 //
-// 8 portions of 512..1024 tokens, 16 / 8 heads of 128: 55 + 155 us, against 645 us token by token.  The walk
+// 8 portions of 512..1024 tokens, 16 / 8 heads of 128: 37 + 150 us, against 645 us token by token.  The walk
 // takes 9.7 us a chunk of 64 columns; its six phases between barriers use the matrix units, the
 // vector units (cutting) and the LDS for about 2.5 us each and hardly overlap: one workgroup per CU is all that
 // LDS and registers hold.  32 columns per workgroup 160 us; all waves in both roles, two workgroups per CU
@@ -87,18 +87,27 @@ struct Product {
 };
 #endif
 
+// bytes of delta_weights_kernel's LDS that hold first the k rows, then the triangular systems
+template <int DP>
+constexpr int weights_room() {
+    constexpr int rows = 3 * C * DP * 2, systems = 2 * C * (C + 4) * 4;
+    return rows > systems ? rows : systems;
+}
+
 template <int DP, bool DELTA>
 __global__ void __launch_bounds__(256, 2)
 delta_weights_kernel(DeltaChunks a) {
 #ifdef __HIP_DEVICE_COMPILE__       // (the host pass only needs the launch stub)
     constexpr int KS = DP / 32, PITCH = C + 4;
     extern __shared__ __attribute__((aligned(256))) char smem[];
+    // the k rows' images make room for the triangular systems: with both at once (86 KB) one workgroup was all a
+    // CU held, and 112 chunks of 8 groups of two heads of 128 took 53 us instead of 37
     char* kparts = smem;                                         // [3] images of the chunk's k rows
-    float* Lm = reinterpret_cast<float*>(smem + 3 * C * DP * 2); // [C][PITCH]
+    float* Lm = reinterpret_cast<float*>(smem);                  // [C][PITCH]
     float* Tm = Lm + C * PITCH;                                  // [C][PITCH]
     const int tid = threadIdx.x, lane = tid & 63, tb = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l16 = lane & 15, q4 = lane >> 4;
-    float* suf = Tm + C * PITCH + tb * 2 * C;                    // per wave: [C] W to a block's end, [C] decays
+    float* suf = reinterpret_cast<float*>(smem + weights_room<DP>()) + tb * 2 * C;   // per wave: [C] W to a block's end, [C] decays
     float* dec = suf + C;
     const int H = a.H, G = a.G, D = a.D, R = H / G, g = blockIdx.y;
 
@@ -234,7 +243,7 @@ delta_weights_kernel(DeltaChunks a) {
             put(ws, s, x);
         }
         if constexpr (DELTA) {
-            if (r > 0) __syncthreads();                   // the last head's inverse has been read
+            __syncthreads();                              // the images, or the last head's inverse, have been read
 #pragma unroll
             for (int kb = 0; kb < 4; ++kb)
                 if (kb <= tb) {
@@ -634,7 +643,7 @@ int allow_lds(F* kernel, int bytes) {
 
 template <int DP, bool DELTA>
 int launch(const DeltaChunks& a, hipStream_t s) {
-    constexpr int lds1 = 3 * C * DP * 2 + (2 * C * (C + 4) + 4 * 2 * C) * 4;
+    constexpr int lds1 = weights_room<DP>() + 4 * 2 * C * 4;
     static const int ok1 = allow_lds(delta_weights_kernel<DP, DELTA>, lds1);
     if (ok1) return ok1;
     hipLaunchKernelGGL((delta_weights_kernel<DP, DELTA>), dim3(a.T / C + a.B, a.G), dim3(256), lds1, s, a);
