@@ -23,6 +23,22 @@ __device__ __forceinline__ void rest(uint32_t w, float& x, float& y) {
     y -= __uint_as_float(w & 0xffff0000u);
 }
 
+// What the number of a row's 16-byte chunk is XORed with in images of 64 (rows of 128 bytes) or 128 columns that
+// 16 x 16 products read.  LDS serves a wave's accesses in groups of lanes, and a group has to find its
+// bytes in different banks (a line of 256 bytes, two rows of 64 columns):
+//   rows, 16 bytes a lane: rows 0-3 and 12-15 of one chunk with 4-11 of the next: distinct XOR [4 <= row < 12];
+//   transposed, 8 bytes a lane: 32 bytes of rows 0-7 (8-15), or of 0-3 and 8-11 (4-7 and 12-15): half of it distinct;
+//   stores of 8 bytes a lane, a column's chunk of 16 rows: distinct.
+// swizzle (hybrid_tiles.h), which is for transposed reads of 64 bytes of four rows, had every such read of 32
+// bytes take twice as long: a third of the delta rule's LDS cycles (its walk 150 -> 147 us; the matrix LSTM's does not
+// wait for them).
+template <int DP>
+__device__ __forceinline__ int rows16(int row) {
+    if (DP % 128 == 0) return (((row ^ (row >> 1 & 4)) & 7) << 1) | (row >> 3 & 1);
+    const int i = row >> 1;
+    return (((i ^ (i >> 1 & 2)) & 3) << 1) | (i >> 2 & 1);
+}
+
 // eight numbers as three bfloat16 fragments whose sum they are
 __device__ __forceinline__ void split8(const float* x, bf16x8* p) {
     uint32_t w[3][4];

@@ -58,14 +58,19 @@ struct Gates {
 
 template <int DP>
 struct Lds {
-    char q[C * DP * 2], k[C * DP * 2];     // images (hybrid_tiles.h) of the chunk's rows
-    char v[C * EB * 2];                    // plain rows of 64 bytes
-    char wv[3][C * EB * 2];                // W_end v in three parts, laid out as v
+    char q[C * DP * 2], k[C * DP * 2];     // images (rows16) of the chunk's rows
+    char v[C * EB * 2];                    // rows of 64 bytes, halves swapped where v_at says so
+    char wv[3][C * EB * 2];                // W_end v in three parts, likewise
     char s[3][EB * DP * 2];                // the state's parts, a row per state column
     char n[3][DP * 2];                     // the normaliser's parts
     Gates g;
     int lost;                              // an output or a state is not finite
 };
+
+// Place of a byte of a row of v (wv).  Transposed reads take 32 bytes of rows 0-7 (of 0-3 and 8-11): the halves of the
+// second four are swapped, so that they are in the banks that the first four leave.
+__device__ __forceinline__ int v_at(int row, int byte) { return row * (EB * 2) + (byte ^ (row << 3 & 32)); }
+__device__ __forceinline__ int wv_at(int row, int byte) { return row * (EB * 2) + (byte ^ (row << 2 & 32)); }
 
 __device__ __forceinline__ float logsigmoid_(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
@@ -266,18 +271,18 @@ mlstm_chunks_kernel(MlstmChunks a) {
     auto stash = [&]() {
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
-            const int c = i * 512 + tid, row = c / (DP / 8), ch = (c % (DP / 8)) ^ swizzle<DP>(row);
+            const int c = i * 512 + tid, row = c / (DP / 8), ch = (c % (DP / 8)) ^ rows16<DP>(row);
             *reinterpret_cast<uint4*>(L.q + row * DP * 2 + ch * 16) = qr[i];
             *reinterpret_cast<uint4*>(L.k + row * DP * 2 + ch * 16) = kr[i];
         }
-        *reinterpret_cast<uint2*>(L.v + tid * 8) = vr;
+        *reinterpret_cast<uint2*>(L.v + v_at(tid >> 3, (tid & 7) * 8)) = vr;
     };
     // the state's parts: a row per column of the state
     auto publish = [&]() {
 #pragma unroll
         for (int j = 0; j < DT; ++j) {
             const int d = 16 * (tb + 4 * j) + 4 * q4, row = 16 * et + l16;
-            put_parts(S[j], [&](int k) { return L.s[k] + row * DP * 2 + (((d >> 3) ^ swizzle<DP>(row)) << 4) + (d & 4) * 2; });
+            put_parts(S[j], [&](int k) { return L.s[k] + row * DP * 2 + (((d >> 3) ^ rows16<DP>(row)) << 4) + (d & 4) * 2; });
             if (et == 0 && l16 == 0) put_parts(N[j], [&](int k) { return L.n[k] + d * 2; });
         }
     };
@@ -297,11 +302,11 @@ mlstm_chunks_kernel(MlstmChunks a) {
         const Gates& g = L.g;
         if (ch + 1 < nchunks) fetch(ch + 1);
         {   // W_end v, four columns of a token per thread
-            const uint2 raw = *reinterpret_cast<const uint2*>(L.v + tid * 8);
+            const uint2 raw = *reinterpret_cast<const uint2*>(L.v + v_at(tid >> 3, (tid & 7) * 8));
             const float w = g.wl[tid >> 3];
             const f32x4 x = {w * __uint_as_float(raw.x << 16), w * __uint_as_float(raw.x & 0xffff0000u),
                              w * __uint_as_float(raw.y << 16), w * __uint_as_float(raw.y & 0xffff0000u)};
-            put_parts(x, [&](int k) { return L.wv[k] + tid * 8; });
+            put_parts(x, [&](int k) { return L.wv[k] + wv_at(tid >> 3, (tid & 7) * 8); });
         }
         // ---- this wave's 16 queries: t = 16 tb + l16
         const int t = 16 * tb + l16, left = n - ch * C;
@@ -309,13 +314,13 @@ mlstm_chunks_kernel(MlstmChunks a) {
         bf16x8 qf[KS];
 #pragma unroll
         for (int s = 0; s < KS; ++s)
-            qf[s] = *reinterpret_cast<const bf16x8*>(L.q + t * DP * 2 + (((4 * s + q4) ^ swizzle<DP>(t)) << 4));
+            qf[s] = *reinterpret_cast<const bf16x8*>(L.q + t * DP * 2 + (((4 * s + q4) ^ rows16<DP>(t)) << 4));
         f32x4 O = {0.f, 0.f, 0.f, 0.f}, O1 = O, O2 = O, nq = O;
         {
             const int row = 16 * et + l16;
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
-                const int at = row * DP * 2 + (((4 * s + q4) ^ swizzle<DP>(row)) << 4);
+                const int at = row * DP * 2 + (((4 * s + q4) ^ rows16<DP>(row)) << 4);
                 O2 = mfma(*reinterpret_cast<const bf16x8*>(L.s[2] + at), qf[s], O2);
                 O1 = mfma(*reinterpret_cast<const bf16x8*>(L.s[1] + at), qf[s], O1);
                 O = mfma(*reinterpret_cast<const bf16x8*>(L.s[0] + at), qf[s], O);
@@ -333,7 +338,7 @@ mlstm_chunks_kernel(MlstmChunks a) {
             const int row = 16 * kb + l16;
 #pragma unroll
             for (int i = 0; i < KS; ++i)
-                s = mfma(*reinterpret_cast<const bf16x8*>(L.k + row * DP * 2 + (((4 * i + q4) ^ swizzle<DP>(row)) << 4)), qf[i], s);
+                s = mfma(*reinterpret_cast<const bf16x8*>(L.k + row * DP * 2 + (((4 * i + q4) ^ rows16<DP>(row)) << 4)), qf[i], s);
             float w[4];
             if (kb == tb) {
                 const int i3 = 4 * q4 + 3;
@@ -374,7 +379,7 @@ mlstm_chunks_kernel(MlstmChunks a) {
             weighted(2 * s, x);
             bf16x8 p[3];
             split8(x, p);
-            const char* at = L.v + (32 * s + 4 * q4 + (l16 >> 2)) * (EB * 2) + et * 32 + (l16 & 3) * 8;
+            const char* at = L.v + v_at(32 * s + 4 * q4 + (l16 >> 2), et * 32 + (l16 & 3) * 8);
             const bf16x8 vf = join(read_tr(at), read_tr(at + 16 * EB * 2));
 #pragma unroll
             for (int k = 2; k >= 0; --k) O = mfma(vf, p[k], O);
@@ -401,14 +406,14 @@ mlstm_chunks_kernel(MlstmChunks a) {
             bf16x8 wf[3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                const char* at = L.wv[k] + row * (EB * 2) + et * 32 + (l16 & 3) * 8;
+                const char* at = L.wv[k] + wv_at(row, et * 32 + (l16 & 3) * 8);
                 wf[k] = join(read_tr(at), read_tr(at + 4 * EB * 2));
             }
 #pragma unroll
             for (int j = 0; j < DT; ++j) {
                 const int chunk = 2 * (tb + 4 * j) + ((l16 & 3) >> 1);
-                const bf16x8 kf = join(read_tr(L.k + row * DP * 2 + ((chunk ^ swizzle<DP>(row)) << 4) + (l16 & 1) * 8),
-                                       read_tr(L.k + (row + 4) * DP * 2 + ((chunk ^ swizzle<DP>(row + 4)) << 4) + (l16 & 1) * 8));
+                const bf16x8 kf = join(read_tr(L.k + row * DP * 2 + ((chunk ^ rows16<DP>(row)) << 4) + (l16 & 1) * 8),
+                                       read_tr(L.k + (row + 4) * DP * 2 + ((chunk ^ rows16<DP>(row + 4)) << 4) + (l16 & 1) * 8));
 #pragma unroll
                 for (int k = 2; k >= 0; --k) S[j] = mfma(kf, wf[k], S[j]);
                 if (et == 0) N[j] = mfma(kf, *reinterpret_cast<const bf16x8*>(&g.wp[min(l16, 2)][32 * s + 8 * q4]), N[j]);

@@ -139,7 +139,7 @@ delta_weights_kernel(DeltaChunks a) {
             split8(y, qf[s]);
 #pragma unroll
             for (int p = 0; p < 3; ++p)
-                *reinterpret_cast<bf16x8*>(kparts + p * C * DP * 2 + t * DP * 2 + (((4 * s + q4) ^ swizzle<DP>(t)) << 4)) = kf[s][p];
+                *reinterpret_cast<bf16x8*>(kparts + p * C * DP * 2 + t * DP * 2 + (((4 * s + q4) ^ rows16<DP>(t)) << 4)) = kf[s][p];
         }
         __syncthreads();
 #pragma unroll
@@ -154,7 +154,7 @@ delta_weights_kernel(DeltaChunks a) {
                 bf16x8 x[3];
 #pragma unroll
                 for (int p = 0; p < 3; ++p)
-                    x[p] = *reinterpret_cast<const bf16x8*>(kparts + p * C * DP * 2 + row * DP * 2 + (((4 * s + q4) ^ swizzle<DP>(row)) << 4));
+                    x[p] = *reinterpret_cast<const bf16x8*>(kparts + p * C * DP * 2 + row * DP * 2 + (((4 * s + q4) ^ rows16<DP>(row)) << 4));
                 if (DELTA) pk.add(x, kf[s]);
                 pq.add(x, qf[s]);
             }
@@ -322,7 +322,7 @@ delta_weights_kernel(DeltaChunks a) {
 template <int DP, int ET>
 struct Lds {
     static constexpr int EB = 32 * ET, ROW = EB * 2;
-    char k[3][C * DP * 2];             // images (hybrid_tiles.h) of the chunk's k rows, in parts
+    char k[3][C * DP * 2];             // images (rows16) of the chunk's k rows, in parts
     union {
         char s[3][EB * DP * 2];        // the state's parts, a row per state column
         struct { char x[3][C * ROW], u[3][C * ROW]; };   // rows of tokens: V - diag(c) K S, later diag(W_end) U; U
@@ -438,7 +438,7 @@ delta_chunks_kernel(DeltaChunks a) {
 #pragma unroll
             for (int x = 0; x < ET; ++x) {
                 const int d = 16 * (tb + 4 * j) + 4 * q4, row = 16 * (eh * ET + x) + l16;
-                put_parts(S[j][x], [&](int k) { return L.s[k] + row * DP * 2 + (((d >> 3) ^ swizzle<DP>(row)) << 4) + (d & 4) * 2; });
+                put_parts(S[j][x], [&](int k) { return L.s[k] + row * DP * 2 + (((d >> 3) ^ rows16<DP>(row)) << 4) + (d & 4) * 2; });
             }
     };
     auto stash = [&]() {
@@ -449,12 +449,12 @@ delta_chunks_kernel(DeltaChunks a) {
             if (update)
 #pragma unroll
                 for (int k = 0; k < 3; ++k)
-                    *reinterpret_cast<bf16x8*>(L.k[k] + t * DP * 2 + (((4 * s + q4) ^ swizzle<DP>(t)) << 4)) = xp[s][k];
+                    *reinterpret_cast<bf16x8*>(L.k[k] + t * DP * 2 + (((4 * s + q4) ^ rows16<DP>(t)) << 4)) = xp[s][k];
         }
     };
     // a token row's 16-byte chunk in the x / u images
     auto place = [&](int row, int chunk) {
-        return row * ROW + ((chunk ^ (ET == 1 ? (row >> 2) & 3 : swizzle<64>(row))) << 4);
+        return row * ROW + ((chunk ^ (ET == 1 ? (row >> 1 & 2) | (row >> 3 & 1) : rows16<64>(row))) << 4);
     };
     auto put_cols = [&](char (*im)[C * ROW], int x, f32x4 v) {        // this lane's token, four of the columns 16 x ..
         const int at = place(t, 2 * x + (q4 >> 1)) + (q4 & 1) * 8;
@@ -535,7 +535,7 @@ delta_chunks_kernel(DeltaChunks a) {
                     bf16x8 sf[3];
 #pragma unroll
                     for (int k = 0; k < 3; ++k)
-                        sf[k] = *reinterpret_cast<const bf16x8*>(L.s[k] + row * DP * 2 + (((4 * s + q4) ^ swizzle<DP>(row)) << 4));
+                        sf[k] = *reinterpret_cast<const bf16x8*>(L.s[k] + row * DP * 2 + (((4 * s + q4) ^ rows16<DP>(row)) << 4));
                     p.add(sf, xp[s]);
                     __builtin_amdgcn_sched_barrier(0);       // (reads hoisted over the products cost registers)
                 }
@@ -598,8 +598,8 @@ delta_chunks_kernel(DeltaChunks a) {
                 bf16x8 kp[3];
 #pragma unroll
                 for (int k = 0; k < 3; ++k)
-                    kp[k] = join(read_tr(L.k[k] + row * DP * 2 + ((chunk ^ swizzle<DP>(row)) << 4) + (l16 & 1) * 8),
-                                 read_tr(L.k[k] + (row + 16) * DP * 2 + ((chunk ^ swizzle<DP>(row + 16)) << 4) + (l16 & 1) * 8));
+                    kp[k] = join(read_tr(L.k[k] + row * DP * 2 + ((chunk ^ rows16<DP>(row)) << 4) + (l16 & 1) * 8),
+                                 read_tr(L.k[k] + (row + 16) * DP * 2 + ((chunk ^ rows16<DP>(row + 16)) << 4) + (l16 & 1) * 8));
 #pragma unroll
                 for (int x = 0; x < ET; ++x) S[j][x] = mfma6(kp, up[x], S[j][x]);
                 __builtin_amdgcn_sched_barrier(0);
