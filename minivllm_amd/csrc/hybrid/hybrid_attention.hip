@@ -620,7 +620,7 @@ static int launch_split(const void* q, long q_row, long q_head, const void* k_ca
                         const void* v_cache, const void* block_tables, int max_blocks,
                         int block_size, const void* context_lens, const void* sink,
                         const void* gate, long gate_row, void* out, void* ws, float scale, int B,
-                        int H, int G, int splits, KeyRule rule, hipStream_t s) {
+                        int H, int G, int splits, KeyRule rule, int clear, hipStream_t s) {
     constexpr int E = 16 * VPL;
     constexpr bool ONCE = sizeof(T) == 2;
     const int R = H / G;
@@ -646,7 +646,7 @@ static int launch_split(const void* q, long q_row, long q_head, const void* k_ca
     if (hipGetLastError() != hipSuccess) return 2;
     hipLaunchKernelGGL(sink_attention_merge_kernel<T>, dim3(B * H), dim3(E >= 128 ? 128 : 64), 0, s,
                        (const float*)ws, (const float*)sink, (const T*)gate, gate_row,
-                       (const int*)context_lens, (T*)out, H, E, splits);
+                       (const int*)context_lens, (T*)out, H, E, splits, clear);
     return HYB_LAUNCH_OK();
 }
 
@@ -657,7 +657,8 @@ int hyb_sink_attention_split_ok(int D, int E) {
     return (D == 64 || D == 128 || D == 256) && (E == 64 || E == 128);
 }
 
-// Decode rows (row b = sequence b); ws: fp32 workspace of B * H * splits * (E + 2) floats.
+// Decode rows (row b = sequence b); ws: fp32 workspace of B * H * splits * (E + 2) floats; clear: rows without a
+// context become zeros.
 int hyb_sink_attention_split(const void* q, long q_row, long q_head, const void* k_cache,
                              const void* v_cache, const void* block_tables, int max_blocks,
                              int block_size, const void* context_lens, const void* sink,
@@ -665,7 +666,7 @@ int hyb_sink_attention_split(const void* q, long q_row, long q_head, const void*
                              int B, int H, int G, int D, int E, int splits, int window,
                              int keep_first, const void* slopes, int v_stride, const void* temps,
                              float softcap, int pool, int pool_rows, long pool_base, int chunk,
-                             int dt, hipStream_t s) {
+                             int clear, int dt, hipStream_t s) {
     const KeyRule rule{window, keep_first, (const float*)slopes, v_stride > 0 ? v_stride : E,
                        (const float*)temps, softcap, pool, pool_rows, pool_base, chunk};
     if (B <= 0) return 0;
@@ -674,7 +675,7 @@ int hyb_sink_attention_split(const void* q, long q_row, long q_head, const void*
     if (rule.v_stride < E || rule.v_stride % 8) return 1;      // 16-byte runs of a value row
     if (((size_t)k_cache | (size_t)v_cache | (size_t)q) % 16 || (q_row * (dt == 0 ? 2 : 4)) % 16) return 1;
 #define SPLIT_ARGS q, q_row, q_head, k_cache, v_cache, block_tables, max_blocks, block_size, \
-                   context_lens, sink, gate, gate_row, out, ws, scale, B, H, G, splits, rule, s
+                   context_lens, sink, gate, gate_row, out, ws, scale, B, H, G, splits, rule, clear, s
 #define SPLIT_E(T, EPL)                                                  \
     do {                                                                 \
         if (E == 64) return launch_split<T, EPL, 4>(SPLIT_ARGS);         \
@@ -707,7 +708,8 @@ int hyb_sink_attention_tiles_form(const void* q, long q_row, long q_head, const 
 }
 
 // Sequences seq0 .. seq0 + nseq - 1 of a prefill-form step (cu_q / block_tables indexed by the
-// absolute sequence number); max_q: longest portion among them.
+// absolute sequence number); max_q: longest portion among them.  clear_end > 0 (form 2 only): rows clear_first ..
+// clear_end - 1 that none of them owns become zeros.
 int hyb_sink_attention_tiles(const void* q, long q_row, long q_head, const void* k_cache,
                              const void* v_cache, const void* block_tables, int max_blocks,
                              int block_size, const void* cu_q, const void* positions,
@@ -715,7 +717,7 @@ int hyb_sink_attention_tiles(const void* q, long q_row, long q_head, const void*
                              float scale, int nseq, int seq0, int max_q, int H, int G, int D,
                              int E, int window, int keep_first, const void* slopes, int v_stride,
                              const void* temps, float softcap, int pool, int pool_rows,
-                             long pool_base, int chunk, int dt, hipStream_t s) {
+                             long pool_base, int chunk, long clear_first, long clear_end, int dt, hipStream_t s) {
     const KeyRule rule{window, keep_first, (const float*)slopes, v_stride > 0 ? v_stride : E,
                        (const float*)temps, softcap, pool, pool_rows, pool_base, chunk};
     if (nseq <= 0 || max_q <= 0) return 0;
@@ -726,7 +728,11 @@ int hyb_sink_attention_tiles(const void* q, long q_row, long q_head, const void*
                    positions, sink, gate, gate_row, out, scale, nseq, seq0, max_q, H, G, D, E
     const int form = hyb_sink_attention_tiles_form(q, q_row, q_head, k_cache, v_cache, out, nseq, max_q, D, E,
                                                    rule.v_stride, dt);
-    if (form == 2) return dt == 0 ? prompt_attention(TILES_ARGS, rule, s) : prompt_attention_f32(TILES_ARGS, rule, s);
+    if (form == 2) {
+        const RowSpan clear{clear_first, clear_end};
+        return dt == 0 ? prompt_attention(TILES_ARGS, rule, clear, s) : prompt_attention_f32(TILES_ARGS, rule, clear, s);
+    }
+    if (clear_end > 0) return 1;
 #define TILES_E(T, DP)                                                                       \
     do {                                                                                     \
         if (E <= 64) return launch_tiles<T, DP, 64>(TILES_ARGS, form == 1, rule, s);         \

@@ -68,6 +68,19 @@ inline bool pool_rule_ok(const KeyRule& r) {
                            r.pool_rows > 0 && r.pool_base > 0);
 }
 
+// Output rows of a step that no sequence owns are zeros where the kernel is asked to see to it (end > 0): those of
+// [first, end) ahead of its first sequence's and behind its last one's.  By the workgroups (head, sequence, part) of a grid.
+struct RowSpan { long first, end; };
+template <typename T>
+__device__ __forceinline__ void clear_rest(T* out, const int* cu_q, const RowSpan& span, int h, int H, int E) {
+    auto clear = [&](long from, long to) {
+        for (long r = from + blockIdx.z; r < to; r += gridDim.z)
+            for (int e = threadIdx.x; e < E; e += blockDim.x) out[(r * H + h) * E + e] = T(0);
+    };
+    if (blockIdx.y == 0) clear(span.first, cu_q[0]);
+    if (blockIdx.y + 1 == gridDim.y) clear(cu_q[gridDim.y], span.end);
+}
+
 // hybrid_prompts.hip: prompt portions over bfloat16 and (_f32) float caches, operands as
 // hyb_sink_attention_tiles; _ok: sizes in whole runs of eight numbers, 16-byte addresses, a grid that can
 // be launched
@@ -77,13 +90,13 @@ int prompt_attention(const void* q, long q_row, long q_head, const void* k_cache
                      const void* block_tables, int max_blocks, int block_size, const void* cu_q,
                      const void* positions, const void* sink, const void* gate, long gate_row, void* out,
                      float scale, int nseq, int seq0, int max_q, int H, int G, int D, int E,
-                     const KeyRule& rule, hipStream_t s);
+                     const KeyRule& rule, RowSpan clear, hipStream_t s);
 
 int prompt_attention_f32(const void* q, long q_row, long q_head, const void* k_cache, const void* v_cache,
                          const void* block_tables, int max_blocks, int block_size, const void* cu_q,
                          const void* positions, const void* sink, const void* gate, long gate_row, void* out,
                          float scale, int nseq, int seq0, int max_q, int H, int G, int D, int E,
-                         const KeyRule& rule, hipStream_t s);
+                         const KeyRule& rule, RowSpan clear, hipStream_t s);
 
 // the same over formed keys and values of latent attention (hybrid_latent_form.hip, with the operands of
 // hyb_latent_formed_prompts); _pages_ok: what the pages have to be

@@ -543,7 +543,7 @@ int hyb_latent_attention(const void* qa, long qa_row, long qa_head, const void* 
     if (rc || splits == 1) return rc;
     hipLaunchKernelGGL(sink_attention_merge_kernel<bf16_t>, dim3(nseq * H), dim3(R >= 128 ? 128 : 64), 0, s,
                        (const float*)ws, (const float*)sink, (const bf16_t*)nullptr, 0L,
-                       (const int*)lens, (bf16_t*)out, H, R, splits);
+                       (const int*)lens, (bf16_t*)out, H, R, splits, 0);
     return HYB_LAUNCH_OK();
 }
 

@@ -15,9 +15,13 @@ __global__ void sink_attention_merge_kernel(const float* __restrict__ ws,
                                             const float* __restrict__ sink,
                                             const T* __restrict__ gate, long gate_row,
                                             const int* __restrict__ context_lens,
-                                            T* __restrict__ out, int H, int E, int splits) {
+                                            T* __restrict__ out, int H, int E, int splits, int clear) {
     const int b = blockIdx.x / H, h = blockIdx.x % H;
-    if (context_lens[b] <= 0) return;
+    if (context_lens[b] <= 0) {                        // no sequence's row: zeros if the output is new, else as it is
+        if (clear)
+            for (int e = threadIdx.x; e < E; e += blockDim.x) st(out + ((long)b * H + h) * E + e, 0.f);
+        return;
+    }
     const int PS = E + 2;
     const float* p = ws + ((long)b * H + h) * splits * PS;
     float M = sink ? sink[h] : NO_SINK_MAX;

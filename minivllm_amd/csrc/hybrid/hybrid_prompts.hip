@@ -24,8 +24,8 @@
 // taken against the last reference, and formed again where that turns out too low.  The scalar work of a tile
 // (where the next lies) was a fifth of its time as expressions of the tile's number: it is kept up instead.
 //
-// 8 prompts of 512..1024 tokens, 16 / 8 heads of 128, sink and gate: 68 -> 63.8 us for the layer, 5 to 7 of which the clearing
-// of the output takes; one of 1024 tokens alone 46 -> 36 (a tile in 2260 cycles of a lone wave: 1024 of products,
+// 8 prompts of 512..1024 tokens, 16 / 8 heads of 128, sink and gate: 68 -> 59 us for the layer, 65 of which as long as a
+// fill of the output ran ahead of it; one of 1024 tokens alone 46 -> 36 (a tile in 2260 cycles of a lone wave: 1024 of products,
 // some 1000 of vector issue beside them; two waves on a SIMD take 1600 each).  Before that the waves formed score
 // product, softmax and value product one after the other (a tile of 32 in 3350 cycles).  What is left: the clock (1.9
 // GHz under this load), 6 us at the two ends of a workgroup, and the last workgroups, of which not all CUs have one.
@@ -52,6 +52,7 @@ struct PromptArgs {
     const uint16_t* q_turned; long turned_row;     // [T, H, P]
     const uint16_t* latents; int latent_row, P;    // cache rows of latent_row numbers
     long formed_rows;
+    RowSpan clear;
     uint32_t page_magic;                           // key / block_size == key * page_magic >> 32 for every key there can be (0: none)
 };
 
@@ -158,6 +159,7 @@ prompt_attention_kernel(PromptArgs a) {
     const int H = a.H, hx = blockIdx.x;
     const int h = H % 8 == 0 ? (hx & 7) * (H >> 3) + (hx >> 3) : hx;
     const int b = blockIdx.y + a.seq0, tile_q0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * 128;
+    if (a.clear.end > 0) clear_rest(a.out, a.cu_q + a.seq0, a.clear, h, H, a.E);
     const int row0 = __builtin_amdgcn_readfirstlane(a.cu_q[b]), qlen = __builtin_amdgcn_readfirstlane(a.cu_q[b + 1]) - row0;
     if (tile_q0 >= qlen) return;
     const int start = __builtin_amdgcn_readfirstlane(a.positions[row0]), G = a.G, g = h / (H / G);
@@ -723,6 +725,7 @@ struct PromptArgs32 {
     float scale;
     int H, G, D, E, seq0;
     KeyRule rule;
+    RowSpan clear;
 };
 
 template <int DP, int EP, bool EXT>
@@ -738,6 +741,7 @@ prompt_attention_f32_kernel(PromptArgs32 a) {
     const int H = a.H, hx = blockIdx.x;
     const int h = H % 8 == 0 ? (hx & 7) * (H >> 3) + (hx >> 3) : hx;
     const int b = blockIdx.y + a.seq0, tile_q0 = ((int)gridDim.z - 1 - (int)blockIdx.z) * 128;
+    if (a.clear.end > 0) clear_rest(a.out, a.cu_q + a.seq0, a.clear, h, H, a.E);
     const int row0 = a.cu_q[b], qlen = a.cu_q[b + 1] - row0;
     if (tile_q0 >= qlen) return;
     const int start = a.positions[row0], G = a.G, g = h / (H / G);
@@ -999,10 +1003,10 @@ int prompt_attention(const void* q, long q_row, long q_head, const void* k_cache
                      const void* block_tables, int max_blocks, int block_size, const void* cu_q,
                      const void* positions, const void* sink, const void* gate, long gate_row, void* out,
                      float scale, int nseq, int seq0, int max_q, int H, int G, int D, int E,
-                     const KeyRule& rule, hipStream_t s) {
+                     const KeyRule& rule, RowSpan clear, hipStream_t s) {
     const PromptArgs a{(const uint16_t*)q, q_row, q_head, (const uint16_t*)k_cache, (const uint16_t*)v_cache,
                        (const int*)block_tables, max_blocks, block_size, (const int*)cu_q, (const int*)positions,
-                       (const float*)sink, (const bf16_t*)gate, gate_row, (uint16_t*)out, scale, H, G, D, E, seq0, rule, nullptr, 0, nullptr, 0, 0, 0, 
+                       (const float*)sink, (const bf16_t*)gate, gate_row, (uint16_t*)out, scale, H, G, D, E, seq0, rule, nullptr, 0, nullptr, 0, 0, 0, clear,
                        page_magic(block_size, max_blocks, 2L * G * (D > rule.v_stride ? D : rule.v_stride))};
 #define PICK(DP, EP) if (D <= DP && E <= EP) return launch<DP, EP>(a, nseq, max_q, s)
     PICK(64, 64);
@@ -1021,10 +1025,10 @@ int prompt_attention_f32(const void* q, long q_row, long q_head, const void* k_c
                          const void* block_tables, int max_blocks, int block_size, const void* cu_q,
                          const void* positions, const void* sink, const void* gate, long gate_row, void* out,
                          float scale, int nseq, int seq0, int max_q, int H, int G, int D, int E,
-                         const KeyRule& rule, hipStream_t s) {
+                         const KeyRule& rule, RowSpan clear, hipStream_t s) {
     const PromptArgs32 a{(const float*)q, q_row, q_head, (const float*)k_cache, (const float*)v_cache,
                          (const int*)block_tables, max_blocks, block_size, (const int*)cu_q, (const int*)positions,
-                         (const float*)sink, (const float*)gate, gate_row, (float*)out, scale, H, G, D, E, seq0, rule};
+                         (const float*)sink, (const float*)gate, gate_row, (float*)out, scale, H, G, D, E, seq0, rule, clear};
     if (D <= 64) return E <= 64 ? launch_f32<64, 64>(a, nseq, max_q, s) : launch_f32<64, 128>(a, nseq, max_q, s);
     return E <= 64 ? launch_f32<128, 64>(a, nseq, max_q, s) : launch_f32<128, 128>(a, nseq, max_q, s);
 }
@@ -1045,7 +1049,7 @@ int latent_prompts(const void* q, long q_row, long q_head, const void* qr, long 
                        (const int*)block_tables, max_blocks, block_size, (const int*)cu_q, (const int*)positions,
                        (const float*)sink, nullptr, 0, (uint16_t*)out, scale, H, 1, D, E, 0, rule,
                        (const uint16_t*)qr, qr_row, (const uint16_t*)cache, R + P, P, formed_rows,
-                       page_magic(block_size, max_blocks, 2L * (R + P))};
+                       RowSpan{0, 0}, page_magic(block_size, max_blocks, 2L * (R + P))};
     return P <= 64 ? launch_form<128, 64, 128, 2, false, true>(a, nseq, max_q, s)
                    : launch_form<128, 128, 128, 2, false, true>(a, nseq, max_q, s);
 }

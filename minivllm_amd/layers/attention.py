@@ -243,9 +243,10 @@ class SinkAttention(nn.Module):
         if self.k_cache is None:
             raise RuntimeError("attention needs an allocated KV cache")
         T = q.shape[0]
-        out = torch.zeros((T, self.num_heads, self.v_head_dim), dtype=q.dtype, device=q.device)
+        # (the calls clear the rows that belong to no sequence)
+        out = torch.empty((T, self.num_heads, self.v_head_dim), dtype=q.dtype, device=q.device)
         a = (self.k_cache, self.v_cache)
-        opt = dict(window=self.window, keep_first=self.keep_first, slopes=self.slopes)
+        opt = dict(clear=True, window=self.window, keep_first=self.keep_first, slopes=self.slopes)
         if self.temps is not None or self.softcap or self.pool:
             opt.update(temps=self.temps, softcap=self.softcap, pool=self.pool, k_pool=self.k_pool,
                        v_pool=self.v_pool)
@@ -263,6 +264,8 @@ class SinkAttention(nn.Module):
                                            ctx.block_tables[Bd:], self.scale, self.sink, gate, out,
                                            positions=ctx.positions, max_q=ctx.max_seqlen_q or None,
                                            row_seq=ctx.row_seq, first_seq=Bd, **opt)
+            else:
+                out[Bd:].zero_()
             if Bd:
                 ops.sink_attention_decode(q[:Bd], *a, ctx.block_tables[:Bd], ctx.context_lens,
                                           self.scale, self.sink,

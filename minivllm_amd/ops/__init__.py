@@ -277,7 +277,7 @@ def pair_rope_mix_store(q, k, v, positions, cos_sin, rot_dims, v_first, lam, v_m
 def sink_attention_prefill(q, k_cache, v_cache, cu_q, cu_k, block_tables, scale, sink, gate, out,
                            positions=None, max_q=None, row_seq=None, first_seq=0,
                            window=0, keep_first=0, slopes=None, temps=None, softcap=0.0, pool=0,
-                           k_pool=None, v_pool=None, chunk=0):
+                           k_pool=None, v_pool=None, chunk=0, clear=False):
     """``temps`` [H] fp32: a score multiplier per head; ``softcap`` > 0: score <- softcap
     tanh(score / softcap); ``pool`` > 0 with ``k_pool`` / ``v_pool``: one pooled key / value per
     block of ``pool`` tokens that has passed out of the window as a whole
@@ -288,14 +288,17 @@ def sink_attention_prefill(q, k_cache, v_cache, cu_q, cu_k, block_tables, scale,
     everything from ``cu_q`` / ``cu_k``.  ``sink`` None: no sink term.  ``window`` > 0: a query at
     position i sees key j <= i only if i - j < window or j < keep_first.  ``slopes`` [H] fp32:
     slope_h * (i - j) is taken off the score.  ``chunk`` > 0: a query sees only keys of its own run of
-    ``chunk`` positions, counted from position 0 of the sequence."""
+    ``chunk`` positions, counted from position 0 of the sequence.  ``clear``: ``out`` is new, rows from row
+    ``first_seq`` on that no sequence owns become zeros (otherwise they stay as they are)."""
     if _on_gpu(q):
         return _hybrid().sink_attention_prefill(q, k_cache, v_cache, cu_q, cu_k, block_tables,
                                                 scale, sink, gate, out, positions=positions,
                                                 max_q=max_q, row_seq=row_seq, first_seq=first_seq,
                                                 window=window, keep_first=keep_first, slopes=slopes,
                                                 temps=temps, softcap=softcap, pool=pool,
-                                                k_pool=k_pool, v_pool=v_pool, chunk=chunk)
+                                                k_pool=k_pool, v_pool=v_pool, chunk=chunk, clear=clear)
+    if clear:
+        out[first_seq:].zero_()
     return torch_seqmix.sink_attention_prefill(q, k_cache, v_cache, cu_q, cu_k, block_tables,
                                                scale, sink, gate, out, window, keep_first, slopes,
                                                temps, softcap, pool, k_pool, v_pool, chunk)
@@ -311,15 +314,18 @@ def sink_attention_step(q, k_cache, v_cache, block_tables, row_seq, positions, s
 
 def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale, sink, gate, out,
                           max_context_len=None, window=0, keep_first=0, slopes=None, temps=None,
-                          softcap=0.0, pool=0, k_pool=None, v_pool=None, chunk=0):
+                          softcap=0.0, pool=0, k_pool=None, v_pool=None, chunk=0, clear=False):
     """``max_context_len`` (a host integer, an upper bound will do): lets the GPU form size its
-    context splits without reading the lengths back."""
+    context splits without reading the lengths back.  ``clear``: ``out`` is new, rows without a context become
+    zeros (otherwise they stay as they are)."""
     if _on_gpu(q):
         return _hybrid().sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens,
                                                scale, sink, gate, out, max_context_len,
                                                window=window, keep_first=keep_first, slopes=slopes,
                                                temps=temps, softcap=softcap, pool=pool,
-                                               k_pool=k_pool, v_pool=v_pool, chunk=chunk)
+                                               k_pool=k_pool, v_pool=v_pool, chunk=chunk, clear=clear)
+    if clear:
+        out.zero_()
     return torch_seqmix.sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens,
                                               scale, sink, gate, out, window, keep_first, slopes,
                                               temps, softcap, pool, k_pool, v_pool, chunk)

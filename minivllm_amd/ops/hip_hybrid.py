@@ -43,13 +43,13 @@ _POOL = (_P, _F, _I, _I, _L, _I)
 _attn = _sig("hyb_sink_attention_rows", _P, _L, _L, _P, _P, _P, _I, _I, _P, _P, _I, _P, _P, _L, _P,
              _F, _L, _I, _I, _I, _I, _I, _I, _I, _P, _I, *_POOL, _I, _P)
 _tiles = _sig("hyb_sink_attention_tiles", _P, _L, _L, _P, _P, _P, _I, _I, _P, _P, _P, _P, _L, _P, _F,
-              _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, *_POOL, _I, _P)
+              _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, *_POOL, _L, _L, _I, _P)
 _tiles_ok = _lib.hyb_sink_attention_tiles_ok
 _tiles_ok.argtypes = [_I, _I]
 _tiles_ok.restype = _I
 _tiles_form = _sig("hyb_sink_attention_tiles_form", _P, _L, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I)
 _split = _sig("hyb_sink_attention_split", _P, _L, _L, _P, _P, _P, _I, _I, _P, _P, _P, _L, _P, _P, _F,
-              _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, *_POOL, _I, _P)
+              _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, *_POOL, _I, _I, _P)
 _split_heads = _sig("hyb_sink_attention_split_heads", _I)
 _split_ok = _lib.hyb_sink_attention_split_ok
 _split_ok.argtypes = [_I, _I]
@@ -282,17 +282,20 @@ def sink_attention_step(q, k_cache, v_cache, block_tables, row_seq, positions, s
 def sink_attention_prefill(q, k_cache, v_cache, cu_q, cu_k, block_tables, scale, sink, gate, out,
                            positions=None, max_q=None, row_seq=None, first_seq=0,
                            window=0, keep_first=0, slopes=None, temps=None, softcap=0.0, pool=0,
-                           k_pool=None, v_pool=None, chunk=0):
+                           k_pool=None, v_pool=None, chunk=0, clear=False):
     """The prompt portions of a step: sequence b owns rows cu_q[b] .. cu_q[b+1] (absolute rows
     of q / out / positions) and block table row b.  Runs the matrix-core tile kernel (fp32
     scores, weights and sums); head sizes it has no instance for go row by row.  ``cu_k`` is
-    not needed (a row's context is its position + 1)."""
+    not needed (a row's context is its position + 1).  ``clear``: ``out`` is new, rows from
+    ``first_seq`` on that none of the sequences owns become zeros (otherwise they stay as they are)."""
     T, H, D = q.shape
     G, E = k_cache.shape[2], v_cache.shape[3]
     nseq = cu_q.shape[0] - 1
     assert positions is not None, "the GPU form takes the rows' positions"
     if not _tiles_ok(D, E):
         assert row_seq is not None
+        if clear:
+            out[first_seq:].zero_()
         # ``first_seq``: number of the step's sequences ahead of these (its decode riders)
         return sink_attention_step(q, k_cache, v_cache, block_tables, row_seq, positions, scale,
                                    sink, gate, out, seq_base=first_seq, window=window,
@@ -306,6 +309,11 @@ def sink_attention_prefill(q, k_cache, v_cache, cu_q, cu_k, block_tables, scale,
     assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1
     if gate is not None:
         assert gate.stride(1) == 1 and gate.dtype == q.dtype
+    if clear and (nseq <= 0 or max_q <= 0 or _tiles_form(
+            q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), nseq,
+            max_q, D, E, vs, _dt(q)) != 2):
+        out[first_seq:].zero_()
+        clear = False
     _check(_tiles(q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(),
                   block_tables.data_ptr(), block_tables.stride(0), k_cache.shape[1],
                   _i32c(cu_q).data_ptr(), _i32(positions).data_ptr(),
@@ -313,7 +321,7 @@ def sink_attention_prefill(q, k_cache, v_cache, cu_q, cu_k, block_tables, scale,
                   _ptr(gate), gate.stride(0) if gate is not None else 0, out.data_ptr(), scale,
                   nseq, 0, max_q, H, G, D, E, int(window), int(keep_first), _slopes(slopes, H), vs,
                   *_pool_args(k_cache, v_cache, vs, H, temps, softcap, pool, k_pool, v_pool), int(chunk),
-                  _dt(q), _stream()), "sink_attention_prefill")
+                  first_seq if clear else 0, T if clear else 0, _dt(q), _stream()), "sink_attention_prefill")
     return out
 
 
@@ -335,11 +343,12 @@ def decode_splits(batch: int, kv_heads: int, heads: int, max_context_len) -> int
 
 def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale, sink, gate, out,
                           max_context_len=None, window=0, keep_first=0, slopes=None, temps=None,
-                          softcap=0.0, pool=0, k_pool=None, v_pool=None, chunk=0):
+                          softcap=0.0, pool=0, k_pool=None, v_pool=None, chunk=0, clear=False):
     """Single next tokens: row b is sequence b with ``context_lens[b]`` keys.  Head sizes the
     split-context kernel has an instance for (D in 64 / 128 / 256, E in 64 / 128) stream K / V
     rows with coalesced 16-byte loads over several workgroups per sequence and are merged by a
-    second small kernel; other sizes go through the row kernel."""
+    second small kernel; other sizes go through the row kernel.  ``clear``: ``out`` is new, rows without a
+    context become zeros (otherwise they stay as they are)."""
     B, H, D = q.shape
     G, E = k_cache.shape[2], v_cache.shape[3]
     es = q.element_size()
@@ -364,9 +373,11 @@ def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale
                       ws.data_ptr(), scale, B, H, G, D, E, splits, int(window), int(keep_first),
                       _slopes(slopes, H), vs,
                       *_pool_args(k_cache, v_cache, vs, H, temps, softcap, pool, k_pool, v_pool), int(chunk),
-                      _dt(q), _stream()),
+                      int(clear), _dt(q), _stream()),
                "sink_attention_decode")
         return out
+    if clear:
+        out.zero_()
     return _attention_rows(q, k_cache, v_cache, block_tables, None, context_lens, 0, scale, sink,
                            gate, out, 0, window, keep_first, slopes, temps, softcap, pool, k_pool, v_pool,
                            chunk)
