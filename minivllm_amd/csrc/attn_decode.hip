@@ -47,14 +47,16 @@ constexpr int kTile = 32;          // tokens per wave iteration
 // (workgroups of WAVES waves).  The grid of a captured step is sized for the longest context the
 // engine admits, and a split costs the merge (write-through partials, a ticket, reading them
 // back: 2 us, more with every split).  A context of up to 1.25 tiles per wave therefore stays in one
-// workgroup, without partials; a longer one is bound by what one CU reads (a workgroup's
-// 256 tokens take 0.9 us) and takes a split for every half workgroup of tiles (one for every whole one is slower
-// below 2000 tokens: 8.2 us at 512, one for every two tiles 7.4).  4 sequences, 16 / 8 heads of 128, grid for 2048 tokens, us a launch
-// before (16 splits of 4 waves, all of them merged) and now: 128 tokens 8.1 -> 4.5, 264 7.9 -> 6.4,
-// 512 9.2 -> 7.0, 1024 10.0 -> 7.8, 2048 10.4 -> 8.8.
+// workgroup, without partials; a longer one is bound by what one CU reads (a workgroup's 256 tokens take 0.9 us)
+// and takes a split for every half workgroup of tiles (one for every whole one is slower below 2000 tokens:
+// 8.2 us at 512, one for every two tiles 7.4), but from 8 on for every whole one (one sequence of 4096, 32 / 8 heads:
+// 16 splits 8.8 us, 32 10.1).  4 sequences, 16 / 8 heads of 128, grid for 2048 tokens, us a launch
+// before (16 splits of 4 waves, all of them merged) and now: 128 tokens 8.1 -> 4.3, 264 7.9 -> 6.4,
+// 512 9.2 -> 6.8, 1024 10.0 -> 7.6, 2048 10.4 -> 8.6.
 template <int WAVES>
 __device__ __forceinline__ int splits_in_use(int tiles, int nsplit) {
-    return tiles <= WAVES + WAVES / 4 ? 1 : min(nsplit, (2 * tiles + WAVES - 1) / WAVES);
+    if (tiles <= WAVES + WAVES / 4) return 1;
+    return min(nsplit, max(min(8, (2 * tiles + WAVES - 1) / WAVES), (tiles + WAVES - 1) / WAVES));
 }
 
 // Device-scope ("agent") relaxed accesses to global memory: stores are written through to
@@ -265,8 +267,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
 #pragma unroll
             for (int i = 0; i < 8; ++i) ss += x[s][i] * x[s][i];
         }
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
+        ss = pair_sum<32>(pair_sum<16>(ss));
         if (wgt != nullptr) {
             const float rstd = rsqrtf(ss / (float)D + fu.eps);
 #pragma unroll
@@ -383,8 +384,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
                 p[4 * sub + r] = v;
                 m_tile = fmaxf(m_tile, v);
             }
-        m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 16, 64));
-        m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 32, 64));
+        m_tile = pair_max<32>(pair_max<16>(m_tile));
         const float m_new = fmaxf(m_run, m_tile);          // finite: the tile has >= 1 token
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         float psum = 0.f;
@@ -418,8 +418,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
     }
 
     // ---- merge the waves through LDS (each wave reuses its own staging region)
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = pair_sum<32>(pair_sum<16>(l_run));
     float* wbuf = reinterpret_cast<float*>(smem + w * WAVE_LDS);
     if (q4 == 0) { wbuf[c16] = m_run; wbuf[16 + c16] = l_run; }
 #pragma unroll

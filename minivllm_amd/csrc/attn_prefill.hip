@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kThreads, 2) void flash_prefill_kernel(PrefillArgs 
 #pragma unroll
             for (int i = 0; i < 8; ++i) ss += f[i] * f[i];
         }
-        ss += __shfl_xor(ss, 32, 64);                    // the other half of the row
+        ss = pair_sum<32>(ss);                    // the other half of the row
         const float rstd = a.q_w != nullptr ? rsqrtf(ss / (float)D + a.eps) : 1.f;
 #pragma unroll
         for (int s = 0; s < KSTEPS / 2; ++s) {
@@ -486,7 +486,7 @@ __global__ __launch_bounds__(kThreads, 2) void flash_prefill_kernel(PrefillArgs 
                 }
                 m_tile = fmaxf(m_tile, s_acc[sub][e]);
             }
-        m_tile = fmaxf(m_tile, __shfl_xor(m_tile, 32, 64)) * a.scale_log2;   // scale > 0
+        m_tile = pair_max<32>(m_tile) * a.scale_log2;   // scale > 0
         // rescale only when needed (wave-uniform decision; NaN-safe: -inf - -inf counts)
         if (!__all(m_tile - m_run <= kRescaleThr)) {
             const float m_new = fmaxf(m_run, m_tile);
@@ -614,7 +614,7 @@ __global__ __launch_bounds__(kThreads, 2) void flash_prefill_kernel(PrefillArgs 
 
     __builtin_amdgcn_s_setprio(0);
     // ---- epilogue: O[q][d] = O^T / l --------------------------------------------------
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = pair_sum<32>(l_run);
     {
         // A row's 8 d-values of group k = 4 n + g8 are split over the two lane halves (4 + 4), so
         // the natural store is 8 bytes per lane.  One half exchange per dword between groups k

@@ -116,6 +116,34 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// v and its partner's 16 (32) lanes away, in an order that may differ between the two, by a swap inside the vector unit
+// (all lanes active); a __shfl_xor goes through LDS: some 100 cycles instead of 10
+struct LanePair { float a, b; };
+template <int N>
+__device__ __forceinline__ LanePair lane_pair(float v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    static_assert(N == 16 || N == 32);
+    const uint32_t u = __float_as_uint(v);
+    if constexpr (N == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+    }
+#else
+    return {v, v};
+#endif
+}
+template <int N> __device__ __forceinline__ float pair_sum(float v) {
+    const LanePair p = lane_pair<N>(v);
+    return p.a + p.b;
+}
+template <int N> __device__ __forceinline__ float pair_max(float v) {
+    const LanePair p = lane_pair<N>(v);
+    return fmaxf(p.a, p.b);
+}
+
 // Sum over all threads of a block (<= 1024 threads).  `scratch` holds >= 16 floats.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
     v = wave_sum(v);

@@ -556,10 +556,7 @@ sink_attention_split_kernel(const T* __restrict__ q, long q_row, long q_head,
                 float d = 0.f;
 #pragma unroll
                 for (int i = 0; i < EPL; ++i) d += kf[x][i] * qf[r][i];
-                d += __shfl_xor(d, 1, kWave);
-                d += __shfl_xor(d, 2, kWave);
-                d += __shfl_xor(d, 4, kWave);
-                d += __shfl_xor(d, 8, kWave);
+                d = run_sum<16>(d);
                 d = (EXT ? rule.capped(d) : d) - slope[r] * dist;
                 if (d > m[r]) {                    // the running maximum moves: rescale (rare)
                     const float a = expf(m[r] - d);

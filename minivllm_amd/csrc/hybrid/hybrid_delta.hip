@@ -207,7 +207,9 @@ delta_prepare_rows_kernel(const T* __restrict__ proj, long row_stride, int b_off
         }
         if (!ssd) {
             if (exchange) {
-                for (int o = 1; o < lanes; o <<= 1) sq += __shfl_xor(sq, o, kWave);
+                if (lanes == 16) sq = run_sum<16>(sq);                 // (uniform: heads of 128)
+                else
+                    for (int o = 1; o < lanes; o <<= 1) sq += __shfl_xor(sq, o, kWave);
             } else {
                 __syncthreads();                                   // (every thread is in the same row)
                 part[tid] = sq;
@@ -394,8 +396,7 @@ delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
                     d2 += S[4 * i + 2] * k4[i].z; d3 += S[4 * i + 3] * k4[i].w;
                 }
                 float dot = (d0 + d1) + (d2 + d3);
-                dot += __shfl_xor(dot, 1, kWave);
-                dot += __shfl_xor(dot, 2, kWave);
+                dot = run_sum<4>(dot);
                 u = bt * (ve - gd * dot);
             }
             float o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f;
@@ -407,8 +408,7 @@ delta_scan_kernel(const float* __restrict__ qn, const float* __restrict__ kn,
                 S[4 * i + 3] = gd * S[4 * i + 3] + k4[i].w * u; o3 += S[4 * i + 3] * q4[i].w;
             }
             float out = (o0 + o1) + (o2 + o3);
-            out += __shfl_xor(out, 1, kWave);
-            out += __shfl_xor(out, 2, kWave);
+            out = run_sum<4>(out);
             if (col && r == 0) o[((first + ch * CT + tok) * H + h) * (long)E + e] = out;
         }
         if (ch + 1 < nchunks) stash(reg, sm + ((ch + 1) & 1) * BUF);

@@ -214,8 +214,9 @@ gated_head_norm_runs_kernel(const float* __restrict__ o, const float* __restrict
 #pragma unroll
         for (int i = 0; i < 8; ++i) s += v[i] * v[i];
     }
+    s = run_sum<(LPH < 16 ? LPH : 16)>(s);
 #pragma unroll
-    for (int x = 1; x < LPH; x <<= 1) s += __shfl_xor(s, x, kWave);
+    for (int x = 16; x < LPH; x <<= 1) s += __shfl_xor(s, x, kWave);
     if (!live) return;
     const float r = rsqrtf(s / (float)E + eps);
 #pragma unroll

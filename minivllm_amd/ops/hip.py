@@ -411,7 +411,9 @@ def decode_num_splits(batch: int, num_kv_heads: int, max_context_len: Optional[i
     n, waves = (wide, 8) if 2 * wide >= narrow else (narrow, 4)
     if max_context_len is not None:
         tiles = (max_context_len + 31) // 32
-        n = 1 if tiles <= waves + waves // 4 else min(n, (2 * tiles + waves - 1) // waves)
+        if tiles <= waves + waves // 4:
+            return 1
+        n = min(n, max(min(8, -(-2 * tiles // waves)), -(-tiles // waves)))
     return n
 
 
