@@ -12,9 +12,15 @@ from . import torch_ref
 from .partials import PendingReduce, ResidualShard, ResidualSum, ScatteredRows, SplitKPartials
 
 
+_HIP = None
+
+
 def _hip():
-    from . import hip        # raises with a build hint when the .so is absent
-    return hip
+    global _HIP
+    if _HIP is None:             # (the import statement of a loaded module costs each call 0.7 us)
+        from . import hip        # raises with a build hint when the .so is absent
+        _HIP = hip
+    return _HIP
 
 
 def _on_gpu(t: torch.Tensor) -> bool:
@@ -247,9 +253,15 @@ def sample(logits, temperatures, seed=0, step=0, generator=None):
 from . import torch_seqmix
 
 
+_HYBRID = None
+
+
 def _hybrid():
-    from . import hip_hybrid     # raises with a build hint when the library is absent
-    return hip_hybrid
+    global _HYBRID
+    if _HYBRID is None:
+        from . import hip_hybrid     # raises with a build hint when the library is absent
+        _HYBRID = hip_hybrid
+    return _HYBRID
 
 
 def _seqmix(t):

@@ -458,24 +458,30 @@ def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     ``context_lens - 1``.  The kernel norms and rotates q and k itself and writes k / v into the
     caches at those positions: the stand-alone norm + rotate + store kernel is not needed."""
     B, hq, d = q.shape
-    hkv = k_cache.shape[2]
+    block, hkv = k_cache.shape[1:3]
     bt, ctx = _i32(block_tables), _i32(context_lens)
-    qs_b, qs_h = _q_strides(q)
+    qs_b, qs_h, qs_d = q.stride()
+    assert qs_d == 1, "q must be [T, H, D] with contiguous D"
     sb, st, sh = _cache_strides(k_cache)
-    assert _cache_strides(v_cache) == (sb, st, sh)
-    assert bt.stride(1) == 1
+    assert v_cache.stride() == k_cache.stride()
+    bt_row, bt_col = bt.stride()
+    assert bt_col == 1
     ns = num_splits or decode_num_splits(B, hkv, max_context_len)
     if out is None:
         out = torch.empty((B, hq, d), dtype=q.dtype, device=q.device)
-    assert out.shape == (B, hq, d) and out.stride(2) == 1 and out.dtype == q.dtype
+        os_b, os_h = hq * d, d
+    else:
+        os_b, os_h, os_d = out.stride()
+        assert out.shape == (B, hq, d) and os_d == 1 and out.dtype == q.dtype
     if ns > 1:
-        part_acc = torch.empty(B * hq * ns * d, dtype=torch.float32, device=q.device)
-        part_ml = torch.empty(B * hq * ns * 2, dtype=torch.float32, device=q.device)
+        rows = B * hq * ns
+        part = torch.empty(rows * (d + 2), dtype=torch.float32, device=q.device)   # sums, then maxima and normalisers
         need = B * hkv * ((hq // hkv + 15) // 16)
         if tickets is None:
             tickets = decode_ticket_words(q.device, need)
         assert tickets.dtype == torch.int32 and tickets.numel() >= need and tickets.is_contiguous()
-        pa, pm, tk = part_acc.data_ptr(), part_ml.data_ptr(), tickets.data_ptr()
+        pa, tk = part.data_ptr(), tickets.data_ptr()
+        pm = pa + rows * d * 4
     else:
         pa = pm = tk = None
     fuse = (None, None, None, None, None, 0.0)
@@ -498,8 +504,8 @@ def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
                 q_w.data_ptr() if q_w is not None else None,
                 k_w.data_ptr() if k_w is not None else None, float(eps))
     _check(_decode(q.data_ptr(), qs_b, qs_h, k_cache.data_ptr(), v_cache.data_ptr(), sb, st, sh,
-                   bt.data_ptr(), bt.stride(0), ctx.data_ptr(), out.data_ptr(), out.stride(0),
-                   out.stride(1), pa, pm, tk, scale, B, hq, hkv, d, k_cache.shape[1], ns, _dt(q),
+                   bt.data_ptr(), bt_row, ctx.data_ptr(), out.data_ptr(), os_b,
+                   os_h, pa, pm, tk, scale, B, hq, hkv, d, block, ns, _dt(q),
                    _kv_fp8(k_cache), *fuse, _stream()), "paged_attention_decode")
     return out
 
