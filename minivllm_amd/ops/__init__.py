@@ -154,7 +154,7 @@ def linear(x, weight, bias=None, to_norm=False, residual=None):
     if _on_gpu(x) and x.dim() == 2 and x.shape[0] <= 256:
         h = _hip()
         if x.shape[0] <= 16:
-            sp = h.skinny_gemm_splits(x, weight) if to_norm else None
+            sp = h.skinny_gemm_splits(x, weight, bias) if to_norm else None
             if sp:
                 return h.skinny_linear(x, weight, bias, splits=sp, defer=True)
             if sp is None and h.skinny_gemm_pays(x, weight):
@@ -169,7 +169,7 @@ def linear(x, weight, bias=None, to_norm=False, residual=None):
             return h.big_linear_resid(x, weight, bias, residual)
         if h.big_gemm_pays(x, weight):
             return h.big_linear(x, weight, bias)
-        c = h.tiled_gemm_choice(x, weight, to_norm=to_norm)
+        c = h.tiled_gemm_choice(x, weight, to_norm=to_norm, bias=bias)
         if c is not None:
             return h.mid_linear(x, weight, bias, False, c[1], c[2], False, c[0], defer=to_norm)
     return F.linear(x, weight, bias)
@@ -193,7 +193,7 @@ def swiglu_linear(x, weight, bias=None):
         h = _hip()
         if h.big_gemm_pays(x, weight, swiglu=True):
             return h.big_linear(x, weight, bias, swiglu=True)      # prefill: GEMM + SwiGLU in one kernel
-        c = h.tiled_gemm_choice(x, weight, swiglu=True)
+        c = h.tiled_gemm_choice(x, weight, swiglu=True, bias=bias)
         if c is not None:
             return h.mid_linear(x, weight, bias, True, c[1], c[2], False, c[0])
     return silu_and_mul(F.linear(x, weight, bias))

@@ -511,6 +511,15 @@ def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
 
 
 # ------------------------------------------------------- weight-streaming GEMM
+def _rule_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
+    """What a call has to be for a rule (not a measurement of the engine's own weights) to send it from the library to a
+    kernel: nothing to differentiate, weight and bias where runs of 16 bytes can be read."""
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
+        return False
+    return weight.data_ptr() % 16 == 0 and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous()
+                                                             and bias.data_ptr() % 16 == 0))
+
+
 SKINNY_MAX_ROWS = 16
 SKINNY_PAYS_ROWS = 16                 # up to here the kernel beats the library (see skinny_gemm_pays)
 SKINNY_MIN_WEIGHT_BYTES = 8 << 20     # below this an unmeasured projection goes to the library (see skinny_gemm_pays)
@@ -560,7 +569,7 @@ def skinny_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False
     return swiglu or (n <= 4096 and k <= 4096)
 
 
-def skinny_gemm_splits(x: torch.Tensor, weight: torch.Tensor) -> Optional[int]:
+def skinny_gemm_splits(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> Optional[int]:
     """For a projection whose output goes straight into residual add + RMSNorm: the K split
     (over workgroups) that was measured fastest together with that norm, 0 = library GEMM.
     Never measured: ``skinny_narrow_splits`` where the output is narrow, otherwise None (the caller
@@ -568,7 +577,10 @@ def skinny_gemm_splits(x: torch.Tensor, weight: torch.Tensor) -> Optional[int]:
     if x.dim() != 2 or x.shape[0] > SKINNY_PAYS_ROWS or not skinny_gemm_ok(x, weight):
         return None
     n, k = weight.shape
-    return _SKINNY_CHOICE.get((_row_bucket(x.shape[0]), n, k, "norm"), skinny_narrow_splits(n, k))
+    choice = _SKINNY_CHOICE.get((_row_bucket(x.shape[0]), n, k, "norm"))
+    if choice is None and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and _rule_takes(x, weight, bias):
+        return skinny_narrow_splits(n, k)
+    return choice
 
 
 def skinny_narrow_splits(n: int, k: int) -> Optional[int]:
@@ -714,7 +726,7 @@ def skinny_norm_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = 
         return False
     n, k = weight.shape
     if x.shape[0] > SKINNY_NORM_MAX_ROWS and (k > 1024 or k % 256 or n > 8192 or x.stride(0) % 8
-                                              or x.data_ptr() % 16):
+                                              or (x.data_ptr() | weight.data_ptr()) % 16):
         return False
     return swiglu or n <= 8192
 
@@ -729,7 +741,8 @@ def skinny_norm_partials_pays(part: SplitKPartials, residual: Optional[torch.Ten
     n = weight.shape[0]
     if (slices > 4 or m > SKINNY_MAX_ROWS or n > 8192 or k % 256 or n % (32 if swiglu else 16)
             or weight.dtype != part.dtype or weight.shape[1] != k or not weight.is_contiguous()
-            or part.dtype not in _DT or m * (k + 8) * 2 > _STAGED_ROWS_BYTES):
+            or part.dtype not in _DT or m * (k + 8) * 2 > _STAGED_ROWS_BYTES or weight.data_ptr() % 16
+            or (part.bias is not None and part.bias.data_ptr() % 16)):
         return False
     if residual is not None and (residual.shape != (m, k) or residual.dtype != part.dtype or residual.stride(1) != 1
                                  or residual.stride(0) % 8 or residual.data_ptr() % 16):
@@ -899,10 +912,12 @@ def tiled_gemm_sizes(m: int, n: int, k: int, swiglu: bool, to_norm: bool) -> Opt
     return best and best[1]
 
 
-def tiled_gemm_choice(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False, to_norm: bool = False):
+def tiled_gemm_choice(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False, to_norm: bool = False,
+                      bias: Optional[torch.Tensor] = None):
     """``tiled_gemm_sizes`` for this call, None where the start-up has measured its shape or the operands do not fit."""
     m, (n, k) = x.shape[0], weight.shape
-    if m > 1024 or (big_row_bucket(m), n, k, swiglu) in _BIG_CHOICE or not _mid_operands_ok(x, weight, swiglu):
+    if (m > 1024 or (big_row_bucket(m), n, k, swiglu) in _BIG_CHOICE or not _mid_operands_ok(x, weight, swiglu)
+            or not _rule_takes(x, weight, bias)):
         return None
     return tiled_gemm_sizes(m, n, k, swiglu, to_norm)
 

@@ -828,13 +828,20 @@ def test_skinny_norm_gemm_staged_rows(hip, dtype, M, K, N, swiglu, slices, with_
     assert float((out.double() - want).norm() / want.norm()) < (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
 
 
+@pytest.fixture
+def unmeasured(hip, monkeypatch):
+    """No start-up measurement of an engine before has a say."""
+    for name in ("_BIG_CHOICE", "_SKINNY_CHOICE", "_MID_CHOICE"):
+        monkeypatch.setattr(hip, name, {})
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,N,K,swiglu,to_norm,tile", [
     (257, 1024, 2048, False, True, (64, 64, 3)), (960, 1024, 3072, False, True, (64, 64, 1)),
     (960, 6144, 1024, True, False, (256, 96, 1)), (512, 4096, 1024, False, False, (64, 128, 1)), (500, 1024, 3072, False, True, (64, 64, 2)),
     (1024, 4096, 512, False, False, (128, 128, 1)), (300, 576, 576, False, False, (64, 64, 1)),
     (769, 704, 1536, True, False, None), (321, 4160, 1024, True, False, None)])
-def test_tiled_gemm_of_rows_in_several_tiles(hip, dtype, M, N, K, swiglu, to_norm, tile):
+def test_tiled_gemm_of_rows_in_several_tiles(hip, unmeasured, dtype, M, N, K, swiglu, to_norm, tile):
     """257 to 1024 rows on the mid-batch kernel: last row tiles that are not full, strided rows, every kind of result."""
     from minivllm_amd import ops
     torch.manual_seed(5)
@@ -854,11 +861,34 @@ def test_tiled_gemm_of_rows_in_several_tiles(hip, dtype, M, N, K, swiglu, to_nor
 
 @pytest.mark.parametrize("m,n,k,swiglu", [(256, 1024, 1024, False), (1025, 1024, 1024, False), (960, 6144, 1024, False),
                                           (1024, 8192, 1024, True), (300, 2048, 6144, False), (300, 448, 1024, False), (300, 1024, 448, False)])
-def test_tiled_gemm_leaves_other_sizes_to_the_library(hip, m, n, k, swiglu):
+def test_tiled_gemm_leaves_other_sizes_to_the_library(hip, unmeasured, m, n, k, swiglu):
     assert hip.tiled_gemm_sizes(m, n, k, swiglu, True) is None
     x, w = torch.zeros(960, 1024, device=DEV, dtype=torch.bfloat16), torch.zeros(1024, 1024, device=DEV, dtype=torch.bfloat16)
     assert hip.tiled_gemm_choice(x, w) and not hip.tiled_gemm_choice(x.float(), w.float())
     assert not hip.tiled_gemm_choice(x, w[:, ::2]) and not hip.tiled_gemm_choice(x[:, 1:], w[:, 1:])
+
+
+def test_rules_leave_odd_operands_and_gradients_to_the_library(hip, unmeasured):
+    """Calls that only a rule sends to a kernel: a bias or a weight that does not lie on 16 bytes, a bias of another stride,
+    anything to differentiate."""
+    from minivllm_amd import ops
+    x, w = torch.randn(300, 1024, device=DEV, dtype=torch.bfloat16), torch.randn(1024, 1024, device=DEV, dtype=torch.bfloat16)
+    b = torch.randn(2049, device=DEV, dtype=torch.bfloat16)
+    odd = torch.randn(1024 * 1024 + 8, device=DEV, dtype=torch.bfloat16)[1:1024 * 1024 + 1].view(1024, 1024)
+    for rows in (300, 4):
+        def choice(xx, ww, bb):
+            return hip.tiled_gemm_choice(xx, ww, bias=bb) if rows == 300 else hip.skinny_gemm_splits(xx, ww, bb)
+        y = x[:rows]
+        assert choice(y, w, None) and choice(y, w, b[:1024])
+        assert not choice(y, w, b[1:1025]) and not choice(y, w, b[:2048:2]) and not choice(y, odd, None)
+        wg = w.clone().requires_grad_()
+        with torch.enable_grad():
+            assert not choice(y, wg, None)
+            ops.linear(y, wg, b[1:1025], to_norm=True).float().sum().backward()
+        assert wg.grad is not None
+        want = y.double() @ odd.double().T + b[1:1025].double()
+        got = ops.linear(y, odd, b[1:1025], to_norm=True)
+        assert float((got.double() - want).norm() / want.norm()) < 2.0 ** -8
 
 
 @pytest.mark.parametrize("n,k,want", [(1024, 2048, 2), (1024, 3072, 3), (1024, 4096, 4), (2048, 4096, 2),
