@@ -97,6 +97,15 @@ def test_every_instance_and_option(H, G, D, E, bs, opt, dt):
     compare(H, G, D, E, bs, opt, dt)
 
 
+@pytest.mark.parametrize("bs", [1, 4, 8, 12, 24, 32, 40, 96])
+@pytest.mark.parametrize("opt", [dict(), dict(window=40, keep_first=37), dict(window=70)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_pages_of_every_kind(bs, opt, dt):
+    """Pages of whole tiles of 32 (one descriptor a tile), of whole runs of eight (one a piece) and of neither (every row
+    looked up), powers of two or not, kept first keys that end inside a tile."""
+    compare(4, 2, 128, 64, bs, opt, dt)
+
+
 @pytest.mark.parametrize("H,G,D,E,shift", [(4, 2, 128, 100, 0), (8, 4, 64, 20, 0), (3, 1, 144, 36, 0),    # whole key rows
                                            (4, 2, 36, 64, 0), (2, 1, 64, 64, 1), (2, 2, 128, 128, 3)])    # neither
 @pytest.mark.parametrize("opt", OPTIONS)
