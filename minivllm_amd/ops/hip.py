@@ -513,11 +513,16 @@ def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
 # ------------------------------------------------------- weight-streaming GEMM
 def _rule_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
     """What a call has to be for a rule (not a measurement of the engine's own weights) to send it from the library to a
-    kernel: nothing to differentiate, weight and bias where runs of 16 bytes can be read."""
+    kernel: nothing to differentiate, weight and bias where runs of 16 bytes can be read, a bias value for every column."""
     if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
         return False
-    return weight.data_ptr() % 16 == 0 and (bias is None or (bias.dtype == x.dtype and bias.is_contiguous()
-                                                             and bias.data_ptr() % 16 == 0))
+    return weight.data_ptr() % 16 == 0 and (bias is None or (_bias_fits(bias, weight) and bias.data_ptr() % 16 == 0))
+
+
+def _bias_fits(bias: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Kernels read one bias value per column, next to each other and in the weight's type (the library also takes other
+    strides, and shapes that broadcast to the result's)."""
+    return bias.dtype == weight.dtype and bias.dim() == 1 and bias.shape[0] == weight.shape[0] and bias.is_contiguous()
 
 
 SKINNY_MAX_ROWS = 16
