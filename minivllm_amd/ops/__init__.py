@@ -199,11 +199,11 @@ def swiglu_linear(x, weight, bias=None):
     return silu_and_mul(F.linear(x, weight, bias))
 
 
-def fuses_norm_linear(x, weight, swiglu=False) -> bool:
+def fuses_norm_linear(x, weight, swiglu=False, bias=None) -> bool:
     """True when ``norm_linear`` runs as one kernel for these operands (decode batches of one
     or two rows on the GPU, of up to 16 short ones), provided the weight carries the norm's scale vector."""
     return (_on_gpu(x) and x.dim() == 2 and x.shape[0] <= 16
-            and _hip().skinny_norm_gemm_pays(x, weight, swiglu))
+            and _hip().skinny_norm_gemm_pays(x, weight, swiglu, bias))
 
 
 def norm_linear(x, residual, gamma, eps, weight, bias=None, swiglu=False, gamma_folded=False):
@@ -225,11 +225,11 @@ def norm_linear(x, residual, gamma, eps, weight, bias=None, swiglu=False, gamma_
         raise TypeError("a row-sharded residual stream can only be consumed together with a "
                         "pending row-parallel reduce")
     if _is_partials(x):                                # K-split GEMM slices: summed by the norm
-        if gamma_folded and _hip().skinny_norm_partials_pays(x, residual, weight, swiglu):
+        if gamma_folded and _hip().skinny_norm_partials_pays(x, residual, weight, swiglu, bias):
             return _hip().skinny_norm_linear(x, residual, eps, weight, bias, swiglu)
         h, residual = x.add_rms_norm(residual, gamma, eps)
         return (swiglu_linear(h, weight, bias) if swiglu else linear(h, weight, bias)), residual
-    if gamma_folded and fuses_norm_linear(x, weight, swiglu):
+    if gamma_folded and fuses_norm_linear(x, weight, swiglu, bias):
         return _hip().skinny_norm_linear(x, residual, eps, weight, bias, swiglu)
     if residual is None:
         residual, h = x, rms_norm(x, gamma, eps)

@@ -513,16 +513,19 @@ def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
 # ------------------------------------------------------- weight-streaming GEMM
 def _rule_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
     """What a call has to be for a rule (not a measurement of the engine's own weights) to send it from the library to a
-    kernel: nothing to differentiate, weight and bias where runs of 16 bytes can be read, a bias value for every column."""
+    kernel: ``_only_values``, with weight and bias where runs of 16 bytes can be read."""
+    return (_only_values(x, weight, bias) and weight.data_ptr() % 16 == 0
+            and (bias is None or bias.data_ptr() % 16 == 0))
+
+
+def _only_values(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
+    """Whether a kernel does all that the library would for this projection: nothing is to be differentiated, and the bias
+    is one value per column, next to each other and in the weight's type (the library also takes other strides, and
+    shapes that broadcast to the result's)."""
     if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
         return False
-    return weight.data_ptr() % 16 == 0 and (bias is None or (_bias_fits(bias, weight) and bias.data_ptr() % 16 == 0))
-
-
-def _bias_fits(bias: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Kernels read one bias value per column, next to each other and in the weight's type (the library also takes other
-    strides, and shapes that broadcast to the result's)."""
-    return bias.dtype == weight.dtype and bias.dim() == 1 and bias.shape[0] == weight.shape[0] and bias.is_contiguous()
+    return bias is None or (bias.dtype == weight.dtype and bias.dim() == 1 and bias.shape[0] == weight.shape[0]
+                            and bias.is_contiguous())
 
 
 SKINNY_MAX_ROWS = 16
@@ -720,14 +723,16 @@ SKINNY_NORM_MAX_ROWS = 2          # beyond this the two-kernel path is faster fo
 _STAGED_ROWS_BYTES = 112 << 10    # rows the kernel can hold in LDS (csrc/skinny_norm_gemm.hip)
 
 
-def skinny_norm_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False) -> bool:
+def skinny_norm_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False,
+                          bias: Optional[torch.Tensor] = None) -> bool:
     """Shapes for which (residual add + RMSNorm + projection) runs as ONE weight-streaming
     kernel: 1-2 rows and a projection the plain weight-streaming kernel takes (also QKV-sized
     outputs, where dropping the norm launch outweighs the library's small GEMM advantage), or up to 16 rows
     of up to 1024 values, where every workgroup can afford to form the rows itself (us, two kernels / one, 4, 8
     and 16 rows: 4096 x 1024 7.6 / 4.8, 8.7 / 5.3, 10.6 / 6.4, SwiGLU of 2 x 3072 x 1024 7.6 / 6.0, 8.0 / 6.6,
-    8.4 / 7.7; but 6144 x 4096 16.3 / 17.3, 18.1 / 21.2, 22.3 / 29.4)."""
-    if x.dim() != 2 or not skinny_gemm_ok(x, weight, swiglu):
+    8.4 / 7.7; but 6144 x 4096 16.3 / 17.3, 18.1 / 21.2, 22.3 / 29.4).  A bias that the kernel cannot read and a
+    gradient that it would not form are the two-kernel path's."""
+    if x.dim() != 2 or not skinny_gemm_ok(x, weight, swiglu) or not _only_values(x, weight, bias):
         return False
     n, k = weight.shape
     if x.shape[0] > SKINNY_NORM_MAX_ROWS and (k > 1024 or k % 256 or n > 8192 or x.stride(0) % 8
@@ -737,7 +742,7 @@ def skinny_norm_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = 
 
 
 def skinny_norm_partials_pays(part: SplitKPartials, residual: Optional[torch.Tensor], weight: torch.Tensor,
-                              swiglu: bool = False) -> bool:
+                              swiglu: bool = False, bias: Optional[torch.Tensor] = None) -> bool:
     """The same for the K slices of the projection before, which every workgroup then reads and
     sums (norm kernel that sums + projection / one kernel, us, two slices, 4, 8 and 16 rows: 4096 x 1024 7.4 / 5.2,
     8.4 / 6.2, 10.4 / 8.2; 4096 x 2048 9.5 / 8.2, 10.3 / 10.1, 12.4 / 14.2; SwiGLU of 2 x 3072 x 1024 7.6 / 6.8,
@@ -747,7 +752,7 @@ def skinny_norm_partials_pays(part: SplitKPartials, residual: Optional[torch.Ten
     if (slices > 4 or m > SKINNY_MAX_ROWS or n > 8192 or k % 256 or n % (32 if swiglu else 16)
             or weight.dtype != part.dtype or weight.shape[1] != k or not weight.is_contiguous()
             or part.dtype not in _DT or m * (k + 8) * 2 > _STAGED_ROWS_BYTES or weight.data_ptr() % 16
-            or (part.bias is not None and part.bias.data_ptr() % 16)):
+            or (part.bias is not None and part.bias.data_ptr() % 16) or not _only_values(part.ws, weight, bias)):
         return False
     if residual is not None and (residual.shape != (m, k) or residual.dtype != part.dtype or residual.stride(1) != 1
                                  or residual.stride(0) % 8 or residual.data_ptr() % 16):

@@ -62,3 +62,44 @@ def test_biases(call, rows, n):
     for refused in (torch.randn(n), b[:n - 1]):
         with pytest.raises(RuntimeError):
             call(x, w, refused)
+
+
+def _norm_linear(x, w, b, slices=0, swiglu=False):
+    """Residual add + norm + projection, from a tensor or from the slices of the projection before it."""
+    ones, rows = torch.ones(1024, dtype=BF), torch.zeros_like(x)
+    if slices:
+        x = hip.SplitKPartials(x.detach()[None].float(), None, BF)
+    return ops.norm_linear(x, rows, ones, 1e-6, w, b, swiglu, gamma_folded=True)[0]
+
+
+# entry point, rows: each a call that runs as one kernel
+NORMED = {"1 row": (_norm_linear, 1), "4 rows": (_norm_linear, 4), "16 rows": (_norm_linear, 16),
+          "slices": (lambda x, w, b: _norm_linear(x, w, b, slices=1), 4),
+          "SwiGLU": (lambda x, w, b: _norm_linear(x, w, b, swiglu=True), 4),
+          "slices, SwiGLU": (lambda x, w, b: _norm_linear(x, w, b, 1, True), 3)}
+
+
+@pytest.mark.parametrize("call,rows", NORMED.values(), ids=NORMED)
+def test_biases_behind_a_norm(monkeypatch, call, rows):
+    """As ``test_biases``; what is not for the one kernel is what the norm and the library's projection give."""
+    monkeypatch.setattr(hip.SplitKPartials, "add_rms_norm",
+                        lambda p, r, g, eps: torch_ref.add_rms_norm(p.ws.sum(0).to(p.dtype), r, g, eps))
+    n = 2048
+    x, w = _operands(rows, n)
+    b = torch.randn(2 * n + 1).to(BF)
+    normed = lambda x, w, b: call(x.clone(), w, b)
+    library = lambda x, w, b: F.linear(torch_ref.rms_norm(x, torch.ones(1024, dtype=BF), 1e-6), w, b)
+    for plain in (None, b[:n], b[1:n + 1]):
+        with pytest.raises(Launched):
+            normed(x, w, plain)
+    for other in (b[:1], b[:n].view(1, n), torch.randn(rows, n).to(BF), b[:1].expand(n), b[:2 * n:2]):
+        got, want = normed(x, w, other), library(x, w, other)
+        torch.testing.assert_close(got, want if got.shape == want.shape else torch_ref.silu_and_mul(want))
+    for refused in (torch.randn(n), b[:n - 1]):
+        with pytest.raises(RuntimeError):
+            normed(x, w, refused)
+    wg = w.clone().requires_grad_()
+    normed(x, wg, b[:n]).float().sum().backward()
+    assert wg.grad is not None
+    with torch.no_grad(), pytest.raises(Launched):
+        normed(x, wg, b[:n])
