@@ -230,10 +230,14 @@ __global__ void __launch_bounds__(512, 2) latent_form_kernel(FormArgs a) {
 
 extern "C" {
 
-// 1 when keys of D and values of E numbers can be formed from latents of R and attended to with P shared ones
+int hyb_latent_attention_ok(int R, int P);           // hybrid_latent.hip
+
+// 1 when keys of D and values of E numbers can be formed from latents of R and attended to with P shared ones.
+// R: the ranks of hybrid_latent.hip (up to 512), whose weights are in two parts as they are here; latents of higher
+// ranks are attended to by kernels with weights of 24 bits and more, which forming would take bits from.
 int hyb_latent_formed_ok(int D, int E, int R, int P, int block_size, int max_blocks) {
     if (D < 8 || D > 128 || E < 8 || E > 128 || P < 8 || P > 128 || (D | E | P) % 8) return 0;
-    if (R < 64 || R % 64 || R > 4096 || block_size % 32) return 0;
+    if (R < 64 || R % 64 || !hyb_latent_attention_ok(R, P) || block_size % 32) return 0;
     return latent_prompts_pages_ok(block_size, max_blocks, R + P);
 }
 

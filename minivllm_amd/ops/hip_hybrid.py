@@ -751,7 +751,7 @@ def latent_formed_rows(seqs: int, max_k: int) -> int:
 
 def latent_formed_ok(q, dkv, up_k, up_v, k_cache, block_tables, seqs, max_q, max_k) -> bool:
     """Whether prompt portions run with their keys and values formed: bfloat16, sizes the kernels
-    have, pages of whole tiles of 32, and formed rows that take no more memory than the absorbed
+    have (ranks of up to 512: ``latent_attention_ok``, whose weights are held in as many bits), pages of whole tiles of 32, and formed rows that take no more memory than the absorbed
     queries and the sums of latents of the other form do.  With that a context is at most 2 R / (D + E)
     times (R 512, D = E = 128: four times) the step's new tokens, sequence by sequence as long as the longest.
     On that line the forming pays too: us, absorbed / formed, 16 heads, R 512, 512 tokens behind 1536 146 / 100, 64 behind 192

@@ -114,3 +114,16 @@ def test_when_keys_and_values_are_formed(change, taken):
     got = hk.latent_formed_ok(q, z(c["T"], c["R"] + c["P"]), up_k, z(H, c["R"], c["E"]), z(8, c["bs"], 1, c["R"] + c["P"]),
                               torch.zeros(2, 4, dtype=torch.int32, device="cuda"), c["seqs"], c["max_q"], c["max_k"])
     assert got == taken
+
+
+@pytest.mark.parametrize("R", [64, 448, 512, 576, 640, 960, 1024, 4096])
+@pytest.mark.parametrize("P", [8, 64, 128])
+def test_ranks_whose_weights_have_as_many_bits(R, P):
+    """Formed only where the other form holds its weights in two bfloat16 parts too."""
+    from minivllm_amd.ops import hip_hybrid as hk
+    T, H, D = 64, 2, 128
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)
+    cache = z(2, 32, 1, R + P)
+    taken = hk.latent_formed_ok(z(T, H, D + P), z(T, R + P), z(H, D, R), z(H, R, D), cache,
+                                torch.zeros(1, 2, dtype=torch.int32), 1, 32, 32)
+    assert taken == hk.latent_attention_ok(z(H, T, R), cache, P) == (R <= 512)
