@@ -14,6 +14,7 @@ import os
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from .partials import ResidualSum, SplitKPartials      # the types live where CPU-only code can import them
 
@@ -519,13 +520,24 @@ def _rule_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
 
 
 def _only_values(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
-    """Whether a kernel does all that the library would for this projection: nothing is to be differentiated, and the bias
-    is one value per column, next to each other and in the weight's type (the library also takes other strides, and
-    shapes that broadcast to the result's)."""
-    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
+    """Whether a kernel does all that the library would for this projection: the tensors are plain ones, nothing is
+    differentiated (in either mode), traced, transformed (``vmap``) or cast on the way, and the bias is one value per
+    column, next to each other and in the weight's type (the library also takes other strides, and shapes that
+    broadcast to the result's).  0.8 us of the host, for calls that a rule decides."""
+    if (_compiling() or type(x) not in _PLAIN or type(weight) not in _PLAIN or _dispatch_modes() or _transforming()
+            or _tracing() or _autocast() or forward_ad._current_level >= 0):
         return False
-    return bias is None or (bias.dtype == weight.dtype and bias.dim() == 1 and bias.shape[0] == weight.shape[0]
-                            and bias.is_contiguous())
+    if _grad_enabled() and (x.requires_grad or weight.requires_grad
+                            or (bias is not None and bias.requires_grad)):
+        return False
+    return bias is None or (type(bias) in _PLAIN and bias.dtype == weight.dtype and bias.dim() == 1
+                            and bias.shape[0] == weight.shape[0] and bias.is_contiguous())
+
+
+_PLAIN = frozenset((torch.Tensor, torch.nn.Parameter))
+_compiling, _grad_enabled, _autocast = torch.compiler.is_compiling, torch.is_grad_enabled, torch.is_autocast_enabled
+_dispatch_modes, _tracing = torch._C._len_torch_dispatch_stack, torch._C._is_tracing
+_transforming = torch._C._are_functorch_transforms_active
 
 
 SKINNY_MAX_ROWS = 16
@@ -586,7 +598,7 @@ def skinny_gemm_splits(x: torch.Tensor, weight: torch.Tensor, bias: Optional[tor
         return None
     n, k = weight.shape
     choice = _SKINNY_CHOICE.get((_row_bucket(x.shape[0]), n, k, "norm"))
-    if choice is None and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and _rule_takes(x, weight, bias):
+    if choice is None and x.stride(0) % 8 == 0 and _rule_takes(x, weight, bias) and x.data_ptr() % 16 == 0:
         return skinny_narrow_splits(n, k)
     return choice
 
@@ -732,7 +744,7 @@ def skinny_norm_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = 
     and 16 rows: 4096 x 1024 7.6 / 4.8, 8.7 / 5.3, 10.6 / 6.4, SwiGLU of 2 x 3072 x 1024 7.6 / 6.0, 8.0 / 6.6,
     8.4 / 7.7; but 6144 x 4096 16.3 / 17.3, 18.1 / 21.2, 22.3 / 29.4).  A bias that the kernel cannot read and a
     gradient that it would not form are the two-kernel path's."""
-    if x.dim() != 2 or not skinny_gemm_ok(x, weight, swiglu) or not _only_values(x, weight, bias):
+    if x.dim() != 2 or not _only_values(x, weight, bias) or not skinny_gemm_ok(x, weight, swiglu):
         return False
     n, k = weight.shape
     if x.shape[0] > SKINNY_NORM_MAX_ROWS and (k > 1024 or k % 256 or n > 8192 or x.stride(0) % 8
@@ -747,12 +759,14 @@ def skinny_norm_partials_pays(part: SplitKPartials, residual: Optional[torch.Ten
     sums (norm kernel that sums + projection / one kernel, us, two slices, 4, 8 and 16 rows: 4096 x 1024 7.4 / 5.2,
     8.4 / 6.2, 10.4 / 8.2; 4096 x 2048 9.5 / 8.2, 10.3 / 10.1, 12.4 / 14.2; SwiGLU of 2 x 3072 x 1024 7.6 / 6.8,
     7.8 / 8.1, 8.2 / 10.6; of 2 x 6144 x 2048 16.8 / 21.7 at 4 rows)."""
+    if not _only_values(part.ws, weight, bias):
+        return False
     slices, m, k = part.ws.shape
     n = weight.shape[0]
     if (slices > 4 or m > SKINNY_MAX_ROWS or n > 8192 or k % 256 or n % (32 if swiglu else 16)
             or weight.dtype != part.dtype or weight.shape[1] != k or not weight.is_contiguous()
             or part.dtype not in _DT or m * (k + 8) * 2 > _STAGED_ROWS_BYTES or weight.data_ptr() % 16
-            or (part.bias is not None and part.bias.data_ptr() % 16) or not _only_values(part.ws, weight, bias)):
+            or (part.bias is not None and part.bias.data_ptr() % 16)):
         return False
     if residual is not None and (residual.shape != (m, k) or residual.dtype != part.dtype or residual.stride(1) != 1
                                  or residual.stride(0) % 8 or residual.data_ptr() % 16):
@@ -926,8 +940,8 @@ def tiled_gemm_choice(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = Fals
                       bias: Optional[torch.Tensor] = None):
     """``tiled_gemm_sizes`` for this call, None where the start-up has measured its shape or the operands do not fit."""
     m, (n, k) = x.shape[0], weight.shape
-    if (m > 1024 or (big_row_bucket(m), n, k, swiglu) in _BIG_CHOICE or not _mid_operands_ok(x, weight, swiglu)
-            or not _rule_takes(x, weight, bias)):
+    if (m > 1024 or (big_row_bucket(m), n, k, swiglu) in _BIG_CHOICE or not _rule_takes(x, weight, bias)
+            or not _mid_operands_ok(x, weight, swiglu)):
         return None
     return tiled_gemm_sizes(m, n, k, swiglu, to_norm)
 

@@ -103,3 +103,86 @@ def test_biases_behind_a_norm(monkeypatch, call, rows):
     assert wg.grad is not None
     with torch.no_grad(), pytest.raises(Launched):
         normed(x, wg, b[:n])
+
+
+def _transforms(call):
+    """name -> (function of x, w, b, what a call under that transform gives)."""
+    fw = torch.autograd.forward_ad
+
+    def bias_gradient(x, w, b):
+        b = b.clone().requires_grad_()
+        call(x, w, b).float().sum().backward()
+        return b.grad
+
+    def tangent(of):
+        def f(*args):
+            with fw.dual_level():
+                args = list(args)
+                args[of] = fw.make_dual(args[of], torch.ones_like(args[of]))
+                return fw.unpack_dual(call(*args)).tangent
+        return f
+
+    def other_types(x, w, b):
+        from torch._subclasses import FakeTensorMode
+        with FakeTensorMode() as mode:
+            fake = [mode.from_tensor(t) for t in (x, w, b)]
+        return torch.empty(call(*fake).shape)                # (out of the mode: the tensors carry it)
+
+    def counted(x, w, b):
+        from torch.utils.flop_counter import FlopCounterMode
+        with FlopCounterMode(display=False) as c:
+            call(x, w, b)
+        return torch.tensor(c.get_total_flops())
+
+    def autocast(x, w, b):
+        torch.set_autocast_enabled("cuda", True)
+        try:
+            return call(x, w, b)
+        finally:
+            torch.set_autocast_enabled("cuda", False)
+
+    return {"gradient of the bias": bias_gradient, "tangent of x": tangent(0), "tangent of the weight": tangent(1),
+            "tangent of the bias": tangent(2), "vmap over weights": lambda x, w, b: torch.func.vmap(
+                lambda ww: call(x, ww, b))(torch.stack([w, -w])),
+            "jvp": lambda x, w, b: torch.func.jvp(lambda t: call(x, w, t), (b,), (torch.ones_like(b),))[1],
+            "jit trace": lambda x, w, b: torch.jit.trace(call, (x, w, b), check_trace=False)(2 * x, w, b),
+            "fx trace": lambda x, w, b: torch.fx.experimental.proxy_tensor.make_fx(call)(x, w, b)(2 * x, w, b),
+            "compiled": lambda *a: torch.compile(call, backend="eager", fullgraph=True)(*a),
+            "fake tensors": other_types, "counted": counted, "autocast": autocast}
+
+
+@pytest.mark.filterwarnings("ignore")                        # (of the tracers)
+@pytest.mark.parametrize("call,rows,n", [CALLS["narrow to norm"], CALLS["several row tiles"]])
+@pytest.mark.parametrize("name", list(_transforms(None)))
+def test_transforms(call, rows, n, name):
+    """Calls of which more than the values is wanted: as the library's projection gives it."""
+    import torch.fx.experimental.proxy_tensor                # noqa: F401
+    x, w = _operands(rows, n)
+    b = torch.randn(n).to(BF)
+    got, want = (_transforms(c)[name](x, w, b) for c in (call, F.linear))
+    assert got is not None
+    torch.testing.assert_close(got, want) if name != "fake tensors" else None
+    assert got.shape == want.shape
+    with pytest.raises(Launched):                            # (and nothing is left switched off)
+        call(x, w, b)
+
+
+@pytest.mark.parametrize("rows", [2, 4])
+@pytest.mark.parametrize("slices", [0, 1])
+def test_transforms_behind_a_norm(monkeypatch, rows, slices):
+    monkeypatch.setattr(hip.SplitKPartials, "add_rms_norm",
+                        lambda p, r, g, eps: torch_ref.add_rms_norm(p.ws.sum(0).to(p.dtype), r, g, eps))
+    x, w = _operands(rows, 2048)
+    b = torch.randn(2048).to(BF)
+    call = lambda ww, bb: _norm_linear(x.clone(), ww, bb, slices)
+    bg = b.clone().requires_grad_()
+    call(w, bg).float().sum().backward()
+    assert torch.equal(bg.grad, torch.full_like(b, rows))
+    for wrt in (0, 1):
+        with torch.autograd.forward_ad.dual_level():
+            args = [w, b]
+            args[wrt] = torch.autograd.forward_ad.make_dual(args[wrt], torch.ones_like(args[wrt]))
+            assert torch.autograd.forward_ad.unpack_dual(call(*args)).tangent is not None
+    assert torch.func.vmap(lambda ww: call(ww, b))(torch.stack([w, -w])).shape == (2, rows, 2048)
+    with pytest.raises(Launched):
+        call(w, b)
