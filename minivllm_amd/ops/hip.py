@@ -402,7 +402,8 @@ def decode_num_splits(batch: int, num_kv_heads: int, max_context_len: Optional[i
     per CU, where their number comes as close to that as workgroups of 4, two per CU, do (the
     launcher takes 8 waves for grids of at most 256 workgroups), otherwise of 4; never more
     splits than the longest context uses (``splits_in_use`` of the kernel: shorter ones leave the
-    rest of theirs unused)."""
+    rest of theirs unused), with the waves that the grid it leaves will have.  (KV heads of more than 16 query heads have a
+    workgroup per 16 of them, which are not counted: their grids hold up to that many times the waves.)"""
     wgs = max(batch * num_kv_heads, 1)
     # one workgroup per CU or more: no split (batch 256 x 1 KV head at 1024 tokens: 24.5 us
     # unsplit, 27 us in two splits; what the second split adds is its merge, not bandwidth)
@@ -410,12 +411,16 @@ def decode_num_splits(batch: int, num_kv_heads: int, max_context_len: Optional[i
         return 1
     wide, narrow = min(32, 256 // wgs), min(32, 512 // wgs)
     n, waves = (wide, 8) if 2 * wide >= narrow else (narrow, 4)
-    if max_context_len is not None:
+    if max_context_len is None:
+        return n
+
+    def used(n, waves):
         tiles = (max_context_len + 31) // 32
         if tiles <= waves + waves // 4:
             return 1
-        n = min(n, max(min(8, -(-2 * tiles // waves)), -(-tiles // waves)))
-    return n
+        return min(n, max(min(8, -(-2 * tiles // waves)), -(-tiles // waves)))
+    n = used(n, waves)
+    return used(n, 8) if waves == 4 and n * wgs <= 256 else n
 
 
 # The decode kernel merges its context splits in the workgroup that finishes last; the tickets
