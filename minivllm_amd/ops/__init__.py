@@ -151,6 +151,8 @@ def linear(x, weight, bias=None, to_norm=False, residual=None):
     its own epilogue and return ``ResidualSum`` (the stream, updated in place, not yet
     normalised), which ``norm_linear`` / ``add_rms_norm`` / ``rms_norm`` accept in place of a
     tensor."""
+    if bias is not None and _on_gpu(x) and not _hip().bias_fits(bias, weight):
+        return F.linear(x, weight, bias)               # (broadcast, strided, or refused there)
     if _on_gpu(x) and x.dim() == 2 and x.shape[0] <= 256:
         h = _hip()
         if x.shape[0] <= 16:
@@ -180,6 +182,8 @@ def swiglu_linear(x, weight, bias=None):
     start-up measurements preferred a hand-written one (decode-sized inputs: weight-streaming
     kernels; prefill-sized: the 256 x 256-tile kernel with the SwiGLU epilogue), otherwise
     GEMM + activation kernel."""
+    if bias is not None and _on_gpu(x) and not _hip().bias_fits(bias, weight):
+        return silu_and_mul(F.linear(x, weight, bias))
     if _on_gpu(x) and x.dim() == 2 and x.shape[0] <= 256:
         h = _hip()
         if x.shape[0] <= 16:

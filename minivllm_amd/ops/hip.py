@@ -526,17 +526,21 @@ def _rule_takes(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
 
 def _only_values(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
     """Whether a kernel does all that the library would for this projection: the tensors are plain ones, nothing is
-    differentiated (in either mode), traced, transformed (``vmap``) or cast on the way, and the bias is one value per
-    column, next to each other and in the weight's type (the library also takes other strides, and shapes that
-    broadcast to the result's).  0.8 us of the host, for calls that a rule decides."""
+    differentiated (in either mode), traced, transformed (``vmap``) or cast on the way, and the bias is one that kernels
+    read (``bias_fits``).  0.8 us of the host, for calls that a rule decides."""
     if (_compiling() or type(x) not in _PLAIN or type(weight) not in _PLAIN or _dispatch_modes() or _transforming()
             or _tracing() or _autocast() or forward_ad._current_level >= 0):
         return False
     if _grad_enabled() and (x.requires_grad or weight.requires_grad
                             or (bias is not None and bias.requires_grad)):
         return False
-    return bias is None or (type(bias) in _PLAIN and bias.dtype == weight.dtype and bias.dim() == 1
-                            and bias.shape[0] == weight.shape[0] and bias.is_contiguous())
+    return bias is None or (type(bias) in _PLAIN and bias_fits(bias, weight))
+
+
+def bias_fits(bias: torch.Tensor, weight: torch.Tensor) -> bool:
+    """One value per column, next to each other and in the weight's type (the library also takes other strides, and
+    shapes that broadcast to the result's)."""
+    return bias.dtype == weight.dtype and bias.dim() == 1 and bias.shape[0] == weight.shape[0] and bias.is_contiguous()
 
 
 _PLAIN = frozenset((torch.Tensor, torch.nn.Parameter))

@@ -186,3 +186,24 @@ def test_transforms_behind_a_norm(monkeypatch, rows, slices):
     assert torch.func.vmap(lambda ww: call(ww, b))(torch.stack([w, -w])).shape == (2, rows, 2048)
     with pytest.raises(Launched):
         call(w, b)
+
+
+@pytest.mark.parametrize("rows", [1, 4, 16, 40, 300])
+@pytest.mark.parametrize("call,n,kind", [(ops.linear, 1024, False), (_linear, 1024, "norm"), (ops.swiglu_linear, 2048, True)],
+                         ids=["plain", "to norm", "SwiGLU"])
+def test_biases_of_measured_projections(monkeypatch, rows, call, n, kind):
+    """The same where the start-up timing chose a kernel for the shape."""
+    for b in (1, 8, 16):
+        monkeypatch.setitem(hip._SKINNY_CHOICE, (b, n, 1024, kind), True if kind != "norm" else 2)
+    monkeypatch.setitem(hip._MID_CHOICE, (64, n, 1024, kind), (64, 2, True))
+    monkeypatch.setitem(hip._BIG_CHOICE, (512, n, 1024, kind is True), True)
+    x, w = _operands(rows, n)
+    b = torch.randn(2 * n + 1).to(BF)
+    for plain in (None, b[:n]):
+        with pytest.raises(Launched):
+            call(x, w, plain)
+    for other in (b[:1], b[:n].view(1, n), torch.randn(rows, n).to(BF), b[:1].expand(n), b[:2 * n:2]):
+        _by_library(call, x, w, other)
+    for refused in (torch.randn(n), b[:n - 1]):
+        with pytest.raises(RuntimeError):
+            call(x, w, refused)
