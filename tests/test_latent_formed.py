@@ -127,3 +127,113 @@ def test_ranks_whose_weights_have_as_many_bits(R, P):
     taken = hk.latent_formed_ok(z(T, H, D + P), z(T, R + P), z(H, D, R), z(H, R, D), cache,
                                 torch.zeros(1, 2, dtype=torch.int32), 1, 32, 32)
     assert taken == hk.latent_attention_ok(z(H, T, R), cache, P) == (R <= 512)
+
+
+def _turned(x, pos, base=10000.0):
+    """Entries i and i + n / 2 of the last dimension turn together (64 bits)."""
+    n = x.shape[-1]
+    a = pos.double()[:, None, None] * (base ** (-torch.arange(0, n, 2, dtype=torch.float64) / n))
+    x1, x2 = x[..., :n // 2], x[..., n // 2:]
+    return torch.cat([x1 * a.cos() - x2 * a.sin(), x2 * a.cos() + x1 * a.sin()], -1)
+
+
+@gpu
+@pytest.mark.parametrize("R,bs,formed", [(512, 32, True), (192, 64, True), (576, 32, False), (512, 16, False)])
+@pytest.mark.parametrize("window,sink", [(0, False), (70, True)])
+def test_steps_through_the_layer(monkeypatch, R, bs, formed, window, sink):
+    """A layer's steps over one cache: prompts of several lengths, portions behind a prefix, next tokens, prompts with
+    riders, a prompt behind what those wrote; rows of no sequence in between.  The steps of prompts alone run with keys
+    and values formed where the rule has it, and are no further from 64 bits than with attention in the latents' coordinates."""
+    from minivllm_amd import ops
+    from minivllm_amd.layers.attention import LatentAttention
+    from minivllm_amd.layers.rotary_embedding import HalfRotation
+    from minivllm_amd.ops import hip_hybrid as hk
+    from minivllm_amd.utils.context import set_context
+    torch.manual_seed(R + bs)
+    H, D, P, E, eps, scale, nseq, room = 4, 64, 32, 72, 1e-6, (64 + 32) ** -0.5, 3, 256
+    up_k, up_v = torch.randn(H * D, R) * R ** -0.5, torch.randn(H * E, R) * R ** -0.5
+    norm, weight_sink = 1 + 0.1 * torch.randn(R), torch.randn(H)
+    tables = torch.randperm(nseq * room // bs).to(torch.int32).view(nseq, -1)
+    layers = {}
+    for form in ("rule", "absorbed"):
+        a = LatentAttention(H, D, P, E, R, scale, window, HalfRotation(P, 10000.0), eps, sink=sink).cuda()
+        a.latent_norm.copy_(norm)
+        a.load_expansions(up_k, up_v, torch.empty(0, dtype=torch.bfloat16, device="cuda"))
+        if sink:
+            a.core.sink.copy_(weight_sink)
+        a.core.k_cache = torch.full((tables.numel(), bs, 1, R + P), float("nan"), dtype=torch.bfloat16, device="cuda")
+        a.core.v_cache = a.core.k_cache[..., :R]
+        layers[form] = a
+    taken = []
+    for name in ("latent_formed_prompts", "latent_attention_prefill", "latent_attention_decode"):
+        def spy(*args, _f=getattr(hk, name), _name=name, **kw):
+            taken.append(_name)
+            return _f(*args, **kw)
+        monkeypatch.setattr(hk, name, spy)
+    rule = ops.latent_formed_ok
+    ku, vu = up_k.bfloat16().double().view(H, D, R), up_v.bfloat16().double().view(H, E, R)
+    rows = torch.zeros(nseq, room, R + P, dtype=torch.float64)              # what the cache should hold
+    past, squares = [0] * nseq, dict(rule=0.0, absorbed=0.0, of=0.0)
+
+    def step(seqs, new, riders=0, behind=0):
+        """Tokens of sequences (the first ``riders`` with one each), ``behind`` rows of none after them."""
+        T = sum(new) + behind
+        q, dkv = torch.randn(T, H, D + P).bfloat16(), torch.randn(T, R + P).bfloat16()
+        pos = torch.tensor([past[s] + i for s, n in zip(seqs, new) for i in range(n)] + [0] * behind, dtype=torch.int32)
+        owner = [b for b, n in enumerate(new) for _ in range(n)] + [-1] * behind
+        slots = [int(tables[seqs[b], int(p) // bs]) * bs + int(p) % bs if b >= 0 else -1 for b, p in zip(owner, pos)]
+        total = [past[s] + n for s, n in zip(seqs, new)]
+        ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+        kw = dict(positions=pos.cuda(), num_seqs=len(seqs), block_tables=tables[seqs].cuda(), slot_mapping=ints(slots))
+        prompts = new[riders:]
+        if prompts:
+            cu = lambda ns: ints([0] + torch.tensor(ns).cumsum(0).tolist())
+            kw.update(is_prefill=True, cu_seqlens_q=cu(new), cu_seqlens_k=cu(total), max_seqlen_q=max(new),
+                      max_seqlen_k=max(total), row_seq=ints(owner), num_decode_seqs=riders,
+                      num_prefill_tokens=sum(prompts))
+        if riders:
+            kw.update(context_lens=ints(total[:riders]), max_context_len=max(total[:riders]))
+        got, ways = {}, {}
+        for form, a in layers.items():
+            monkeypatch.setattr(ops, "latent_formed_ok", rule if form == "rule" else lambda *args: False)
+            set_context(**kw)
+            taken.clear()
+            with torch.inference_mode():
+                got[form] = a(q.cuda(), dkv.cuda()).double().cpu()
+            ways[form] = list(taken)
+        c = dkv[:, :R].double()
+        c = c * torch.rsqrt(c.pow(2).mean(-1, keepdim=True) + eps) * norm.double()
+        turned = torch.cat([c, _turned(dkv[:, None, R:].double(), pos)[:, 0]], -1)
+        at = 0
+        for s, n, m in zip(seqs, new, total):
+            rows[s, past[s]:m] = turned[at:at + n]
+            seen = rows[s, :m]
+            k, v = (torch.einsum("nr,hdr->hnd", seen[:, :R], u) for u in (ku, vu))
+            one = slice(at, at + n)
+            w = torch.einsum("thd,hnd->htn", q[one, :, :D].double(), k) \
+                + torch.einsum("thp,np->htn", _turned(q[one, :, D:].double(), pos[one]), seen[:, R:])
+            back = pos[one].long()[:, None] - torch.arange(m)[None]
+            w = (w * scale).masked_fill((back < 0) | ((back >= window) if window else False), -math.inf)
+            if sink:
+                w = torch.cat([w, weight_sink.double()[:, None, None].expand(H, n, 1)], -1)
+            want = torch.einsum("htn,hne->the", w.softmax(-1)[..., :m], v)
+            for form in got:
+                # rounded to bfloat16, 2^-9 of a value each: the cached rows, the turned queries, keys or absorbed queries,
+                # values or sums of latents, the result
+                assert float((got[form][one] - want).norm() / want.norm()) < 5 * 2.0 ** -9, (form, s, n, m)
+                squares[form] += float((got[form][one] - want).pow(2).sum()) * bool(prompts and not riders)
+            past[s] = m
+            at += n
+        if R > 512 and behind:
+            assert not got["rule"][at:].any()
+        return ways["rule"]
+
+    alone = ["latent_formed_prompts"] if formed else ["latent_attention_prefill"] if R <= 512 else []
+    nexts = ["latent_attention_decode"] if R <= 512 else []
+    assert step([0, 1, 2], [5, 65, 96], behind=6) == alone
+    assert step([1, 0], [64, 75], behind=1) == alone                       # behind 65 and 5 tokens
+    assert step([2, 1, 0], [1, 1, 1], riders=3) == nexts
+    assert sorted(step([2, 0], [1, 40], riders=1, behind=3)) == sorted(nexts + ["latent_attention_prefill"] * (R <= 512))
+    assert step([0], [80]) == alone
+    # the two forms round the same number of times: their errors differ by chance only (a tenth allowed)
+    assert squares["rule"] <= 1.21 * squares["absorbed"]
