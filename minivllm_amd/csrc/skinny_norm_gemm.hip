@@ -21,6 +21,7 @@ using namespace mvl;
 
 namespace {
 
+constexpr int kCus = 256;
 constexpr size_t kStagedLds = 112 * 1024;     // rows in LDS, besides at most 20 KB of partial sums
 constexpr int kUnroll = 4;       // 4 k-steps in flight keep the kernel under 96 VGPRs (>= 2 workgroups per CU)
 
@@ -160,18 +161,22 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_norm_gemm_kernel(
 // thread adds up some 16-byte chunks of x (or of the SLABS fp32 K-slices a split projection left,
 // plus that projection's bias) and of the residual, rounds them, and stores them to LDS, from
 // where the waves take their A fragments; the first weights are requested ahead of that and fly
-// meanwhile, those of the next block of k-steps during the products of the present one.
+// meanwhile, those of the next block of k-steps during the products of the present one.  There is a workgroup for
+// every CU at most (132 registers and more: no second one fits beside it), which takes its 16 columns and those 256
+// tiles on in turn: as many workgroups as tiles form the rows again for every round of 256.
 //
-// Bound by latency: at 4 rows, N = 4096, K = 1024 the weights (8 MB) take 1.6 us at the rate of a large
-// copy, a launch 2, the whole 4.7 (5.2 with two slices to sum, where a norm kernel that sums them and the plain
-// product take 7.4).  Rows of 4096 are too much for every workgroup to form: 24 us at 4 rows and N = 6144 against 17.
+// Bound by latency: at 8 rows, N = 4096, K = 1024 the weights (8 MB) take 1.6 us at the rate of a large
+// copy, a launch 2, the whole 5.4 (5.6 with two slices to sum, where a norm kernel that sums them and the plain
+// product take 8.4).  us with two slices, K = 1024, a workgroup per tile / per CU (norm kernel + product): 16 rows, N = 4096
+// 8.5 / 6.8 (10.1), 4112 13.7 / 8.1 (10.4), 8192 15.2 / 8.9 (10.9); 1 row, N = 8192 8.5 / 6.8 (8.3); 16 rows from a
+// tensor, N = 8192 11.3 / 8.6 (11.2).  Rows of 4096 are too much for every workgroup to form: 24 us at 4 rows and N = 6144 against 17.
 template <int CODE, int EPI, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void skinny_norm_staged_kernel(
         const uint16_t* __restrict__ x, long x_stride, const float* __restrict__ slabs, int n_slabs,
         const uint16_t* __restrict__ x_bias, const uint16_t* __restrict__ res_in, long ri_stride,
         uint16_t* __restrict__ res_out, long ro_stride, float eps,
         const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
-        uint16_t* __restrict__ out, long o_stride, int M, int K, int up_row_offset) {
+        uint16_t* __restrict__ out, long o_stride, int M, int K, int up_row_offset, int tiles) {
     using DT = DType<CODE>;
     using vec8 = typename DT::vec8;
     constexpr int NB = EPI == 1 ? 2 : 1;
@@ -183,12 +188,12 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_norm_staged_kernel(
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c16 = lane & 15, q4 = lane >> 4;
-    const int n0 = blockIdx.x * 16;
     const int kslice = K / WAVES;                // a multiple of 32
     const uint16_t* wp[NB];
-    wp[0] = w + (long)(n0 + c16) * K + (long)wv * kslice + 8 * q4;
-    if (NB == 2) wp[NB - 1] = w + (long)(up_row_offset + n0 + c16) * K + (long)wv * kslice + 8 * q4;
-
+    auto point = [&](int tile) {                 // this lane's weights of 16 columns
+        wp[0] = w + (long)(16 * tile + c16) * K + (long)wv * kslice + 8 * q4;
+        if (NB == 2) wp[NB - 1] = w + (long)(up_row_offset + 16 * tile + c16) * K + (long)wv * kslice + 8 * q4;
+    };
     auto request = [&](int k, u32x4_t (&bw)[NB][U]) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -198,6 +203,7 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_norm_staged_kernel(
                     bw[b][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(wp[b] + k + 32 * u));
     };
     u32x4_t bw[NB][U];
+    point(blockIdx.x);
     request(0, bw);
 
     const int per_row = K >> 3, pitch = K + 8;
@@ -240,29 +246,38 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_norm_staged_kernel(
     }
     __syncthreads();
 
-    f32x4_t acc[NB], gram = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     const uint16_t* rp = rows + min(c16, M - 1) * pitch + wv * kslice + 8 * q4;
-    for (int k = 0; k < kslice; k += 32 * U) {
-        u32x4_t next[NB][U];
-        request(k + 32 * U, next);
-        __builtin_amdgcn_sched_barrier(0);       // the next block's loads ahead of this one's waits
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {      // uniform
+        f32x4_t acc[NB], gram = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (k + 32 * u < kslice) {           // uniform
-                const vec8 a = __builtin_bit_cast(vec8, *reinterpret_cast<const u32x4_t*>(rp + k + 32 * u));
-                gram = DT::mfma16(a, a, gram);
+        for (int b = 0; b < NB; ++b) acc[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < kslice; k += 32 * U) {
+            u32x4_t next[NB][U];
+            request(k + 32 * U, next);
+            __builtin_amdgcn_sched_barrier(0);   // the next block's loads ahead of this one's waits
 #pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    acc[b] = DT::mfma16(a, __builtin_bit_cast(vec8, bw[b][u]), acc[b]);
-            }
+            for (int u = 0; u < U; ++u)
+                if (k + 32 * u < kslice) {       // uniform
+                    const vec8 a = __builtin_bit_cast(vec8, *reinterpret_cast<const u32x4_t*>(rp + k + 32 * u));
+                    gram = DT::mfma16(a, a, gram);
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
+                    for (int b = 0; b < NB; ++b)
+                        acc[b] = DT::mfma16(a, __builtin_bit_cast(vec8, bw[b][u]), acc[b]);
+                }
 #pragma unroll
-            for (int u = 0; u < U; ++u) bw[b][u] = next[b][u];
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int u = 0; u < U; ++u) bw[b][u] = next[b][u];
+        }
+        const bool more = tile + (int)gridDim.x < tiles;
+        if (more) {
+            point(tile + gridDim.x);
+            request(0, bw);
+        }
+        finish_rows<CODE, EPI, WAVES>(red, diag, acc, gram, lane, wv, M, K, eps, bias, out, o_stride, 16 * tile,
+                                      up_row_offset);
+        if (more) __syncthreads();               // the sums have been read before the next columns' are written
     }
-    finish_rows<CODE, EPI, WAVES>(red, diag, acc, gram, lane, wv, M, K, eps, bias, out, o_stride, n0, up_row_offset);
 }
 
 template <int CODE, int EPI, bool HAS_RES>
@@ -288,16 +303,16 @@ int launch_r(const void* x, long xs, const void* slabs, int n_slabs, const void*
              int K, int up_off, hipStream_t st) {
     const size_t lds = (size_t)M * (K + 8) * 2;
     // up to 4 rows the loads of x and residual beside the weights cost less than the pass through LDS
-    // and its barrier (us, per k-step / staged, K = 1024: 4.2 / 4.6 at 2 rows, 4.8 / 4.7 at 4, 6.1 / 5.3 at 8, 8.3 /
-    // 6.4 at 16; K = 2048 6.1 / 6.6, 6.4 / 7.1, 8.3 / 8.2, 11.3 / 10.4)
+    // and its barrier (us, per k-step / staged, N = 4096, K = 1024: 4.2 / 4.8 at 2 rows, 4.9 / 4.9 at 4, 6.1 / 5.4 at 8, 8.4 /
+    // 6.4 at 16; K = 2048 6.7 / 7.2, 7.3 / 7.7, 8.2 / 8.4, 11.4 / 10.7)
     if ((slabs != nullptr || M > 4) && K % 256 == 0 && lds <= kStagedLds) {
         auto kern = skinny_norm_staged_kernel<CODE, EPI, 8>;
         static const hipError_t once = hipFuncSetAttribute(
             (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kStagedLds);
         if (once != hipSuccess) return -1;
-        kern<<<tiles, 8 * 64, lds, st>>>(
+        kern<<<min(tiles, kCus), 8 * 64, lds, st>>>(
             (const uint16_t*)x, xs, (const float*)slabs, n_slabs, (const uint16_t*)xb, (const uint16_t*)ri, ris,
-            (uint16_t*)ro, ros, eps, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)out, os, M, K, up_off);
+            (uint16_t*)ro, ros, eps, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)out, os, M, K, up_off, tiles);
         return MVL_CHECK_LAUNCH();
     }
     if (slabs != nullptr) return -1;

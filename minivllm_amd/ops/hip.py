@@ -749,9 +749,12 @@ def skinny_norm_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = 
     """Shapes for which (residual add + RMSNorm + projection) runs as ONE weight-streaming
     kernel: 1-2 rows and a projection the plain weight-streaming kernel takes (also QKV-sized
     outputs, where dropping the norm launch outweighs the library's small GEMM advantage), or up to 16 rows
-    of up to 1024 values, where every workgroup can afford to form the rows itself (us, two kernels / one, 4, 8
-    and 16 rows: 4096 x 1024 7.6 / 4.8, 8.7 / 5.3, 10.6 / 6.4, SwiGLU of 2 x 3072 x 1024 7.6 / 6.0, 8.0 / 6.6,
-    8.4 / 7.7; but 6144 x 4096 16.3 / 17.3, 18.1 / 21.2, 22.3 / 29.4).  A bias that the kernel cannot read and a
+    of up to 1024 values, where every workgroup can afford to form the rows itself (us, two kernels - the second one
+    the faster of the library and the plain weight-streaming kernel, whichever a start-up measurement would choose - / one, 4, 8
+    and 16 rows: 4096 x 1024 7.3 / 4.8, 8.3 / 5.4, 10.3 / 6.5, 8192 x 1024 8.9 / 6.6, 9.9 / 7.5, 11.2 / 8.6, SwiGLU of 2 x 3072 x
+    1024 7.5 / 6.0, 7.9 / 6.6, 8.4 / 7.7; above, it is lost at 16 rows, and earlier the longer they are: 4096 x 2048 9.2 / 6.4, 10.2 / 8.2,
+    11.3 / 10.4, 6144 x 2048 11.4 / 9.8, 11.6 / 11.1, 11.6 / 13.4, SwiGLU of 2 x 3072 x 2048 10.6 / 9.6, 11.0 / 11.3, 11.7 / 13.5,
+    6144 x 4096 16.3 / 17.3, 18.1 / 21.2, 22.3 / 29.4).  A bias that the kernel cannot read and a
     gradient that it would not form are the two-kernel path's."""
     if x.dim() != 2 or not _only_values(x, weight, bias) or not skinny_gemm_ok(x, weight, swiglu):
         return False
@@ -765,9 +768,9 @@ def skinny_norm_gemm_pays(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = 
 def skinny_norm_partials_pays(part: SplitKPartials, residual: Optional[torch.Tensor], weight: torch.Tensor,
                               swiglu: bool = False, bias: Optional[torch.Tensor] = None) -> bool:
     """The same for the K slices of the projection before, which every workgroup then reads and
-    sums (norm kernel that sums + projection / one kernel, us, two slices, 4, 8 and 16 rows: 4096 x 1024 7.4 / 5.2,
-    8.4 / 6.2, 10.4 / 8.2; 4096 x 2048 9.5 / 8.2, 10.3 / 10.1, 12.4 / 14.2; SwiGLU of 2 x 3072 x 1024 7.6 / 6.8,
-    7.8 / 8.1, 8.2 / 10.6; of 2 x 6144 x 2048 16.8 / 21.7 at 4 rows)."""
+    sums (norm kernel that sums + projection / one kernel, us, two slices, 4, 8 and 16 rows: 4096 x 1024 7.3 / 5.1,
+    8.4 / 5.6, 10.1 / 6.8; 8192 x 1024 8.9 / 7.1, 9.9 / 7.7, 10.9 / 8.9; 4 rows, 8192 x 2048 12.7 / 11.9; SwiGLU of 2 x 3072 x 1024
+    7.6 / 6.8, 7.8 / 8.1, 8.2 / 10.6; of 2 x 6144 x 2048 16.8 / 21.7 at 4 rows)."""
     if not _only_values(part.ws, weight, bias):
         return False
     slices, m, k = part.ws.shape

@@ -828,6 +828,23 @@ def test_skinny_norm_gemm_staged_rows(hip, dtype, M, K, N, swiglu, slices, with_
     assert float((out.double() - want).norm() / want.norm()) < (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,N,swiglu,slices", [(16, 256, 4112, False, 0), (5, 1024, 8192, False, 2), (7, 512, 8208, False, 1),
+                                                 (2, 256, 12304, False, 3), (9, 256, 8224, True, 0), (4, 1024, 16416, True, 4)])
+def test_staged_rows_of_more_tiles_than_workgroups(hip, dtype, M, K, N, swiglu, slices):
+    """More tiles of 16 columns than CUs: 257, 512, 513 and 769, the first ones with a second and a third turn."""
+    torch.manual_seed(N)
+    w, bias, res = ((torch.randn(*s, device=DEV) * f).to(dtype) for s, f in (((N, K), 0.03), ((N,), 1.0), ((M, K), 1.0)))
+    x = hip.SplitKPartials(torch.randn(slices, M, K, device=DEV), None, dtype) if slices else torch.randn(M, K, device=DEV, dtype=dtype)
+    out, r = hip.skinny_norm_linear(x, res, 1e-6, w, bias, swiglu)
+    rd = r.double()
+    y = (rd @ w.double().T) * torch.rsqrt(rd.pow(2).mean(-1, keepdim=True) + 1e-6) + bias.double()
+    want = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:] if swiglu else y
+    # one rounding of the result: 2^-9 (bfloat16) or 2^-12 (float16) of it, plus fp32 sums of K terms
+    assert float((out.double() - want).norm() / want.norm()) < (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12)
+    assert float((out.double() - want).norm(dim=0).max() / want.norm(dim=0).mean()) < 2.0 ** -3        # (no column of another tile: those are off by their size)
+
+
 @pytest.fixture
 def unmeasured(hip, monkeypatch):
     """No start-up measurement of an engine before has a say."""
