@@ -608,18 +608,20 @@ def skinny_gemm_splits(x: torch.Tensor, weight: torch.Tensor, bias: Optional[tor
     n, k = weight.shape
     choice = _SKINNY_CHOICE.get((_row_bucket(x.shape[0]), n, k, "norm"))
     if choice is None and x.stride(0) % 8 == 0 and _rule_takes(x, weight, bias) and x.data_ptr() % 16 == 0:
-        return skinny_narrow_splits(n, k)
+        return skinny_narrow_splits(n, k, x.shape[0])
     return choice
 
 
-def skinny_narrow_splits(n: int, k: int) -> Optional[int]:
+def skinny_narrow_splits(n: int, k: int, rows: int = 1) -> Optional[int]:
     """K split of a projection to norm that was never measured, None: no opinion.  Up to 2048
     output columns are at most 128 tiles of 16, so K goes over up to four workgroups, no more than fill the
     chip once, with 1024 of K or more for each.  us at 4 / 16 rows, library, unsplit, split so: 1024 x 2048
     8.0 / 8.0, 5.2 / 7.1, 4.2 / 5.9; 1024 x 3072 9.0 / 9.0, 6.8 / 8.4, 4.4 / 6.0; 2048 x 4096 14.5 / 14.3,
     7.8 / 9.6, 6.2 / 7.8; 2048 x 6144 10.9 / 11.1, 11.3 / 15.7, 7.6 / 9.2; 1536 x 8960 28.9 / 28.9, 16.0 / 21.8,
-    11.5 / 12.9.  Wider ones lose by it: 2560 x 9728 15.0 / 15.5, 17.4 / 22.9, 17.2 / 24.0."""
-    if n > 2048 or n * k * 2 < (1 << 20):
+    11.5 / 12.9.  Wider ones lose by it: 2560 x 9728 15.0 / 15.5, 17.4 / 22.9, 17.2 / 24.0.  So do more than 8 rows where
+    K is below 1024, too short for the eight waves that share it (library / so, both with the norm behind, at 8 and 16 rows: 1536 x 512
+    7.1 / 6.5, 7.1 / 7.7; 1024 x 1024 8.4 / 6.8, 8.5 / 8.0)."""
+    if n > 2048 or n * k * 2 < (1 << 20) or (k < 1024 and rows > 8):
         return None
     return next((s for s in (4, 3, 2) if skinny_splits_ok(k, s) and k // s >= 1024 and n // 16 * s <= _NUM_CUS), 1)
 

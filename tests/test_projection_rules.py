@@ -207,3 +207,15 @@ def test_biases_of_measured_projections(monkeypatch, rows, call, n, kind):
     for refused in (torch.randn(n), b[:n - 1]):
         with pytest.raises(RuntimeError):
             call(x, w, refused)
+
+
+@pytest.mark.parametrize("rows,k,kernel", [(8, 512, True), (9, 512, False), (16, 896, False), (16, 1024, True)])
+def test_short_rows_of_narrow_projections(rows, k, kernel):
+    """More than 8 rows of fewer than 1024 values: the library was measured to be faster."""
+    torch.manual_seed(k)
+    x, w = torch.randn(rows, k).to(BF), torch.randn(2048, k).to(BF)
+    if kernel:
+        with pytest.raises(Launched):
+            _linear(x, w, None)
+    else:
+        _by_library(_linear, x, w, None)
