@@ -931,12 +931,29 @@ def tiled_gemm_sizes(m: int, n: int, k: int, swiglu: bool, to_norm: bool) -> Opt
     kernel does in passing) and 16 MB of weights the chip is hardly filled once, and a tile that fills it beats the library's
     choice; beyond, larger tiles and streams win.  The choice: rounds of the grid over 256 CUs, times k-steps, times what one
     takes; K is split only towards a norm, which sums the slices, at what they cost to write and read.  us, library /
-    kernel: 960 rows, 1024 x 2048 10.7 / 10.3, 1024 x 3072 14.5 / 14.2, SwiGLU of 2 x 3072 x 1024 23.8 / 16.6, 4096 x 1024
-    12.7 / 12.7, 2048 x 2048 14.8 / 14.1; 512 rows, 4096 x 1024 10.1 / 8.9, 1024 x 3072 11.8 / 8.6 (slices for the norm);
-    past the lines 960 rows 6144 x 4096 51.5 / 57.8, 2048 x 6144 39.2 / 44.3, 1500 rows 2048 x 2048 18.0 / 19.8.  And a call of the
-    library costs the host 24 us where tables of its variants are loaded, one of the kernel 8."""
+    kernel: 960 rows, SwiGLU of 2 x 3072 x 1024 23.8 / 16.6, 4096 x 1024 13.8 / 13.3; 512 rows 10.9 / 9.3; with the norm
+    behind, 1024 x 3072 at 512 rows 18.7 / 14.1; past the lines 960 rows 6144 x 4096 51.5 / 57.8, 2048 x 6144 39.2 / 44.3,
+    1500 rows 2048 x 2048 18.0 / 19.8.
+
+    What the grid leaves idle costs more the longer K is, and the library splits K where its grid is small.  So K ends at
+    2048 for SwiGLU (384 rows, 2 x 256 x 3072 12.4 / 15.5, 2 x 256 x 2048 10.6 / 9.7); towards a norm at 1536 above 1024
+    columns (1024 rows, 1536 x 2048 19.3 / 20.4, 1536 x 1536 21.3 / 17.8; split up to four times, 1024 columns and fewer gain at every K:
+    512 rows, 512 x 16384 35.6 / 27.6); for a plain result at 1536 between 1024 and 3072 columns, at 1024
+    elsewhere (384 rows, 512 x 1536 7.0 / 8.0, 3072 x 2048 14.5 / 16.8, 640 rows 4096 x 1536 18.0 / 18.7).  More than 4096
+    columns that are no whole tiles of 128 lose as well (800 rows, 4928 x 704 16.0 / 18.0).  Inside these lines 789
+    measured sizes are at worst as fast as the library, in the middle 1.34 times."""
     if (not BIG_MIN_ROWS <= m <= 1024 or m * n > (6 << 20 if swiglu else 4 << 20) or n * k > 8 << 20
             or n < 512 or k < 512):
+        return None
+    if swiglu:
+        longest = 2048
+    elif n > 4096 and n % 128:
+        return None
+    elif to_norm:
+        longest = 1536 if n > 1024 else k
+    else:
+        longest = 1536 if 1024 <= n <= 3072 else 1024
+    if k > longest:
         return None
     best = None
     for (bm, bn), us in _TILE_US.items():

@@ -219,3 +219,14 @@ def test_short_rows_of_narrow_projections(rows, k, kernel):
             _linear(x, w, None)
     else:
         _by_library(_linear, x, w, None)
+
+
+@pytest.mark.parametrize("m,n,k,kind,kernel", [
+    (384, 512, 2048, "swiglu", True), (384, 512, 2112, "swiglu", False), (321, 4160, 1024, "swiglu", True),
+    (300, 1024, 8192, "norm", True), (1024, 1088, 1536, "norm", True), (1024, 1088, 1600, "norm", False),
+    (300, 1024, 1536, "plain", True), (300, 1024, 1600, "plain", False), (300, 960, 1024, "plain", True),
+    (300, 960, 1088, "plain", False), (300, 3072, 1536, "plain", True), (300, 3136, 1088, "plain", False),
+    (300, 4160, 512, "plain", False), (300, 4224, 512, "plain", True), (300, 4160, 512, "norm", False)])
+def test_lines_of_the_tiled_form(m, n, k, kind, kernel):
+    """257 to 1024 rows: where the grid's idle CUs cost more than the library's split of K."""
+    assert (hip.tiled_gemm_sizes(m, n, k, kind == "swiglu", kind == "norm") is not None) == kernel
