@@ -309,12 +309,14 @@ def sink_attention_prefill(q, k_cache, v_cache, cu_q, cu_k, block_tables, scale,
     assert block_tables.dtype == torch.int32 and block_tables.stride(1) == 1
     if gate is not None:
         assert gate.stride(1) == 1 and gate.dtype == q.dtype
-    if clear and (nseq <= 0 or max_q <= 0 or _tiles_form(
-            q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), nseq,
+    qs_t, qs_h, _ = q.stride()
+    # (sizes and strides that the clearing kernel never takes are told without the library's rule, a call of 2 us)
+    if clear and (nseq <= 0 or max_q <= 0 or (qs_t | qs_h | D | E | vs) % 8 or _tiles_form(
+            q.data_ptr(), qs_t, qs_h, k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), nseq,
             max_q, D, E, vs, _dt(q)) != 2):
-        out[first_seq:].zero_()
+        (out[first_seq:] if first_seq else out).zero_()
         clear = False
-    _check(_tiles(q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(),
+    _check(_tiles(q.data_ptr(), qs_t, qs_h, k_cache.data_ptr(), v_cache.data_ptr(),
                   block_tables.data_ptr(), block_tables.stride(0), k_cache.shape[1],
                   _i32c(cu_q).data_ptr(), _i32(positions).data_ptr(),
                   _f32(sink).data_ptr() if sink is not None else None,
