@@ -760,13 +760,14 @@ def latent_formed_ok(q, dkv, up_k, up_v, k_cache, block_tables, seqs, max_q, max
     42.8 / 39.9, 8 times 32 behind 96 44.4 / 41.0; 16 tokens alone 29.5 / 29.5.  Beyond it a token forms more than it saves, and
     for R 128, where the two come out alike (8 prompts of about 1024: 109.6 / 108.7), the line lies at contexts without a prefix."""
     T, H, width = q.shape
-    D, R, E = up_k.shape[1], up_k.shape[2], up_v.shape[2]
-    P = width - D
-    if not (max_q and max_k and seqs > 0 and T > 0) or max_q > max_k:
+    _, D, R = up_k.shape
+    E, P = up_v.shape[2], width - D
+    # (what turns most steps down first: a layer whose ranks are too low for it asks here on every prompt step)
+    if not (max_q and max_k and seqs > 0 and T > 0) or max_q > max_k \
+            or latent_formed_rows(seqs, max_k) * (D + E) > 2 * T * R:
         return False
-    if any(t is None or t.dtype != torch.bfloat16 for t in (q, dkv, up_k, up_v, k_cache)):
-        return False
-    if latent_formed_rows(seqs, max_k) * (D + E) > 2 * T * R or P <= 0 or dkv.shape[1] != R + P:
+    if any(t is None or t.dtype != torch.bfloat16 for t in (q, dkv, up_k, up_v, k_cache)) \
+            or P <= 0 or dkv.shape[1] != R + P:
         return False
     return bool(k_cache.is_contiguous() and up_k.is_contiguous() and up_v.is_contiguous() and q.stride(2) == 1
                 and q.stride(1) == width and width % 8 == 0 and (T == 1 or q.stride(0) % 8 == 0)
