@@ -22,7 +22,7 @@
 //    tiles only;
 //  * the 1-D grid is remapped so that workgroups sharing an XCD (and its L2) walk the query
 //    heads of one KV head and adjacent Q tiles of one sequence, heaviest Q tiles first, and that
-//    every XCD gets its share of every sequence.
+//    every XCD gets its share of every sequence (a work list has an order of its own).
 #include "common.h"
 #include <type_traits>
 #include <cstdlib>
@@ -688,7 +688,7 @@ extern "C" int mvl_flash_attention_prefill(
     a.B = B; a.Hq = Hq; a.Hkv = Hkv;
     a.n_qtiles = (max_q_len + kBM - 1) / kBM;
     static const char* pair_env = getenv("MVL_PREFILL_PAIR");
-    // One Q tile per workgroup, or one heavy / light pair (MVL_PREFILL_PAIR: 0 = tiles, g = g pairs).
+    // Without a work list: one Q tile per workgroup, or one heavy / light pair (MVL_PREFILL_PAIR: 0 = tiles, g = g pairs).
     // Tiles find better places on 512 slots than pairs do and a lone prompt's chain is half as long; a pair saves
     // one of two prologues, which shows where prompts are short and the chip is filled twice over.
     // us, pairs / tiles, heads of 128: 4 x 256 (16 / 8) 15.0 / 10.0, 1 x 2048 (16 / 8) 48.8 / 43.4, 3 x 1000 (32 / 8)
@@ -698,7 +698,7 @@ extern "C" int mvl_flash_attention_prefill(
     a.n_items = a.pair ? (n_pairs + a.pair - 1) / a.pair : a.n_qtiles;
     a.total_wg = B * Hq * a.n_items;
     a.items = items;
-    if (items != nullptr) {          // one heavy / light pair of one sequence per slot
+    if (items != nullptr) {          // one heavy / light pair of one sequence per slot, whatever the sizes
         a.pair = 1;
         a.n_items = n_item_slots;
         a.total_wg = Hq * n_item_slots;

@@ -5,7 +5,7 @@
 // Against attention in the latents' own coordinates (hybrid_latent.hip), which for a query and a key takes
 // 2 (R + P) + 4 R operations per head where this takes 2 (D + P) + 4 E (two parts per weight in both), and for a token
 // as many for its query and its output as this for its key and value.  With R 512, P 64, D = E = 128: 3200
-// against 896.  8 prompts of 512..1024 tokens, 16 heads: 268 -> 120 us for the layer (12.5 the store, 49 the forming, 61
+// against 896.  8 prompts of 512..1024 tokens, 16 heads: 267 -> 116 us for the layer (12.5 the store, 49 the forming, 61
 // the attention, where the library's two batched products around the other form took 90 and its attention 182), one of 2048
 // 188 -> 100, of 8192 1632 -> 536; 512 tokens behind 1536 146 -> 100.  Which of the two: the caller's rule.
 //

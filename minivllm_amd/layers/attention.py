@@ -336,7 +336,7 @@ class LatentAttention(nn.Module):
     is c (R), run by ``SinkAttention`` (with its window and sink, when asked for), between two
     batched products per head; in bfloat16 on the GPU by a matrix-core kernel of its own that takes
     the two parts of a query where they are (``SinkAttention.forward_latent``).  Prompts that are most of
-    their contexts are the exception: there keys and values ARE formed, in one pass ahead of the attention
+    their contexts, of ranks up to 512 and in steps without next tokens, are the exception: there keys and values ARE formed, in one pass ahead of the attention
     (``ops.latent_formed_prompts``), which takes a quarter of the operations.  ``up_k`` [H, D, R] and ``up_v`` [H, R, E] are the per-head
     expansion matrices, each laid out as the right operand of its product; ``rotation``: a
     ``HalfRotation`` / ``NeighbourRotation`` over the first entries of the P-part.  Only c and r

@@ -919,7 +919,8 @@ def mid_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
     return out
 
 
-# us a k-step of 64 takes in one workgroup per CU (fitted to 64 measured times), by row and column tile
+# us a k-step of 64 takes in one workgroup per CU, by row and column tile (what is reckoned with them and what was
+# measured stand side by side in profiles/projection_rules.txt)
 _TILE_US = {(64, 64): 0.2, (64, 128): 0.31, (128, 64): 0.31, (128, 128): 0.5, (256, 64): 0.5, (256, 96): 0.8,
             (256, 128): 0.88}
 
