@@ -488,7 +488,8 @@ extern "C" int mvl_car_alloc(void** out, size_t bytes, int uncached) {
     if (e != hipSuccess) return (int)e;
     return (int)hipMemset(*out, 0, bytes);
 }
-extern "C" int mvl_car_free(void* p) { return (int)hipFree(p); }
+// (there is no function that frees: uncached memory that a kernel has read must stay allocated, see custom_allreduce.py)
+extern "C" int mvl_car_clear(void* p, size_t bytes) { return (int)hipMemset(p, 0, bytes); }
 extern "C" int mvl_car_ipc_get(void* p, void* handle_out) {
     return (int)hipIpcGetMemHandle((hipIpcMemHandle_t*)handle_out, p);
 }

@@ -33,7 +33,8 @@ from __future__ import annotations
 
 import ctypes
 import os
-from typing import List, Optional
+import threading
+from typing import Dict, List, Optional, Tuple
 
 import torch
 import torch.distributed as dist
@@ -46,6 +47,38 @@ DEFAULT_MAX_BYTES = 8 << 20             # [1024, 4096] bf16
 # longest wait for a peer inside one kernel before the block gives up (status word set, output
 # poisoned with NaN); MINIVLLM_CAR_TIMEOUT_MS
 DEFAULT_TIMEOUT_MS = int(os.environ.get("MINIVLLM_CAR_TIMEOUT_MS", 2000))
+
+
+# Uncached memory that a kernel has read stays allocated until the process ends: tensors that came to lie where such memory
+# had been freed have held wrong values (an engine built behind one that had used these kernels gave logits that were
+# NaN).  Buffers of a closed all-reduce wait here, device -> [(bytes, address)], for the next one of the process, so there
+# are never more than were in use at one time.
+_IDLE: Dict[int, List[Tuple[int, int]]] = {}
+_IDLE_LOCK = threading.Lock()
+
+
+def _take_buffer(lib, device: int, nbytes: int) -> Tuple[int, int]:
+    """(bytes, address) of at least ``nbytes`` of zeroed uncached memory on the current device, ``device``: the smallest
+    waiting buffer that holds them, a new one where none does."""
+    with _IDLE_LOCK:
+        idle = _IDLE.setdefault(device, [])
+        fit = min((b for b in idle if b[0] >= nbytes), default=None)
+        if fit is not None:
+            idle.remove(fit)
+    if fit is None:
+        p = ctypes.c_void_p()
+        CustomAllReduce._ck(lib.mvl_car_alloc(ctypes.byref(p), nbytes, 1), "alloc")
+        return nbytes, p.value
+    rc = lib.mvl_car_clear(ctypes.c_void_p(fit[1]), fit[0])
+    if rc:
+        _give_back(device, [fit])
+    CustomAllReduce._ck(rc, "clear")
+    return fit
+
+
+def _give_back(device: int, buffers) -> None:
+    with _IDLE_LOCK:
+        _IDLE.setdefault(device, []).extend(buffers)
 
 
 class PeerAllReduceError(RuntimeError):
@@ -68,7 +101,7 @@ class CustomAllReduce:
         vp, sz = ctypes.c_void_p, ctypes.c_size_t
         lib.mvl_car_flags_bytes.restype = sz
         lib.mvl_car_alloc.argtypes = [ctypes.POINTER(vp), sz, ctypes.c_int]
-        lib.mvl_car_free.argtypes = [vp]
+        lib.mvl_car_clear.argtypes = [vp, sz]
         lib.mvl_car_ipc_get.argtypes = [vp, ctypes.c_char_p]
         lib.mvl_car_ipc_open.argtypes = [ctypes.c_char_p, ctypes.POINTER(vp)]
         lib.mvl_car_ipc_close.argtypes = [vp]
@@ -92,15 +125,16 @@ class CustomAllReduce:
         assert max_bytes % 16 == 0
         sizes = [lib.mvl_car_flags_bytes(), 2 * max_bytes, max_bytes]
         self._own: List[int] = []
+        self._buffers: List[Tuple[int, int]] = []           # the same, with their sizes
         self._mapped: List[int] = []
         handles, err = [], None
         try:
             for nbytes in sizes:
-                p = vp()
-                self._ck(lib.mvl_car_alloc(ctypes.byref(p), nbytes, 1), "alloc")
-                self._own.append(p.value)
+                buffer = _take_buffer(lib, self._device_index(), nbytes)
+                self._buffers.append(buffer)
+                self._own.append(buffer[1])
                 buf = ctypes.create_string_buffer(self._hbytes)
-                self._ck(lib.mvl_car_ipc_get(p, buf), "ipc_get")
+                self._ck(lib.mvl_car_ipc_get(vp(buffer[1]), buf), "ipc_get")
                 handles.append(buf.raw)
         except Exception as e:
             err = repr(e)
@@ -137,15 +171,20 @@ class CustomAllReduce:
     def _raise_if_any_failed(self, errors: list) -> None:
         bad = [(r, e) for r, e in enumerate(errors) if e is not None]
         if bad:
-            self._release()
+            self._release(idle=True)                        # (no kernel has been launched, here or by a peer)
             raise RuntimeError(f"peer-to-peer all-reduce set-up failed on rank(s) {bad}")
 
-    def _release(self) -> None:
+    def _device_index(self) -> int:
+        return self.device.index if self.device.index is not None else torch.cuda.current_device()
+
+    def _release(self, idle: bool = False) -> None:
+        """``idle``: no kernel of any rank uses this rank's buffers any more, so another all-reduce may; otherwise (peers
+        that are dead, or did not arrive) a peer may still write to them, and they stay allocated and unused."""
         for p in self._mapped:
             self._lib.mvl_car_ipc_close(p)
-        for p in self._own:
-            self._lib.mvl_car_free(p)
-        self._mapped, self._own = [], []
+        if idle and self._buffers:
+            _give_back(self._device_index(), self._buffers)
+        self._mapped, self._own, self._buffers = [], [], []
 
     @staticmethod
     def _ck(rc: int, what: str) -> None:
@@ -312,8 +351,9 @@ class CustomAllReduce:
         torch.cuda.synchronize()
         try:
             dist.barrier(group=self.group)
+            met = True
         except Exception:
-            pass
+            met = False
         if self.loopback:
             self._lib.mvl_car_set_loopback(0)
-        self._release()
+        self._release(idle=met)
