@@ -227,7 +227,8 @@ gated_head_norm_runs_kernel(const float* __restrict__ o, const float* __restrict
 // One workgroup (256 threads) per token: fp32 router logits (the row is read once, eight experts'
 // partial sums per pass), softmax over all experts (sig: the sigmoid of each logit instead), best
 // `keep` of `groups` groups (a group scores its best expert), `top` largest eligible scores; dense
-// [T, NE] out, zero where not chosen.  Ties go to the lower index.  LDS: 2 * NE + 32 floats.
+// [T, NE] out, zero where not chosen.  Ties go to the lower index.  LDS: 2 * NE + 32 floats.  Scores that are not numbers
+// are never chosen (rows of no sequence may hold anything).
 template <typename T>
 __global__ void grouped_route_kernel(const T* __restrict__ h, const float* __restrict__ wr,
                                      float* __restrict__ dense, int W, int NE, int top,
@@ -295,11 +296,13 @@ __global__ void grouped_route_kernel(const T* __restrict__ h, const float* __res
                 for (int j = 1; j < per; ++j) gv = fmaxf(gv, z[g * per + j]);
                 if (gv > bv) { bv = gv; bg = g; }
             }
+            if (bg < 0) break;                               // (scores that are not numbers)
             for (int j = 0; j < per; ++j) elig[bg * per + j] = z[bg * per + j];
         }
         for (int r = 0; r < top; ++r) {
             int be = -1; float bv = -1.f;
             for (int e = 0; e < NE; ++e) if (elig[e] > bv) { bv = elig[e]; be = e; }
+            if (be < 0) break;
             dense[t * NE + be] = z[be];
             elig[be] = -2.f;
         }
