@@ -27,7 +27,7 @@
 // first chunk.  (A flag of the third kernel's own would have to be seen by a workgroup behind all others: with a fence and
 // a ticket in each that kernel took 115 us instead of 26, a fourth kernel is 3 us more.)
 //
-// 8 portions of 512..1024 tokens, 8 heads of 64 x 128, layer with its norm: 333 us token by token, now 76 (35 + 12 + 26 in the
+// 8 portions of 512..1024 tokens, 8 heads of 64 x 128, layer with its norm: 333 us token by token, now 80 (38 + 12 + 26 in the
 // kernels: decays, scores inside blocks and cutting on the vector units; 5 TB/s; 4.6 TB/s over 120 MB); one of 1024
 // 308 -> 38.  WKV, 16 heads of 64: 334 -> 100, 310 -> 41.  From 64 bits: outputs 1.5e-7, state 1.2e-7, token by token 1.6e-7
 // and 1.3e-7.
@@ -53,13 +53,13 @@ __host__ __device__ inline long item_count(long T, int B) { return T / C + B; }
 
 constexpr float LARGE = 1e9f, LARGE_STATE = 1e25f;      // 64 channels of q u k v: 6e37
 
-// sigmoid(z)^(1/tau) and exp(-exp(z)).  The logarithm of 1 + e^-|z| is taken without care for small e^-|z|: the decay is
-// the exponential of it over tau, to which its last bit makes 6e-8 / tau.
+// sigmoid(z)^(1/tau) and exp(-exp(z)), as the recurrence has them: log1pf and not the logarithm of 1 + e^-|z|, whose rounding is
+// the whole of a slow decay's error and adds up over a portion (600 tokens of one decay each, tau 0.25: outputs 2.7e-5 from 64 bits,
+// 4.3e-6 with log1pf and token by token; the layer's call below 73 us and 80).
 template <int RULE>
 __device__ __forceinline__ float decay_of(float z, float tau_inv) {
     if (RULE == CHANNEL_WKV) return expf(-expf(z));
-    const float l = __builtin_amdgcn_logf(1.f + expf(-fabsf(z))) * 0.693147180559945f;
-    return expf(((z < 0.f ? z : 0.f) - l) * tau_inv);
+    return expf((fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) * tau_inv);
 }
 
 // the sequence that chunk slot `i` belongs to (chunk c of sequence b has slot cu_q[b] / C + b + c), -1: none
