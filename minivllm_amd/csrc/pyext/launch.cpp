@@ -3,8 +3,8 @@
 // the same with an object and a conversion table for every argument: a launcher of 25 arguments costs 4.6 us a call
 // through it and 0.4 like this, where the smallest attention call takes 10 to 13 us altogether.
 //
-// `types`: a letter per argument, i - an integer or a pointer (an int of either sign, taken modulo 2^64, or None for 0),
-// f - a float; then one for the result, I (int) or L (long).  x86-64 System V only: there integers go to six
+// `types`: a letter per argument, p - a pointer (an int, or None for 0), i - an integer (of either sign, taken modulo 2^64),
+// f - a float; then one for the result, I (int) or L (long).  What is none of it is a TypeError, as through ctypes.  x86-64 System V only: there integers go to six
 // registers and then to the stack in their order, floats to registers of their own (up to eight here), so that every
 // signature is called through one type; words on the stack that a function does not have are the caller's to remove.
 #define PY_SSIZE_T_CLEAN
@@ -48,9 +48,13 @@ PyObject* call(PyObject* self, PyObject* const* args, Py_ssize_t n) {
             const double x = PyFloat_AsDouble(args[i]);
             if (x == -1.0 && PyErr_Occurred()) return nullptr;
             f[nf++] = (float)x;
-        } else if (args[i] == Py_None) {
+        } else if (c->types[i] == 'p' && args[i] == Py_None) {
             w[nw++] = 0;
         } else {
+            if (c->types[i] == 'p' && !PyLong_Check(args[i])) {
+                PyErr_Format(PyExc_TypeError, "argument %zd: a pointer expected, an int or None", i + 1);
+                return nullptr;
+            }
             if (PyFloat_Check(args[i])) {
                 PyErr_Format(PyExc_TypeError, "argument %zd: int expected instead of float", i + 1);
                 return nullptr;
@@ -84,9 +88,9 @@ PyObject* bind(PyObject*, PyObject* args) {
     int words = 0, floats = 0;
     bool ok = address != 0 && len >= 1 && len - 1 <= ARGS && (types[len - 1] == 'I' || types[len - 1] == 'L');
     for (Py_ssize_t i = 0; ok && i + 1 < len; ++i) {
-        words += types[i] == 'i';
         floats += types[i] == 'f';
-        ok = types[i] == 'i' || types[i] == 'f';
+        words += types[i] != 'f';
+        ok = types[i] == 'p' || types[i] == 'i' || types[i] == 'f';
     }
     if (!ok || words > REGS + STACK || floats > FLOATS) {
         PyErr_SetString(PyExc_ValueError, "no such call");

@@ -25,15 +25,15 @@ def _load():
 
 
 _native = _load()
+_LETTERS = {ctypes.c_void_p: "p", ctypes.c_int: "i", ctypes.c_long: "i", ctypes.c_uint64: "i", ctypes.c_float: "f"}
 
 
 def bind(lib: ctypes.CDLL, name: str, argtypes, restype=ctypes.c_int):
-    """The function ``name`` of ``lib`` as a callable; integers and pointers are Python ints (None: 0), ``restype``
-    ``c_int`` or ``c_long``."""
+    """The function ``name`` of ``lib`` as a callable; ``restype`` ``c_int`` or ``c_long``.  Pointers are Python ints or None."""
     f = getattr(lib, name)
     f.argtypes = list(argtypes)
     f.restype = restype
-    if _native is None:
+    if _native is None or not all(t in _LETTERS for t in argtypes):
         return f
-    letters = "".join("f" if t is ctypes.c_float else "i" for t in argtypes)
+    letters = "".join(_LETTERS[t] for t in argtypes)
     return _native.bind(ctypes.cast(f, ctypes.c_void_p).value, letters + ("L" if restype is ctypes.c_long else "I"))

@@ -48,6 +48,18 @@ def test_what_is_refused(lib):
     for bad in (args[:-1], args + [0], [1.0] + args[1:], ["x"] + args[1:], args[:4] + ["x"] + args[5:], args[:4] + [None] + args[5:]):
         with pytest.raises(TypeError):
             f(*bad)
+    # None is a pointer and no number; a pointer is an int and nothing that stands for one (a tensor's item would be waited for)
+    class Index:
+        def __index__(self):
+            return 5
+    for i, t in enumerate(MANY):
+        bad = args[:i] + [Index() if t is P else None] + args[i + 1:]
+        with pytest.raises(TypeError):
+            f(*bad)
+        with pytest.raises(ctypes.ArgumentError):
+            lib.many(*bad)
+    assert f(*[None if t is P else Index() if t is not F else 0 for t in MANY]) == \
+        lib.many(*[None if t is P else Index() if t is not F else 0 for t in MANY])
     for types in ("", "i", "iX", "f" * 9 + "I", "i" * 47 + "I"):
         with pytest.raises(ValueError):
             native_call._native.bind(1, types)
