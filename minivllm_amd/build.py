@@ -5,17 +5,19 @@
 * ``_hip_hybrid.so``   - the kernels of hybrid decoders under ``csrc/hybrid/*.hip`` (a library of
   its own, so that a program serving only such a model builds, and loads, nothing else).
 * ``_host_core.so``    - host-side C++ (csrc/host/*.cpp), no GPU code.
-* ``_launch.so``       - the extension module that calls the kernel libraries' launchers (csrc/pyext/launch.cpp).
+* ``_launch_<source><ABI>.so`` - the extension module that calls the kernel libraries' launchers (csrc/pyext/launch.cpp).
 
 ``python -m minivllm_amd.build`` builds whatever is out of date; ``--force`` rebuilds all.
-The libraries are loaded with ctypes, so no torch headers are involved (Python's for ``_launch.so`` alone, which can be
-done without) and hipcc cross-compiles on a machine without a GPU.
+The libraries are loaded with ctypes, so no torch headers are involved (Python's for the launchers' module alone, which can
+be done without) and hipcc cross-compiles on a machine without a GPU.
 """
 from __future__ import annotations
 
 import argparse
 import glob
+import hashlib
 import os
+import platform
 import shutil
 import subprocess
 import sysconfig
@@ -26,7 +28,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "csrc", "build")
 HIP_LIB = os.path.join(HERE, "_hip_kernels.so")
 HOST_LIB = os.path.join(HERE, "_host_core.so")
-LAUNCH_LIB = os.path.join(HERE, "_launch.so")
+LAUNCH_SRC = os.path.join(CSRC, "pyext", "launch.cpp")
 # further kernel libraries: name -> (source folder under csrc, library file)
 GROUPS = {"hybrid": ("hybrid", os.path.join(HERE, "_hip_hybrid.so"))}
 ARCH = "gfx950"
@@ -116,20 +118,37 @@ def build_host(force: bool = False, verbose: bool = True) -> str:
     return HOST_LIB
 
 
+def launch_lib() -> str:
+    """Where the launchers' module of this source and this interpreter lies, built or not: unlike the other libraries it depends
+    on Python, and one of another source may look for other arguments."""
+    with open(LAUNCH_SRC, "rb") as f:
+        source = hashlib.sha256(f.read()).hexdigest()[:12]
+    return os.path.join(HERE, f"_launch_{source}{sysconfig.get_config_var('EXT_SUFFIX') or '.so'}")
+
+
 def build_launch(force: bool = False, verbose: bool = True) -> str:
-    """The extension module that calls the launchers; nothing where Python's headers are not there (ctypes then does)."""
-    src = os.path.join(CSRC, "pyext", "launch.cpp")
-    include = sysconfig.get_paths()["include"]
-    if not os.path.exists(os.path.join(include, "Python.h")):
-        return ""
-    if force or not _newer(LAUNCH_LIB, [src]):
-        cxx = shutil.which("g++") or shutil.which("c++")
-        tmp = f"{LAUNCH_LIB}.{os.getpid()}.tmp"
-        _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-I{include}", "-o", tmp, src])
-        os.replace(tmp, LAUNCH_LIB)
+    """The extension module that calls the launchers; "" where it cannot be built (ctypes then makes the calls)."""
+    lib, include = launch_lib(), sysconfig.get_paths()["include"]
+    if os.path.exists(lib) and not force:
+        return lib
+    cxx = shutil.which("g++") or shutil.which("c++")
+    lack = ("an x86-64 machine with the System V calling convention" if platform.machine() != "x86_64" or os.name != "posix"
+            else "Python's headers" if not os.path.exists(os.path.join(include, "Python.h"))
+            else "a C++ compiler" if cxx is None else "")
+    if lack:
         if verbose:
-            print(f"[build] linked {LAUNCH_LIB}", flush=True)
-    return LAUNCH_LIB
+            print(f"[build] the launchers' module wants {lack}: ctypes makes the calls", flush=True)
+        return ""
+    tmp = f"{lib}.{os.getpid()}.tmp"
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-I{include}", "-o", tmp, LAUNCH_SRC])
+    os.replace(tmp, lib)
+    abi = lib[lib.rindex("_launch_") + len("_launch_") + 12:]
+    for old in glob.glob(os.path.join(HERE, "_launch_*" + abi)):           # of other sources; other interpreters keep theirs
+        if old != lib:
+            os.remove(old)
+    if verbose:
+        print(f"[build] linked {lib}", flush=True)
+    return lib
 
 
 def build_all(force: bool = False, verbose: bool = True) -> None:

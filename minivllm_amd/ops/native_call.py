@@ -1,27 +1,30 @@
-"""How the kernel libraries' launchers are called: through ``_launch.so`` (``csrc/pyext/launch.cpp``), which makes a call of
-25 arguments in 0.4 us, or, where it cannot be built or loaded (no Python headers, no x86-64), through ctypes, which takes
-3 to 5.  The library is built on first use like the kernel libraries."""
+"""How the kernel libraries' launchers are called: through an extension module (``csrc/pyext/launch.cpp``), which makes a call of
+25 arguments in 0.4 us, or, where it cannot be built or loaded (no Python headers, no compiler, no x86-64), through ctypes, which
+takes 3 to 5, with a warning.  The module is built on first use like the kernel libraries; its name says which source and which
+interpreter it is for (``build.launch_lib``)."""
 from __future__ import annotations
 
 import ctypes
 import importlib.machinery
 import importlib.util
-import os
+import warnings
 
-_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "_launch.so")
+from minivllm_amd import build
 
 
 def _load():
+    why = "it cannot be built here"
     try:
-        if not os.path.exists(_PATH):
-            from minivllm_amd import build
-            build.build_launch(verbose=False)
-        loader = importlib.machinery.ExtensionFileLoader("_launch", _PATH)
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_launch", loader))
-        loader.exec_module(module)
-        return module
-    except Exception:                      # noqa: BLE001  (ctypes takes the calls)
-        return None
+        path = build.build_launch(verbose=False)
+        if path:
+            loader = importlib.machinery.ExtensionFileLoader("_launch", path)
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_launch", loader))
+            loader.exec_module(module)
+            return module
+    except Exception as e:                 # noqa: BLE001  (ctypes takes the calls)
+        why = str(e)
+    warnings.warn(f"kernels are launched through ctypes, 3 to 5 us a call slower than by the launchers' module: {why}")
+    return None
 
 
 _native = _load()

@@ -1,11 +1,15 @@
 """Calls of C functions by address (``ops.native_call``): every argument arrives where the function looks for it, as
 through ctypes, and what is no number is refused."""
 import ctypes
+import os
+import platform
 import shutil
 import subprocess
+import sysconfig
 
 import pytest
 
+from minivllm_amd import build
 from minivllm_amd.ops import native_call
 
 SOURCE = r"""
@@ -70,3 +74,39 @@ def test_without_it(lib, monkeypatch):
     monkeypatch.setattr(native_call, "_native", None)
     f = native_call.bind(lib, "many", MANY, L)
     assert f(*[1] * len(MANY)) == lib.many(*[1] * len(MANY))
+
+
+@pytest.fixture
+def empty_package(monkeypatch, tmp_path):
+    """The builder with a package folder of its own, and a source in it."""
+    (tmp_path / "launch.cpp").write_bytes(open(build.LAUNCH_SRC, "rb").read())
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
+    monkeypatch.setattr(build, "LAUNCH_SRC", str(tmp_path / "launch.cpp"))
+    return tmp_path
+
+
+@pytest.mark.parametrize("lack", ["machine", "headers", "compiler"])
+def test_done_without_where_it_cannot_be_built(empty_package, monkeypatch, lack):
+    if lack == "machine":
+        monkeypatch.setattr(platform, "machine", lambda: "aarch64")
+    elif lack == "headers":
+        monkeypatch.setattr(sysconfig, "get_paths", lambda: {"include": str(empty_package)})
+    else:
+        monkeypatch.setattr(shutil, "which", lambda name: None)
+    assert build.build_launch(verbose=False) == "" and build.build_launch(force=True) == ""
+    with pytest.warns(UserWarning, match="ctypes"):
+        assert native_call._load() is None
+
+
+def test_named_by_source_and_interpreter(lib, empty_package):
+    first = build.build_launch(verbose=False)
+    assert first.endswith(sysconfig.get_config_var("EXT_SUFFIX")) and os.path.exists(first)
+    stamp = os.stat(first).st_mtime_ns
+    assert build.build_launch(verbose=False) == first and os.stat(first).st_mtime_ns == stamp
+    (empty_package / "launch.cpp").open("a").write("// another source\n")
+    second = build.build_launch(verbose=False)
+    assert second != first and os.listdir(empty_package).count(os.path.basename(first)) == 0
+    assert native_call._load() is not None
+    (empty_package / "launch.cpp").write_text("no C++\n")
+    with pytest.warns(UserWarning, match="command failed"):
+        assert native_call._load() is None
