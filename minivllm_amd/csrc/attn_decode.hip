@@ -360,6 +360,9 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
             if (tile + 2 * kWaves < t1) load_block_ids(tile + 2 * kWaves, ids_next);
         }
 
+        // (lanes read what others have written: the hardware keeps a wave's LDS instructions in order, this the compiler)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         // ---- S^T[token][head] = K . Q^T : two 16-token sub-tiles
         f32x4_t s_acc[2];
 #pragma unroll
@@ -415,6 +418,8 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
             const s16x8_t a = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
             acc_o[n] = DT::mfma16(__builtin_bit_cast(vec8, a), pfrag, acc_o[n]);
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 
     // ---- merge the waves through LDS (each wave reuses its own staging region)

@@ -172,6 +172,7 @@ channel_chunk_kernel(const ChannelChunks a) {
             for (int y = 0; y < 3; ++y) *reinterpret_cast<bf16x8*>(L.vp[y] + at_v<EP>(row, e >> 3)) = p[y];
         }
     }
+    lanes_meet();                                               // (a wave reads its own block's rows)
     // ---- scores inside the block: lane = (key s, a quarter of the channels), s + j is the query of step j
     {
         float kd[DC], p[16];
@@ -223,6 +224,7 @@ channel_chunk_kernel(const ChannelChunks a) {
             if (t < 16) L.diag[w][t][s] = p4[j];
         }
     }
+    lanes_meet();                                               // q's rows are about to change
     // ---- q with the decays from its block's start, k with those to its block's end
 #pragma unroll
     for (int i = 0; i < NC; ++i) {

@@ -11,6 +11,14 @@ namespace hyb {
 
 constexpr int kWave = 64;
 
+// Between LDS that lanes of a wave have written and other lanes of it read, or the other way round: the hardware keeps a wave's
+// LDS instructions in order, this keeps the compiler from moving them, to which lanes are threads of their own.  No
+// instruction.
+__device__ __forceinline__ void lanes_meet() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 struct bf16_t { uint16_t v; };
 
 template <typename T> __device__ __forceinline__ float ld(const T* p);

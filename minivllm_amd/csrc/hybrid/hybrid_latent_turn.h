@@ -58,8 +58,7 @@ __device__ __forceinline__ void latent_turn_store(long t, float* cs, const T* __
         sincosf(p * inv_freq[i], &s_, &c_);
         cs[i] = c_ * mult; sn[i] = s_ * mult;
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");          // cs / sn: written and read by this wave
-    __builtin_amdgcn_wave_barrier();
+    lanes_meet();                                                   // cs / sn: written and read by this wave
     const float r = rsqrtf(wave_sum(ss) / (float)R + eps);
     const int DK = R + P;
     if (store) {

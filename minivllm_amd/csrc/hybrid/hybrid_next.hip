@@ -150,6 +150,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) next_attention_kernel(const Nex
             fetch(t + WAVES);
             if (t + 2 * WAVES < t1) look(t + 2 * WAVES);
         }
+        lanes_meet();                              // the images are there
         // scores of two blocks of 16 keys: lane = head c16, keys 16 x + 4 q4 + r
         float p[8], top = -INFINITY;
 #pragma unroll
@@ -192,6 +193,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2) next_attention_kernel(const Nex
 #pragma unroll
             for (int k = 2; k >= 0; --k) acc[n] = mfma(vf, pf[k], acc[n]);
         }
+        lanes_meet();                              // and have been read
     }
     // ---- the waves' sums through LDS, each in its own place
     l_run += __shfl_xor(l_run, 16, kWave);
