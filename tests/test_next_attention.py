@@ -98,3 +98,35 @@ def test_against_exact(D, E, G, R, rule, bs):
         assert bool(out[10, :R].isnan().all())
     else:
         compare(out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,E,n", [(128, 128, 1024), (64, 64, 300), (128, 64, 700)])
+@pytest.mark.parametrize("spread", [1.0, 2.0, 4.0])
+def test_sums_are_no_further_from_float64_than_on_the_vector_units(D, E, n, spread):
+    """The partial results of two splits, which are fp32, ahead of the rounding that hides what is below it."""
+    dev, B, G, H, bs, S = "cuda", 8, 4, 8, 64, 2
+    pages, ratios = -(-n // bs), []
+    for seed in range(6):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        kc, vc = (torch.randn(B * pages, bs, G, m, generator=g, device=dev).bfloat16() for m in (D, E))
+        q = (spread * torch.randn(B, H, D, generator=g, device=dev)).bfloat16()
+        sink = torch.randn(H, generator=g, device=dev)
+        tables = torch.arange(B * pages, device=dev, dtype=torch.int32).view(B, pages)
+        lens = torch.full((B,), n, dtype=torch.int32, device=dev)
+        out = torch.empty(B, H, E, dtype=torch.bfloat16, device=dev)
+        want = torch.stack([_exact(q[b], *(c[b * pages:(b + 1) * pages].reshape(-1, G, c.shape[3])[:n] for c in (kc, vc)),
+                                   D ** -0.5, 0, 0, None, sink, None) for b in range(B)])
+        err = []
+        for launch, own, last in ((hk._nxa, [], []), (hk._split, hk._pool_args(kc, vc, E, H, None, 0.0, 0, None, None), [0])):
+            ws = torch.zeros(B, H, S, E + 2, device=dev)
+            hk._check(launch(q.data_ptr(), H * D, D, kc.data_ptr(), vc.data_ptr(), tables.data_ptr(), pages, bs, lens.data_ptr(),
+                             sink.data_ptr(), None, 0, out.data_ptr(), ws.data_ptr(), D ** -0.5, B, H, G, D, E, S, 0, 0, None, E,
+                             *own, 0, 0, *last, hk._stream()), "attention")
+            m, l, o = ws[..., 0].double(), ws[..., 1].double(), ws[..., 2:].double()
+            top = torch.maximum(m.amax(-1), sink.double())
+            f = (m - top[..., None]).exp()
+            err.append(((o * f[..., None]).sum(2) / ((l * f).sum(-1) + (sink.double() - top).exp())[..., None] - want).norm())
+        ratios.append(math.log(float(err[0] / err[1])))
+    # the mean of six; a tenth for their spread (single ones differ by up to a quarter)
+    assert sum(ratios) / len(ratios) <= math.log(1.1), ratios
