@@ -890,14 +890,10 @@ def _latent(q_abs, q_rot, k_cache, tables, cu_q, positions, lens, scale, sink, o
 
 
 def latent_attention_prefill(q_abs, q_rot, k_cache, cu_q, block_tables, positions, scale, sink, out,
-                             max_q, window=0, around=None):
+                             max_q, window=0):
     """Prompt portions: ``q_abs`` [H, T, R] and ``q_rot`` [T, H, P] are the two parts of the queries,
     sequence b owns rows cu_q[b] .. cu_q[b+1] (absolute rows) and block table row b; ``max_q``: the
-    longest portion (a host integer).  ``around``: the whole step's call, queries and ``out`` before and behind the
-    expansions (``latent_rows``)."""
-    if around is not None:
-        _check(_latr(*around), "latent_rows")
-        return out
+    longest portion (a host integer)."""
     nseq = cu_q.shape[0] - 1
     if max_q is None:
         max_q = int((cu_q[1:] - cu_q[:-1]).max())
@@ -906,11 +902,8 @@ def latent_attention_prefill(q_abs, q_rot, k_cache, cu_q, block_tables, position
 
 
 def latent_attention_decode(q_abs, q_rot, k_cache, block_tables, context_lens, scale, sink, out,
-                            max_context_len=None, window=0, around=None):
-    """Single next tokens: row b is sequence b with ``context_lens[b]`` keys.  ``around``: as above."""
-    if around is not None:
-        _check(_latr(*around), "latent_rows")
-        return out
+                            max_context_len=None, window=0):
+    """Single next tokens: row b is sequence b with ``context_lens[b]`` keys."""
     B, H, R = out.shape
     return _latent(q_abs, q_rot, k_cache, block_tables, None, None, _i32c(context_lens), scale, sink, out,
                    B, 1, window, latent_splits(B, H, R, max_context_len, window))
@@ -953,15 +946,13 @@ def latent_rows(q, dkv, norm_w, eps, positions, inv_freq, rot_dims, neighbours, 
     assert block_tables.shape[0] >= nseq
     ws = torch.empty((_latr_ws(T, H, P, R, splits),), dtype=torch.uint8, device=q.device)
     out = torch.empty((T, H, E), dtype=q.dtype, device=q.device)
-    around = (qp, q_row, dp, dkv_row, _f32(norm_w).data_ptr(), eps, _i32(positions).data_ptr(), _f32(inv_freq).data_ptr(),
-              int(rot_dims), int(neighbours), float(mult), cp, _i32(slot_mapping).data_ptr(), kp, vp,
-              block_tables.data_ptr(), block_tables.stride(0), k_cache.shape[1],
-              None if cu_q is None else _i32c(cu_q).data_ptr(), None if cu_q is not None else _i32c(lens).data_ptr(),
-              None if sink is None else _f32(sink).data_ptr(), ws.data_ptr(), out.data_ptr(), float(scale), T, nseq,
-              int(max_q), H, D, P, R, E, int(window), splits, _stream())
-    if cu_q is None:
-        return latent_attention_decode(None, None, k_cache, block_tables, lens, scale, sink, out, around=around)
-    return latent_attention_prefill(None, None, k_cache, cu_q, block_tables, positions, scale, sink, out, max_q, around=around)
+    _check(_latr(qp, q_row, dp, dkv_row, _f32(norm_w).data_ptr(), eps, _i32(positions).data_ptr(), _f32(inv_freq).data_ptr(),
+                 int(rot_dims), int(neighbours), float(mult), cp, _i32(slot_mapping).data_ptr(), kp, vp,
+                 block_tables.data_ptr(), block_tables.stride(0), k_cache.shape[1],
+                 None if cu_q is None else _i32c(cu_q).data_ptr(), None if cu_q is not None else _i32c(lens).data_ptr(),
+                 None if sink is None else _f32(sink).data_ptr(), ws.data_ptr(), out.data_ptr(), float(scale), T, nseq,
+                 int(max_q), H, D, P, R, E, int(window), splits, _stream()), "latent_rows")
+    return out
 
 
 def latent_formed_rows(seqs: int, max_k: int) -> int:

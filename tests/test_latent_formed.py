@@ -143,7 +143,8 @@ def _turned(x, pos, base=10000.0):
 def test_steps_through_the_layer(monkeypatch, R, bs, formed, window, sink):
     """A layer's steps over one cache: prompts of several lengths, portions behind a prefix, next tokens, prompts with
     riders, a prompt behind what those wrote; rows of no sequence in between.  The steps of prompts alone run with keys
-    and values formed where the rule has it, and are no further from 64 bits than with attention in the latents' coordinates."""
+    and values formed where the rule has it, steps of few rows in one call, and are no further from 64 bits than with
+    attention in the latents' coordinates, call by call."""
     from minivllm_amd import ops
     from minivllm_amd.layers.attention import LatentAttention
     from minivllm_amd.layers.rotary_embedding import HalfRotation
@@ -164,13 +165,16 @@ def test_steps_through_the_layer(monkeypatch, R, bs, formed, window, sink):
         a.core.k_cache = torch.full((tables.numel(), bs, 1, R + P), float("nan"), dtype=torch.bfloat16, device="cuda")
         a.core.v_cache = a.core.k_cache[..., :R]
         layers[form] = a
+    monkeypatch.setattr(hk, "LATENT_ROWS", 100 * R)                       # (the steps lie on both sides of it)
     taken = []
-    for name in ("latent_formed_prompts", "latent_attention_prefill", "latent_attention_decode"):
+    for name in ("latent_formed_prompts", "latent_rows", "latent_attention_prefill", "latent_attention_decode"):
         def spy(*args, _f=getattr(hk, name), _name=name, **kw):
-            taken.append(_name)
-            return _f(*args, **kw)
+            out = _f(*args, **kw)
+            if out is not None or _name != "latent_rows":
+                taken.append(_name)
+            return out
         monkeypatch.setattr(hk, name, spy)
-    rule = ops.latent_formed_ok
+    rule, few = ops.latent_formed_ok, ops.latent_rows
     ku, vu = up_k.bfloat16().double().view(H, D, R), up_v.bfloat16().double().view(H, E, R)
     rows = torch.zeros(nseq, room, R + P, dtype=torch.float64)              # what the cache should hold
     past, squares = [0] * nseq, dict(rule=0.0, absorbed=0.0, of=0.0)
@@ -196,6 +200,7 @@ def test_steps_through_the_layer(monkeypatch, R, bs, formed, window, sink):
         got, ways = {}, {}
         for form, a in layers.items():
             monkeypatch.setattr(ops, "latent_formed_ok", rule if form == "rule" else lambda *args: False)
+            monkeypatch.setattr(ops, "latent_rows", few if form == "rule" else lambda *args: None)
             set_context(**kw)
             taken.clear()
             with torch.inference_mode():
@@ -226,14 +231,17 @@ def test_steps_through_the_layer(monkeypatch, R, bs, formed, window, sink):
             at += n
         if R > 512 and behind:
             assert not got["rule"][at:].any()
-        return ways["rule"]
+        has = lambda *names: sorted(names) if R <= 512 else []
+        assert sorted(ways["absorbed"]) == has(*["latent_attention_decode"] * bool(riders), *["latent_attention_prefill"] * bool(prompts))
+        return sorted(ways["rule"]) if R <= 512 else ways["rule"] or None
 
-    alone = ["latent_formed_prompts"] if formed else ["latent_attention_prefill"] if R <= 512 else []
-    nexts = ["latent_attention_decode"] if R <= 512 else []
-    assert step([0, 1, 2], [5, 65, 96], behind=6) == alone
-    assert step([1, 0], [64, 75], behind=1) == alone                       # behind 65 and 5 tokens
-    assert step([2, 1, 0], [1, 1, 1], riders=3) == nexts
-    assert sorted(step([2, 0], [1, 40], riders=1, behind=3)) == sorted(nexts + ["latent_attention_prefill"] * (R <= 512))
-    assert step([0], [80]) == alone
+    one_call = ["latent_rows"] if R <= 512 else None
+    call_by_call = ["latent_attention_prefill"] if R <= 512 else None
+    formed_or = lambda other: ["latent_formed_prompts"] if formed else other
+    assert step([0, 1, 2], [5, 65, 96], behind=6) == formed_or(call_by_call)
+    assert step([1, 0], [64, 75], behind=1) == formed_or(call_by_call)     # behind 65 and 5 tokens
+    assert step([2, 1, 0], [1, 1, 1], riders=3) == one_call
+    assert step([2, 0], [1, 40], riders=1, behind=3) == (["latent_attention_decode", "latent_attention_prefill"] if R <= 512 else None)
+    assert step([0], [80]) == formed_or(one_call)
     # the two forms round the same number of times: their errors differ by chance only (a tenth allowed)
     assert squares["rule"] <= 1.21 * squares["absorbed"]
