@@ -32,6 +32,7 @@
 // Two parts per weight instead of three would hold 16 bits of it.
 #include "hybrid_row_by_keys.h"
 #include "hybrid_chunks.h"
+#include <algorithm>
 
 using namespace hyb;
 
@@ -980,20 +981,55 @@ int launch_f32_as(const PromptArgs32& a, int nseq, int max_q, hipStream_t s) {
     return HYB_LAUNCH_OK();
 }
 
+// The most keys that a workgroup walks: contexts fit their pages, and queries see no more than a window or a chunk has.
+long longest_walk(int max_blocks, int block_size, const KeyRule& rule) {
+    long n = (long)max_blocks * block_size;
+    if (rule.window > 0) n = std::min(n, (long)rule.window + rule.keep_first + 127);
+    if (rule.chunk > 0) n = std::min(n, (long)rule.chunk + 127);
+    return n;
+}
+
+// Which form takes a launch of float rows, F32_QUERIES * 10 + F32_GROUPS: 41, one group of four waves; 42, two groups; 22 and 24,
+// two and four groups of two waves on 64 queries.  rows: of the step, 0 if that is not known.
+//
+// More groups shorten the chain of a workgroup and cost their meeting, LDS and, with 24 and 42, the second workgroup of a CU;
+// they pay for long walks and where there is at most a workgroup for every CU.  us, 41 / 42 / 24 / 22, 8 heads, prompts of
+// equal length, 64 + 64, 128 + 64 and (41 / 42 / 22) 128 + 128 columns:
+//   4 of 128 keys                  14 / 14 / 11 / 11      18 / 18 / 16 / 14      21 / 22 / 17
+//   32 of 128                      16 / 15 / 19 / 13      21 / 21 / 33 / 26      26 / 29 / 34
+//   64 of 128                      23 / 30 / 39 / 24      31 / 39 / 63 / 50      49 / 54 / 67
+//   256 of 32                      28 / 51 / 59 / 30      35 / 68 / 84 / 66      68 / 89 / 81
+//   4 of 512                       45 / 35 / 24 / 29      58 / 44 / 33 / 38      69 / 56 / 46
+//   16 of 512                      49 / 48 / 62 / 48      64 / 64 / 91 / 91      92 / 87 / 113
+//   2 of 2048                     165 / 118 / 83 / 101   216 / 148 / 114 / 143  253 / 186 / 177
+//   4 of 2048                     168 / 133 / 157 / 148  222 / 173 / 222 / 278  276 / 236 / 342
+//   16 of 2048                    487 / 526 / 627 / 546  658 / 700 / 894 / 1107 1097 / 953 / 1366
+// Over 420 such launches (32 to 2048 keys, 24 to 2048 tiles of 128 queries, also of uneven lengths) the choice below is at worst
+// 1.02 times as slow as 41 and in the mean 1.01 times the best of the four; by the number of tiles alone it was 1.16, and
+// up to 1.9 times 41 for many short prompts.
+int f32_form(int columns, long keys, int H, int nseq, int max_q, long rows) {
+    auto tiles = [&](int q) {
+        const long most = (long)H * nseq * ((max_q + q - 1) / q);
+        return rows > 0 ? std::min(most, H * (rows / q + (nseq + 1) / 2)) : most;
+    };
+    const bool wide = columns > 192;
+    const long t64 = tiles(64), t128 = tiles(128);
+    if (keys <= 32) return 41;
+    if (t64 <= 256) return !wide && keys >= (columns > 128 ? 256 : 96) ? 24 : 22;
+    if (t64 <= 512 && (keys >= 192 || columns <= 128)) return !wide && (keys >= 1024 || (keys >= 512 && t64 <= 384)) ? 24 : 22;
+    if (wide) return keys >= 384 ? 42 : 41;
+    return (keys >= 384 && t128 <= 384) || (keys >= 512 && t128 <= 512) || (keys >= 1024 && t128 <= 640) ? 42 : 41;
+}
+
 template <int DP, int EP>
 int launch_f32(const PromptArgs32& a, int nseq, int max_q, hipStream_t s) {
     if (a.rule.temps || a.rule.softcap > 0.f || a.rule.pool > 0) return launch_f32_as<DP, EP, true, 4, 1>(a, nseq, max_q, s);
-    // tiles of 128 queries, us: one group of four waves / two / two groups of two / four (three at 128 + 128 columns)
-    // of two.  64 + 64 columns: 120 (window 256) 36.7 / 32.7 / 27.2 / 23.8, 128 (one of 2048) 170 / 124 / 107 / 79, 512 98 / 80 /
-    // 81 / 94; 128 + 64: 80 69 / 52 / 46 / 38, 512 111 / 82 / 104 / 95; 128 + 128: 48 47 / 39 / 34 / 41, 256 258 / 199 / 184 /
-    // 219, 384 50.8 / 50.2 / 46.6 / 62, 512 80 / 76 / 93 / 115, 1024 284 / 255 / 308 / 376.
-    const long tiles = (long)a.H * nseq * ((max_q + 127) / 128);
-    if constexpr (DP + EP <= 192) {
-        if (tiles <= 256) return launch_f32_as<DP, EP, false, 2, 4>(a, nseq, max_q, s);
-    } else {
-        if (tiles <= 384) return launch_f32_as<DP, EP, false, 2, 2>(a, nseq, max_q, s);
+    switch (f32_form(DP + EP, longest_walk(a.max_blocks, a.block_size, a.rule), a.H, nseq, max_q, a.clear.end - a.clear.first)) {
+        case 24: if constexpr (DP + EP <= 192) return launch_f32_as<DP, EP, false, 2, 4>(a, nseq, max_q, s);
+        case 22: return launch_f32_as<DP, EP, false, 2, 2>(a, nseq, max_q, s);
+        case 42: return launch_f32_as<DP, EP, false, 4, 2>(a, nseq, max_q, s);
+        default: return launch_f32_as<DP, EP, false, 4, 1>(a, nseq, max_q, s);
     }
-    return launch_f32_as<DP, EP, false, 4, 2>(a, nseq, max_q, s);
 }
 
 template <int DP, int RP, int EP, int PARTS, bool EXT, bool WHOLE, int KG>
@@ -1009,13 +1045,26 @@ int launch_groups(const PromptArgs& a, int nseq, int max_q, hipStream_t s) {
     return HYB_LAUNCH_OK();
 }
 
+// Groups of waves on a workgroup's queries, for images of so many key and value columns (`columns`: both).  A second group shortens each one's
+// run of tiles; it pays where there is a workgroup for every CU at most, and where the run is long enough for the groups'
+// meeting.  us, one group / two, 8 heads, prompts of equal length, 128 workgroups:
+//   keys a prompt      64        128       256       384       512       1024      2048
+//   64 + 64           10 / 9    10 / 10   13 / 12   16 / 14   18 / 16   31 / 25   55 / 41
+//   128 + 128         10 / 10   11 / 13   15 / 16   19 / 18   23 / 21   38 / 32   68 / 53
+//   64 + 256          11 / 14   15 / 19   20 / 23   25 / 26   30 / 30   50 / 45   89 / 77
+//   256 + 128         10 / 12   13 / 16   17 / 19   22 / 23   26 / 26   43 / 39   76 / 65
+// The two last spill some 20 registers with two groups of waves on a CU, which one group has room for.  Keys and values formed
+// from latents, 16 heads: 4 of 256 41.7 / 41.8, 5 of 384 50 / 48.5, one of 1024 68.5 / 62.
+int groups_of(int columns, int value_columns, long keys, long workgroups) {
+    const bool spills = value_columns > 128 || columns > 320;
+    return workgroups <= 256 && keys >= (spills ? 640 : 384) ? 2 : 1;
+}
+
 template <int DP, int RP, int EP, int PARTS, bool EXT, bool WHOLE>
 int launch_form(const PromptArgs& a, int nseq, int max_q, hipStream_t s) {
     if constexpr (!EXT && 2 * 32 * 2 * (3 * (DP + RP) + 4 * EP) <= 160 * 1024) {
-        // a workgroup for every CU at most: a second group of waves on it shortens each one's run of tiles.  us, one group / two,
-        // 16 heads of 128: 128 workgroups (one of 1024) 39.7 / 35.3, 256 (one of 2048) 72.1 / 59.5, two of 1024 42.6 /
-        // 37.3, 512 (8 of 500) 29.7 / 33.1; 8 heads of 64, 128 (one of 2048) 56.9 / 43.1.
-        if ((long)a.H * nseq * ((max_q + 127) / 128) <= 256) return launch_groups<DP, RP, EP, PARTS, EXT, WHOLE, 2>(a, nseq, max_q, s);
+        if (groups_of(DP + EP, EP, longest_walk(a.max_blocks, a.block_size, a.rule), (long)a.H * nseq * ((max_q + 127) / 128)) == 2)
+            return launch_groups<DP, RP, EP, PARTS, EXT, WHOLE, 2>(a, nseq, max_q, s);
     }
     return launch_groups<DP, RP, EP, PARTS, EXT, WHOLE, 1>(a, nseq, max_q, s);
 }
@@ -1095,3 +1144,20 @@ int latent_prompts(const void* q, long q_row, long q_head, const void* qr, long 
 }
 
 }  // namespace hyb
+
+extern "C" {
+
+// The rules above, for tests of where their lines lie.
+int hyb_prompt_f32_form(int columns, long keys, int H, int nseq, int max_q, long rows) {
+    return f32_form(columns, keys, H, nseq, max_q, rows);
+}
+int hyb_prompt_groups(int columns, int value_columns, long keys, long workgroups) {
+    return groups_of(columns, value_columns, keys, workgroups);
+}
+int hyb_prompt_longest_walk(int max_blocks, int block_size, int window, int keep_first, int chunk) {
+    KeyRule rule{};
+    rule.window = window; rule.keep_first = keep_first; rule.chunk = chunk;
+    return (int)std::min(longest_walk(max_blocks, block_size, rule), 1L << 30);
+}
+
+}  // extern "C"

@@ -45,6 +45,9 @@ _attn = _sig("hyb_sink_attention_rows", _P, _L, _L, _P, _P, _P, _I, _I, _P, _P, 
 _tiles = _sig("hyb_sink_attention_tiles", _P, _L, _L, _P, _P, _P, _I, _I, _P, _P, _P, _P, _L, _P, _F,
               _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, *_POOL, _L, _L, _I, _P)
 _tiles_ok = bind(_lib, "hyb_sink_attention_tiles_ok", [_I, _I], _I)
+_f32_form = bind(_lib, "hyb_prompt_f32_form", [_I, _L, _I, _I, _I, _L], _I)
+_prompt_groups = bind(_lib, "hyb_prompt_groups", [_I, _I, _L, _L], _I)
+_longest_walk = bind(_lib, "hyb_prompt_longest_walk", [_I] * 5, _I)
 _tiles_form = _sig("hyb_sink_attention_tiles_form", _P, _L, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I)
 _split = _sig("hyb_sink_attention_split", _P, _L, _L, _P, _P, _P, _I, _I, _P, _P, _P, _L, _P, _P, _F,
               _I, _I, _I, _I, _I, _I, _I, _I, _P, _I, *_POOL, _I, _I, _P)

@@ -51,3 +51,34 @@ def test_heads_of_a_decode_workgroup():
     (64, 8, 16, 0, 2), (1, 8, 16, None, 8)])
 def test_splits_of_a_decode_batch(batch, kv_heads, heads, longest, splits):
     assert hk.decode_splits(batch, kv_heads, heads, longest) == splits
+
+
+@pytest.mark.parametrize("columns,keys,H,nseq,max_q,rows,form", [
+    (128, 32, 8, 4, 32, 0, 41), (128, 33, 8, 4, 33, 0, 22), (128, 95, 8, 4, 95, 0, 22), (128, 96, 8, 4, 96, 0, 24),
+    (192, 255, 8, 4, 128, 0, 22), (192, 256, 8, 4, 128, 0, 24), (256, 4096, 8, 4, 256, 0, 22),
+    # 256 tiles of 64 queries, 264; 512, 520
+    (192, 1023, 8, 4, 512, 0, 24), (192, 511, 8, 3, 704, 0, 22), (192, 512, 8, 3, 704, 0, 24), (192, 191, 8, 3, 704, 0, 41),
+    (128, 191, 8, 3, 704, 0, 22), (256, 191, 8, 3, 704, 0, 41), (256, 192, 8, 3, 704, 0, 22), (192, 512, 8, 4, 1024, 0, 22),
+    (192, 1024, 8, 4, 1024, 0, 24), (192, 383, 8, 5, 832, 0, 41), (192, 384, 8, 5, 832, 0, 42), (256, 383, 8, 5, 832, 0, 41),
+    (256, 384, 8, 500, 832, 0, 42),
+    # tiles of 128 queries: 384, 392; 512, 520; 640, 648
+    (128, 384, 8, 16, 384, 0, 42), (128, 384, 8, 49, 128, 0, 41), (128, 512, 8, 64, 128, 0, 42), (128, 512, 8, 65, 128, 0, 41),
+    (128, 1024, 8, 80, 128, 0, 42), (128, 1024, 8, 81, 128, 0, 41),
+    # rows that are known: 8 * (4000 / 64 + 5) tiles at most
+    (128, 1024, 8, 9, 1024, 4000, 42), (128, 1024, 8, 9, 1024, 0, 42), (128, 384, 8, 9, 1024, 4000, 42), (128, 384, 8, 9, 1024, 0, 41)])
+def test_prompt_attention_form_of_float_rows(columns, keys, H, nseq, max_q, rows, form):
+    assert hk._f32_form(columns, keys, H, nseq, max_q, rows) == form
+
+
+@pytest.mark.parametrize("D,E,keys,workgroups,groups", [
+    (128, 128, 384, 256, 2), (128, 128, 383, 256, 1), (128, 128, 4096, 257, 1), (256, 64, 384, 1, 2), (64, 256, 639, 1, 1),
+    (64, 256, 640, 1, 2), (256, 128, 639, 1, 1), (256, 128, 640, 256, 2)])
+def test_prompt_attention_groups(D, E, keys, workgroups, groups):
+    assert hk._prompt_groups(D + E, E, keys, workgroups) == groups
+
+
+@pytest.mark.parametrize("blocks,size,window,keep,chunk,walk", [
+    (6, 64, 0, 0, 0, 384), (6, 64, 256, 0, 0, 383), (6, 64, 256, 4, 0, 384), (100, 64, 256, 4, 0, 387), (100, 64, 0, 0, 512, 639),
+    (1 << 30, 1 << 20, 0, 0, 0, 1 << 30)])
+def test_longest_walk(blocks, size, window, keep, chunk, walk):
+    assert hk._longest_walk(blocks, size, window, keep, chunk) == walk

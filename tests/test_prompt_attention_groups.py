@@ -66,3 +66,36 @@ def test_forms(D, E, H, window, keep, dt, bs):
             # fp32 sums of up to 333 terms and exponentials of fp32 differences; the result in its type
             assert float((got - want).norm() / want.norm()) < (1e-6 if dt == torch.float32 else 2.0 ** -8), (b, broken)
             at += n
+
+
+@pytest.mark.parametrize("D,E", [(64, 64), (128, 64), (128, 128), (64, 256), (256, 64), (256, 128)])
+@pytest.mark.parametrize("H", [2, 32, 96])
+@pytest.mark.parametrize("new,past", [([1, 33, 129, 300], [700, 0, 95, 900]), ([96, 65, 31, 1, 64, 96, 80], [0] * 7)])
+@pytest.mark.parametrize("window", [0, 300])
+@pytest.mark.parametrize("dt,bs", [(torch.float32, 32), (torch.bfloat16, 64), (torch.bfloat16, 16)])
+def test_long_and_short_walks(D, E, H, new, past, window, dt, bs):
+    if dt == torch.float32 and max(D, E) > 128:
+        pytest.skip("float rows of more than 128 have another kernel")
+    g = torch.Generator().manual_seed(D + E + H)
+    G, total = 2, [n + p for n, p in zip(new, past)]
+    pages = [-(-n // bs) for n in total]
+    perm, tables, at = torch.randperm(sum(pages), generator=g).int(), torch.zeros(len(new), max(pages), dtype=torch.int32), 0
+    for b, n in enumerate(pages):
+        tables[b, :n] = perm[at:at + n]
+        at += n
+    kc, vc = (torch.randn(sum(pages), bs, G, n, generator=g).to(dt).cuda() for n in (D, E))
+    T = sum(new)
+    q, sink, scale = torch.randn(T, H, D, generator=g).to(dt).cuda(), torch.randn(H, generator=g).cuda(), D ** -0.5
+    cu, cu_k = (torch.tensor([0] + x).cumsum(0).int().cuda() for x in (new, total))
+    pos = torch.cat([torch.arange(p, p + n) for n, p in zip(new, past)]).int().cuda()
+    out = torch.full((T, H, E), 7.0, dtype=dt, device="cuda")
+    hk.sink_attention_prefill(q, kc, vc, cu, cu_k, tables.cuda(), scale, sink, None, out, positions=pos, max_q=max(new),
+                              row_seq=None, window=window)
+    at = 0
+    for b, (n, p) in enumerate(zip(new, past)):
+        rows = tables[b].long().cuda()
+        k, v = (c[rows].reshape(-1, G, c.shape[3])[:n + p] for c in (kc, vc))
+        want, got = _exact(q[at:at + n], k, v, p, scale, window, 0, sink), out[at:at + n].double()
+        # fp32 sums of up to 1200 terms and exponentials of fp32 differences; the result in its type
+        assert float((got - want).norm() / want.norm()) < (1e-6 if dt == torch.float32 else 2.0 ** -8), b
+        at += n
