@@ -490,14 +490,22 @@ def _delta_next_sizes(H, G, D, E, taps) -> bool:
     return bool(_next_ok(H, G, D, E, taps))
 
 
+def delta_next_pays(B: int, H: int, D: int, E: int) -> bool:
+    """Whether single next tokens of ``B`` sequences are fewer than the three calls pay for.  From 256 MB of state the card's
+    time is the state's alone, and the step's own kernel, with smaller workgroups, moves it faster; heads of small states
+    are bound by their workgroups.  One kernel / three, us, bfloat16: 16 / 8 heads of 128 x 128 64 sequences 32 / 55, 192 78 /
+    84, 256 116 / 109; 32 / 8 of them 96 81 / 82, 128 122 / 110; 16 / 8 of 64 x 64 256 44 / 53, 512 78 / 64."""
+    return B * H * D * E < 1 << 26 and B * H <= 4096
+
+
 def delta_next(proj, a, gate, sizes, conv_w, a_log, dt_bias, norm_w, conv_state, state, positions, slots, eps, out_dtype, act):
     """Single next tokens: ``delta_prepare``, ``delta_scan`` and ``gated_head_norm`` in one kernel, their sums in the same order; None where
-    it has no instance (the caller then makes the three calls).  ``proj`` [T, ..] = [q | k | v | gate | beta | decay | ..]
+    it has no instance or they are too many (``delta_next_pays``; the caller then makes the three calls).  ``proj`` [T, ..] = [q | k | v | gate | beta | decay | ..]
     with ``a`` and ``gate`` None, or [q | k | v | beta | ..] with ``a`` [T, H*D] (a decay per key channel) and ``gate`` [T, H*E]."""
     H, G, D, E = sizes
     T, C, taps = proj.shape[0], 2 * G * D + H * E, conv_w.shape[1]
-    if not (T > 0 and slots.shape[0] == T and proj.dtype == out_dtype and out_dtype in _DT and _delta_next_sizes(H, G, D, E, taps)
-            and proj.stride(1) == 1 and conv_w.shape[0] == C and state.data_ptr() % 16 == 0):
+    if not (T > 0 and slots.shape[0] == T and proj.dtype == out_dtype and out_dtype in _DT and delta_next_pays(T, H, D, E)
+            and _delta_next_sizes(H, G, D, E, taps) and proj.stride(1) == 1 and conv_w.shape[0] == C and state.data_ptr() % 16 == 0):
         return None
     base, row, es = proj.data_ptr(), proj.stride(0), proj.element_size()
     if a is None:

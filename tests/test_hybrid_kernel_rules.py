@@ -82,3 +82,12 @@ def test_prompt_attention_groups(D, E, keys, workgroups, groups):
     (1 << 30, 1 << 20, 0, 0, 0, 1 << 30)])
 def test_longest_walk(blocks, size, window, keep, chunk, walk):
     assert hk._longest_walk(blocks, size, window, keep, chunk) == walk
+
+
+@pytest.mark.parametrize("B,H,D,E,one", [
+    (64, 16, 128, 128, True), (255, 16, 128, 128, True), (256, 16, 128, 128, False), (127, 32, 128, 128, True),
+    (128, 32, 128, 128, False), (512, 8, 256, 64, False), (256, 16, 64, 64, True), (257, 16, 64, 64, False),
+    (1024, 4, 48, 40, True), (1025, 4, 48, 40, False)])
+def test_next_tokens_of_the_delta_rule(B, H, D, E, one):
+    """One kernel up to 256 MB of state and 4096 heads, the three calls beyond."""
+    assert hk.delta_next_pays(B, H, D, E) is one
