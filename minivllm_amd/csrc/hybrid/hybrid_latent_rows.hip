@@ -9,7 +9,7 @@
 // chain load -> LDS -> product -> store of one workgroup, and with it by how many kernels stand behind each other.  As
 // two library products, rotation and store, attention and merge (five kernels, 12 us of the host each for the library's two),
 // one token with 432 keys, 16 heads, R 128: 88 us a call,
-// 30 of them on the card; now 27 (the limits: LATENT_ROWS in ops/hip_hybrid.py).
+// 30 of them on the card; now 27 (the limits: latent_rows_pay in ops/hip_hybrid.py).
 #include "hybrid_chunks.h"
 #include "hybrid_latent.h"
 #include "hybrid_latent_turn.h"

@@ -920,22 +920,33 @@ def latent_attention_decode(q_abs, q_rot, k_cache, block_tables, context_lens, s
                    B, 1, window, latent_splits(B, H, R, max_context_len, window))
 
 
-# Rows times rank up to which few rows pay against the library's two products and the calls around them, which take 83
-# to 90 us whatever the step (this / those, us, 16 heads): R 512 8 portions of 64 50 / 82, one of 500 75 / 86, 8 of 128 82 /
-# 84, one of 1000 132 / 105; R 256 8 of 128 46 / 85, one of 1000 85 / 88, of 2000 156 / 134; R 128 one of 1000 65 / 83, of
-# 2000 113 / 113, 8 of 500 92 / 84.  Single next tokens: one of 432 keys 30 / 88, 64 of 1000 51 / 88, 128 of 500 54 / 93.
+# Up to where few rows pay against the library's two products and the calls around them, which take 80 to 90 us
+# until the card is full: by the rows of the caches and of the weights that a workgroup walks (rows times rank), and by the
+# products (rows times rank times heads; single next tokens are split over their contexts, with sums to be joined, and
+# fill the card sooner).  This / those, us:
+#   16 heads: R 512 8 portions of 64 53 / 88, of 128 82 / 83, one of 200 58 / 84, of 500 108 / 105; R 256 8 of 128 50 / 84,
+#   one of 1000 124 / 125, of 2000 225 / 208; R 128 one of 1000 71 / 84, of 2000 119 / 120
+#   64 heads: R 512 8 portions of 16 53 / 87, one of 200 109 / 89, 64 of 8 130 / 82; R 256 2 of 128 53 / 90, 8 of 128 109 / 83;
+#   R 128 64 of 8 39 / 80, one of 1000 114 / 102; 128 heads, R 512: one of 64 67 / 87, 8 of 16 96 / 85
+#   single next tokens, 512 keys each: 16 heads, R 512 one 29 / 79, 64 45 / 83, 256 56 / 80; 128 heads, R 512 32 84 / 88, 64
+#   135 / 101, R 256 64 69 / 90, 128 101 / 99; 64 heads, R 512 64 79 / 89, 256 134 / 104
 LATENT_ROWS = 1 << 18
+
+
+def latent_rows_pay(T: int, H: int, R: int, prompts: bool) -> bool:
+    """Whether ``T`` rows are few enough for ``latent_rows``."""
+    return T * R <= LATENT_ROWS and T * R * H <= (5 << 20 if prompts else 3 << 20)
 
 
 def latent_rows(q, dkv, norm_w, eps, positions, inv_freq, rot_dims, neighbours, mult, k_cache, slot_mapping, up_k, up_v,
                 block_tables, cu_q, lens, scale, sink, max_q, max_context_len, window=0):
     """A step of few rows from its projections to [T, H, E], in the latents' coordinates, in one call: prompt portions
     (``cu_q``, ``max_q``) or single next tokens (``lens``).  None where the calls are to be made one by one: beyond
-    ``LATENT_ROWS`` (rows times rank), other types than bfloat16, sizes or addresses that are no whole runs of eight."""
+    ``latent_rows_pay``, other types than bfloat16, sizes or addresses that are no whole runs of eight."""
     T, H, width = q.shape
     _, D, R = up_k.shape
     E, P = up_v.shape[2], width - D
-    if T * R > LATENT_ROWS or T == 0 or q.dtype != torch.bfloat16 or not _latr_ok(H, D, P, R, E, int(rot_dims), int(neighbours)):
+    if not latent_rows_pay(T, H, R, cu_q is not None) or T == 0 or q.dtype != torch.bfloat16 or not _latr_ok(H, D, P, R, E, int(rot_dims), int(neighbours)):
         return None
     if k_cache is None or any(t.dtype != torch.bfloat16 for t in (dkv, up_k, up_v, k_cache)) or dkv.shape[1] != R + P \
             or slot_mapping is None or block_tables is None:

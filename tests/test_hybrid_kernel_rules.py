@@ -91,3 +91,14 @@ def test_longest_walk(blocks, size, window, keep, chunk, walk):
 def test_next_tokens_of_the_delta_rule(B, H, D, E, one):
     """One kernel up to 256 MB of state and 4096 heads, the three calls beyond."""
     assert hk.delta_next_pays(B, H, D, E) is one
+
+
+@pytest.mark.parametrize("T,H,R,prompts,few", [
+    # rows of the caches and the weights: up to 2^18 of them times the rank, as the heads allow
+    (512, 16, 512, True, True), (513, 16, 512, True, False), (4096, 8, 64, True, True), (4097, 8, 64, True, False),
+    # ... times the heads: prompts up to 5 x 2^20, single next tokens up to 3 x 2^20
+    (160, 64, 512, True, True), (161, 64, 512, True, False), (80, 128, 512, True, True), (1200, 64, 64, True, True),
+    (96, 64, 512, False, True), (97, 64, 512, False, False), (48, 128, 512, False, True), (64, 128, 512, False, False),
+    (256, 16, 512, False, True), (1, 128, 512, False, True)])
+def test_few_rows_in_latents(T, H, R, prompts, few):
+    assert hk.latent_rows_pay(T, H, R, prompts) is few
