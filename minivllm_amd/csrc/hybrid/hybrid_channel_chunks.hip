@@ -637,15 +637,27 @@ int launch(const ChannelChunks& a, hipStream_t s) {
 
 namespace hyb {
 
-// Three kernels, of which each portion costs at least a chunk, against a token after the other.  Layer of 8 heads of 64 x
-// 128, us, chunks / tokens: 8 portions of 32 30.5 / 26.9, of 64 31.6 / 30.6, of 128 32.8 / 51.8; 64 of 17 57 / 33, of 64 74 / 78,
-// of 128 97 / 141; 128 of 64 132 / 131; 63 single tokens and one of 128 54 / 84; 255 and one of 128 132 / 101, of 512 135 / 323;
-// 511 and one of 600 304 / 393.  Without the norm inside, 16 heads of 64 x 64: 8 of 64 33.4 / 30.2, of 96 36.3 / 41.2; 32 of
-// 64 59 / 44, of 128 74 / 75; 128 of 64 194 / 144.  So `each` tokens a portion, or a longest one of as many and half
-// a token for every portion (0: not known).
-static bool channel_chunks_pay(const ChannelChunks& a, int longest) {
+// Three kernels, of which each portion costs at least a chunk, against a token after the other, by what both take on the
+// card, us: the tokens a walk as long as the longest portion and their share of the card (by rows of the outputs and by states),
+// the chunks a share by their number.  Layer of 8 heads of 64 x 128, bfloat16, with the norm, us, chunks / tokens: 8 portions of 32
+// 30.5 / 26.9, of 64 31.6 / 30.6, of 128 32.8 / 51.8; 64 of 17 57 / 33, of 64 74 / 78, of 128 97 / 141; 63 single tokens
+// and one of 128 54 / 84; 255 and one of 128 132 / 101, of 512 135 / 323.  Without it, 16 heads of 64 x 64: 8 of 96 36 / 41, 32
+// of 64 59 / 44, of 128 74 / 75, 128 of 64 194 / 144; 8 heads of 32 x 32, 256 of 64, up to 3.9 times as long.  Over 1342
+// steps of either (1 to 256 portions of 16 to 1024 tokens, 4 to 32 heads of 32 to 64 x 32 to 128, both types) the rule's way takes
+// 1.009 of the shorter one in the mean, and 1.16 of the tokens' at the most; below `each` tokens a portion and half a
+// token for every portion it was not measured, and is the tokens'.  longest 0: not known.
+static bool channel_chunks_pay(const ChannelChunks& a, int longest, int dt) {
     const long each = a.y ? 64 : 96;
-    return a.T >= each * a.B || 2L * longest >= 2 * each + a.B;
+    if (a.T < each * a.B && 2L * longest < 2 * each + a.B) return false;
+    const bool f32 = dt == 2, wide = a.E > 64;
+    const float n = longest > 0 ? (float)longest : (float)a.T / a.B, T = (float)a.T, B = (float)a.B;
+    const float columns = a.H * ((a.E + 15) / 16) / 4.f;       // in 64s
+    const float tokens = a.D <= 32 ? 12.f + .22f * n + columns * (.00027f * T + .0136f * B)
+                             : f32 ? 9.f + .25f * n + columns * (.0012f * T + .0415f * B)
+                                   : 11.f + .28f * n + columns * (.0005f * T + .009f * B);
+    const float share = f32 ? (wide ? .084f : .059f) : (wide ? .053f : .0355f);
+    const float chunks = (wide ? 29.f : 25.5f) + (a.y ? 0.f : 2.f) + share * a.H * (T / 64.f + B);
+    return chunks * 1.03f < tokens;
 }
 
 long channel_chunks_bytes(const ChannelChunks& a, int dt) {
@@ -675,14 +687,15 @@ int channel_chunks(const ChannelChunks& a, int rule, int dt, hipStream_t s) {
 extern "C" {
 
 // Bytes of workspace hyb_channel_chunks wants (0: it does not take the call).  `aligned`: v, gate and norm_w on 16 bytes,
-// v in rows of whole runs of eight, gates of four; longest: the longest portion's tokens, 0 if that is not known
+// v in rows of whole runs of eight, gates of four; longest: the longest portion's tokens, 0 if that is not known, -1 for what it
+// would want of any step of that size
 long hyb_channel_chunks_bytes(long T_, int B, int longest, int H, int D, int E, int aligned, int norm, int dt) {
     ChannelChunks a{};
     a.cu_q = (const int*)256;
     a.T = T_; a.B = B; a.H = H; a.D = D; a.E = E;
     if (!aligned) return 0;
     if (norm) a.y = (void*)256;
-    return channel_chunks_pay(a, longest) ? channel_chunks_bytes(a, dt) : 0;
+    return longest < 0 || channel_chunks_pay(a, longest, dt) ? channel_chunks_bytes(a, dt) : 0;
 }
 
 // rule 0: GLA (tau; bonus null), 1: WKV (bonus [H*D]).  y null: o [T, H, E] fp32; else y [T, H*E] of the activation type,

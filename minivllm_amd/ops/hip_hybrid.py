@@ -718,7 +718,7 @@ def _channel_chunks(rule, q, k, v, a_raw, a_bias, bonus, tau, qscale, state, cu_
     """Prompt portions in chunks side by side, None where the rows are to be walked token by token."""
     T, H, D = q.shape
     E, B = v.shape[2], slots.shape[0]
-    if T < 96 * B and 2 * longest < 192 + B:           # (the library's rule; most steps that it turns down end here)
+    if T < 96 * B and 2 * longest < 192 + B:           # (of the library's rule; most steps that it turns down end here)
         return None
     dt, v_row = _dt(q), _rows(v)
     n = _channel_bytes(T, B, longest, H, D, E, v.data_ptr() % 16 == 0 and v_row % (8 if dt == 0 else 4) == 0, False, dt)
@@ -734,9 +734,10 @@ def _channel_chunks(rule, q, k, v, a_raw, a_bias, bonus, tau, qscale, state, cu_
 
 
 def channel_scan_workspace(tokens: int, seqs: int, H: int, D: int, E: int) -> int:
-    """The most bytes ``gla_scan`` / ``wkv_scan`` take for themselves in a step of up to that many tokens and sequences."""
+    """Bytes that ``gla_scan`` / ``wkv_scan`` take at most for themselves in a step of up to that many tokens and sequences:
+    they grow with both, and steps of too few tokens for their sequences take none."""
     seqs = min(seqs, max(tokens // 64, (2 * tokens - 126) // 3))
-    return _channel_bytes(tokens, seqs, max(tokens - seqs + 1, 0), H, D, E, True, True, 0) if seqs > 0 else 0
+    return _channel_bytes(tokens, seqs, -1, H, D, E, True, True, 0) if seqs > 0 else 0
 
 
 def _check_gla(q, k, v, a_raw, a_bias, state):
@@ -775,7 +776,7 @@ def gla_norm(proj, a_raw, sizes, a_bias, tau, norm_w, state, cu_q, positions, sl
         return None
     base, row, es, n = proj.data_ptr(), _rows(proj), 2 if dt == 0 else 4, 0
     v, gate, wp = base + 2 * HD * es, base + (2 * HD + HE) * es, _f32(norm_w).data_ptr()
-    if cu_q is not None and (T >= 64 * B or 2 * (longest or 0) >= 128 + B):      # (the library's rule)
+    if cu_q is not None and (T >= 64 * B or 2 * (longest or 0) >= 128 + B):      # (of the library's rule)
         n = _channel_bytes(T, B, int(longest or 0), H, D, E, (v | gate | wp) % 16 == 0 and row % (8 if dt == 0 else 4) == 0,
                            True, dt)
     assert state.shape[1:] == (H, D, E) and a_bias.numel() == HD and norm_w.numel() in (E, HE)
