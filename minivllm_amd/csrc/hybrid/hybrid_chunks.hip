@@ -14,7 +14,8 @@
 // Two kernels.  mlstm_weights_kernel, a workgroup per (chunk, head, 128 columns), takes m' of a chunk that begins with m =
 // -inf, and so depends on no state: A' = (Q K^T) o W', A' V, the sums of A', W'_end.  With F_t = f_1 + .. + f_t, where the chunk
 // follows a maximum m it is m_t = max(m + F_t, m'_t), c_t = e^(m + F_t - m_t) and W = e^(m'_t - m_t) W', one of the two
-// factors being 1.  mlstm_chunks_kernel, a workgroup per (sequence, head, 32 state columns), walks the chunks.
+// factors being 1.  mlstm_chunks_kernel, a workgroup per (sequence, head, 32 state columns), walks the chunks.  Many small heads
+// in bfloat16 are one kernel's, mlstm_whole_kernel.
 //
 // Every factor inside a chunk is a product of a and b, all <= 1: no quotients, no logarithms of products.  W' comes from the
 // products inside blocks of 16 tokens: in a pair of different blocks it is (a .. to t inside its block) (whole blocks between)
@@ -334,11 +335,11 @@ struct Lds {
 // second four are swapped, so that they are in the banks that the first four leave.
 __device__ __forceinline__ int wv_at(int row, int byte) { return row * (EB * 2) + (byte ^ (row << 2 & 32)); }
 
-// The portion's tokens one after the other: thread = a column and a 32nd of the channels, sums through LDS
-// (`red`: 16 KB).
-template <typename T, int DP>
+// The portion's tokens one after the other: thread = a column and a GROUPS-th of the channels, sums through LDS
+// (`red`: 16 bytes a thread).
+template <typename T, int DP, int THREADS>
 __device__ __forceinline__ void walk_tokens(const MlstmChunks a, float* red) {
-    constexpr int CH = DP / 32;
+    constexpr int GROUPS = THREADS / 32, CH = DP / GROUPS;
     const int b = blockIdx.x, h = blockIdx.y, e0 = blockIdx.z * EB, slot = a.slots[b];
     const long first = a.cu_q[b];
     const int n = a.cu_q[b + 1] - (int)first;
@@ -372,15 +373,15 @@ __device__ __forceinline__ void walk_tokens(const MlstmChunks a, float* red) {
             N[i] = fs * N[i] + is * k;
             pn += N[i] * q;
         }
-        float* at = red + (x & 1) * 2048;              // two of them: one barrier per token
+        float* at = red + (x & 1) * (2 * THREADS);              // two of them: one barrier per token
         at[r * 32 + c] = po;
-        at[1024 + r * 32 + c] = pn;
+        at[THREADS + r * 32 + c] = pn;
         __syncthreads();
         if (r == 0 && e < E) {
             po = pn = 0.f;
-            for (int i = 0; i < 32; ++i) {
+            for (int i = 0; i < GROUPS; ++i) {
                 po += at[i * 32 + c];
-                pn += at[1024 + i * 32 + c];
+                pn += at[THREADS + i * 32 + c];
             }
             a.o[(t * H + h) * (long)E + e] = po / (fmaxf(fabsf(pn), expf(-m)) + 1e-6f);
         }
@@ -643,7 +644,7 @@ mlstm_chunks_kernel(MlstmChunks a) {
     if (lost) {
         __threadfence();                                    // (the outputs are written again, by other waves)
         __syncthreads();
-        walk_tokens<T, DP>(arguments_anew<MlstmChunks>(), reinterpret_cast<float*>(smem));
+        walk_tokens<T, DP, 1024>(arguments_anew<MlstmChunks>(), reinterpret_cast<float*>(smem));
         return;
     }
     // ---- the state after the portion
@@ -663,6 +664,332 @@ mlstm_chunks_kernel(MlstmChunks a) {
 #endif
 }
 
+// ---- All of a portion in one kernel, for bfloat16 heads of up to 64 channels (`whole` has when): every workgroup of 32 columns
+// works the weights out for itself, in eight waves that both keep the state and form the outputs, but two of it share a CU,
+// which the walk above, with 16 waves of 82 registers, has to itself (at 64 registers it spills: 64 portions of 64, 16 heads of
+// 64 x 64, 63 us; this 52).  Bound by the vector instructions around the products.
+// per token of a chunk, in LDS
+struct Gates {
+    alignas(16) float a[C], b[C];          // decay, input
+    alignas(16) float bs[C];               // b times the decays behind the token inside its block of 16
+    float pre[C];              // the decays up to the token inside its block
+    float c[C];                // ... from the chunk's start
+    float wl[C];               // W_end
+    float em[C];               // e^(-m)
+    float blk[4];              // a block's decays
+    alignas(16) uint16_t wp[3][C];         // wl in three parts
+};
+
+struct WholeLds {
+    static constexpr int DP = 64;
+    char q[C * DP * 2], k[C * DP * 2];     // images (rows16) of the chunk's rows
+    char v[C * EB * 2];                    // rows of 64 bytes, halves swapped where v_at says so
+    char wv[3][C * EB * 2];                // W_end v in three parts, likewise
+    char s[3][EB * DP * 2];                // the state's parts, a row per state column
+    char n[3][DP * 2];                     // the normaliser's parts
+    Gates g;
+    int lost;                              // an output or a state is not finite
+};
+
+// Place of a byte of a row of v (wv).  Transposed reads take 32 bytes of rows 0-7 (of 0-3 and 8-11): the halves of the
+// second four are swapped, so that they are in the banks that the first four leave.
+__device__ __forceinline__ int v_at(int row, int byte) { return row * (EB * 2) + (byte ^ (row << 3 & 32)); }
+__global__ void __launch_bounds__(512, 4)                   // (two workgroups on a CU)
+mlstm_whole_kernel(MlstmChunks a) {
+#ifdef __HIP_DEVICE_COMPILE__       // (the host pass only needs the launch stub)
+    constexpr int DP = 64, KS = DP / 32;           // key channels; steps over them
+    static_assert(C * DP / 8 == 512);              // a piece of 16 bytes of a q (or k) image per thread
+    extern __shared__ __attribute__((aligned(256))) char smem[];
+    WholeLds& L = *reinterpret_cast<WholeLds*>(smem);
+    const int b = blockIdx.x, h = blockIdx.y, e0 = blockIdx.z * EB;
+    const int H = a.H, D = a.D, E = a.E;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tb = wave & 3, et = wave >> 2;       // this wave's queries and channels; its 16 state columns
+    const int l16 = lane & 15, q4 = lane >> 4;
+    const int slot = a.slots[b];
+    const long first = a.cu_q[b];
+    const int n = a.cu_q[b + 1] - (int)first;
+    clear_unowned(a.o, a.cu_q, a.slots, b, gridDim.x, a.T, H, h, E, e0, EB);
+    if (slot < 0 || n <= 0) return;
+    const bool has_past = a.positions[first] > 0;
+    const int ZG = (E + 15) / 16;
+
+    // ---- the state: S holds channels 16 tb + 4 q4 + r of column e, the first column of N a channel's normaliser (the waves of
+    // the first 16 columns keep it)
+    const int e = e0 + 16 * et + l16;
+    f32x4 S, N;
+    float* sp = a.state + ((long)slot * H + h) * D * E;
+    float* np = a.nstate + (((long)slot * H + h) * ZG + e0 / 16) * D;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int d = 16 * tb + 4 * q4 + r;
+        S[r] = has_past && d < D && e < E ? sp[(long)d * E + e] : 0.f;
+        N[r] = has_past && d < D && l16 == 0 ? np[d] : 0.f;
+    }
+    float m_run = has_past ? a.mstate[((long)slot * H + h) * ZG + e0 / 16] : 0.f;
+
+    // ---- the next chunk on its way: rows behind the portion and columns behind a head are out of the
+    // buffers' range and read as zeros
+    uint4 qr, kr;
+    uint2 vr;
+    float gi = 0.f, gf = 0.f;
+    const int row = tid / (DP / 8), piece = tid % (DP / 8), d = piece * 8;
+    const int q_off = d < D ? (row * (int)a.q_row + d) * 2 : NOWHERE, k_off = d < D ? (row * (int)a.k_row + d) * 2 : NOWHERE;
+    const int v_off = e0 + (tid & 7) * 4 < E ? ((tid >> 3) * (int)a.v_row + (tid & 7) * 4) * 2 : NOWHERE;
+    constexpr int GATES = 4;                       // the wave that works the gates out (few key blocks, no N)
+    auto fetch = [&](int ch) {
+        const int nt = min(C, n - ch * C);
+        const long t0 = first + (long)ch * C;
+        const __amdgpu_buffer_rsrc_t qb = rows_of<bf16_t>(a.q, t0 * a.q_row + h * D, a.q_row, nt, D);
+        const __amdgpu_buffer_rsrc_t kb = rows_of<bf16_t>(a.k, t0 * a.k_row + h * D, a.k_row, nt, D);
+        const __amdgpu_buffer_rsrc_t vb = rows_of<bf16_t>(a.v, t0 * a.v_row + (long)h * E + e0, a.v_row, nt, E - e0);
+        qr = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(qb, q_off, 0, 0));
+        kr = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(kb, k_off, 0, 0));
+        vr = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(vb, v_off, 0, 0));
+        if (wave == GATES) {
+            const long t = t0 + min(lane, nt - 1);
+            gi = ld((const bf16_t*)a.gi + t * a.g_row + h);
+            gf = ld((const bf16_t*)a.gf + t * a.g_row + h);
+        }
+    };
+    const float bi = a.bi[h], bf = a.bf[h];
+    struct { float a, b, bs, pre, c, wl, em; } G;
+    // the factors of every token of the chunk fetched last (lane = token)
+    auto gates = [&](int ch) {
+        const bool ok = lane < min(C, n - ch * C);             // tokens behind the portion change nothing
+        const float i = ok ? a.cap * tanhf((gi + bi) / a.cap) : NEG_INF;
+        const float f = ok ? logsigmoid_(a.cap * tanhf((gf + bf) / a.cap)) : 0.f;
+        float F = f, M = i;                                    // inclusive scan of (sum of f, max), 16 tokens at a time
+        static_for<0, 4>([&](auto dc) {
+            constexpr int d = 1 << decltype(dc)::value;
+            M = fmaxf(M, from_left<d>(M, NEG_INF) + F);
+            F += from_left<d>(F, 0.f);
+        });
+        float before = m_run, m0 = m_run;                      // the maximum ahead of this lane's block
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (k == q4) m0 = before;
+            before = fmaxf(lane_of(M, 16 * k + 15), before + lane_of(F, 16 * k + 15));
+        }
+        m_run = before;
+        const float m = fmaxf(M, m0 + F), mp = from_left<1>(m, m0);
+        // (of the difference that decides the maximum, as in the recurrence, and not of m, whose own rounding would
+        // come on top; not by fminf, which would lose a NaN)
+        const float x = f + mp - i;
+        const float fa = ok ? expf(x >= 0.f ? 0.f : x) : 1.f, fb = ok ? expf(x <= 0.f ? 0.f : -x) : 0.f;
+        float pre = fa, suf = fa;
+        static_for<0, 4>([&](auto dc) {
+            constexpr int d = 1 << decltype(dc)::value;
+            pre *= from_left<d>(pre, 1.f);
+            suf *= from_right<d>(suf, 1.f);
+        });
+        suf = from_right<1>(suf, 1.f);
+        float ahead = 1.f, behind = 1.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float bk = lane_of(pre, 16 * k + 15);
+            if (k < q4) ahead *= bk;
+            if (k > q4) behind *= bk;
+        }
+        G.a = fa; G.b = fb; G.bs = fb * suf; G.pre = pre; G.c = pre * ahead; G.wl = fb * suf * behind;
+        G.em = expf(-m);
+    };
+    auto publish_gates = [&]() {
+        Gates& g = L.g;
+        g.a[lane] = G.a;
+        g.b[lane] = G.b;
+        g.bs[lane] = G.bs;
+        g.pre[lane] = G.pre;
+        g.c[lane] = G.c;
+        g.wl[lane] = G.wl;
+        g.em[lane] = G.em;
+        if (l16 == 15) g.blk[q4] = G.pre;
+        float x = G.wl, y = 0.f;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const uint32_t w = rounded(x, y);
+            g.wp[k][lane] = (uint16_t)w;
+            rest(w, x, y);
+        }
+    };
+    // what was fetched last into LDS
+    auto stash = [&]() {
+        const int at = row * DP * 2 + ((piece ^ rows16<DP>(row)) << 4);
+        *reinterpret_cast<uint4*>(L.q + at) = qr;
+        *reinterpret_cast<uint4*>(L.k + at) = kr;
+        *reinterpret_cast<uint2*>(L.v + v_at(tid >> 3, (tid & 7) * 8)) = vr;
+    };
+    // the state's parts: a row per column of the state
+    auto publish = [&]() {
+        const int d = 16 * tb + 4 * q4, row = 16 * et + l16;
+        put_parts(S, [&](int k) { return L.s[k] + row * DP * 2 + (((d >> 3) ^ rows16<DP>(row)) << 4) + (d & 4) * 2; });
+        if (et == 0 && l16 == 0) put_parts(N, [&](int k) { return L.n[k] + d * 2; });
+    };
+
+    const int nchunks = (n + C - 1) / C;
+    float seen = 0.f;                              // the sum of all outputs and states: finite if they are
+    if (tid == 0) L.lost = 0;
+    fetch(0);
+    if (wave == GATES) {
+        gates(0);
+        publish_gates();
+    }
+    stash();
+    publish();
+    __syncthreads();
+    for (int ch = 0; ch < nchunks; ++ch) {
+        const Gates& g = L.g;
+        if (ch + 1 < nchunks) fetch(ch + 1);
+        {   // W_end v, four columns of a token per thread
+            const uint2 raw = *reinterpret_cast<const uint2*>(L.v + v_at(tid >> 3, (tid & 7) * 8));
+            const float w = g.wl[tid >> 3];
+            const f32x4 x = {w * __uint_as_float(raw.x << 16), w * __uint_as_float(raw.x & 0xffff0000u),
+                             w * __uint_as_float(raw.y << 16), w * __uint_as_float(raw.y & 0xffff0000u)};
+            put_parts(x, [&](int k) { return L.wv[k] + wv_at(tid >> 3, (tid & 7) * 8); });
+        }
+        // ---- this wave's 16 queries: t = 16 tb + l16
+        const int t = 16 * tb + l16, left = n - ch * C;
+        if (16 * tb < left) {
+        bf16x8 qf[KS];
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            qf[s] = *reinterpret_cast<const bf16x8*>(L.q + t * DP * 2 + (((4 * s + q4) ^ rows16<DP>(t)) << 4));
+        f32x4 O = {0.f, 0.f, 0.f, 0.f}, O1 = O, O2 = O, nq = O;
+        {
+            const int row = 16 * et + l16;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const int at = row * DP * 2 + (((4 * s + q4) ^ rows16<DP>(row)) << 4);
+                O2 = mfma(*reinterpret_cast<const bf16x8*>(L.s[2] + at), qf[s], O2);
+                O1 = mfma(*reinterpret_cast<const bf16x8*>(L.s[1] + at), qf[s], O1);
+                O = mfma(*reinterpret_cast<const bf16x8*>(L.s[0] + at), qf[s], O);
+                nq = mfma(*reinterpret_cast<const bf16x8*>(L.n[min(l16, 2)] + (4 * s + q4) * 16), qf[s], nq);
+            }
+        }
+        const float ct = g.c[t] * a.qscale;
+        O = (O + (O1 + O2)) * ct;
+        float den = __shfl(nq[0] + (nq[1] + nq[2]), l16, kWave) * ct;         // rows 0 .. 2 lie in lanes 0 .. 15
+        float sum = 0.f, mid = 1.f;
+        // key blocks from the diagonal down, two of 16 per step of the value product
+        const float pre = g.pre[t] * a.qscale;
+        auto weighted = [&](int kb, float* x) {                               // x[r]: key 16 kb + 4 q4 + r
+            f32x4 s = {0.f, 0.f, 0.f, 0.f};
+            const int row = 16 * kb + l16;
+#pragma unroll
+            for (int i = 0; i < KS; ++i)
+                s = mfma(*reinterpret_cast<const bf16x8*>(L.k + row * DP * 2 + (((4 * i + q4) ^ rows16<DP>(row)) << 4)), qf[i], s);
+            float w[4];
+            if (kb == tb) {
+                const int i3 = 4 * q4 + 3;
+                float ga[16];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float4 x4 = reinterpret_cast<const float4*>(g.a + 16 * kb)[j];
+                    ga[4 * j] = x4.x; ga[4 * j + 1] = x4.y; ga[4 * j + 2] = x4.z; ga[4 * j + 3] = x4.w;
+                }
+                float p = 1.f;
+#pragma unroll
+                for (int j = 4; j < 16; ++j) p *= ((j > i3) & (j <= l16)) ? ga[j] : 1.f;
+                const float4 a4 = reinterpret_cast<const float4*>(g.a + 16 * kb)[q4];
+                const float4 b4 = reinterpret_cast<const float4*>(g.b + 16 * kb)[q4];
+                const float ar[4] = {a4.x, a4.y, a4.z, a4.w}, br[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+                for (int r = 3; r >= 0; --r) {
+                    const bool seen = 4 * q4 + r <= l16;
+                    w[r] = seen ? br[r] * p * a.qscale : 0.f;
+                    p *= seen ? ar[r] : 1.f;
+                }
+            } else {
+                const float f = pre * mid;
+                const float4 b4 = reinterpret_cast<const float4*>(g.bs + 16 * kb)[q4];
+                w[0] = f * b4.x; w[1] = f * b4.y; w[2] = f * b4.z; w[3] = f * b4.w;
+                mid *= g.blk[kb];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                x[r] = s[r] * w[r];
+                sum += x[r];
+            }
+        };
+        for (int s = tb >> 1; s >= 0; --s) {
+            float x[8];
+            if (2 * s + 1 <= tb) weighted(2 * s + 1, x + 4);
+            else { x[4] = 0.f; x[5] = 0.f; x[6] = 0.f; x[7] = 0.f; }
+            weighted(2 * s, x);
+            bf16x8 p[3];
+            split8(x, p);
+            const char* at = L.v + v_at(32 * s + 4 * q4 + (l16 >> 2), et * 32 + (l16 & 3) * 8);
+            const bf16x8 vf = join(read_tr(at), read_tr(at + 16 * EB * 2));
+#pragma unroll
+            for (int k = 2; k >= 0; --k) O = mfma(vf, p[k], O);
+        }
+        sum += __shfl_xor(sum, 16, kWave);
+        sum += __shfl_xor(sum, 32, kWave);
+        den = 1.f / (fmaxf(fabsf(den + sum), g.em[t]) + 1e-6f);
+        O *= den;
+        if (t < left && e0 + 16 * et + 4 * q4 < E)
+            *reinterpret_cast<f32x4*>(a.o + ((first + ch * C + t) * H + h) * (long)E + e0 + 16 * et + 4 * q4) = O;
+        seen += (O[0] + O[1]) + (O[2] + O[3]);              // (zeros behind the portion, as q is)
+        }
+        if (wave == GATES && ch + 1 < nchunks) gates(ch + 1);
+        __syncthreads();                                    // W_end v is there
+        const float ce = g.c[C - 1];
+        f32x4 n = {0.f, 0.f, 0.f, 0.f};                     // the chunk's, a column for each part of W_end
+        S *= ce;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int row = 32 * s + 8 * q4 + (l16 >> 2), piece = 2 * tb + ((l16 & 3) >> 1);
+            bf16x8 wf[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const char* at = L.wv[k] + wv_at(row, et * 32 + (l16 & 3) * 8);
+                wf[k] = join(read_tr(at), read_tr(at + 4 * EB * 2));
+            }
+            const bf16x8 kf = join(read_tr(L.k + row * DP * 2 + ((piece ^ rows16<DP>(row)) << 4) + (l16 & 1) * 8),
+                                   read_tr(L.k + (row + 4) * DP * 2 + ((piece ^ rows16<DP>(row + 4)) << 4) + (l16 & 1) * 8));
+#pragma unroll
+            for (int k = 2; k >= 0; --k) S = mfma(kf, wf[k], S);
+            if (et == 0) n = mfma(kf, *reinterpret_cast<const bf16x8*>(&g.wp[min(l16, 2)][32 * s + 8 * q4]), n);
+        }
+        if (et == 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {                   // (what the first sum rounds off goes with the small ones)
+                const float x = fmaf(N[r], ce, n[r]), off = fmaf(N[r], ce, n[r] - x);
+                N[r] = x + (off + (from_right<1>(n[r], 0.f) + from_right<2>(n[r], 0.f)));
+            }
+        }
+        if (ch + 1 < nchunks) {
+            __syncthreads();                                // everybody has read this chunk's images
+            if (wave == GATES) publish_gates();
+            stash();
+            publish();
+            __syncthreads();
+        }
+    }
+    seen += (S[0] + S[1]) + (S[2] + S[3]);
+    if (et == 0 && l16 == 0) seen += (N[0] + N[1]) + (N[2] + N[3]);
+    if (seen * 0.f != 0.f) L.lost = 1;
+    __syncthreads();
+    if (L.lost) {
+        __threadfence();                                    // (the outputs are written again, by other waves)
+        __syncthreads();
+        walk_tokens<bf16_t, DP, 512>(arguments_anew<MlstmChunks>(), reinterpret_cast<float*>(smem));
+        return;
+    }
+    // ---- the state after the portion
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int d = 16 * tb + 4 * q4 + r;
+        if (d < D && e < E) sp[(long)d * E + e] = S[r];
+        if (et == 0 && l16 == 0 && d < D) {
+            np[d] = N[r];
+            if (e0 / 16 + 1 < ZG) np[D + d] = N[r];
+        }
+    }
+    if (wave == GATES && lane < 2 && e0 / 16 + lane < ZG) a.mstate[((long)slot * H + h) * ZG + e0 / 16 + lane] = m_run;
+#endif
+}
+
 template <typename T, int DP>
 int launch(const MlstmChunks& a, int B, hipStream_t s) {
     constexpr int NP = sizeof(T) == 2 ? 1 : 3, images = sizeof(Lds<DP, NP>), lds = images <= 56 * 1024 ? 2 * images : images;
@@ -677,6 +1004,17 @@ int launch(const MlstmChunks& a, int B, hipStream_t s) {
     hipLaunchKernelGGL((mlstm_chunks_kernel<T, DP>), dim3(B, a.H, (a.E + EB - 1) / EB), dim3(1024), lds, s, a);
     return HYB_LAUNCH_OK();
 }
+
+int launch_whole(const MlstmChunks& a, hipStream_t s) {
+    static_assert(sizeof(WholeLds) <= 64 * 1024);
+    hipLaunchKernelGGL(mlstm_whole_kernel, dim3(a.B, a.H, (a.E + EB - 1) / EB), dim3(512), sizeof(WholeLds), s, a);
+    return HYB_LAUNCH_OK();
+}
+
+// Whether one kernel does it all: where the walks are more than the CUs.  bfloat16, us, one / two kernels: 4 heads of 64 x 256
+// (32 walks a sequence) 16 portions of 100 24 / 31, of 256 36 / 44, 64 of 32 42 / 50, of 128 72 / 74; 16 heads of 64 x 64 16 of
+// 512 59 / 71, 64 of 64 52 / 66; 256 of 32, 4 heads of 48 x 40 40 / 49.  256 walks: 8 of 512, 16 heads of 64 x 64 47 / 41.
+bool whole(const MlstmChunks& a, int dt) { return dt == 0 && a.D <= 64 && (long)a.B * a.H * ((a.E + EB - 1) / EB) > 256; }
 
 }  // namespace
 
@@ -694,10 +1032,11 @@ long mlstm_chunks_bytes(const MlstmChunks& a, int dt) {
     for (long row : {a.q_row, a.k_row, a.v_row})
         if (row % (dt == 0 ? 8 : 4) || row < 0 || row >= (dt == 0 ? 1 << 23 : 1 << 22)) return 0;      // (64 rows are addressed in 31 bits)
     if ((long)a.H * a.E >= 1 << 22) return 0;
-    return (a.T / C + B) * (long)a.H * (long)sizeof(Slot);
+    return whole(a, dt) ? 256 : (a.T / C + B) * (long)a.H * (long)sizeof(Slot);
 }
 
 int mlstm_chunks(const MlstmChunks& a, int dt, hipStream_t s) {
+    if (whole(a, dt)) return launch_whole(a, s);
     if (dt == 0) return a.D <= 64 ? launch<bf16_t, 64>(a, a.B, s) : launch<bf16_t, 128>(a, a.B, s);
     return a.D <= 64 ? launch<float, 64>(a, a.B, s) : launch<float, 128>(a, a.B, s);
 }

@@ -67,7 +67,9 @@ def _exact(proj, H, D, E, bi, bf, cap, init, cu):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 48, 40), (1, 64, 136), (2, 72, 264), (1, 8, 8)])
+@pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 48, 40), (1, 64, 136), (2, 72, 264), (1, 8, 8),
+                                   # more walks of 32 columns than CUs: bfloat16 in one kernel
+                                   (15, 48, 40), (8, 64, 136), (29, 8, 8), (16, 64, 64)])
 @pytest.mark.parametrize("gates", [1.0, 6.0])
 def test_against_exact_and_tokens(dt, H, D, E, gates):
     g = torch.Generator().manual_seed(D + E)
@@ -115,7 +117,7 @@ def test_against_exact_and_tokens(dt, H, D, E, gates):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 48, 40), (3, 20, 24), (1, 64, 136)])
+@pytest.mark.parametrize("H,D,E", [(2, 128, 128), (3, 48, 40), (3, 20, 24), (1, 64, 136), (15, 48, 40)])
 @pytest.mark.parametrize("step", ["prompts", "tokens", "one"])
 @pytest.mark.parametrize("extra", [0, 1])
 def test_rows_call_is_the_two_calls(dt, H, D, E, step, extra):
