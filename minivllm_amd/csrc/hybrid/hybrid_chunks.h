@@ -142,9 +142,11 @@ struct MlstmChunks {
     float qscale;
 };
 
-// bytes of workspace, 0 when the recurrence is to be walked token by token.  It takes portions (cu_q) that are long
-// enough, up to 128 key channels, sizes in whole runs of eight and 16-byte addresses
+// bytes of workspace, 0 where there is no such way: it takes portions (cu_q), up to 128 key channels, sizes in whole runs
+// of eight and 16-byte addresses
 long mlstm_chunks_bytes(const MlstmChunks& a, int dt);
+// whether it is the faster one; longest: the longest portion's tokens, 0 if that is not known
+bool mlstm_chunks_pay(const MlstmChunks& a, int longest, int dt);
 int mlstm_chunks(const MlstmChunks& a, int dt, hipStream_t s);
 
 struct DeltaChunks {

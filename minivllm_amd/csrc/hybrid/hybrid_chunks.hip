@@ -1011,22 +1011,44 @@ int launch_whole(const MlstmChunks& a, hipStream_t s) {
     return HYB_LAUNCH_OK();
 }
 
+long walks_of(const MlstmChunks& a) { return (long)a.B * a.H * ((a.E + EB - 1) / EB); }
+
 // Whether one kernel does it all: where the walks are more than the CUs.  bfloat16, us, one / two kernels: 4 heads of 64 x 256
 // (32 walks a sequence) 16 portions of 100 24 / 31, of 256 36 / 44, 64 of 32 42 / 50, of 128 72 / 74; 16 heads of 64 x 64 16 of
 // 512 59 / 71, 64 of 64 52 / 66; 256 of 32, 4 heads of 48 x 40 40 / 49.  256 walks: 8 of 512, 16 heads of 64 x 64 47 / 41.
-bool whole(const MlstmChunks& a, int dt) { return dt == 0 && a.D <= 64 && (long)a.B * a.H * ((a.E + EB - 1) / EB) > 256; }
+bool whole(const MlstmChunks& a, int dt) { return dt == 0 && a.D <= 64 && walks_of(a) > 256; }
 
 }  // namespace
 
 namespace hyb {
 
-// A portion of a few tokens costs a whole chunk, so the rows must make up for the sequences: ten per sequence, or a thousand
-// beyond the first of each, as with a prompt next to many single tokens, which are walked in 0.5 us each.  Layer of 8 heads of
-// 128, us, chunks / tokens, bfloat16: 64 portions of 10 54 / 50, of 16 56 / 83, of 32 60 / 120, of 128 103 / 453; floats: of
-// 10 73 / 98, of 16 77 / 131, of 32 89 / 185, of 128 201 / 494.  (Up to 8 portions of 64 the call itself takes longer, 26 us.)
+// A portion of a few tokens costs a whole chunk, so the rows must make up for the portions: by the walks (workgroups of
+// mlstm_chunks_kernel), as few of either way take a call's 21 to 26 us and a token 0.3 us of it, and by how fast either way
+// is.  Or one portion is long beside many short ones, and walked at 0.6 us a token.  us, chunks / tokens:
+//   64 < D, bfloat16: 32 walks 24 tokens a portion 27 / 25, 32 26 / 28; 256 16 27 / 22, 24 27 / 28; 512 12 27 / 24, 16 26 / 26; 1024 10 35 /
+//   37; 4096 10 97 / 124; 8192 8 178 / 214; floats: 32 walks 16 26 / 26, 24 26 / 31; 256 12 26 / 25, 16 26 / 28; 512 10 32 / 32; 1024
+//   10 46 / 56; 8192 8 245 / 346
+//   up to 64, bfloat16: 256 walks 32 27 / 26, 48 26 / 33; 512 16 24 / 21, 24 24 / 26; 1024 16 25 / 24, 24 26 / 32; 2048 12 38 / 35, 16
+//   38 / 39; 8192 16 121 / 127; floats: 128 32 28 / 25, 48 26 / 33; 512 24 26 / 28; 1024 24 38 / 33, 32 38 / 38; 4096 16 106 / 84, 24 109 / 110
+//   one portion beside single tokens: 255 of these, 8 heads of 128 x 128, bfloat16, one of 64 176 / 235, of 256 198 / 597; 127 and 4
+//   of 48 x 40 one of 64 24 / 53, of 1024 81 / 666; 255 and 16 of 64 x 64, floats, one of 96 197 / 144, of 1024 329 / 794
+static long tokens_that_pay(const MlstmChunks& a, int dt) {
+    const long walks = walks_of(a);
+    if (a.D > 64) {
+        if (walks >= 512) return walks >= 4096 ? 8 : walks >= 1024 || dt == 2 ? 10 : 16;
+        return dt == 2 ? (walks >= 256 ? 16 : 24) : (walks >= 256 ? 24 : 32);
+    }
+    if (dt == 2) return walks >= 256 ? 32 : 40;
+    return walks > 1024 ? 16 : walks > 256 ? 24 : 40;
+}
+
+bool mlstm_chunks_pay(const MlstmChunks& a, int longest, int dt) {
+    const long walks = walks_of(a), alone = 40 + walks / (dt == 2 && a.D <= 64 ? 64 : 200);
+    return a.T >= tokens_that_pay(a, dt) * a.B || (longest > 0 ? longest >= alone : a.T - a.B >= 1024);
+}
+
 long mlstm_chunks_bytes(const MlstmChunks& a, int dt) {
     const int B = a.B;
-    if (a.T < 10L * B && a.T - B < 1024) return 0;
     if (!a.cu_q || B <= 0 || a.D < 8 || a.D > 128 || a.D % 8 || a.E % 8 || a.H > 65535 || (dt != 0 && dt != 2)) return 0;
     if (((size_t)a.q | (size_t)a.k | (size_t)a.v) % 16) return 0;
     for (long row : {a.q_row, a.k_row, a.v_row})

@@ -589,14 +589,15 @@ int hyb_wkv_scan(const void* r, const void* k, const void* v, long r_row, long k
     return 1;
 }
 
-// Bytes of workspace with which hyb_mlstm_scan takes prompt portions in chunks; 0: none, token by token
+// Bytes of workspace with which hyb_mlstm_scan takes prompt portions in chunks; 0: none, token by token.  longest: the longest
+// portion's tokens, 0 if that is not known, -1 for what it would want of any step of that size
 long hyb_mlstm_chunks_bytes(const void* q, const void* k, const void* v, long q_row, long k_row, long v_row, long T_, int B,
-                            int H, int D, int E, int dt) {
+                            int longest, int H, int D, int E, int dt) {
     MlstmChunks c{};
     c.q = q; c.k = k; c.v = v; c.q_row = q_row; c.k_row = k_row; c.v_row = v_row;
     c.cu_q = (const int*)256;
     c.T = T_; c.B = B; c.H = H; c.D = D; c.E = E;
-    return mlstm_chunks_bytes(c, dt);
+    return B > 0 && (longest < 0 || mlstm_chunks_pay(c, longest, dt)) ? mlstm_chunks_bytes(c, dt) : 0;
 }
 
 // gi, gf [T, H] raw gate projections (activation type, element stride g_row); nstate

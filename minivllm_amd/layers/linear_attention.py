@@ -82,14 +82,15 @@ class MatrixLSTM(nn.Module):
             raise RuntimeError("the matrix memory needs allocated state slots")
         T = proj.shape[0]
         H, D, E = self.num_heads, self.head_dim, self.v_head_dim
-        lay = _layout(get_context())
+        ctx = get_context()
+        lay = _layout(ctx)
         y = ops.mlstm_norm(proj, (H, D, E), self.i_bias, self.f_bias, self.gate_cap, self.norm_weight, self.state,
-                           self.norm_state, self.max_state, *lay, self.eps, out_dtype)
+                           self.norm_state, self.max_state, *lay, self.eps, out_dtype, ctx.max_seqlen_q)
         if y is not None:
             return y
         q, k, v, gate, ig, fg = proj.split(self.split_sizes(), dim=-1)
         o = ops.mlstm_scan(q.view(T, H, D), k.view(T, H, D), v.view(T, H, E), ig, fg, self.i_bias,
-                           self.f_bias, self.gate_cap, self.state, self.norm_state, self.max_state, *lay)
+                           self.f_bias, self.gate_cap, self.state, self.norm_state, self.max_state, *lay, ctx.max_seqlen_q)
         return ops.gated_head_norm(o, self.norm_weight, gate, self.eps, out_dtype,
                                    "sigmoid").view(T, H * E)
 

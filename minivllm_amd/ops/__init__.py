@@ -418,9 +418,10 @@ def tanh_cap_(z, cap):
 
 
 def mlstm_scan(q, k, v, i_raw, f_raw, i_bias, f_bias, cap, state, norm_state, max_state,
-               cu_q, positions, slots):
-    return _seqmix(q).mlstm_scan(q, k, v, i_raw, f_raw, i_bias, f_bias, cap, state, norm_state,
-                                 max_state, cu_q, positions, slots)
+               cu_q, positions, slots, longest=0):
+    """``longest``: as for ``gla_scan``."""
+    a = (q, k, v, i_raw, f_raw, i_bias, f_bias, cap, state, norm_state, max_state, cu_q, positions, slots)
+    return _hybrid().mlstm_scan(*a, longest) if _on_gpu(q) else torch_seqmix.mlstm_scan(*a)
 
 
 def gla_scan(q, k, v, a_raw, a_bias, tau, state, cu_q, positions, slots, longest=0):

@@ -71,7 +71,7 @@ _mlstm = _sig("hyb_mlstm_scan", _P, _P, _P, _L, _L, _L, _P, _P, _L, _P, _P, _F, 
               _P, _P, _L, _I, _I, _I, _I, _I, _P)
 _mlstm_rows = _sig("hyb_mlstm_rows", _P, _L, _P, _P, _F, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _F, _L, _I, _I, _I, _I, _I, _P)
 _gla_rows = _sig("hyb_gla_rows", _P, _L, _P, _L, _P, _F, _P, _P, _P, _P, _P, _P, _P, _I, _F, _L, _I, _I, _I, _I, _I, _P)
-_mlstm_bytes = bind(_lib, "hyb_mlstm_chunks_bytes", [_P, _P, _P, _L, _L, _L, _L, _I, _I, _I, _I, _I], _L)
+_mlstm_bytes = bind(_lib, "hyb_mlstm_chunks_bytes", [_P, _P, _P, _L, _L, _L, _L] + [_I] * 6, _L)
 _chan = _sig("hyb_channel_chunks", _I, _P, _P, _P, _L, _L, _L, _P, _L, _P, _P, _F, _F, _P, _P, _P, _P, _P, _P, _P, _P, _L, _P,
              _I, _F, _I, _L, _I, _I, _I, _I, _I, _P)
 _chan_bytes = bind(_lib, "hyb_channel_chunks_bytes", [_L] + [_I] * 8, _L)
@@ -657,7 +657,7 @@ def _heads_view(t, n):
 
 
 def mlstm_scan(q, k, v, i_raw, f_raw, i_bias, f_bias, cap, state, norm_state, max_state,
-               cu_q, positions, slots):
+               cu_q, positions, slots, longest=0):
     T, H, D = q.shape
     E = v.shape[2]
     ZG = (E + 15) // 16
@@ -669,7 +669,7 @@ def mlstm_scan(q, k, v, i_raw, f_raw, i_bias, f_bias, cap, state, norm_state, ma
     o = _rows_out(T, H, E, slots, q.device)
     rows, ws = (q.data_ptr(), k.data_ptr(), v.data_ptr(), _heads_view(q, D), _heads_view(k, D), _heads_view(v, E)), None
     if cu_q is not None:
-        n = _mlstm_bytes(*rows, T, slots.shape[0], H, D, E, _dt(q))
+        n = _mlstm_bytes(*rows, T, slots.shape[0], int(longest or 0), H, D, E, _dt(q))
         if n:
             ws = torch.empty((n,), dtype=torch.uint8, device=q.device)
     _check(_mlstm(*rows, i_raw.data_ptr(), f_raw.data_ptr(), _rows(i_raw),
@@ -680,7 +680,8 @@ def mlstm_scan(q, k, v, i_raw, f_raw, i_bias, f_bias, cap, state, norm_state, ma
     return o
 
 
-def mlstm_norm(proj, sizes, i_bias, f_bias, cap, norm_w, state, norm_state, max_state, cu_q, positions, slots, eps, out_dtype):
+def mlstm_norm(proj, sizes, i_bias, f_bias, cap, norm_w, state, norm_state, max_state, cu_q, positions, slots, eps, out_dtype,
+               longest=0):
     """``mlstm_scan`` and ``gated_head_norm`` (sigmoid) in one call: ``proj`` [T, ..] = [q | k | v | gate | input gate | forget
     gate] -> [T, H*E].  None where the two calls are to be made.  (8 next tokens: a layer's call 35 us as two, 22 as one.)"""
     H, D, E = sizes
@@ -692,7 +693,7 @@ def mlstm_norm(proj, sizes, i_bias, f_bias, cap, norm_w, state, norm_state, max_
     assert norm_w.numel() in (E, HE)
     base, row, es, n = proj.data_ptr(), _rows(proj), 2 if dt == 0 else 4, 0
     if cu_q is not None:
-        n = _mlstm_bytes(base, base + HD * es, base + 2 * HD * es, row, row, row, T, B, H, D, E, dt)
+        n = _mlstm_bytes(base, base + HD * es, base + 2 * HD * es, row, row, row, T, B, int(longest or 0), H, D, E, dt)
     out = -(-T * HE * 4 // 256) * 256
     ws = torch.empty((out + n,), dtype=torch.uint8, device=proj.device)
     y = torch.empty((T, HE), dtype=out_dtype, device=proj.device)

@@ -102,3 +102,29 @@ def test_next_tokens_of_the_delta_rule(B, H, D, E, one):
     (256, 16, 512, False, True), (1, 128, 512, False, True)])
 def test_few_rows_in_latents(T, H, R, prompts, few):
     assert hk.latent_rows_pay(T, H, R, prompts) is few
+
+
+@pytest.mark.parametrize("B,H,D,E,each", [
+    # walks of 32 columns: 32, 256, 512, 1024, 4096; (bfloat16, float) tokens a portion
+    (1, 8, 128, 128, (32, 24)), (8, 8, 128, 128, (24, 16)), (8, 16, 128, 128, (16, 10)), (32, 8, 128, 128, (10, 10)),
+    (128, 8, 128, 128, (8, 8)), (32, 16, 72, 264, (8, 8)),
+    # up to 64 channels: 16, 256, 257, 1024, 1026, 4096
+    (1, 8, 64, 64, (40, 40)), (16, 8, 64, 64, (40, 32)), (257, 1, 8, 8, (24, 32)), (64, 8, 64, 64, (24, 32)),
+    (171, 3, 48, 40, (16, 32)), (256, 8, 64, 64, (16, 32))])
+def test_matrix_lstm_portions_in_chunks(B, H, D, E, each):
+    """As many tokens as make up for the portions, or one long portion among them; many small bfloat16 heads in one kernel."""
+    walks = B * H * -(-E // 32)
+    for dt in (0, 2):
+        at = lambda T, longest, q=AT, row=8192, D=D: hk._mlstm_bytes(q, AT, AT, row, row, row, T, B, longest, H, D, E, dt)
+        n = each[dt // 2]
+        alone = 40 + walks // (64 if dt == 2 and D <= 64 else 200)
+        assert at(n * B, n) and not at(n * B - 1, n - 1)
+        if alone + B - 1 < n * B:
+            assert at(alone + B - 1, alone) and not at(alone + B - 2, alone - 1)
+        # an unknown length: as if it was all the rows beyond the first of each
+        if B + 1024 < n * B:
+            assert at(B + 1024, 0) and not at(B + 1023, 0)
+        whole = dt == 0 and D <= 64 and walks > 256
+        for T in (n * B, n * B + 640):
+            assert at(T, n) == at(T, -1) == (256 if whole else (T // 64 + B) * H * 1024) <= hk.mlstm_scan_workspace(T, B, H, D, E)
+        assert at(B, -1) and not at(n * B, n, AT + 2) and not at(n * B, n, AT, 8190) and not at(n * B, n, D=136)
