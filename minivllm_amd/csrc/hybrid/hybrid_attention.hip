@@ -637,9 +637,7 @@ static int launch_split(const void* q, long q_row, long q_head, const void* k_ca
         else if (hyb_sink_attention_split_heads(R) == 3) SPLIT_LAUNCH_X(3, false, EXT);           \
         else SPLIT_LAUNCH_X(4, false, EXT);                                                       \
     } while (0)
-    // (the 16-bit rows of 64 / 128 without any of these are next_attention_kernel's)
-    if (rule.temps || rule.softcap > 0.f || rule.pool > 0 || (sizeof(T) == 2 && EPL < 16)) SPLIT_LAUNCH(true);
-    else if constexpr (sizeof(T) == 4 || EPL == 16) SPLIT_LAUNCH(false);
+    if (rule.temps || rule.softcap > 0.f || rule.pool > 0) SPLIT_LAUNCH(true); else SPLIT_LAUNCH(false);
 #undef SPLIT_LAUNCH
 #undef SPLIT_LAUNCH_X
     if (hipGetLastError() != hipSuccess) return 2;

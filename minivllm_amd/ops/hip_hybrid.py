@@ -363,13 +363,28 @@ def next_splits(batch: int, kv_heads: int, heads: int, seen) -> int:
     return min(16, max(1, 256 // groups, min(2048 // groups, -(-seen // 2048))), max(1, -(-seen // 512)))
 
 
+def next_pays(groups: int, R: int, width: int, seen) -> bool:
+    """Whether bfloat16 next tokens are the matrix cores': ``groups`` of a sequence and a KV head with ``R`` query heads, keys and
+    values of ``width`` together, ``seen`` keys (an upper bound, None if there is none).  A workgroup of theirs takes four waves
+    and tiles of 32 keys for any context; many short contexts of one or two heads leave most of both idle, where the kernel on
+    the vector units has 16 lanes a key.  us, matrix cores / vector units, 128 + 128 wide: one head, 2048 groups of 64 keys 27 / 25, of
+    128 33 / 31, 4096 of 16 49 / 24, of 128 60 / 58, of 256 100 / 110, 8192 of 16 93 / 32, of 192 158 / 138; two heads, 1024 of 128 19 / 24,
+    2048 of 64 27 / 25, 4096 of 64 50 / 39, of 512 189 / 177; four heads, 2048 of 16 30 / 28, of 64 30 / 35; 64 + 64, one head: 4096 of 64
+    25 / 25, 6144 of 16 33 / 25, of 96 38 / 40, 8192 of 64 44 / 40, of 128 56 / 61.  Beyond 192 keys either by
+    up to a tenth: one head, 2048 of 512 99 / 92, 2560 of 512 120 / 127; two, 2048 of 512 99 / 104."""
+    if not seen or R > 4:
+        return True
+    if width <= 128:
+        return R > 2 or groups < 6144 or seen > 64
+    return groups < 2048 or (seen > 16 if R > 2 else seen > 192 and (groups < 2560) == (R == 2))
+
+
 def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale, sink, gate, out,
                           max_context_len=None, window=0, keep_first=0, slopes=None, temps=None,
                           softcap=0.0, pool=0, k_pool=None, v_pool=None, chunk=0, clear=False):
     """Single next tokens: row b is sequence b with ``context_lens[b]`` keys.  bfloat16 rows of 64 / 128 go to the
-    matrix cores (``hybrid_next.hip``) unless pooled rows, temperatures or a soft cap belong to the call; those, floats and
-    keys of 256 to the split-context kernel on the vector units (64 sequences of 1024 keys 52 us there, 46 here); both
-    fold the splits by a second small kernel.  Other sizes go through the row kernel.  ``clear``: ``out`` is new, rows without a
+    matrix cores (``hybrid_next.hip``) where that is faster (``next_pays``), unless pooled rows, temperatures or a soft cap
+    belong to the call; those, floats and keys of 256 to the split-context kernel on the vector units; both fold the splits by a second small kernel.  Other sizes go through the row kernel.  ``clear``: ``out`` is new, rows without a
     context become zeros (otherwise they stay as they are)."""
     B, H, D = q.shape
     G, E = k_cache.shape[2], v_cache.shape[3]
@@ -383,7 +398,8 @@ def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale
             seen = min(int(seen), int(window) + int(keep_first) + (int(seen) // pool if pool else 0))
         if chunk and seen:
             seen = min(int(seen), int(chunk))
-        if q.dtype == torch.bfloat16 and _nxa_ok(D, E) and temps is None and not softcap and not pool:
+        if q.dtype == torch.bfloat16 and _nxa_ok(D, E) and temps is None and not softcap and not pool \
+                and next_pays(B * G, H // G, D + E, seen):
             splits = next_splits(B, G, H, seen)
             ws = torch.empty((B * H * splits * (E + 2),), dtype=torch.float32, device=q.device) if splits > 1 else None
             if gate is not None:

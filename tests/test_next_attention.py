@@ -15,6 +15,15 @@ def test_splits(batch, kv_heads, heads, seen, splits):
     assert hk.next_splits(batch, kv_heads, heads, seen) == splits
 
 
+@pytest.mark.parametrize("groups,R,width,seen,matrix", [
+    (512, 2, 256, 1024, True), (2047, 1, 256, 16, True), (2048, 1, 256, 192, False), (2048, 1, 256, 193, False), (2048, 2, 192, 192, False),
+    (2559, 2, 256, 193, True), (2560, 2, 256, 193, False), (2560, 1, 256, 193, True), (2048, 3, 256, 16, False), (2048, 4, 256, 17, True),
+    (8192, 5, 256, 1, True), (6143, 1, 128, 16, True), (6144, 2, 128, 64, False), (6144, 2, 128, 65, True), (8192, 3, 128, 16, True),
+    (8192, 1, 256, None, True), (8192, 1, 256, 0, True)])
+def test_units(groups, R, width, seen, matrix):
+    assert hk.next_pays(groups, R, width, seen) is matrix
+
+
 def _exact(q, k, v, scale, lo, keep, slopes, sink, gate):
     r = q.shape[0] // k.shape[1]
     kt, vt = (x.double().transpose(0, 1).repeat_interleave(r, 0) for x in (k, v))
@@ -37,7 +46,9 @@ def _exact(q, k, v, scale, lo, keep, slopes, sink, gate):
 @pytest.mark.parametrize("G,R", [(2, 1), (1, 5), (2, 16), (1, 20), (48, 2)])    # (48: workgroups of four waves)
 @pytest.mark.parametrize("rule", [{}, {"window": 40, "keep_first": 5}, {"window": 300}, {"chunk": 256}, {"slopes": True}])
 @pytest.mark.parametrize("bs", [32, 12])
-def test_against_exact(D, E, G, R, rule, bs):
+@pytest.mark.parametrize("matrix", [True, False])
+def test_against_exact(D, E, G, R, rule, bs, matrix, monkeypatch):
+    monkeypatch.setattr(hk, "next_pays", lambda *a: matrix)               # (the steps are too few for the vector units)
     lens = [1, 31, 0, 32, 33, 256, 257, 513, 0, 1025, 2100]
     dev, H, B = "cuda", G * R, len(lens)
     g = torch.Generator().manual_seed(D + E + G + R)
