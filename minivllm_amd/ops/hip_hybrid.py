@@ -365,18 +365,23 @@ def next_splits(batch: int, kv_heads: int, heads: int, seen) -> int:
 
 def next_pays(groups: int, R: int, width: int, seen) -> bool:
     """Whether bfloat16 next tokens are the matrix cores': ``groups`` of a sequence and a KV head with ``R`` query heads, keys and
-    values of ``width`` together, ``seen`` keys (an upper bound, None if there is none).  A workgroup of theirs takes four waves
-    and tiles of 32 keys for any context; many short contexts of one or two heads leave most of both idle, where the kernel on
-    the vector units has 16 lanes a key.  us, matrix cores / vector units, 128 + 128 wide: one head, 2048 groups of 64 keys 27 / 25, of
-    128 33 / 31, 4096 of 16 49 / 24, of 128 60 / 58, of 256 100 / 110, 8192 of 16 93 / 32, of 192 158 / 138; two heads, 1024 of 128 19 / 24,
-    2048 of 64 27 / 25, 4096 of 64 50 / 39, of 512 189 / 177; four heads, 2048 of 16 30 / 28, of 64 30 / 35; 64 + 64, one head: 4096 of 64
-    25 / 25, 6144 of 16 33 / 25, of 96 38 / 40, 8192 of 64 44 / 40, of 128 56 / 61.  Beyond 192 keys either by
-    up to a tenth: one head, 2048 of 512 99 / 92, 2560 of 512 120 / 127; two, 2048 of 512 99 / 104."""
+    values of ``width`` together, ``seen`` keys (an upper bound, None if there is none).  A workgroup of theirs takes four waves,
+    which walk tiles of 32 keys: 128 keys at a time, and for one or two heads much of the tiles is idle, where the kernel on the
+    vector units takes keys one by one.  That shows once the card is full of workgroups, until a context is long.  us, matrix
+    cores / vector units:
+      one head, 128 + 128 wide: 768 groups of 130 keys 23 / 25, 1024 of 128 19 / 25, of 130 26 / 24, of 260 37 / 33, of 512 56 / 53, of 1030 100 /
+      103, 1536 of 200 40 / 34, of 1500 197 / 189, 2560 of 64 32 / 24, of 512 120 / 127, 4096 of 16 49 / 24, of 250 100 / 90, of 256 99 / 93;
+      64 + 128: 1024 of 260 32 / 30, of 700 57 / 62, 1536 of 200 34 / 30, of 1030 115 / 104, 8192 of 16 87 / 32
+      two heads, 128 + 128: 512 of 260 21 / 24, 1024 of 260 37 / 34, of 512 58 / 56, 2048 of 128 33 / 36, of 512 99 / 104, 4096 of 64 50 / 39, of
+      512 189 / 177; four: 1536 of 200 42 / 53, 2048 of 16 30 / 28, of 64 30 / 35
+      64 + 64, one head: 1536 of 260 30 / 31, 4096 of 64 25 / 25, 6144 of 16 33 / 25, of 96 38 / 40, 8192 of 64 44 / 40, of 128 56 / 61"""
     if not seen or R > 4:
         return True
+    if R > 2:
+        return width <= 128 or groups < 2048 or seen > 16
     if width <= 128:
-        return R > 2 or groups < 6144 or seen > 64
-    return groups < 2048 or (seen > 16 if R > 2 else seen > 192 and (groups < 2560) == (R == 2))
+        return groups < 6144 or seen > 64
+    return groups * width < (1 << 18 if seen > 128 else 1 << 19) or seen > 1536
 
 
 def sink_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale, sink, gate, out,

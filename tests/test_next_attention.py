@@ -16,9 +16,9 @@ def test_splits(batch, kv_heads, heads, seen, splits):
 
 
 @pytest.mark.parametrize("groups,R,width,seen,matrix", [
-    (512, 2, 256, 1024, True), (2047, 1, 256, 16, True), (2048, 1, 256, 192, False), (2048, 1, 256, 193, False), (2048, 2, 192, 192, False),
-    (2559, 2, 256, 193, True), (2560, 2, 256, 193, False), (2560, 1, 256, 193, True), (2048, 3, 256, 16, False), (2048, 4, 256, 17, True),
-    (8192, 5, 256, 1, True), (6143, 1, 128, 16, True), (6144, 2, 128, 64, False), (6144, 2, 128, 65, True), (8192, 3, 128, 16, True),
+    (512, 2, 256, 1024, True), (1023, 1, 256, 129, True), (1024, 1, 256, 129, False), (2047, 2, 256, 128, True), (2048, 2, 256, 128, False), (1024, 2, 256, 1536, False), (1024, 2, 256, 1537, True),
+    (1365, 1, 192, 200, True), (1366, 2, 192, 200, False), (2047, 3, 256, 16, True), (2048, 3, 256, 16, False), (2048, 4, 256, 17, True),
+    (2048, 4, 128, 1, True), (8192, 5, 256, 1, True), (6143, 1, 128, 16, True), (6144, 2, 128, 64, False), (6144, 2, 128, 65, True),
     (8192, 1, 256, None, True), (8192, 1, 256, 0, True)])
 def test_units(groups, R, width, seen, matrix):
     assert hk.next_pays(groups, R, width, seen) is matrix
