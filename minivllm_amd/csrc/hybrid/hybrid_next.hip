@@ -10,11 +10,12 @@
 //
 // Reading the keys and values bounds it.  A workgroup that has a context to itself writes the result; the splits of a
 // context are folded by a second kernel (how many: next_splits).  A page is looked up two tiles ahead of its use: one
-// ahead, the rows behind it are asked for late (64 x 1024 keys 48.1 us, two ahead 46.0).
-// A call, in us, against the kernel on the vector units (scores by exchanges between 16 lanes) and its fold; 16 / 8 heads of 128:
-// 64 x 1024 keys 46 (4.6 TB/s; the kernel alone 43) and 52, 128 x 1024 80 and 89, 32 x 1024 24 and 31, 16 x 2048 28 and 33,
-// 64 of 200 and one of 8192 90 and 152, 1 x 512 19 and 25, 64 x 1024 under a window of 128 20 and 25, 1 x 2048 25 and 25 (both
-// the launches).  Error 1.7e-3 of the result, its rounding, in both.
+// ahead, the rows behind it are asked for late (64 x 1024 keys two us more).
+// 64 sequences of about 1024 keys, 16 / 8 heads of 128: 44.4 us a call among many (4.7 TB/s; the kernel alone 43).  A call among
+// eight, in us, against the kernel on the vector units (scores by exchanges between 16 lanes) and its fold: 64 x 1024 keys
+// 47 and 52, 128 x 1024 84 and 91, 32 x 1024 27 and 33, 16 x 2048 30 and 35, 64 of 200 and one of 8192 94 and 157, 1 x 512 19 and
+// 25, 64 x 1024 under a window of 128 20 and 25, 1 x 2048 24 and 25 (both the launches).  Where the vector units are ahead:
+// next_pays in ops/hip_hybrid.py.  Error 1.7e-3 of the result, its rounding, in both.
 #include "hybrid_chunks.h"
 #include "hybrid_row_by_keys.h"
 

@@ -19,8 +19,9 @@
 // per-token scalars.  GLA, WKV and
 // MLSTM read the raw projections (bfloat16 or float rows of a wider projection output) and do
 // the gates' fp32 arithmetic while staging; CDELTA reads the fp32 outputs of delta_prepare.
-// MLSTM's prompt portions run on the matrix cores instead (hybrid_chunks.hip).
-// Its running maximum is a sequential max-plus chain over tokens: wave 0 walks it once per chunk
+// Prompt portions that are long enough run on the matrix cores instead: MLSTM's in hybrid_chunks.hip, GLA's and WKV's of up to
+// 64 channels in hybrid_channel_chunks.hip.
+// MLSTM's running maximum is a sequential max-plus chain over tokens: wave 0 walks it once per chunk
 // (two dependent operations per token) and leaves the three factors of every token in LDS;
 // the normaliser n is kept by every lane group (its d-slice), since every column divides by n . q.
 // WKV's output is S^T q + (q . (u * k)) v: the factor of v is the same number for all columns and is
