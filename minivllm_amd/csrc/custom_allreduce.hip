@@ -488,7 +488,7 @@ extern "C" int mvl_car_alloc(void** out, size_t bytes, int uncached) {
     if (e != hipSuccess) return (int)e;
     return (int)hipMemset(*out, 0, bytes);
 }
-// (there is no function that frees: uncached memory that a kernel has read must stay allocated, see custom_allreduce.py)
+// (no function frees or unmaps: uncached memory that a kernel has read must stay where it is, see custom_allreduce.py)
 extern "C" int mvl_car_clear(void* p, size_t bytes) { return (int)hipMemset(p, 0, bytes); }
 extern "C" int mvl_car_ipc_get(void* p, void* handle_out) {
     return (int)hipIpcGetMemHandle((hipIpcMemHandle_t*)handle_out, p);
@@ -498,7 +498,6 @@ extern "C" int mvl_car_ipc_open(const void* handle, void** out) {
     memcpy(&h, handle, sizeof(h));
     return (int)hipIpcOpenMemHandle(out, h, hipIpcMemLazyEnablePeerAccess);
 }
-extern "C" int mvl_car_ipc_close(void* p) { return (int)hipIpcCloseMemHandle(p); }
 
 static long g_loopback = 0;
 

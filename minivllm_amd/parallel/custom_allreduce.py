@@ -52,9 +52,14 @@ DEFAULT_TIMEOUT_MS = int(os.environ.get("MINIVLLM_CAR_TIMEOUT_MS", 2000))
 # Uncached memory that a kernel has read stays allocated until the process ends: tensors that came to lie where such memory
 # had been freed have held wrong values (an engine built behind one that had used these kernels gave logits that were
 # NaN).  Buffers of a closed all-reduce wait here, device -> [(bytes, address)], for the next one of the process, so there
-# are never more than were in use at one time.
+# are never more than were in use at one time.  For the same reason what this process has mapped of a peer's stays mapped
+# (unmapping gives its addresses, and with the peer's end its pages, to other tensors): _MAPPED, (the peer's process, its buffer's
+# address, this device) -> address here, found again when the peer offers the same buffer.  That is 24 MB for a peer that was a process of
+# its own, with the default sizes.
 _IDLE: Dict[int, List[Tuple[int, int]]] = {}
+_MAPPED: Dict[tuple, int] = {}
 _IDLE_LOCK = threading.Lock()
+_PROCESS = os.urandom(16)               # (process numbers come again)
 
 
 def _take_buffer(lib, device: int, nbytes: int) -> Tuple[int, int]:
@@ -81,6 +86,17 @@ def _give_back(device: int, buffers) -> None:
         _IDLE.setdefault(device, []).extend(buffers)
 
 
+def _map_peer(lib, device: int, owner: tuple, handle: bytes) -> int:
+    """Address, on the current device, ``device``, of the peer's buffer ``owner`` (its process and address there)."""
+    key = owner + (device,)
+    with _IDLE_LOCK:
+        if key not in _MAPPED:
+            q = ctypes.c_void_p()
+            CustomAllReduce._ck(lib.mvl_car_ipc_open(handle, ctypes.byref(q)), "ipc_open")
+            _MAPPED[key] = q.value
+        return _MAPPED[key]
+
+
 class PeerAllReduceError(RuntimeError):
     """A peer-to-peer all-reduce kernel gave up waiting for a peer: activations of that step
     (and everything computed from them) are invalid."""
@@ -104,7 +120,6 @@ class CustomAllReduce:
         lib.mvl_car_clear.argtypes = [vp, sz]
         lib.mvl_car_ipc_get.argtypes = [vp, ctypes.c_char_p]
         lib.mvl_car_ipc_open.argtypes = [ctypes.c_char_p, ctypes.POINTER(vp)]
-        lib.mvl_car_ipc_close.argtypes = [vp]
         lib.mvl_car_status.argtypes = [vp]
         lib.mvl_car_all_reduce.argtypes = [ctypes.POINTER(vp)] * 3 + [
             ctypes.c_int, ctypes.c_int, vp, ctypes.c_long, ctypes.c_int, ctypes.c_int, ctypes.c_long, vp]
@@ -126,7 +141,6 @@ class CustomAllReduce:
         sizes = [lib.mvl_car_flags_bytes(), 2 * max_bytes, max_bytes]
         self._own: List[int] = []
         self._buffers: List[Tuple[int, int]] = []           # the same, with their sizes
-        self._mapped: List[int] = []
         handles, err = [], None
         try:
             for nbytes in sizes:
@@ -135,7 +149,7 @@ class CustomAllReduce:
                 self._own.append(buffer[1])
                 buf = ctypes.create_string_buffer(self._hbytes)
                 self._ck(lib.mvl_car_ipc_get(vp(buffer[1]), buf), "ipc_get")
-                handles.append(buf.raw)
+                handles.append(((os.getpid(), _PROCESS, buffer[1]), buf.raw))
         except Exception as e:
             err = repr(e)
         # every rank takes part in both exchanges whatever happened locally, and all ranks give
@@ -150,10 +164,7 @@ class CustomAllReduce:
                     if r == rank or loopback:
                         arr[r] = self._own[k]
                     else:
-                        q = vp()
-                        self._ck(lib.mvl_car_ipc_open(everyone[r][1][k], ctypes.byref(q)), "ipc_open")
-                        self._mapped.append(q.value)
-                        arr[r] = q.value
+                        arr[r] = _map_peer(lib, self._device_index(), *everyone[r][1][k])
                 tables.append(arr)
             torch.cuda.synchronize()
         except Exception as e:
@@ -180,11 +191,9 @@ class CustomAllReduce:
     def _release(self, idle: bool = False) -> None:
         """``idle``: no kernel of any rank uses this rank's buffers any more, so another all-reduce may; otherwise (peers
         that are dead, or did not arrive) a peer may still write to them, and they stay allocated and unused."""
-        for p in self._mapped:
-            self._lib.mvl_car_ipc_close(p)
         if idle and self._buffers:
             _give_back(self._device_index(), self._buffers)
-        self._mapped, self._own, self._buffers = [], [], []
+        self._own, self._buffers = [], []
 
     @staticmethod
     def _ck(rc: int, what: str) -> None:
