@@ -51,3 +51,22 @@ def test_small_results(fast):
     z = -torch.linspace(87.0, 88.72, 64 * H * E).view(64, -1)
     y, want = filtered(z.cuda(), 4, fast).double(), z.double() * torch.sigmoid(z.double())
     assert ((y - want).abs() <= 3 * 2.0 ** -24 * want.abs()).all()
+
+
+# where log2(e)'s lower part, rounded instead of cut to 24 bits, puts the exponential one place off expf
+PLACES = [-87.6323853, -79.0445404, -76.9907761, -74.7452698, -73.0642929, -61.6797829, -60.720314, -57.0911827, -54.5741081, -46.1522217,
+          -40.9672012, -30.360157, -29.5498428, -19.8694191, -15.3136673, -7.82923794]
+
+
+@pytest.mark.parametrize("taps,fast", [(4, True), (4, False), (3, True), (5, False)])
+def test_bits(taps, fast):
+    """Bit by bit z / (1 + expf(-z)), as torch has it in fp32: one of every 8191 arguments from the lowest to the highest, all from -89 to
+    -87, and those above.  (All 2^32 were compared once, in a program that calls both functions.)"""
+    bits = torch.arange(0, 1 << 32, 8191, dtype=torch.int64)
+    z = torch.cat([(bits - (bits >> 31 << 32)).to(torch.int32).view(torch.float32), torch.tensor(PLACES),
+                   -(87.0 + torch.arange(1 << 18) * 2.0 ** -17)])
+    z = z[z.isfinite()]
+    z = torch.cat([z, z.new_zeros(-z.numel() % (H * E))]).view(-1, H * E).cuda()
+    y, want = filtered(z, taps, fast), (z / (1 + torch.exp(-z))).cpu()
+    differ = (y.view(torch.int32) != want.view(torch.int32)) & ~((y == 0) & (z.cpu() == 0))    # (the filter's sum makes 0 of -0)
+    assert not differ.any(), z.cpu()[differ]
