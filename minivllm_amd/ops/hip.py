@@ -169,10 +169,10 @@ def _kv_fp8(cache: Optional[torch.Tensor]) -> int:
 
 def _cache_strides(cache: torch.Tensor):
     """cache is logically [block, token, kv_head, d] with arbitrary physical order (dimensions behind these: of one element)."""
-    sb, st, sh, sd, *_ = cache.stride()
-    if sd != 1:
+    s = cache.stride()
+    if s[3] != 1:
         raise ValueError("KV cache head_dim must be contiguous")
-    return sb, st, sh
+    return s[:3]
 
 
 def _rows_like(q: torch.Tensor, qs_b: int, qs_h: int) -> torch.Tensor:
